@@ -14,17 +14,18 @@
 //     row vector work per key row its pairs name, with the dk weight of each pair stored by
 //     bwd_dq_pairs (no V, no matrix cores), the tile's other gradient rows stored as zeros.
 // Gradient rows are streaming (non-temporal) stores: nothing reads them back soon.
-// The tile passes take the rest (lists past the cap, or no lists at all), driven by the bitmask:
-//   * bwd_dq_fast: per (branch, query tile), several to a wave when lists exist (their counts
-//     tested in one round); walks the set bits of the bitmask row, so only key tiles with a
-//     non-zero score are touched; dq_br is finished (F.normalize backward) at the end.
-//   * bwd_dkv_fast: per key tile, from the queue bwd_dkv_pairs fills when lists exist; walks
-//     the set bits of the bitmask column of each branch; dv accumulates over both branches
-//     (A1 - lam A2), dk_br is finished per branch.
-// The tile passes fetch each visited tile with direct global->LDS loads into a wave-private,
-// chunk-swizzled row-major tile that serves both as row fragments (ds_read_b128) and, through
-// the LDS transpose read, as transposed fragments.  dbeta / dlambda partials: one pair per
-// (branch, query tile), summed in a fixed order by bwd_finish.
+// The block tile passes take the rest (lists past the cap, or no lists at all), driven by the
+// bitmask: four consecutive tiles of one head per workgroup, one wave each, sharing every streamed
+// tile's rows through LDS:
+//   * bwd_dq_blk: four query tiles of one (branch, head); walks the set bits of their bitmask
+//     rows, so only key tiles with a non-zero score are touched; dq_br is finished (F.normalize
+//     backward) at the end.
+//   * bwd_dkv_blk: four key tiles of one head; walks the set bits of the bitmask columns of each
+//     branch; dv accumulates over both branches (A1 - lam A2), dk_br is finished per branch.
+//   * bwd_tiles: both in one launch over the blocks that the key-major pair pass queued (with
+//     normalisation, where usually every list fits and the queue is empty).
+// dbeta / dlambda partials: one pair per (branch, query tile), summed in a fixed order by
+// bwd_finish.
 #include "tda_common.hpp"
 #include "tda_params.hpp"
 #include "tda_pos.hpp"
@@ -32,47 +33,9 @@
 namespace tda {
 
 
-// Direct global->LDS load of rows r0..r0+31 of a (N, D) row set (row stride st elements;
-// rows >= n clamped to n-1, their values only meet zero weights) into a swizzled tile.
-// One instruction moves 1 KiB: 64 lanes x 16 bytes.
-template <int D>
-__device__ __forceinline__ void dma_tile(const bf16* rows, int64_t st, int r0, int n, bf16* tile) {
-  constexpr int CH = D / 8, RPI = 64 / CH;
-  const int l = lane_id();
-#pragma unroll
-  for (int u = 0; u < 32 / RPI; ++u) {
-    const int r = u * RPI + l / CH;
-    const int c = (l % CH) ^ bswz<D>(r);
-    const bf16* src = rows + (int64_t)min(r0 + r, n - 1) * st + 8 * c;
-    __builtin_amdgcn_global_load_lds((const void*)src, LDS_PTR(void, tile + u * RPI * D), 16, 0, 0);
-  }
-}
-// 32 floats (one per tile row) by direct load; rows >= n clamped.
-__device__ __forceinline__ void dma_row_vals(const float* vals, int r0, int n, float* dst) {
-  const int l = lane_id();
-  if (l < 32) __builtin_amdgcn_global_load_lds((const void*)(vals + min(r0 + l, n - 1)), LDS_PTR(void, dst), 4, 0, 0);
-}
-__device__ __forceinline__ void wait_all_loads() { __builtin_amdgcn_s_waitcnt(0); }
-
-// The same loads through a buffer descriptor per tile: the tile sets the descriptor's base and
-// size, the lanes add 32-bit offsets within the tile; rows past n read as zeros (the
-// descriptor's range check).
+// Descriptor of one tile's rows: loads past `bytes` read as zeros (its range check).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
-template <int D>
-__device__ __forceinline__ void dma_tile_b(const bf16* rows, int64_t st, int r0, int n, bf16* tile) {
-  constexpr int CH = D / 8, RPI = 64 / CH;
-  const int l = lane_id();
-  const int nr = min(32, n - r0);
-  const __amdgpu_buffer_rsrc_t rs = rows_rsrc(rows + (int64_t)r0 * st, (uint32_t)(((int64_t)(nr - 1) * st + D) * 2));
-  const uint32_t st2 = (uint32_t)(2 * st);  // row stride in bytes (at most 2^26)
-#pragma unroll
-  for (int u = 0; u < 32 / RPI; ++u) {
-    const int r = u * RPI + l / CH;
-    const uint32_t off = (uint32_t)r * st2 + 16u * (uint32_t)((l % CH) ^ bswz<D>(r));
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS_PTR(void, tile + u * RPI * D), 16, off, 0, 0, 0);
-  }
 }
 // Lane-distributed pair list: lane e < n holds entry e (key, query row in the tile, x).
 struct PairLanes {
@@ -88,11 +51,6 @@ __device__ __forceinline__ PairLanes load_pairs(const uint32_t* ent, uint32_t n)
   // to element 0 (the key index)
   const f32x4 ef = __builtin_bit_cast(f32x4, e);
   return PairLanes{(int)e[0], (int)e[1], ef[2], e[3]};
-}
-
-__device__ __forceinline__ void dma_row_vals_b(const float* vals, int r0, int n, float* dst) {
-  const __amdgpu_buffer_rsrc_t rs = rows_rsrc(vals + r0, (uint32_t)(min(32, n - r0) * 4));
-  if (lane_id() < 32) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, LDS_PTR(void, dst), 4, 4 * lane_id(), 0, 0, 0);
 }
 
 // Row fragment t of a swizzled tile: lane (m, g) gets elements 16t + 8g .. +7 of row m.
@@ -164,185 +122,6 @@ __device__ __forceinline__ void store_grad_rows(const f32x16 (&acc)[D / 32], con
       }
       store4(grow + 32 * c + 8 * u + 4 * g, o[0], o[1], o[2], o[3]);
     }
-}
-
-template <int D>
-struct BwdWaveLds {
-  bf16 a[32 * D];  // K (dq pass) or Q (dkv pass) tile
-  bf16 b[32 * D];  // V (dq pass) or dO (dkv pass) tile
-  float rows[32];  // key inverse norms (dq) or query inverse norms (dkv)
-  float taus[32];  // tau coefficients of the query rows (dkv)
-};
-
-// Waves per workgroup of both passes.  The work per item varies with its number of non-zero
-// tiles; single-wave workgroups retire independently.
-constexpr int kBwdWaves = 1;
-
-// ------------------------------------------------------------------ query-major pass, tiles
-// One wave per (branch, query tile) whose pair list did not fit (or with no lists at all): it
-// walks the set bits of the branch's bitmask row.  A branch's resident operands (its query
-// fragments, dO, one dq accumulator) are half of both branches', which lets two waves share a
-// SIMD.
-// (branch, head, query tile) of query-major tile-pass item `item`: longest first (query tiles
-// from the last); the two branches of a (head, query tile) adjacent.
-template <int BR>
-__device__ __forceinline__ void dq_item(int64_t item, int BH, int nqt, int& br, int& qt, int& bh) {
-  br = BR == 2 ? (int)(item & 1) : 0;
-  const int64_t rest = BR == 2 ? item >> 1 : item;
-  qt = nqt - 1 - (int)(rest / BH);
-  bh = (int)(rest % BH);
-}
-
-// The tile pass over one (branch, query tile) item: one wave, W its LDS.
-template <int D, int BR, int PK, bool NORM>
-__device__ __forceinline__ void bwd_dq_tile(const BwdParams& P, BwdWaveLds<D>& W, int64_t item) {
-  constexpr int NT = D / 16, ND = D / 32;
-  const int l = lane_id(), n32 = l & 31, g = l >> 5;
-  const int BH = P.B * P.H;
-  int br, qt, bh;
-  dq_item<BR>(item, BH, P.nqt, br, qt, bh);
-  const int b = bh / P.H, h = bh % P.H;
-  const int Nq = P.Nq, Nk = P.Nk, qoff = P.qoff;
-  const int i = qt * 32 + n32;
-  const bool qvalid = i < Nq;
-  const int ic = min(i, Nq - 1);
-  const int pq = qoff + i;                   // the lane's query position
-  const int ktl = kt_last(qt, qoff, P.nkt);  // last key tile the query tile sees
-  auto base = [&](int slot) {
-    return (const bf16*)P.in[slot] + (int64_t)b * P.s[slot][0] + (int64_t)h * P.s[slot][1];
-  };
-  const int qslot = br == 0 ? B_Q1 : B_Q2, kslot = br == 0 ? B_K1 : B_K2;
-
-  // row operands, all issued before the first wait: dO and query fragments, the inverse query
-  // norm, bitmask words 0..63 of the branch's row (lane w holds word w)
-  const int nw = (ktl >> 5) + 1;  // bitmask words covering key tiles 0..ktl
-  // the forward's pair list of (branch, head, query tile), when it fit (else the tile path)
-  const int64_t lidx = ((int64_t)br * BH + bh) * P.nqt + qt;
-  const uint32_t npairs = P.pairs ? P.pairs[pair_lists(BR, BH, P.nqt) * 4 * kPairCap + lidx] : kPairOverflow;
-  if (npairs <= (uint32_t)kPairCap) return;  // bwd_dq_pairs handles the lists that fit
-  bf16x8 DO[NT], Q[NT];
-  {
-    const bf16* r = base(B_DO) + (int64_t)ic * P.s[B_DO][2];
-    const bf16* rq_ = base(qslot) + (int64_t)ic * P.s[qslot][2];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      DO[t] = *reinterpret_cast<const bf16x8*>(r + 16 * t + 8 * g);
-      Q[t] = *reinterpret_cast<const bf16x8*>(rq_ + 16 * t + 8 * g);
-    }
-  }
-  const float rq = NORM ? P.norms[norm_base(P, br == 0 ? N_Q1 : N_Q2, bh) + ic] : 1.f;
-  const uint32_t* occrow = P.occ ? P.occ + (((int64_t)br * BH + bh) * P.nqt + qt) * P.occ_w : nullptr;
-  const uint32_t lw0 = l < nw ? (occrow ? occrow[l] : 0xffffffffu) : 0u;
-  const float ci = tau_coeff(pq, P.inv_d);
-  const float tau = (*P.beta) * ci;
-  const float pw = P.p;
-  float coef = 1.f;
-  if constexpr (BR == 2) coef = br == 0 ? 1.f : -clamp01(*P.lam);
-  const bool want_l = BR == 2 && br == 1;  // dlambda comes from branch 2 alone
-  const bf16* vb = base(B_V);
-  const int64_t sv = P.s[B_V][2];
-  const bf16* kb = base(kslot);
-  const int64_t sk = P.s[kslot][2];
-  const float* nk = nullptr;
-  if constexpr (NORM) nk = P.norms + norm_base(P, br == 0 ? N_K1 : N_K2, bh);
-  float bsum = 0.f, lsum = 0.f;
-  unsigned visited = 0, computed = 0;
-
-  f32x16 A[ND];
-#pragma unroll
-  for (int c = 0; c < ND; ++c) A[c] = f32x16{};
-
-  for (int w0 = 0; w0 < nw; w0 += 64) {
-    const uint32_t lw = w0 == 0 ? lw0 : (w0 + l < nw) ? (occrow ? occrow[w0 + l] : 0xffffffffu) : 0u;
-    for (int w = w0; w < min(nw, w0 + 64); ++w) {
-      uint32_t bits = __builtin_amdgcn_readlane(lw, w - w0);
-      if (w == (ktl >> 5)) bits &= (ktl & 31) == 31 ? 0xffffffffu : ((2u << (ktl & 31)) - 1u);
-      while (bits) {
-        const int kt = 32 * w + __builtin_ctz(bits);
-        bits &= bits - 1u;
-        ++visited;
-        const int k0 = 32 * kt;
-        dma_tile_b<D>(kb, sk, k0, Nk, W.a);
-        dma_tile_b<D>(vb, sv, k0, Nk, W.b);
-        if constexpr (NORM) dma_row_vals_b(nk, k0, Nk, W.rows);
-        wait_all_loads();
-        f32x16 S = f32x16{}, Dp = f32x16{};
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          S = PolBF16::mma(tile_row_frag<D>(W.a, t), Q[t], S);
-          Dp = PolBF16::mma(tile_row_frag<D>(W.b, t), DO[t], Dp);
-        }
-        float rk[16];
-        if constexpr (NORM) crow_vals(W.rows, rk);
-        f32x16 E;
-        bool any = false;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = k0 + crow(r, g);
-          const bool valid = qvalid && key <= pq && key < Nk;  // rows past Nk read as zeros
-          const float sr = NORM ? S[r] * rk[r] : S[r];
-          const float x = __builtin_fmaf(sr, rq, -tau);
-          const bool pos = valid && x > 0.f;
-          const float ds = pos ? coef * dpow_p<PK>(x, pw) * Dp[r] : 0.f;
-          bsum += ds;
-          lsum = __builtin_fmaf(pos && want_l ? pow_p<PK>(x, pw) : 0.f, Dp[r], lsum);
-          any = any || pos;
-          E[r] = NORM ? ds * rk[r] : ds;
-        }
-        if (!occrow && wave_ballot(any) == 0ull) continue;
-        ++computed;
-        const bf16x8 E0 = PolBF16::pack_c(E, 0), E1 = PolBF16::pack_c(E, 1);
-#pragma unroll
-        for (int c = 0; c < ND; ++c) {
-          A[c] = PolBF16::mma(tile_tr_frag<D>(W.a, 0, c), E0, A[c]);
-          A[c] = PolBF16::mma(tile_tr_frag<D>(W.a, 1, c), E1, A[c]);
-        }
-      }
-    }
-  }
-  if (qvalid) {
-    // the query row for the normalize backward, loaded after the tiles (held during them, it
-    // would push the wave past the register budget of two waves per SIMD)
-    GradRow<D> XR;
-    if constexpr (NORM) load_grad_row<D>(base(qslot) + (int64_t)ic * P.s[qslot][2], XR);
-    const int gslot = br == 0 ? B_DQ1 : B_DQ2;
-    bf16* grow = (bf16*)P.grad[br == 0 ? 0 : 2] + (int64_t)b * P.s[gslot][0] + (int64_t)h * P.s[gslot][1] +
-                 (int64_t)i * P.s[gslot][2];
-    store_grad_rows<D, NORM>(A, XR, grow, rq);
-  }
-
-  const float pb = wave_sum(-ci * bsum);
-  const float pl = wave_sum(-lsum);
-  if (l == 0) {
-    P.ws[2 * lidx + 0] = pb;  // slot of (branch, head, query tile), whichever pass takes it
-    P.ws[2 * lidx + 1] = pl;
-    if (P.stats) {
-      atomicAdd(P.stats + 0, (unsigned long long)visited);
-      atomicAdd(P.stats + 1, (unsigned long long)computed);
-    }
-  }
-}
-
-// One wave per workgroup and `per_wave` consecutive items per wave.  With pair lists, the items
-// whose list fit belong to bwd_dq_pairs: the wave tests its items' counts in one lane-parallel
-// round and runs only the others (per_wave 8: a launch where every list fits costs two waves per
-// SIMD); without lists every item runs (per_wave 1).
-template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_fast(BwdParams P, int per_wave) {
-  __shared__ __attribute__((aligned(16))) BwdWaveLds<D> W;
-  const int l = lane_id();
-  const int BH = P.B * P.H;
-  const int64_t n = (int64_t)BR * BH * P.nqt, first = (int64_t)blockIdx.x * per_wave;
-  bool need = false;
-  if (l < per_wave && first + l < n) {
-    need = true;
-    if (P.pairs) {
-      int br, qt, bh;
-      dq_item<BR>(first + l, BH, P.nqt, br, qt, bh);
-      need = P.pairs[pair_lists(BR, BH, P.nqt) * 4 * kPairCap + ((int64_t)br * BH + bh) * P.nqt + qt] > (uint32_t)kPairCap;
-    }
-  }
-  for (uint64_t m = wave_ballot(need); m; m &= m - 1ull) bwd_dq_tile<D, BR, PK, NORM>(P, W, first + __builtin_ctzll(m));
 }
 
 // ------------------------------------------------------------------ query-major pass, pairs
@@ -475,6 +254,17 @@ __device__ __forceinline__ void zero_rows(T* tile0, int64_t st, int nrows, uint3
   }
 }
 
+// Tiles per workgroup of the block tile passes.
+constexpr int kBwdBlk = 4;
+
+// The tile-pass queue (P.dkvq, bf16 with normalisation), u32 words: [0] key blocks queued, [1]
+// query blocks queued, [2] tickets taken, up to kTileqHead; one mask per key block (head, key
+// tile / kBwdBlk): its key tiles that the pair pass left; the queued key blocks (as many as there
+// are); the queued query blocks (of BR B H ceil(nqt / kBwdBlk)).  Head and masks are zeroed by the
+// query-major pair pass, the rest filled by the key-major one.  It fits where nkt <= 64 nqt:
+// 2 ceil(nkt / 4) + 2 ceil(nqt / 4) <= 64 nqt words per head.
+constexpr int kTileqHead = 64;
+
 // Pairs whose row loads the pair passes keep in flight together: the query-major pass 4 (64
 // VGPRs, eight waves per SIMD: 23.6 us against 24.8 with 8 at B4 H16 N4096 d128), the
 // key-major pass 8.
@@ -523,8 +313,14 @@ __global__ void __launch_bounds__(64) bwd_dq_pairs(BwdParams P) {
   // the count and every entry slot at once (slots past the count are never used)
   const PairLanes PL = load_pairs(P.pairs + lidx * (4 * kPairCap), (uint32_t)kPairCap);
   const uint32_t npairs = P.pairs[pair_lists(BR, BH, P.nqt) * 4 * kPairCap + lidx];
-  if (P.dkvq && item == 0 && l == 0) P.dkvq[0] = 0u;  // the key-major pair pass fills it later
-  if (npairs > (uint32_t)kPairCap) return;  // bwd_dq_fast walks the tiles
+  if (P.dkvq) {  // the key-major pair pass fills the queue later
+    if (item == 0 && l < kTileqHead) P.dkvq[l] = 0u;
+    if constexpr (sizeof(T) == 2) {  // the key blocks' masks
+      const int64_t nkb = (int64_t)BH * ((P.nkt + kBwdBlk - 1) / kBwdBlk);
+      for (int64_t x = item * 64 + l; x < nkb; x += (int64_t)BR * BH * P.nqt * 64) P.dkvq[kTileqHead + x] = 0u;
+    }
+  }
+  if (npairs > (uint32_t)kPairCap) return;  // the block tile pass walks the tiles
 
   auto base = [&](int slot) {
     return (const T*)P.in[slot] + (int64_t)b * P.s[slot][0] + (int64_t)h * P.s[slot][1];
@@ -634,30 +430,6 @@ __global__ void __launch_bounds__(64) bwd_dq_pairs(BwdParams P) {
 }
 
 // ------------------------------------------------------------------ key-major pass, pairs
-// Whether the bitmask column of key tile kt (query tiles qtf.., every branch) has a query tile
-// whose pair list did not fit: the key tile then goes to the tile pass, else to the pair pass.
-// Both key-major passes decide with this test.
-template <int BR>
-__device__ __forceinline__ bool column_overflows(const BwdParams& P, int bh, int kt, int qtf) {
-  const int BH = P.B * P.H, l = lane_id();
-  const uint32_t* counts = P.pairs + pair_lists(BR, BH, P.nqt) * 4 * kPairCap;
-  bool ovf = false;
-  for (int q0c = qtf; q0c < P.nqt; q0c += 64) {
-    const int qt = q0c + l;
-    const bool in = qt < P.nqt;
-    uint32_t w[BR], c[BR];
-#pragma unroll
-    for (int br = 0; br < BR; ++br) {  // every load of the chunk before the first use
-      const int64_t row = ((int64_t)br * BH + bh) * P.nqt + (in ? qt : P.nqt - 1);
-      w[br] = P.occ[row * P.occ_w + (kt >> 5)];
-      c[br] = counts[row];
-    }
-#pragma unroll
-    for (int br = 0; br < BR; ++br) ovf = ovf || (in && ((w[br] >> (kt & 31)) & 1u) && c[br] > (uint32_t)kPairCap);
-  }
-  return wave_ballot(ovf) != 0ull;
-}
-
 // LDS slots of the key-major pair pass: pairs of one column gathered at once.
 constexpr int kColPairs = 64;
 static_assert(kColCap == kColPairs && kColCap == 64, "a column bucket: one entry per lane, as many as the slots");
@@ -673,6 +445,19 @@ struct ColEntry {
   float x;     // exact forward value
   float wk;    // dk weight from the query-major pair pass
 };
+
+// Query block k of the queue, numbered from the last query tiles (the longest rows) of every (head,
+// branch): the list count of its tile `lane` (0 past the block).
+template <int BR>
+__device__ __forceinline__ uint32_t query_block_count(const BwdParams& P, const uint32_t* counts, int64_t k) {
+  const int BH = P.B * P.H, nqt = P.nqt, l = lane_id();
+  const int nqb = (nqt + kBwdBlk - 1) / kBwdBlk;
+  if (k >= (int64_t)BR * BH * nqb) return 0u;
+  const int jb = nqb - 1 - (int)(k / (BR * BH)), rem = (int)(k % (BR * BH));
+  const int br = BR == 2 ? rem & 1 : 0, bh = BR == 2 ? rem >> 1 : rem;
+  const int qt = kBwdBlk * jb + l;
+  return l < kBwdBlk && qt < nqt ? counts[((int64_t)br * BH + bh) * nqt + qt] : 0u;
+}
 
 // One wave per key tile whose column has only lists that fit.  Its pairs come from the column's
 // bucket when the forward filled one with all of them (every entry with its dk weight: one round
@@ -696,7 +481,7 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
 
   const int l = lane_id();
   const int BH = P.B * P.H;
-  const int64_t item = blockIdx.x;  // (key tile, head), in the order of bwd_dkv_fast
+  const int64_t item = blockIdx.x;  // (key tile, head), the first key tiles (most queries) first
   if (item >= (int64_t)BH * P.nkt) return;
   const int kt = (int)(item / BH), bh = (int)(item % BH);
   const int b = bh / P.H, h = bh % P.H;
@@ -712,12 +497,17 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
   const float pw = P.p;
   float lam = 0.f;
   if constexpr (BR == 2) lam = clamp01(*P.lam);
+  // query block `item` (and every B H nkt-th after it) goes to the tile-pass queue when one of its
+  // tiles' lists did not fit; its counts are loaded here and tested once the bucket has arrived
+  const bool queue = sizeof(T) == 2 && NORM && P.dkvq;
+  uint32_t qcount = 0u;
+  if (queue) qcount = query_block_count<BR>(P, counts, item);
 
   // Walk the column's lists in the order (query-tile chunk of 64, branch, query tile): the
   // bitmask bits and counts of 128 query tiles per load round, then 2 kWalkRounds lists per
   // step, all loaded before the first is used (lanes 0-31 and 32-63 take one list each per
   // round); body(entry) once per round.  Returns false, before any body call of that chunk pair, when a
-  // list of the column did not fit (the same test as column_overflows: the tile pass takes the
+  // list of the column did not fit (the same test as bwd_dkv_blk's: the tile pass takes the
   // key tile); the caller has then written nothing.
   auto walk = [&](auto&& body) -> bool {
     for (int q0c = qtf; q0c < P.nqt; q0c += 128) {
@@ -837,6 +627,16 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
     }
   }
 
+  if (queue) {
+    const int64_t nkb = (int64_t)BH * ((P.nkt + kBwdBlk - 1) / kBwdBlk);
+    const int64_t nb = (int64_t)BR * BH * ((P.nqt + kBwdBlk - 1) / kBwdBlk), step = (int64_t)BH * P.nkt;
+    for (int64_t k = item; k < nb; k += step) {
+      if (k != item) qcount = query_block_count<BR>(P, counts, k);
+      if (wave_ballot(qcount > (uint32_t)kPairCap) != 0ull && l == 0)
+        P.dkvq[kTileqHead + 2 * nkb + atomicAdd(P.dkvq + 1, 1u)] = (uint32_t)k;
+    }
+  }
+
   // ---- else the first walk: rows named, pairs into the slots while they fit
   const bool fits = from_bucket || walk([&](const ColEntry& c) {
     const bool match = c.valid && (c.key >> 5) == kt;
@@ -857,8 +657,16 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
     }
     np += (uint32_t)__builtin_popcountll(mm);
   });
-  if (!fits) {  // bwd_dkv_fast takes the key tile
-    if (P.dkvq && l == 0) P.dkvq[1 + atomicAdd(P.dkvq, 1u)] = (uint32_t)item;
+  if (!fits) {  // the tile pass takes the key tile
+    if (P.dkvq && l == 0) {
+      if constexpr (sizeof(T) == 2) {  // its block of key tiles, queued by the first of them
+        const int64_t nkb = (P.nkt + kBwdBlk - 1) / kBwdBlk, blk = (int64_t)bh * nkb + kt / kBwdBlk;
+        uint32_t* masks = P.dkvq + kTileqHead;
+        if (atomicOr(masks + blk, 1u << (kt % kBwdBlk)) == 0u) masks[BH * nkb + atomicAdd(P.dkvq, 1u)] = (uint32_t)blk;
+      } else {
+        P.dkvq[1 + atomicAdd(P.dkvq, 1u)] = (uint32_t)item;
+      }
+    }
     return;
   }
   wave_lds_sync();  // slots written by other lanes
@@ -1060,244 +868,12 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
   }
 }
 
-// ------------------------------------------------------------------ key-major pass
-// The tile pass over one key tile (item = (key tile, head)): one wave, W its LDS.
-template <int D, int BR, int PK, bool NORM>
-__device__ __forceinline__ void bwd_dkv_tile(const BwdParams& P, BwdWaveLds<D>& W, int64_t item) {
-  constexpr int NT = D / 16, ND = D / 32;
-  const int l = lane_id(), n32 = l & 31, g = l >> 5;
-  const int BH = P.B * P.H;
-  const int kt = (int)(item / BH);
-  const int bh = (int)(item % BH);
-  const int b = bh / P.H, h = bh % P.H;
-  const int Nq = P.Nq, Nk = P.Nk, qoff = P.qoff;
-  const int j = kt * 32 + n32;
-  const bool kvalid = j < Nk;
-  const int jc = min(j, Nk - 1);
-  const int qtf = qt_first(kt, qoff);  // first query tile that sees the key tile
-  auto base = [&](int slot) {
-    return (const bf16*)P.in[slot] + (int64_t)b * P.s[slot][0] + (int64_t)h * P.s[slot][1];
-  };
-
-  bf16x8 V[NT];
-  {
-    const bf16* r = base(B_V) + (int64_t)jc * P.s[B_V][2];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) V[t] = *reinterpret_cast<const bf16x8*>(r + 16 * t + 8 * g);
-  }
-  const float beta = *P.beta;
-  const float pw = P.p;
-  float lam = 0.f;
-  if constexpr (BR == 2) lam = clamp01(*P.lam);
-  const bf16* dob = base(B_DO);
-  const int64_t sdo = P.s[B_DO][2];
-  f32x16 AV[ND];
-#pragma unroll
-  for (int c = 0; c < ND; ++c) AV[c] = f32x16{};
-  unsigned visited = 0, computed = 0;
-
-  // Both branches' row operands, issued with V so that one memory round trip covers them:
-  // inverse key norms, and the bitmask column bits of query tiles qtf .. qtf+63 (lane q holds
-  // tile qtf + q).  The key fragments are loaded by the tile path, which alone needs them.
-  float RK[BR];
-  bool HAS[BR];
-#pragma unroll
-  for (int br = 0; br < BR; ++br) {
-    RK[br] = NORM ? P.norms[norm_base(P, br == 0 ? N_K1 : N_K2, bh) + jc] : 1.f;
-    const uint32_t* occcol = P.occ ? P.occ + ((int64_t)br * BH + bh) * P.nqt * P.occ_w + (kt >> 5) : nullptr;
-    const int qtl = qtf + l;
-    HAS[br] = qtl < P.nqt && (!occcol || ((occcol[(int64_t)qtl * P.occ_w] >> (kt & 31)) & 1u));
-  }
-
-#pragma unroll
-  for (int br = 0; br < BR; ++br) {
-    const int qslot = br == 0 ? B_Q1 : B_Q2, kslot = br == 0 ? B_K1 : B_K2;
-    const bf16* qb = base(qslot);
-    const int64_t sq = P.s[qslot][2];
-    const bf16* krow = base(kslot) + (int64_t)jc * P.s[kslot][2];
-    const float rk = RK[br];
-    const float* nq = nullptr;
-    if constexpr (NORM) nq = P.norms + norm_base(P, br == 0 ? N_Q1 : N_Q2, bh);
-    const float coef = br == 0 ? 1.f : -lam;
-    f32x16 AK[ND];
-#pragma unroll
-    for (int c = 0; c < ND; ++c) AK[c] = f32x16{};
-    // bitmask column: bit kt % 32 of word (br, bh, qt, kt / 32) for qt = qtf .. nqt-1
-    const uint32_t* occcol = P.occ ? P.occ + ((int64_t)br * BH + bh) * P.nqt * P.occ_w + (kt >> 5) : nullptr;
-
-    for (int q0c = qtf; q0c < P.nqt; q0c += 64) {
-      const int qtl = q0c + l;
-      const bool has = q0c == qtf ? HAS[br] : qtl < P.nqt && (!occcol || ((occcol[(int64_t)qtl * P.occ_w] >> (kt & 31)) & 1u));
-      uint64_t mask = wave_ballot(has);
-      while (mask) {
-        const int qt = q0c + __builtin_ctzll(mask);
-        mask &= mask - 1ull;
-        ++visited;
-        const int q0 = 32 * qt;
-        bf16x8 K[NT];  // the key fragments, for the score recompute
-#pragma unroll
-        for (int t = 0; t < NT; ++t) K[t] = *reinterpret_cast<const bf16x8*>(krow + 16 * t + 8 * g);
-        dma_tile<D>(qb, sq, q0, Nq, W.a);
-        dma_tile<D>(dob, sdo, q0, Nq, W.b);
-        if constexpr (NORM) dma_row_vals(nq, q0, Nq, W.rows);
-        if (l < 32) W.taus[l] = beta * tau_coeff(qoff + q0 + l, P.inv_d);
-        wait_all_loads();
-        f32x16 S = f32x16{}, Dp = f32x16{};
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          S = PolBF16::mma(tile_row_frag<D>(W.a, t), K[t], S);
-          Dp = PolBF16::mma(tile_row_frag<D>(W.b, t), V[t], Dp);
-        }
-        float rq[16], tq[16];
-        if constexpr (NORM) crow_vals(W.rows, rq);
-        crow_vals(W.taus, tq);
-        f32x16 EV, EK;
-        bool any = false;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int qi = q0 + crow(r, g);
-          const bool valid = kvalid && qi < Nq && j <= qoff + qi;
-          const float sr = NORM ? S[r] * rk : S[r];
-          const float x = __builtin_fmaf(sr, NORM ? rq[r] : 1.f, -tq[r]);
-          const bool pos = valid && x > 0.f;
-          EV[r] = pos ? coef * pow_p<PK>(x, pw) : 0.f;
-          const float ds = pos ? coef * dpow_p<PK>(x, pw) * Dp[r] : 0.f;
-          EK[r] = NORM ? ds * rq[r] : ds;
-          any = any || pos;
-        }
-        if (!occcol && wave_ballot(any) == 0ull) continue;
-        ++computed;
-        const bf16x8 V0 = PolBF16::pack_c(EV, 0), V1 = PolBF16::pack_c(EV, 1);
-        const bf16x8 K0 = PolBF16::pack_c(EK, 0), K1 = PolBF16::pack_c(EK, 1);
-#pragma unroll
-        for (int c = 0; c < ND; ++c) {
-          AV[c] = PolBF16::mma(tile_tr_frag<D>(W.b, 0, c), V0, AV[c]);
-          AV[c] = PolBF16::mma(tile_tr_frag<D>(W.b, 1, c), V1, AV[c]);
-          AK[c] = PolBF16::mma(tile_tr_frag<D>(W.a, 0, c), K0, AK[c]);
-          AK[c] = PolBF16::mma(tile_tr_frag<D>(W.a, 1, c), K1, AK[c]);
-        }
-      }
-    }
-    if (kvalid) {
-      GradRow<D> XR;  // the key row for the normalize backward
-      if constexpr (NORM) load_grad_row<D>(krow, XR);
-      const int gslot = br == 0 ? B_DK1 : B_DK2;
-      bf16* grow = (bf16*)P.grad[br == 0 ? 1 : 3] + (int64_t)b * P.s[gslot][0] + (int64_t)h * P.s[gslot][1] +
-                   (int64_t)j * P.s[gslot][2];
-      store_grad_rows<D, NORM>(AK, XR, grow, rk);
-    }
-  }
-  if (kvalid) {
-    bf16* vrow = (bf16*)P.grad[4] + (int64_t)b * P.s[B_DV][0] + (int64_t)h * P.s[B_DV][1] + (int64_t)j * P.s[B_DV][2];
-    store_grad_rows<D, false>(AV, GradRow<D>{}, vrow, 1.f);
-  }
-  if (P.stats && l == 0) {
-    atomicAdd(P.stats + 0, (unsigned long long)visited);
-    atomicAdd(P.stats + 1, (unsigned long long)computed);
-  }
-}
-
-// Bit k set when the column of key-major item first + k (k < count <= 4) has a list that did
-// not fit (the test of column_overflows): the bitmask bits and counts of the first 128 query
-// tiles of every column in one round, longer columns' rest column by column.
-template <int BR>
-__device__ __forceinline__ uint32_t columns_overflow(const BwdParams& P, int64_t first, int count) {
-  const int BH = P.B * P.H, l = lane_id();
-  const uint32_t* counts = P.pairs + pair_lists(BR, BH, P.nqt) * 4 * kPairCap;
-  int kt[4], bh[4], qtf[4];
-  bool ovf[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t item = first + (k < count ? k : 0);
-    kt[k] = (int)(item / BH);
-    bh[k] = (int)(item % BH);
-    qtf[k] = qt_first(kt[k], P.qoff);
-    ovf[k] = false;
-  }
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int br = 0; br < BR; ++br) {
-        const int qt = qtf[k] + 64 * c + l;
-        const bool in = k < count && qt < P.nqt;
-        const int64_t row = ((int64_t)br * BH + bh[k]) * P.nqt + (in ? qt : P.nqt - 1);
-        const uint32_t w = P.occ[row * P.occ_w + (kt[k] >> 5)];
-        const uint32_t n = counts[row];
-        ovf[k] = ovf[k] || (in && ((w >> (kt[k] & 31)) & 1u) && n > (uint32_t)kPairCap);
-      }
-  uint32_t out = 0u;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (k >= count) continue;
-    bool o = wave_ballot(ovf[k]) != 0ull;
-    if (!o && qtf[k] + 128 < P.nqt) o = column_overflows<BR>(P, bh[k], kt[k], qtf[k] + 128);
-    out |= o ? 1u << k : 0u;
-  }
-  return out;
-}
-
-// One wave per workgroup and `per_wave` consecutive items per wave.  With pair lists, the key
-// tiles whose columns have only lists that fit belong to bwd_dkv_pairs: the wave tests its
-// items' columns in one round and runs only the others (per_wave 4); without lists every item
-// runs (per_wave 1).
-// With the key-tile queue (per_wave 0), the waves take the queued key tiles in turn instead.
-template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(64) bwd_dkv_fast(BwdParams P, int per_wave) {
-  __shared__ __attribute__((aligned(16))) BwdWaveLds<D> W;
-  if (per_wave == 0) {
-    const uint32_t queued = P.dkvq[0];
-    for (uint32_t k = blockIdx.x; k < queued; k += gridDim.x) bwd_dkv_tile<D, BR, PK, NORM>(P, W, P.dkvq[1 + k]);
-    return;
-  }
-  const int64_t n = (int64_t)P.B * P.H * P.nkt, first = (int64_t)blockIdx.x * per_wave;
-  const int count = (int)min((int64_t)per_wave, n - first);
-  if (count <= 0) return;
-  uint32_t run = count >= 32 ? 0xffffffffu : (1u << count) - 1u;
-  if (P.pairs) run = columns_overflow<BR>(P, first, count);
-  for (; run; run &= run - 1u) bwd_dkv_tile<D, BR, PK, NORM>(P, W, first + __builtin_ctz(run));
-}
-
-// ------------------------------------------------------------------ both tile passes, one launch
-// With pair lists and the key-tile queue: single-wave workgroups that first run the
-// query-major tile pass for the lists that did not fit (64 list counts tested per round, the
-// lists in order) and then take the key tiles the key-major pair pass queued.  The query-major
-// items do not depend on the key-major pass, so they run after it here, which saves the launch
-// of a separate query-major tile pass.  (Adding the dbeta / dlambda sum here, by the last
-// workgroup to finish, cost more than the launch it saved: every workgroup's release fence
-// wrote back its XCD's L2.)
-template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(64) bwd_tiles(BwdParams P) {
-  __shared__ __attribute__((aligned(16))) BwdWaveLds<D> W;
-  const int l = lane_id();
-  const int BH = P.B * P.H;
-  const int64_t lists = (int64_t)BR * BH * P.nqt, lists_h = (int64_t)BH * P.nqt;
-  const uint32_t* counts = P.pairs + pair_lists(BR, BH, P.nqt) * 4 * kPairCap;
-  for (int64_t f = (int64_t)blockIdx.x * 64; f < lists; f += (int64_t)gridDim.x * 64) {
-    const bool need = f + l < lists && counts[f + l] > (uint32_t)kPairCap;
-    for (uint64_t m = wave_ballot(need); m; m &= m - 1ull) {
-      const int64_t lx = f + __builtin_ctzll(m);  // list (branch, head, query tile) -> tile-pass item
-      const int br = (int)(lx / lists_h);
-      const int64_t rem = lx % lists_h;
-      const int bh = (int)(rem / P.nqt), qt = (int)(rem % P.nqt);
-      const int64_t rest = (int64_t)(P.nqt - 1 - qt) * BH + bh;
-      bwd_dq_tile<D, BR, PK, NORM>(P, W, BR == 2 ? 2 * rest + br : rest);
-    }
-  }
-  const uint32_t queued = P.dkvq[0];
-  for (uint32_t k = blockIdx.x; k < queued; k += gridDim.x) bwd_dkv_tile<D, BR, PK, NORM>(P, W, P.dkvq[1 + k]);
-}
-
 // ------------------------------------------------------------------ block tile passes
-// For the backwards whose forward ran the block tile pass (no candidate lists, every query tile
-// runs): kBwdBlk consecutive tiles of one head per workgroup, one wave each, walking the union of
-// their bitmask tiles in step; each streamed tile's rows are loaded once per workgroup (each wave
-// a quarter, one tile ahead into registers) into a two-stage LDS ring of swizzled tiles (the
-// layout of dma_tile_b: tile_row_frag / tile_tr_frag read it), one fence-free barrier per tile.
-// A wave computes only its own tiles, with the arithmetic of bwd_dq_tile / bwd_dkv_tile, the
-// masks branch-free and only on the tiles that need them.
-constexpr int kBwdBlk = 4;
+// kBwdBlk consecutive tiles of one head per workgroup, one wave each, walking the union of their
+// bitmask tiles in step; each streamed tile's rows are loaded once per workgroup (each wave a
+// quarter, one tile ahead into registers) into a two-stage LDS ring of chunk-swizzled tiles
+// (tile_row_frag / tile_tr_frag read them), one fence-free barrier per tile.  A wave computes only
+// its own tiles, the masks branch-free and only on the tiles that need them.
 
 // max(x, 0) of 16 values on their bits: a float is > 0 iff its bits as an int32 are.
 __device__ __forceinline__ f32x16 relu_bits(const f32x16& x) {
@@ -1306,6 +882,14 @@ __device__ __forceinline__ f32x16 relu_bits(const f32x16& x) {
 #pragma unroll
   for (int r = 0; r < 16; ++r) b[r] = max(b[r], 0);
   return __builtin_bit_cast(f32x16, b);
+}
+// The same with a NaN taken to 0: with normalisation a score of a non-finite row has no weight.
+template <bool NORM>
+__device__ __forceinline__ f32x16 relu16(f32x16 x) {
+  if constexpr (!NORM) return relu_bits(x);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) x[r] = fmaxf(x[r], 0.f);
+  return x;
 }
 
 // This wave's share of a 32-row tile of D columns: rows RPI (LPW wv + i) + l / CH, chunk l % CH.
@@ -1334,20 +918,21 @@ struct BlkRows {
   }
 };
 
-// Query-major: kBwdBlk query tiles of one (branch, head), streaming K, V and the key norms.
+// Query-major: kBwdBlk query tiles of one (branch, head), streaming K, V and the key norms.  The
+// block takes its tiles whose lists did not fit (or all, without lists).
+template <int D>
+struct DqBlkLds {
+  bf16 ring[2 * 2 * 32 * D];  // two stages of a K tile and a V tile
+  float norms[2][32];
+};
 template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_blk(BwdParams P) {
+__device__ __forceinline__ void dq_block(const BwdParams& P, DqBlkLds<D>& L, int jb, int br, int bh) {
   constexpr int W = kBwdBlk, NT = D / 16, ND = D / 32;
   constexpr int STAGE = 2 * 32 * D;  // K tile, V tile
-  __shared__ __attribute__((aligned(16))) bf16 ring[2 * STAGE];
-  __shared__ __attribute__((aligned(16))) float nring[2][32];
+  bf16* ring = L.ring;
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int BH = P.B * P.H, nqt = P.nqt, Nq = P.Nq, Nk = P.Nk, qoff = P.qoff;
-  const int nqb = (nqt + W - 1) / W;
-  // longest blocks (last query tiles) of every (head, branch) first, the branches adjacent
-  const int bid = blockIdx.x, jb = nqb - 1 - bid / (BR * BH), rem = bid % (BR * BH);
-  const int br = BR == 2 ? rem & 1 : 0, bh = BR == 2 ? rem >> 1 : rem;
   const int b = bh / P.H, h = bh % P.H;
   const uint32_t* counts = P.pairs ? P.pairs + pair_lists(BR, BH, nqt) * 4 * kPairCap : nullptr;
   const int64_t lrow0 = ((int64_t)br * BH + bh) * nqt + W * jb;  // list / bitmask row of the block's first tile
@@ -1449,7 +1034,7 @@ __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_
   while (kt >= 0) {
     bf16* kst = ring + (it & 1) * STAGE;
     bf16* vst = kst + 32 * D;
-    float* nst = nring[it & 1];
+    float* nst = L.norms[it & 1];
     kr.store(kst, wv);
     vr.store(vst, wv);
     if (NORM && wv == 0 && l < 8) *reinterpret_cast<f32x4*>(nst + 4 * l) = nr;
@@ -1487,7 +1072,7 @@ __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_
         // relu on the bits (a float is > 0 iff its bits as an int32 are): t = max(x, 0) with no
         // comparison per value; 2 t and t^2 vanish with t.  (Whole-vector bit casts: hipcc
         // compiled a bit cast of one element of an ext_vector to element 0.)
-        const f32x16 T = relu_bits(X);
+        const f32x16 T = relu16<NORM>(X);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float ds = coef * (T[r] + T[r]) * Dp[r];
@@ -1545,56 +1130,25 @@ __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_
 }
 
 // Key-major: kBwdBlk consecutive key tiles of one head (aligned: one bitmask word holds their
-// bits), streaming per branch the query tiles' Q and dO rows, query norms and tau values.  A key
-// tile takes this pass when a list of its column did not fit (the test bwd_dkv_pairs queues
-// by; it writes nothing for such a key tile), or always without lists.
+// bits), streaming per branch the query tiles' Q and dO rows, query norms and tau values.  needm:
+// the block's key tiles to take (at least one).
+template <int D>
+struct DkvBlkLds {
+  bf16 ring[2 * 2 * 32 * D];     // two stages of a Q tile and a dO tile
+  float vals[2][2][32];          // [stage][query norms, tau values]
+  bf16 ktiles[kBwdBlk][32 * D];  // each wave's key rows (swizzled)
+};
 template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(BR == 2 ? (D <= 64 ? 2 : 1) : (D <= 64 ? 3 : 2)))) bwd_dkv_blk(BwdParams P) {
+__device__ __forceinline__ void dkv_block(const BwdParams& P, DkvBlkLds<D>& L, int jb, int bh, uint32_t needm) {
   constexpr int W = kBwdBlk, NT = D / 16, ND = D / 32;
   constexpr int STAGE = 2 * 32 * D;  // Q tile, dO tile
-  __shared__ __attribute__((aligned(16))) bf16 ring[2 * STAGE];
-  __shared__ __attribute__((aligned(16))) float vring[2][2][32];  // [stage][query norms, tau values]
-  __shared__ __attribute__((aligned(16))) bf16 ktiles[W][32 * D];  // each wave's key rows (swizzled)
-  __shared__ uint32_t needs[W];
+  bf16* ring = L.ring;
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int BH = P.B * P.H, nqt = P.nqt, nkt = P.nkt, Nq = P.Nq, Nk = P.Nk, qoff = P.qoff;
-  const int nkb = (nkt + W - 1) / W;
-  // longest blocks (first key tiles) of every head first
-  const int bid = blockIdx.x, jb = bid / BH, bh = bid % BH;
   const int b = bh / P.H, h = bh % P.H;
   const int kt0 = W * jb, kt = kt0 + wv;
   const int qtf_b = qt_first(kt0, qoff);  // first query tile of the block
-  const uint32_t* counts = P.pairs ? P.pairs + pair_lists(BR, BH, nqt) * 4 * kPairCap : nullptr;
-  // this wave's key tile: does a list of its column not fit (every branch, query tiles from
-  // the first that sees it)?
-  {
-    bool nd = kt < nkt;
-    if (nd && counts) {
-      const int qtf = qt_first(kt, qoff);
-      bool ovf = false;
-      for (int q0c = qtf; q0c < nqt && !ovf; q0c += 64) {
-        bool o = false;
-#pragma unroll
-        for (int br = 0; br < BR; ++br) {
-          const int qtl = q0c + l;
-          const bool in = qtl < nqt;
-          const int64_t row = ((int64_t)br * BH + bh) * nqt + (in ? qtl : nqt - 1);
-          const uint32_t w = P.occ ? P.occ[row * P.occ_w + (kt >> 5)] : 0xffffffffu;
-          o = o || (in && ((w >> (kt & 31)) & 1u) && counts[row] > (uint32_t)kPairCap);
-        }
-        ovf = wave_ballot(o) != 0ull;
-      }
-      nd = ovf;
-    }
-    if (l == 0) needs[wv] = nd ? 1u : 0u;
-  }
-  __syncthreads();
-  uint32_t needm = 0u;
-#pragma unroll
-  for (int r = 0; r < W; ++r) needm |= needs[r] ? 1u << r : 0u;
-  needm = (uint32_t)__builtin_amdgcn_readfirstlane((int)needm);
-  if (!needm) return;
   const bool need = (needm >> wv) & 1u;
   const int j = 32 * kt + n32;
   const bool kvalid = need && j < Nk;
@@ -1621,7 +1175,7 @@ __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_
   for (int c = 0; c < ND; ++c) AV[c] = f32x16{};
   unsigned visited = 0, computed = 0;
   int it = 0;  // ring position, continued across the branches
-  bf16* kti = ktiles[wv];
+  bf16* kti = L.ktiles[wv];
 
 #pragma unroll
   for (int br = 0; br < BR; ++br) {
@@ -1685,8 +1239,8 @@ __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_
     while (qt >= 0) {
       bf16* qst = ring + (it & 1) * STAGE;
       bf16* dst = qst + 32 * D;
-      float* rqs = vring[it & 1][0];
-      float* tqs = vring[it & 1][1];
+      float* rqs = L.vals[it & 1][0];
+      float* tqs = L.vals[it & 1][1];
       qr.store(qst, wv);
       dr.store(dst, wv);
       if (wv == 0 && l < 32) {
@@ -1728,7 +1282,7 @@ __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_
         }
         f32x16 EV, EK;
         if constexpr (PK == 2) {  // relu on the bits, as in bwd_dq_blk
-          const f32x16 T = relu_bits(X);
+          const f32x16 T = relu16<NORM>(X);
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             EV[r] = coef * (T[r] * T[r]);
@@ -1785,66 +1339,139 @@ __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_
   }
 }
 
+// One workgroup per block of query tiles: longest blocks (last query tiles) of every (head,
+// branch) first, the branches adjacent.
+template <int D, int BR, int PK, bool NORM>
+__global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_blk(BwdParams P) {
+  __shared__ __attribute__((aligned(16))) DqBlkLds<D> L;
+  const int BH = P.B * P.H, nqb = (P.nqt + kBwdBlk - 1) / kBwdBlk;
+  const int bid = blockIdx.x, jb = nqb - 1 - bid / (BR * BH), rem = bid % (BR * BH);
+  dq_block<D, BR, PK, NORM>(P, L, jb, BR == 2 ? rem & 1 : 0, BR == 2 ? rem >> 1 : rem);
+}
+
+// Waves per SIMD that the key-major pass is compiled for: one branch without normalisation three
+// at d = 64 and two at d = 128 (2 and 20 VGPRs spilled; dense steps (4, 16, 2048, d) of 242 and 473
+// us against 244 and 539 with one fewer); two branches spill 21 and 38-54 there (467-472 against
+// 501-514 us at d = 64), normalisation 26 and 41, so they run one fewer.
+template <int D, int BR, bool NORM>
+constexpr int dkv_waves() {
+  return (BR == 2 || NORM ? 1 : 2) + (D <= 64 ? 1 : 0);
+}
+
+// One workgroup per block of key tiles: longest blocks (first key tiles) of every head first.  A
+// key tile takes this pass when a list of its column did not fit (the test bwd_dkv_pairs leaves
+// it by; it writes nothing for such a key tile), or always without lists.
+template <int D, int BR, int PK, bool NORM>
+__global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, NORM>()))) bwd_dkv_blk(BwdParams P) {
+  constexpr int W = kBwdBlk;
+  __shared__ __attribute__((aligned(16))) DkvBlkLds<D> L;
+  __shared__ uint32_t needs[W];
+  const int l = lane_id();
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int BH = P.B * P.H, nqt = P.nqt;
+  const int bid = blockIdx.x, jb = bid / BH, bh = bid % BH, kt = W * jb + wv;
+  const uint32_t* counts = P.pairs ? P.pairs + pair_lists(BR, BH, nqt) * 4 * kPairCap : nullptr;
+  // this wave's key tile: does a list of its column not fit (every branch, query tiles from
+  // the first that sees it)?
+  {
+    bool nd = kt < P.nkt;
+    if (nd && counts) {
+      const int qtf = qt_first(kt, P.qoff);
+      bool ovf = false;
+      for (int q0c = qtf; q0c < nqt && !ovf; q0c += 64) {
+        bool o = false;
+#pragma unroll
+        for (int br = 0; br < BR; ++br) {
+          const int qtl = q0c + l;
+          const bool in = qtl < nqt;
+          const int64_t row = ((int64_t)br * BH + bh) * nqt + (in ? qtl : nqt - 1);
+          const uint32_t w = P.occ ? P.occ[row * P.occ_w + (kt >> 5)] : 0xffffffffu;
+          o = o || (in && ((w >> (kt & 31)) & 1u) && counts[row] > (uint32_t)kPairCap);
+        }
+        ovf = wave_ballot(o) != 0ull;
+      }
+      nd = ovf;
+    }
+    if (l == 0) needs[wv] = nd ? 1u : 0u;
+  }
+  __syncthreads();
+  uint32_t needm = 0u;
+#pragma unroll
+  for (int r = 0; r < W; ++r) needm |= needs[r] ? 1u << r : 0u;
+  needm = (uint32_t)__builtin_amdgcn_readfirstlane((int)needm);
+  if (needm) dkv_block<D, BR, PK, NORM>(P, L, jb, bh, needm);
+}
+
+// Both block passes over the queue of the key-major pair pass, in one launch: the workgroups
+// take tickets, the key blocks (the longer ones) first, each kind longest blocks first as nearly as
+// the queue's order has it.  With every list fitting the queue is empty and a workgroup leaves
+// after one load (5.0 us); at a threshold scale of 0.5 nearly every block is queued
+// (TDA (2, 16, 1500, 64): 178 us, 2632 us with one wave per query or key tile fetching
+// its own rows).
+template <int D, int BR, int PK>
+__global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, true>()))) bwd_tiles(BwdParams P) {
+  union Lds {
+    DqBlkLds<D> dq;
+    DkvBlkLds<D> dkv;
+  };
+  __shared__ __attribute__((aligned(16))) Lds L;
+  __shared__ uint32_t ticket;
+  const uint32_t nk = P.dkvq[0], total = nk + P.dkvq[1];
+  if (total == 0u) return;
+  const int BH = P.B * P.H, nqb = (P.nqt + kBwdBlk - 1) / kBwdBlk, nkb = (P.nkt + kBwdBlk - 1) / kBwdBlk;
+  const uint32_t* masks = P.dkvq + kTileqHead;
+  while (true) {
+    __syncthreads();  // every wave is done with the previous block's LDS and ticket
+    if (threadIdx.x == 0) ticket = atomicAdd(P.dkvq + 2, 1u);
+    __syncthreads();
+    const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)ticket);
+    if (t >= total) return;
+    if (t < nk) {
+      const uint32_t blk = (uint32_t)__builtin_amdgcn_readfirstlane((int)masks[(int64_t)BH * nkb + t]);
+      dkv_block<D, BR, PK, true>(P, L.dkv, (int)(blk % nkb), (int)(blk / nkb),
+                                 (uint32_t)__builtin_amdgcn_readfirstlane((int)masks[blk]));
+    } else {
+      const uint32_t k = (uint32_t)__builtin_amdgcn_readfirstlane((int)masks[2 * (int64_t)BH * nkb + (t - nk)]);
+      const int rem = (int)(k % (uint32_t)(BR * BH));
+      dq_block<D, BR, PK, true>(P, L.dq, nqb - 1 - (int)(k / (uint32_t)(BR * BH)), BR == 2 ? rem & 1 : 0,
+                                BR == 2 ? rem >> 1 : rem);
+    }
+  }
+}
+
 // ------------------------------------------------------------------ dispatch
+// With pair lists the pair passes take the lists that fit, then the block tile passes the rest,
+// then the sum.  With normalisation most calls leave nothing, so the block passes run from a queue
+// in one launch (when the workspace holds it); without, nearly every list is past its cap and each
+// pass launches a workgroup per block.
 template <int D, int BR, int PK, bool NORM>
 static int launch_t(const BwdParams& p, void* stream) {
   const int64_t qitems = (int64_t)BR * p.B * p.H * p.nqt, kitems = (int64_t)p.B * p.H * p.nkt;
   hipStream_t s = (hipStream_t)stream;
-  if constexpr (!NORM) {
-    // The forward ran its block tile pass (every query tile): the pair passes take the lists
-    // that fit, then the block tile passes everything else (no key-tile queue), the sum.
-    BwdParams q = p;
-    q.dkvq = nullptr;
-    if (q.pairs) {
-      hipLaunchKernelGGL((bwd_dq_pairs<D, BR, PK, NORM>), dim3((unsigned)qitems), dim3(64), 0, s, q);
-      launched(s, "bwd_dq_pairs");
-      hipLaunchKernelGGL((bwd_dkv_pairs<D, BR, PK, NORM>), dim3((unsigned)kitems), dim3(64), 0, s, q);
-      launched(s, "bwd_dkv_pairs");
-    }
-    const int BH = q.B * q.H;
-    hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM>), dim3((unsigned)(BR * BH * ((q.nqt + kBwdBlk - 1) / kBwdBlk))),
-                       dim3(64 * kBwdBlk), 0, s, q);
-    launched(s, "bwd_dq_blk");
-    hipLaunchKernelGGL((bwd_dkv_blk<D, BR, PK, NORM>), dim3((unsigned)(BH * ((q.nkt + kBwdBlk - 1) / kBwdBlk))),
-                       dim3(64 * kBwdBlk), 0, s, q);
-    launched(s, "bwd_dkv_blk");
-    const int e = (int)hipGetLastError();
-    return e ? e : launch_bwd_finish(q, BR, qitems, stream);
-  }
-  if (p.pairs && p.dkvq) {  // the pair passes, both tile passes in one launch, the sum
-    hipLaunchKernelGGL((bwd_dq_pairs<D, BR, PK, NORM>), dim3((unsigned)qitems), dim3(64), 0, s, p);
+  BwdParams q = p;
+  if (!NORM) q.dkvq = nullptr;
+  if (q.pairs) {
+    hipLaunchKernelGGL((bwd_dq_pairs<D, BR, PK, NORM>), dim3((unsigned)qitems), dim3(64), 0, s, q);
     launched(s, "bwd_dq_pairs");
-    hipLaunchKernelGGL((bwd_dkv_pairs<D, BR, PK, NORM>), dim3((unsigned)kitems), dim3(64), 0, s, p);
+    hipLaunchKernelGGL((bwd_dkv_pairs<D, BR, PK, NORM>), dim3((unsigned)kitems), dim3(64), 0, s, q);
     launched(s, "bwd_dkv_pairs");
-    // one wave per SIMD (the key-major tile body's registers)
-    hipLaunchKernelGGL((bwd_tiles<D, BR, PK, NORM>), dim3(1024u), dim3(64), 0, s, p);
+  }
+  const int BH = q.B * q.H;
+  const unsigned qblocks = (unsigned)(BR * BH * ((q.nqt + kBwdBlk - 1) / kBwdBlk));
+  const unsigned kblocks = (unsigned)(BH * ((q.nkt + kBwdBlk - 1) / kBwdBlk));
+  if (NORM && q.pairs && q.dkvq) {
+    // as many workgroups as the GPU's 256 CUs hold at dkv_waves waves per SIMD
+    const unsigned most = 256u * dkv_waves<D, BR, true>(), blocks = qblocks + kblocks;
+    hipLaunchKernelGGL((bwd_tiles<D, BR, PK>), dim3(blocks < most ? blocks : most), dim3(64 * kBwdBlk), 0, s, q);
     launched(s, "bwd_tiles");
-    const int e = (int)hipGetLastError();
-    return e ? e : launch_bwd_finish(p, BR, qitems, stream);
-  }
-  if (p.pairs) {
-    hipLaunchKernelGGL((bwd_dq_pairs<D, BR, PK, NORM>), dim3((unsigned)qitems), dim3(64), 0, s, p);
-    launched(s, "bwd_dq_pairs");
-  }
-  const int dq_per_wave = p.pairs ? 8 : 1;  // with pair lists most items exit at once
-  hipLaunchKernelGGL((bwd_dq_fast<D, BR, PK, NORM>), dim3((unsigned)((qitems + dq_per_wave - 1) / dq_per_wave)),
-                     dim3(64), 0, s, p, dq_per_wave);
-  launched(s, "bwd_dq_fast");
-  if (p.pairs) {
-    hipLaunchKernelGGL((bwd_dkv_pairs<D, BR, PK, NORM>), dim3((unsigned)kitems), dim3(64), 0, s, p);
-    launched(s, "bwd_dkv_pairs");
-  }
-  if (p.dkvq) {  // the key tiles the pair pass could not take, from its queue: one wave per SIMD
-    hipLaunchKernelGGL((bwd_dkv_fast<D, BR, PK, NORM>), dim3((unsigned)(kitems < 1024 ? kitems : 1024)), dim3(64), 0, s,
-                       p, 0);
   } else {
-    const int dkv_per_wave = p.pairs ? 4 : 1;  // with pair lists most key tiles exit at once
-    hipLaunchKernelGGL((bwd_dkv_fast<D, BR, PK, NORM>), dim3((unsigned)((kitems + dkv_per_wave - 1) / dkv_per_wave)),
-                       dim3(64), 0, s, p, dkv_per_wave);
+    hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM>), dim3(qblocks), dim3(64 * kBwdBlk), 0, s, q);
+    launched(s, "bwd_dq_blk");
+    hipLaunchKernelGGL((bwd_dkv_blk<D, BR, PK, NORM>), dim3(kblocks), dim3(64 * kBwdBlk), 0, s, q);
+    launched(s, "bwd_dkv_blk");
   }
-  launched(s, "bwd_dkv_fast");
   const int e = (int)hipGetLastError();
-  return e ? e : launch_bwd_finish(p, BR, qitems, stream);
+  return e ? e : launch_bwd_finish(q, BR, qitems, stream);
 }
 template <int D, int BR, int PK>
 static int sel_norm(const BwdParams& p, const KernelKey& k, void* s) {

@@ -20,13 +20,13 @@
 //               of its rows against the candidate keys (the same MFMA sequence and operand
 //               values as fwd_pv, so the same scores), the exact weights and coef A V over the
 //               candidates' V rows, the branches' sums added through LDS; the bitmask row is
-//               rewritten exactly.  Query tiles whose lists overflow go to a queue for fwd_pv.
-//   fwd_pv      the tile pass for the queued query tiles, one wave per query tile: walks the set
-//               bits of both branches, recomputes the score tile, forms the exact weights
-//               ReLU(x)^p with the causal mask, and accumulates out += coef A V.  Tiles whose
-//               exact weights are all zero lose their bit, so the bitmask ends exact.
-// Without normalisation one launch, fwd_pv_blk: every query tile, four per workgroup sharing
-// each key tile's rows, scores every causal key tile and forms the weights, A V and the exact
+//               rewritten exactly.
+//   fwd_pv_blk  the tile pass for the query tiles whose lists overflowed, four consecutive query
+//               tiles per workgroup sharing each key tile's rows: walks the set bits of both
+//               branches, recomputes the score tile, forms the exact weights ReLU(x)^p with the
+//               causal mask, and accumulates out += coef A V.  Tiles whose exact weights are all
+//               zero lose their bit, so the bitmask ends exact.
+// Without normalisation one launch, fwd_pv_blk over every query tile: scores every causal key tile and forms the weights, A V and the exact
 // bitmask itself (a screen would compute the same bf16 scores once more); its workgroups also
 // clear the call's zero range, a share each after their own tiles.
 // The screen tests every key of the tile, including keys after the query on the diagonal tile:
@@ -735,7 +735,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) f
   screen_count<QPW>(P, it, live, ktl);
 }
 
-// ------------------------------------------------------------------ fwd_pv
 // Transposed A fragment of one 32-column block and one 16-row step from a row-major tile
 // with row stride VS: lane (n, g) gets column n of the block at tile rows crow(8*st + j, g),
 // j = 0..7, by two LDS transpose reads.  `p` already includes this lane's base offset.
@@ -746,255 +745,32 @@ __device__ __forceinline__ bf16x8 tr_frag(const bf16* p) {
   return bf16x8{a[0], a[1], a[2], a[3], c[0], c[1], c[2], c[3]};
 }
 
-// The tile pass over one query tile (bh, qt): one wave; vt / ktl its LDS tiles.
-template <int D, int BR, int PK, bool NORM>
-__device__ __forceinline__ void fwd_pv_tile(const FwdParams& P, bf16* vt_, bf16* kt_, int bh, int qt) {
-  constexpr int NT = D / 16, ND = D / 32;
-  constexpr int VS = D + 32;     // LDS row stride of a V tile: conflict-free transpose reads
-  constexpr int CPR = D / 8;     // 16-byte chunks per row
-  constexpr int RPI = 64 / CPR;  // rows per V load instruction
-  constexpr int VL = 32 / RPI;   // V load instructions per tile
-  constexpr int KS = D + 8;      // LDS row stride of a K tile: conflict-free row-fragment reads
-  const int l = lane_id(), n32 = l & 31, g = l >> 5;
-  const int BH = P.B * P.H, Nq = P.Nq, Nk = P.Nk, nqt = P.nqt, qoff = P.qoff;
-  const int b = bh / P.H, h = bh % P.H;
-  const int iq = 32 * qt + n32;
-  const bool valid = iq < Nq;
-  const int pq = qoff + iq;                  // the lane's query position
-  const int klast = kt_last(qt, qoff, P.nkt);  // last key tile the query tile sees
-  const float tau = *P.beta * tau_coeff(pq, P.inv_d);
-  const float pw = P.p;
-  float lam = 0.f;
-  if constexpr (BR == 2) lam = clamp01(*P.lam);
-
-  bf16* vt = vt_;
-  bf16* ktl = kt_;
-  const int vrow = l / CPR, vch = l % CPR;
-  const int bk = l >> 4, jj = l & 15;
-  const int voff = (4 * (bk >> 1) + (jj >> 2)) * VS + 16 * (bk & 1) + 4 * (jj & 3);
-
-  f32x16 O[ND];
-#pragma unroll
-  for (int c = 0; c < ND; ++c) O[c] = f32x16{};
-  unsigned computed = 0, checked = 0;
-
-#pragma unroll
-  for (int br = 0; br < BR; ++br) {
-    const int qslot = br ? F_Q2 : F_Q1, kslot = br ? F_K2 : F_K1;
-    uint32_t* orow = P.occ + ((int64_t)(br * BH + bh) * nqt + qt) * P.occ_w;
-    const bf16* khead = (const bf16*)P.in[kslot] + (int64_t)b * P.s[kslot][0] + (int64_t)h * P.s[kslot][1];
-    const bf16* vhead = (const bf16*)P.in[F_V] + (int64_t)b * P.s[F_V][0] + (int64_t)h * P.s[F_V][1];
-    const int64_t sk = P.s[kslot][2], sv = P.s[F_V][2];
-    const __amdgpu_buffer_rsrc_t rn =
-        make_rsrc(NORM ? P.norms + norm_base(P, br ? N_K2 : N_K1, bh) : nullptr, NORM ? (uint32_t)Nk * 4 : 0u);
-    const float coef = br == 0 ? 1.f : -lam;
-    bool have_q = false;
-    bf16x8 Q[NT];
-    float rq = 1.f;
-    // pair list of (branch, head, query tile): npairs entries written so far (may pass the cap)
-    const int64_t lidx = ((int64_t)br * BH + bh) * nqt + qt;
-    uint32_t* pent = P.pairs ? P.pairs + lidx * (4 * kPairCap) : nullptr;
-    uint32_t npairs = 0;
-    for (int w = 0; w <= (klast >> 5); ++w) {
-      const uint32_t bits0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)orow[w]);
-      uint32_t bits = bits0, keep = bits0;
-      while (bits) {
-        const int kt = 32 * w + __builtin_ctz(bits);
-        bits &= bits - 1u;
-        ++checked;
-        if (!have_q) {
-          // query tile rows with whole-row loads, through the (still free) K tile buffer
-          const bf16* qhead = (const bf16*)P.in[qslot] + (int64_t)b * P.s[qslot][0] + (int64_t)h * P.s[qslot][1];
-          const __amdgpu_buffer_rsrc_t rq_ = tile_rsrc<D>(qhead, P.s[qslot][2], qt, Nq);
-          u32x4 qr[VL];
-#pragma unroll
-          for (int i = 0; i < VL; ++i)
-            qr[i] = buf_load16(rq_, (uint32_t)(((vrow + RPI * i) * P.s[qslot][2] + 8 * vch) * 2));
-#pragma unroll
-          for (int i = 0; i < VL; ++i) *reinterpret_cast<u32x4*>(ktl + (vrow + RPI * i) * KS + 8 * vch) = qr[i];
-          wave_lds_sync();
-          const bf16* qp = ktl + n32 * KS + 8 * g;
-#pragma unroll
-          for (int t = 0; t < NT; ++t) Q[t] = *reinterpret_cast<const bf16x8*>(qp + 16 * t);
-          wave_lds_sync();
-          if constexpr (NORM) rq = P.norms[norm_base(P, br ? N_Q2 : N_Q1, bh) + min(iq, Nq - 1)];
-          have_q = true;
-        }
-        // loads of the key tile (A operand rows), the V tile and the key norms
-        const __amdgpu_buffer_rsrc_t rk = tile_rsrc<D>(khead, sk, kt, Nk);
-        const __amdgpu_buffer_rsrc_t rv = tile_rsrc<D>(vhead, sv, kt, Nk);
-        // whole rows per load instruction (coalesced), staged through LDS like V
-        u32x4 kr[VL];
-#pragma unroll
-        for (int i = 0; i < VL; ++i) kr[i] = buf_load16(rk, (uint32_t)(((vrow + RPI * i) * sk + 8 * vch) * 2));
-        u32x4 vr[VL];
-#pragma unroll
-        for (int i = 0; i < VL; ++i) vr[i] = buf_load16(rv, (uint32_t)(((vrow + RPI * i) * sv + 8 * vch) * 2));
-        f32x4 rk4[4] = {{1.f, 1.f, 1.f, 1.f}, {1.f, 1.f, 1.f, 1.f}, {1.f, 1.f, 1.f, 1.f}, {1.f, 1.f, 1.f, 1.f}};
-        if constexpr (NORM) {
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            rk4[u] = __builtin_bit_cast(f32x4, buf_load16(rn, (uint32_t)(32 * kt + 8 * u + 4 * g) * 4));
-        }
-#pragma unroll
-        for (int i = 0; i < VL; ++i) *reinterpret_cast<u32x4*>(ktl + (vrow + RPI * i) * KS + 8 * vch) = kr[i];
-        wave_lds_sync();
-        f32x16 S = {};
-        const bf16* kp = ktl + n32 * KS + 8 * g;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) S = PolBF16::mma(*reinterpret_cast<const bf16x8*>(kp + 16 * t), Q[t], S);
-#pragma unroll
-        for (int i = 0; i < VL; ++i) *reinterpret_cast<u32x4*>(vt + (vrow + RPI * i) * VS + 8 * vch) = vr[i];
-
-        // exact weights: keys after the query's position and padding keys past Nk are masked
-        // (only tiles reaching past the position of the tile's first row, or past Nk, have any)
-        const bool edge = 32 * kt + 31 > min(qoff + 32 * qt, Nk - 1);
-        f32x16 C;
-        bool pos_any = false;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int r = 4 * u + e;
-            const float x = __builtin_fmaf(NORM ? S[r] * rk4[u][e] : S[r], rq, -tau);
-            const int key = 32 * kt + crow(r, g);
-            const bool pos = (!edge || (key <= pq && key < Nk)) && x > 0.f;
-            C[r] = pos ? coef * pow_p<PK>(x, pw) : 0.f;
-            pos_any |= pos;
-            if (pent) {
-              // list entry of each non-zero weight, in the order (value r, lane)
-              const bool hit = valid && pos;
-              const uint64_t bal = wave_ballot(hit);
-              const uint32_t slot = npairs + __builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32),
-                                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-              if (hit && slot < (uint32_t)kPairCap)
-                *reinterpret_cast<u32x4*>(pent + 4 * slot) = u32x4{(uint32_t)key, (uint32_t)n32, __builtin_bit_cast(uint32_t, x), kNoSlot};
-              npairs += (uint32_t)__builtin_popcountll(bal);
-            }
-          }
-        if (wave_ballot(valid && pos_any) == 0ull) {
-          keep &= ~(1u << (kt & 31));
-          continue;
-        }
-        // pairs of the tile pass are in no column bucket: the key-major backward walks the lists
-        if (P.colcnt && l == 0) atomicOr(P.colcnt + (int64_t)bh * P.nkt + kt, kColTaint);
-        ++computed;
-        const bf16x8 PF0 = PolBF16::pack_c(C, 0), PF1 = PolBF16::pack_c(C, 1);
-        wave_lds_sync();
-        const bf16* vp = vt + voff;
-#pragma unroll
-        for (int c = 0; c < ND; ++c) {
-          O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c), PF0, O[c]);
-          O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c + 16 * VS), PF1, O[c]);
-        }
-        wave_lds_sync();
-      }
-      if (keep != bits0 && l == 0) orow[w] = keep;
-    }
-    if (pent && l == 0) P.pairs[pair_lists(P.nbr, BH, nqt) * 4 * kPairCap + lidx] = npairs;
-  }
-
-  // Output rows through LDS (the K tile buffer): lane (n, g) holds elements 32c + crow(r, g) of
-  // row n; stores then cover whole rows, 16 bytes per lane.
-  wave_lds_sync();
-#pragma unroll
-  for (int c = 0; c < ND; ++c)
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      store4(ktl + n32 * KS + 32 * c + 8 * u + 4 * g, O[c][4 * u], O[c][4 * u + 1], O[c][4 * u + 2], O[c][4 * u + 3]);
-  wave_lds_sync();
-  {
-    bf16* ohead = (bf16*)P.out + (int64_t)b * P.s[F_OUT][0] + (int64_t)h * P.s[F_OUT][1];
-#pragma unroll
-    for (int i = 0; i < VL; ++i) {
-      const int r = vrow + RPI * i, row = 32 * qt + r;
-      if (row < Nq)
-        __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(ktl + r * KS + 8 * vch),
-                                    reinterpret_cast<u32x4*>(ohead + (int64_t)row * P.s[F_OUT][2] + 8 * vch));
-    }
-  }
-  if (P.stats && l == 0 && checked) {
-    atomicAdd(P.stats + 1, (unsigned long long)computed);
-    atomicAdd(P.stats + 2, (unsigned long long)checked);
-  }
-}
-
-// Query tile of tile-pass item `item`: one head's query tiles consecutive on one XCD (when the
-// heads fill the eight XCDs), longest (last query tile) first.
-__device__ __forceinline__ void pv_item(int item, int BH, int nqt, int& bh, int& qt) {
-  if (BH % 8 == 0) {
-    const int x = item & 7, j = item >> 3;
-    bh = x + 8 * (j / nqt);
-    qt = nqt - 1 - j % nqt;
-  } else {
-    bh = item / nqt;
-    qt = nqt - 1 - item % nqt;
-  }
-}
-
-// One wave per workgroup and `per_wave` consecutive items per wave: the work per query tile
-// varies with its number of non-zero tiles, and single-wave workgroups retire independently.
-// With candidate lists (normalised bf16) the items whose lists all fit belong to fwd_pv_cand:
-// the wave tests its items' counts in one lane-parallel round and runs only the others, so a
-// launch where every list fits costs a few waves per SIMD (per_wave 4) instead of one per
-// query tile; without lists every item runs (per_wave 1).
-// With the candidate pass's queue (per_wave 0), the waves take the queued query tiles in turn.
-template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) fwd_pv(FwdParams P, int per_wave) {
-  constexpr int VS = D + 32, KS = D + 8;
-  __shared__ __attribute__((aligned(16))) bf16 vst[32 * VS];
-  __shared__ __attribute__((aligned(16))) bf16 kst[32 * KS];
-  const int l = lane_id();
-  const int BH = P.B * P.H, nqt = P.nqt, n = BH * nqt;
-  if (per_wave == 0) {
-    const uint32_t queued = P.pvq[0];
-    for (uint32_t k = blockIdx.x; k < queued; k += gridDim.x) {
-      const int v = (int)P.pvq[1 + k];
-      fwd_pv_tile<D, BR, PK, NORM>(P, vst, kst, v / nqt, v % nqt);
-    }
-    return;
-  }
-  const int first = (int)blockIdx.x * per_wave;
-  bool need = false;
-  if (l < per_wave && first + l < n) {
-    int bh, qt;
-    pv_item(first + l, BH, nqt, bh, qt);
-    need = true;
-    if (NORM && P.cand) {
-      const uint32_t* counts = P.cand + pair_lists(BR, BH, nqt) * kCandCap;
-      bool fit = true;
-#pragma unroll
-      for (int br = 0; br < BR; ++br) fit = fit && counts[((int64_t)br * BH + bh) * nqt + qt] <= (uint32_t)kCandCap;
-      need = !fit;
-    }
-  }
-  for (uint64_t m = wave_ballot(need); m; m &= m - 1ull) {
-    int bh, qt;
-    pv_item(first + __builtin_ctzll(m), BH, nqt, bh, qt);
-    fwd_pv_tile<D, BR, PK, NORM>(P, vst, kst, bh, qt);
-  }
-}
-
 // ------------------------------------------------------------------ fwd_pv_blk
-// The tile pass of the forwards without candidate lists (every query tile runs), over kBlkTiles
-// consecutive query tiles of one head, one wave each.  The waves walk the union of their bitmask
-// rows' kept key tiles in step and share each key tile's K and V rows (and key norms): the
-// workgroup loads them once, each wave a quarter of the rows, one tile ahead into registers,
-// then into a two-stage LDS ring (one barrier per tile: a stage is rewritten two tiles after it
-// was read, and every wave has passed the barrier between).  A wave computes only the tiles its
-// own row keeps, exactly as fwd_pv_tile does (the same MFMA sequence on the same operands: the
-// same rows, bitmask rewrite, pair lists and counters).  Once a pair list has passed its cap
-// the wave only counts its non-zero weights (one wave sum at the end) instead of placing them.
-// WALK (no screen ran before it): every causal key tile of a row counts as kept, the row's
-// bitmask words are all written (the words past its last key tile as zeros) and the causal
-// tiles are counted into stats[0].  ZR (with WALK): the workgroup then clears its even share of
-// the call's zero range.  K and V tiles load through one descriptor per head at a per-tile
-// offset when the head's offsets fit 31 bits, else through one descriptor per tile.
+// The tile pass, over kBlkTiles consecutive query tiles of one head, one wave each.  The waves
+// walk the union of their bitmask rows' kept key tiles in step and share each key tile's K and V
+// rows (and key norms): the workgroup loads them once, each wave a quarter of the rows, one tile
+// ahead into registers, then into a two-stage LDS ring (one barrier per tile: a stage is rewritten
+// two tiles after it was read, and every wave has passed the barrier between).  A wave computes
+// only the tiles its own row keeps.  Once a pair list has passed its cap the wave only counts its
+// non-zero weights (one wave sum at the end) instead of placing them.  K and V tiles load through
+// one descriptor per head at a per-tile offset when the head's offsets fit 31 bits, else through
+// one descriptor per tile.
+// Without normalisation (no screen ran before it) every query tile runs and every causal key tile
+// of a row counts as kept; the row's bitmask words are all written (the words past its last key
+// tile as zeros) and the causal tiles are counted into stats[0].  ZR: the workgroup then clears
+// its even share of the call's zero range.
+// With normalisation it takes the query tiles whose candidate lists overflowed (a count past
+// kCandCap in some branch; fwd_pv_cand took the others): a workgroup with none of them leaves
+// after one round of loads, a wave whose own lists fit only helps to load.  At a threshold scale
+// of 0.5 nearly every list overflows and a third of the kept tiles' weights are zero: bound by the
+// per-element work of the weights (TDA (2, 16, 1500, 64), beta 0.5: 237 us with one wave per query
+// tile, 109 us so); with every list fitting the launch costs 5.1 us.
 constexpr int kBlkTiles = 4;
 
-template <int D, int BR, int PK, bool NORM, bool WALK = false, bool ZR = false>
+template <int D, int BR, int PK, bool NORM, bool ZR = false>
 __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2))) fwd_pv_blk(FwdParams P) {
-  static_assert(!ZR || WALK, "the zero range is cleared by the walk");
+  static_assert(!ZR || !NORM, "with normalisation the screen clears the zero range");
+  constexpr bool WALK = !NORM;
   constexpr int W = kBlkTiles;
   constexpr int NT = D / 16, ND = D / 32;
   constexpr int VS = D + 32;     // LDS row stride of a V tile: conflict-free transpose reads
@@ -1026,10 +802,20 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
       jb = nqb - 1 - bid / BH;
     }
   }
+  // the block's query tiles this pass takes (the same for every wave)
+  uint32_t needm = nqt - W * jb >= W ? (1u << W) - 1u : (1u << (nqt - W * jb)) - 1u;
+  if constexpr (NORM) {
+    const uint32_t* counts = P.cand + pair_lists(BR, BH, nqt) * kCandCap + (int64_t)bh * nqt + W * jb;
+    bool ovf = false;  // lane r of a branch's W lanes: query tile r's list overflowed
+    if (l < BR * W && W * jb + l % W < nqt) ovf = counts[(int64_t)(l / W) * BH * nqt + l % W] > (uint32_t)kCandCap;
+    const uint64_t m = wave_ballot(ovf);
+    needm = (uint32_t)(BR == 2 ? m | (m >> W) : m) & ((1u << W) - 1u);
+    if (!needm) return;
+  }
   const int b = bh / P.H, h = bh % P.H;
   const int qt = W * jb + wv;
-  const bool act = qt < nqt;  // wave-uniform: waves past the last query tile only load
-  const int qtc = act ? qt : nqt - 1;
+  const bool act = (needm >> wv) & 1u;  // wave-uniform: the other waves only load
+  const int qtc = min(qt, nqt - 1);
   const int iq = 32 * qt + n32;
   const bool valid = act && iq < Nq;
   const bool rowpad = 32 * qt + 31 >= Nq;  // the query tile has rows past Nq (uniform)
@@ -1078,9 +864,8 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
 
     // word w of row r of the block, masked to the key tiles the row sees (uniform)
     auto row_word = [&](int r, int w) -> uint32_t {
-      const int q = W * jb + r;
-      if (q >= nqt) return 0u;
-      const int kl = kt_last(q, qoff, P.nkt);
+      if (!((needm >> r) & 1u)) return 0u;
+      const int kl = kt_last(W * jb + r, qoff, P.nkt);
       if (w > (kl >> 5)) return 0u;
       uint32_t x = WALK ? 0xffffffffu : (uint32_t)__builtin_amdgcn_readfirstlane((int)orow0[(int64_t)r * P.occ_w + w]);
       if (w == (kl >> 5) && (kl & 31) != 31) x &= (2u << (kl & 31)) - 1u;
@@ -1183,15 +968,20 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
         // weights coef relu(x)^p and the lane's largest x (some weight of the tile is non-zero
         // iff a lane's is > 0), on the bits: a float is > 0 iff its bits as an int32 are, so the
         // integer max(bits, 0) is relu(x) (no NaN handling to pay for in float max); p other than
-        // 1, 2 select on x > 0.  (Whole-vector bit casts: hipcc compiled a bit cast of one
-        // element of an ext_vector to element 0.)
+        // 1, 2 select on x > 0.  With normalisation a NaN score (a non-finite row) has no weight:
+        // the float max takes it to 0 first.  (Whole-vector bit casts: hipcc compiled a bit cast
+        // of one element of an ext_vector to element 0.)
         typedef int i32x16 __attribute__((ext_vector_type(16)));
+        if constexpr (NORM) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) X[r] = fmaxf(X[r], 0.f);
+        }
         const i32x16 XB = __builtin_bit_cast(i32x16, X);
         i32x16 TB;
         int xmb = XB[0];
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          TB[r] = max(XB[r], 0);
+          TB[r] = NORM ? XB[r] : max(XB[r], 0);
           if (r) xmb = max(xmb, XB[r]);
         }
         const f32x16 T = __builtin_bit_cast(f32x16, TB);
@@ -1356,10 +1146,7 @@ __global__ void __launch_bounds__(64 * BR) __attribute__((amdgpu_waves_per_eu(3)
   bool fit = true;
 #pragma unroll
   for (int br = 0; br < BR; ++br) fit = fit && nc[br] <= (uint32_t)kCandCap;
-  if (!fit) {  // fwd_pv walks the bitmask tiles (both waves leave: the test is the same)
-    if (l == 0 && wv == 0) P.pvq[1 + atomicAdd(P.pvq, 1u)] = (uint32_t)(bh * nqt + qt);
-    return;
-  }
+  if (!fit) return;  // fwd_pv_blk walks the bitmask tiles (both waves leave: the test is the same)
   if (P.screen_items > (Nq + 255) / 256) {
     // the screen split some key ranges over several items, which append in any order: sort each
     // list (lanes 0-31: branch 0, lanes 32-63: branch 1; its keys are distinct) by rank
@@ -1603,9 +1390,9 @@ int launch_sparse_t(const FwdParams& p, hipStream_t s) {
     const unsigned blocks = (unsigned)(BH * ((p.nqt + kBlkTiles - 1) / kBlkTiles));
     const bool zr = p.zero && p.zero_units > 0 && p.zero_units <= (int64_t)blocks * 65536;
     if (zr)
-      hipLaunchKernelGGL((fwd_pv_blk<D, BR, PK, NORM, true, true>), dim3(blocks), dim3(64 * kBlkTiles), 0, s, p);
-    else
       hipLaunchKernelGGL((fwd_pv_blk<D, BR, PK, NORM, true>), dim3(blocks), dim3(64 * kBlkTiles), 0, s, p);
+    else
+      hipLaunchKernelGGL((fwd_pv_blk<D, BR, PK, NORM>), dim3(blocks), dim3(64 * kBlkTiles), 0, s, p);
     launched(s, "fwd_pv");
     const int e = (int)hipGetLastError();
     return e || zr ? e : launch_zero(p, s);
@@ -1613,16 +1400,11 @@ int launch_sparse_t(const FwdParams& p, hipStream_t s) {
     const dim3 grid((unsigned)(BR * BH) * (unsigned)p.screen_items);
     hipLaunchKernelGGL((fwd_screen_i8<D, bf16>), grid, dim3(256), 0, s, p, BR);
     launched(s, "fwd_screen");
-    if (p.cand) {
-      hipLaunchKernelGGL((fwd_pv_cand<D, BR, PK>), dim3((unsigned)(BH * p.nqt)), dim3(64 * BR), 0, s, p);
-      launched(s, "fwd_pv_cand");
-      // the query tiles the candidate pass could not take, from its queue
-      const int items = BH * p.nqt;
-      hipLaunchKernelGGL((fwd_pv<D, BR, PK, NORM>), dim3((unsigned)(items < 2048 ? items : 2048)), dim3(64), 0, s, p, 0);
-    } else {  // every query tile runs: blocks of query tiles sharing their key tiles
-      const unsigned blocks = (unsigned)(BH * ((p.nqt + kBlkTiles - 1) / kBlkTiles));
-      hipLaunchKernelGGL((fwd_pv_blk<D, BR, PK, NORM>), dim3(blocks), dim3(64 * kBlkTiles), 0, s, p);
-    }
+    hipLaunchKernelGGL((fwd_pv_cand<D, BR, PK>), dim3((unsigned)(BH * p.nqt)), dim3(64 * BR), 0, s, p);
+    launched(s, "fwd_pv_cand");
+    // the query tiles the candidate pass could not take
+    const unsigned blocks = (unsigned)(BH * ((p.nqt + kBlkTiles - 1) / kBlkTiles));
+    hipLaunchKernelGGL((fwd_pv_blk<D, BR, PK, NORM>), dim3(blocks), dim3(64 * kBlkTiles), 0, s, p);
     launched(s, "fwd_pv");
     return (int)hipGetLastError();
   }

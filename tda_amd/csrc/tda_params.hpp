@@ -86,8 +86,8 @@ struct FwdParams {
   uint32_t* colbuf;
   int nbr;                   // branches
   uint32_t* cand;            // candidate keys (workspace; null for a single query tile)
-  uint32_t* pvq;             // with cand: query tiles for the tile pass ([0] count, then bh nqt + qt),
-                             // zeroed by the screen, filled by the candidate pass (workspace)
+  uint32_t* pvq;             // with cand: query tiles for the fp32 tile pass ([0] count, then bh nqt +
+                             // qt), zeroed by key_prep, filled by the candidate pass (workspace)
   void* zero;                // may be null: 16-byte units [0, zero_units) the call sets to zero
   int64_t zero_units;
   int zero_per_it;           // units each screen workgroup clears per key tile it walks
@@ -119,9 +119,9 @@ struct BwdParams {
                              // the query-major pair pass, read by the key-major one
   const uint32_t* colcnt;    // may be null: the forward's column buckets (counts, entries; the
   uint32_t* colbuf;          // query-major pair pass writes each entry's dk weight)
-  uint32_t* dkvq;            // may be null: key tiles for the key-major tile pass ([0] count, then
-                             // items), zeroed by the query-major pair pass, filled by the key-major
-                             // pair pass (workspace)
+  uint32_t* dkvq;            // may be null: queue of the tile passes (workspace), zeroed by the
+                             // query-major pair pass, filled by the key-major one: bf16 blocks of
+                             // tiles (tda_bwd_fast.hip), fp32 key tiles ([0] count, then items)
   int grads_zeroed;          // the gradient rows hold zeros: the pair passes store named rows only
 };
 

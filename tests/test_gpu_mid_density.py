@@ -1,0 +1,74 @@
+"""Normalised calls whose threshold scale lets a few per cent of the weights through: the candidate
+and pair lists overflow, so the tile passes (fwd_pv_blk after the screen; bwd_tiles over the queue
+of blocks, or bwd_dq_blk and bwd_dkv_blk without a queue) take most query and key tiles, beside
+some that still fit.  Output and every gradient against the fp64 oracle."""
+import pytest
+import torch
+
+import tda_amd
+from oracle.formula import rel_err, tda_grads
+from tda_amd import ops
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-2  # bf16 weights, results and gradients (2^-9 each) in sums of up to a few hundred terms
+
+
+def _inputs(b, h, nq, nk, d, br, dtype, seed):
+    g = torch.Generator("cpu").manual_seed(seed)
+    mk = lambda n: torch.randn((b, h, n, d), generator=g).to(dtype)  # noqa: E731
+    return [mk(nq) for _ in range(br)] + [mk(nk) for _ in range(br + 1)], mk(nq)
+
+
+@pytest.mark.parametrize("nq,nk,d,br,p,beta", [
+    (33, 33, 64, 2, 2.0, 0.0),       # two query tiles, a partial block, every causal weight sign
+    (128, 128, 128, 2, 2.0, 0.5),    # exactly one block of tiles
+    (129, 129, 64, 1, 1.0, 0.4),     # a block of one tile with one row
+    (300, 300, 64, 2, 1.5, 0.6),     # lists that fit beside lists that do not
+    (520, 520, 128, 1, 2.0, 0.5),
+    (100, 700, 64, 2, 2.0, 0.5),     # fewer query tiles than key tiles (a key cache)
+    (200, 90, 128, 2, 3.0, 0.4),     # fewer key tiles than query tiles
+    (33, 4200, 64, 2, 2.0, 0.5),     # more key tiles than the queue holds: no queue
+])
+def test_overflowing_lists_against_the_oracle(nq, nk, d, br, p, beta):
+    off = max(nk - nq, 0)
+    rows, do = _inputs(1, 3, nq, nk, d, br, torch.bfloat16, 31)
+    leaves = [x.cuda().requires_grad_(True) for x in rows]
+    bt = torch.tensor(beta, device="cuda", requires_grad=True)
+    lt = torch.tensor(0.4, device="cuda", requires_grad=True)
+    if br == 2:
+        out = tda_amd.differential_threshold_rela_triton(*leaves, bt, lt, relu_power=p, normalize=True)
+        q1, q2, k1, k2, v = (x.double() for x in rows)
+    else:
+        out = tda_amd.threshold_rela_triton(*leaves, bt, relu_power=p, normalize=True)
+        (q1, k1, v), q2, k2 = (x.double() for x in rows), None, None
+    out.backward(do.cuda())
+    ref = tda_grads(q1, q2, k1, k2, v, do.double(), beta, 0.4 if br == 2 else 0.0, p, True, br, q_offset=off)
+    assert rel_err(out, ref["out"]) <= TOL
+    names = ["dq1", "dq2", "dk1", "dk2", "dv"] if br == 2 else ["dq1", "dk1", "dv"]
+    for leaf, name in zip(leaves, names):
+        assert rel_err(leaf.grad, ref[name]) <= TOL, name
+    # the scalars are sums of terms of both signs, each with the rounding of bf16 products' inputs only
+    assert abs(bt.grad.item() - ref["dbeta"].item()) <= 1e-3 * abs(ref["dbeta"].item()) + 1e-5
+
+
+@pytest.mark.parametrize("d,br", [(64, 2), (128, 1)])
+def test_queue_and_direct_launches_agree(d, br):
+    """The backward from pair lists and a queue, and from the bitmask alone, give the same block
+    sums for what both compute with the tile passes (bf16 rounding of dS apart in the rest)."""
+    rows, do = _inputs(2, 2, 400, 400, d, br, torch.bfloat16, 32)
+    xs = [x.cuda() for x in rows]
+    do = do.cuda()
+    q1, q2, k1, k2, v = xs if br == 2 else (xs[0], None, xs[1], None, xs[2])
+    beta, lam = torch.tensor(0.3, device="cuda"), torch.tensor(0.5, device="cuda") if br == 2 else None
+    norms, occ = ops.side_buffers(q1.shape, br, True, "cuda")
+    pairs = ops.pair_buffer(q1.shape, br, "cuda")
+    with torch.no_grad():
+        ops.forward(q1, k1, q2, k2, v, beta, lam, 2.0, True, br, norms, occ, pairs=pairs)
+        a = ops.backward(q1, k1, q2, k2, v, do, beta, lam, 2.0, True, br, norms, occ, pairs=pairs)
+        again = ops.backward(q1, k1, q2, k2, v, do, beta, lam, 2.0, True, br, norms, occ, pairs=pairs)
+        b = ops.backward(q1, k1, q2, k2, v, do, beta, lam, 2.0, True, br, norms, occ)
+    for x, y, z in zip(a, again, b):
+        if x is None:
+            continue
+        assert torch.equal(x, y)  # whatever order the queue was filled in
+        assert rel_err(x, z.double().cpu()) <= TOL
