@@ -173,7 +173,7 @@ class ThresholdRelaFunction(torch.autograd.Function):
             _, occ = ops.side_buffers(qc.shape, 1, False, qc.device, kc.shape[2])
             if cdt == torch.bfloat16:
                 pairs = ops.pair_buffer(qc.shape, 1, qc.device)
-                if all(ctx.needs_input_grad[:3]) and ops.grad_prealloc_enabled():
+                if all(ctx.needs_input_grad[:3]) and dk <= 128 and ops.grad_prealloc_enabled():
                     gbuf, grads = ops.grad_buffers(qc, kc, None, None, vc, 1)
         out = ops.forward(qc, kc, None, None, vc, beta_t, None, p, False, 1, None, occ, q_offset=off,
                           pairs=pairs, zero=gbuf)

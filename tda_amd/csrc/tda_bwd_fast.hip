@@ -70,55 +70,52 @@ __device__ __forceinline__ void crow_vals(const float* tab, float (&v)[16]) {
   }
 }
 
-// This lane's elements of an input row in the transposed C layout of a gradient tile
+// This lane's elements of NC input columns in the transposed C layout of a gradient tile
 // (elements 32c + 8u + 4g .. +3), for the F.normalize backward.
-template <int D>
+template <int NC>
 struct GradRow {
-  bf16x4 x[D / 32][4];
+  bf16x4 x[NC / 32][4];
 };
-template <int D>
-__device__ __forceinline__ void load_grad_row(const bf16* xrow, GradRow<D>& r) {
+template <int NC>
+__device__ __forceinline__ void load_grad_row(const bf16* xrow, GradRow<NC>& r) {
   const int g = lane_id() >> 5;
 #pragma unroll
-  for (int c = 0; c < D / 32; ++c)
+  for (int c = 0; c < NC / 32; ++c)
 #pragma unroll
     for (int u = 0; u < 4; ++u) r.x[c][u] = *reinterpret_cast<const bf16x4*>(xrow + 32 * c + 8 * u + 4 * g);
 }
 
-// Apply the F.normalize backward to a gradient tile in the transposed C layout (lane = row,
-// value r of column block c = element 32c + crow(r, g)) and store it (see finish_rows in
-// tda_bwd.hip; same arithmetic).  xr: the input row (NORM only).
-template <int D, bool NORM>
-__device__ __forceinline__ void store_grad_rows(const f32x16 (&acc)[D / 32], const GradRow<D>& xr, bf16* grow,
-                                                float rinv) {
-  constexpr int ND = D / 32;
-  const int g = lane_id() >> 5;
+// The row dot x^ . acc over the NC columns of a gradient tile in the transposed C layout (lane =
+// row, value r of column block c = element 32c + crow(r, g)), the same in both lanes of the row.
+template <int NC>
+__device__ __forceinline__ float grad_row_dot(const f32x16 (&acc)[NC / 32], const GradRow<NC>& xr, float rinv) {
   float dot = 0.f;
-  f32x4 xh[ND][4];
-  if constexpr (NORM) {
 #pragma unroll
-    for (int c = 0; c < ND; ++c)
+  for (int c = 0; c < NC / 32; ++c)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          xh[c][u][e] = (float)xr.x[c][u][e] * rinv;
-          dot = __builtin_fmaf(xh[c][u][e], acc[c][4 * u + e], dot);
-        }
-      }
-    dot += __shfl_xor(dot, 32);
-  }
+      for (int e = 0; e < 4; ++e) dot = __builtin_fmaf((float)xr.x[c][u][e] * rinv, acc[c][4 * u + e], dot);
+  return dot + __shfl_xor(dot, 32);
+}
+// Apply the F.normalize backward (see finish_rows in tda_bwd.hip) to scale times the tile and store
+// it; xr, rinv, dot: the input row, its inverse norm and the whole row's x^ . acc (NORM only).
+template <int NC, bool NORM>
+__device__ __forceinline__ void store_grad_rows(const f32x16 (&acc)[NC / 32], const GradRow<NC>& xr, bf16* grow,
+                                                float rinv, float dot, float scale) {
+  const int g = lane_id() >> 5;
   const bool clamped = NORM && rinv >= 1.0f / kNormEps;
+  const float rs = rinv * scale;
 #pragma unroll
-  for (int c = 0; c < ND; ++c)
+  for (int c = 0; c < NC / 32; ++c)
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       float o[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const float a = acc[c][4 * u + e];
-        if constexpr (NORM) o[e] = clamped ? a * rinv : (a - xh[c][u][e] * dot) * rinv;
-        else o[e] = a;
+        if constexpr (NORM) o[e] = clamped ? a * rs : (a - (float)xr.x[c][u][e] * rinv * dot) * rs;
+        else o[e] = a * scale;
       }
       store4(grow + 32 * c + 8 * u + 4 * g, o[0], o[1], o[2], o[3]);
     }
@@ -446,17 +443,14 @@ struct ColEntry {
   float wk;    // dk weight from the query-major pair pass
 };
 
-// Query block k of the queue, numbered from the last query tiles (the longest rows) of every (head,
-// branch): the list count of its tile `lane` (0 past the block).
+// Query block j of a head's BR ceil(nqt / kBwdBlk), from the last query tiles (the longest rows), the
+// branches adjacent: the list count of its tile `lane` (0 past the block).
 template <int BR>
-__device__ __forceinline__ uint32_t query_block_count(const BwdParams& P, const uint32_t* counts, int64_t k) {
-  const int BH = P.B * P.H, nqt = P.nqt, l = lane_id();
-  const int nqb = (nqt + kBwdBlk - 1) / kBwdBlk;
-  if (k >= (int64_t)BR * BH * nqb) return 0u;
-  const int jb = nqb - 1 - (int)(k / (BR * BH)), rem = (int)(k % (BR * BH));
-  const int br = BR == 2 ? rem & 1 : 0, bh = BR == 2 ? rem >> 1 : rem;
-  const int qt = kBwdBlk * jb + l;
-  return l < kBwdBlk && qt < nqt ? counts[((int64_t)br * BH + bh) * nqt + qt] : 0u;
+__device__ __forceinline__ uint32_t query_block_count(const BwdParams& P, const uint32_t* counts, int bh, int j) {
+  const int nqt = P.nqt, l = lane_id(), nqb = (nqt + kBwdBlk - 1) / kBwdBlk;
+  if (j >= BR * nqb) return 0u;
+  const int br = BR == 2 ? j & 1 : 0, qt = kBwdBlk * (nqb - 1 - (BR == 2 ? j >> 1 : j)) + l;
+  return l < kBwdBlk && qt < nqt ? counts[((int64_t)br * (P.B * P.H) + bh) * nqt + qt] : 0u;
 }
 
 // One wave per key tile whose column has only lists that fit.  Its pairs come from the column's
@@ -497,11 +491,11 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
   const float pw = P.p;
   float lam = 0.f;
   if constexpr (BR == 2) lam = clamp01(*P.lam);
-  // query block `item` (and every B H nkt-th after it) goes to the tile-pass queue when one of its
-  // tiles' lists did not fit; its counts are loaded here and tested once the bucket has arrived
+  // query block kt of the head (and every nkt-th after it) goes to the tile-pass queue when one of
+  // its tiles' lists did not fit; its counts are loaded here and tested once the bucket has arrived
   const bool queue = sizeof(T) == 2 && NORM && P.dkvq;
   uint32_t qcount = 0u;
-  if (queue) qcount = query_block_count<BR>(P, counts, item);
+  if (queue) qcount = query_block_count<BR>(P, counts, bh, kt);
 
   // Walk the column's lists in the order (query-tile chunk of 64, branch, query tile): the
   // bitmask bits and counts of 128 query tiles per load round, then 2 kWalkRounds lists per
@@ -628,12 +622,13 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
   }
 
   if (queue) {
-    const int64_t nkb = (int64_t)BH * ((P.nkt + kBwdBlk - 1) / kBwdBlk);
-    const int64_t nb = (int64_t)BR * BH * ((P.nqt + kBwdBlk - 1) / kBwdBlk), step = (int64_t)BH * P.nkt;
-    for (int64_t k = item; k < nb; k += step) {
-      if (k != item) qcount = query_block_count<BR>(P, counts, k);
-      if (wave_ballot(qcount > (uint32_t)kPairCap) != 0ull && l == 0)
-        P.dkvq[kTileqHead + 2 * nkb + atomicAdd(P.dkvq + 1, 1u)] = (uint32_t)k;
+    const int nb = BR * ((P.nqt + kBwdBlk - 1) / kBwdBlk);
+    for (int j = kt; j < nb; j += P.nkt) {
+      if (j != kt) qcount = query_block_count<BR>(P, counts, bh, j);
+      if (wave_ballot(qcount > (uint32_t)kPairCap) != 0ull && l == 0) {
+        const int64_t nkb = (int64_t)BH * ((P.nkt + kBwdBlk - 1) / kBwdBlk);
+        P.dkvq[kTileqHead + 2 * nkb + atomicAdd(P.dkvq + 1, 1u)] = (uint32_t)(bh * nb + j);
+      }
     }
   }
 
@@ -871,9 +866,41 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
 // ------------------------------------------------------------------ block tile passes
 // kBwdBlk consecutive tiles of one head per workgroup, one wave each, walking the union of their
 // bitmask tiles in step; each streamed tile's rows are loaded once per workgroup (each wave a
-// quarter, one tile ahead into registers) into a two-stage LDS ring of chunk-swizzled tiles
+// quarter, one or two tiles ahead into registers) into a two-stage LDS ring of chunk-swizzled tiles
 // (tile_row_frag / tile_tr_frag read them), one fence-free barrier per tile.  A wave computes only
-// its own tiles, the masks branch-free and only on the tiles that need them.
+// its own tiles, the masks branch-free and only on the tiles that need them.  The per-element work
+// sets the pace, so what is the same for a whole branch stays out of it: dS = coef p x^(p-1) dP is
+// accumulated without coef and, at p = 2, without the factor 2 (ds_scale times it, exactly, in
+// the epilogue and in the dbeta sum), and the branch that counts -lambda in dv runs first, its sum
+// scaled before the other's is added.
+// At d = 256 a tile's row fragments and accumulators do not fit one wave's registers, so two waves
+// share each tile (kSplit): each contracts its half of the d elements of the scores and of dP, adds
+// the other's half through LDS (the same sums in both, so the same decisions) and owns its half of
+// the gradient columns; the normalize backward's row dots are added the same way.
+// TDA (2, 8, 1000, 256): 47 + 107 us against 113 + 224 with two waves per tile fetching their own rows.
+// The split key-major blocks hold two tiles, four waves with a SIMD each (four tiles, two waves per
+// SIMD, spill 76-195 VGPRs).
+template <int D>
+constexpr int kSplit = D > 128 ? 2 : 1;
+template <int D>
+constexpr int kKeyBlk = D > 128 ? 2 : kBwdBlk;
+template <int D>
+constexpr int kQryThreads = 64 * kBwdBlk * kSplit<D>;
+template <int D>
+constexpr int kKeyThreads = 64 * kKeyBlk<D> * kSplit<D>;
+
+// The partial values of a tile's two waves added through LDS: give writes the wave's, take (after
+// a barrier) returns half 0's plus half 1's.
+__device__ __forceinline__ void give16(float (*x)[64], const f32x16& v) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) x[r][lane_id()] = v[r];
+}
+__device__ __forceinline__ f32x16 take16(const float (*other)[64], const f32x16& v) {
+  f32x16 o;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) o[r] = v[r] + other[r][lane_id()];
+  return o;
+}
 
 // max(x, 0) of 16 values on their bits: a float is > 0 iff its bits as an int32 are.
 __device__ __forceinline__ f32x16 relu_bits(const f32x16& x) {
@@ -892,11 +919,12 @@ __device__ __forceinline__ f32x16 relu16(f32x16 x) {
   return x;
 }
 
-// This wave's share of a 32-row tile of D columns: rows RPI (LPW wv + i) + l / CH, chunk l % CH.
-template <int D>
+// This wave's share (of NW waves) of a 32-row tile of D columns: rows RPI (LPW wv + i) + l / CH,
+// chunk l % CH.
+template <int D, int NW>
 struct BlkRows {
-  static constexpr int CH = D / 8, RPI = 64 / CH, LPW = 32 / RPI / kBwdBlk;
-  static_assert(LPW >= 1 && LPW * RPI * kBwdBlk == 32, "tile rows split evenly over the waves");
+  static constexpr int CH = D / 8, RPI = 64 / CH, LPW = 32 / RPI / NW;
+  static_assert(LPW >= 1 && LPW * RPI * NW == 32, "tile rows split evenly over the waves");
   u32x4 v[LPW];
   __device__ __forceinline__ void load(const bf16* rows, int64_t st, int r0, int n, int wv) {
     const int l = lane_id();
@@ -920,18 +948,33 @@ struct BlkRows {
 
 // Query-major: kBwdBlk query tiles of one (branch, head), streaming K, V and the key norms.  The
 // block takes its tiles whose lists did not fit (or all, without lists).
-template <int D>
-struct DqBlkLds {
-  bf16 ring[2 * 2 * 32 * D];  // two stages of a K tile and a V tile
-  float norms[2][32];
+//
+// The block functions' LDS, arrays of the kernel.
+template <int D, int W>
+struct BlkLds {
+  bf16* ring;             // two stages of two tiles of D columns
+  float (*vals)[2][32];   // [stage]: key norms; query norms and tau values
+  bf16 (*rows)[32 * D];   // key-major, one wave per tile: each wave's key rows (swizzled)
+  float (*xch)[32][64];   // a split tile's waves: partial scores and dP
+  float (*dots)[2][32];   // and row dots
 };
+// Their declaration: W tiles; ROWS as above.
+#define TDA_BLK_LDS(D, W, ROWS)                                                               \
+  __shared__ __attribute__((aligned(16))) bf16 lds_ring[2 * 2 * 32 * D];                      \
+  __shared__ __attribute__((aligned(16))) float lds_vals[2][2][32];                           \
+  __shared__ __attribute__((aligned(16))) bf16 lds_rows[(ROWS) && kSplit<D> == 1 ? W : 1][(ROWS) && kSplit<D> == 1 ? 32 * D : 8]; \
+  __shared__ __attribute__((aligned(16))) float lds_xch[kSplit<D> == 2 ? 2 * W : 1][kSplit<D> == 2 ? 32 * 64 : 4]; \
+  __shared__ float lds_dots[W][kSplit<D> == 2 ? 64 : 1];                                      \
+  const BlkLds<D, W> L{lds_ring, lds_vals, reinterpret_cast<bf16(*)[32 * D]>(&lds_rows[0][0]),             \
+                       reinterpret_cast<float(*)[32][64]>(&lds_xch[0][0]), reinterpret_cast<float(*)[2][32]>(&lds_dots[0][0])}
 template <int D, int BR, int PK, bool NORM>
-__device__ __forceinline__ void dq_block(const BwdParams& P, DqBlkLds<D>& L, int jb, int br, int bh) {
-  constexpr int W = kBwdBlk, NT = D / 16, ND = D / 32;
+__device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBwdBlk>& L, int jb, int br, int bh) {
+  constexpr int W = kBwdBlk, SP = kSplit<D>, NT = D / 16 / SP, ND = D / 32 / SP;
   constexpr int STAGE = 2 * 32 * D;  // K tile, V tile
   bf16* ring = L.ring;
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
-  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wv = wid / SP, hh = wid % SP;  // the wave's tile of the block, its half of d and of the columns
   const int BH = P.B * P.H, nqt = P.nqt, Nq = P.Nq, Nk = P.Nk, qoff = P.qoff;
   const int b = bh / P.H, h = bh % P.H;
   const uint32_t* counts = P.pairs ? P.pairs + pair_lists(BR, BH, nqt) * 4 * kPairCap : nullptr;
@@ -963,8 +1006,8 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, DqBlkLds<D>& L, int
     const bf16* rq_ = base(qslot) + (int64_t)ic * P.s[qslot][2];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      DO[t] = *reinterpret_cast<const bf16x8*>(r + 16 * t + 8 * g);
-      Q[t] = *reinterpret_cast<const bf16x8*>(rq_ + 16 * t + 8 * g);
+      DO[t] = *reinterpret_cast<const bf16x8*>(r + 16 * (t + NT * hh) + 8 * g);
+      Q[t] = *reinterpret_cast<const bf16x8*>(rq_ + 16 * (t + NT * hh) + 8 * g);
     }
   }
   const float rq = NORM ? P.norms[norm_base(P, br == 0 ? N_Q1 : N_Q2, bh) + ic] : 1.f;
@@ -973,6 +1016,7 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, DqBlkLds<D>& L, int
   const float pw = P.p;
   float coef = 1.f;
   if constexpr (BR == 2) coef = br == 0 ? 1.f : -clamp01(*P.lam);
+  const float ds_scale = PK == 2 ? 2.f * coef : coef;
   const bool want_l = BR == 2 && br == 1;  // dlambda comes from branch 2 alone
   const bf16* vb = base(B_V);
   const int64_t sv = P.s[B_V][2];
@@ -980,7 +1024,9 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, DqBlkLds<D>& L, int
   const int64_t sk = P.s[kslot][2];
   const float* nk = nullptr;
   if constexpr (NORM) nk = P.norms + norm_base(P, br == 0 ? N_K1 : N_K2, bh);
-  float bsum = 0.f, lsum = 0.f;
+  // dbeta / dlambda sums: a tile's in fp32, over the tiles in fp64 (terms of both signs: the sums'
+  // own rounding was the larger part of the scalars' error)
+  double bsum = 0., lsum = 0.;
   unsigned visited = 0, computed = 0;
 
   f32x16 A[ND];
@@ -1018,41 +1064,46 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, DqBlkLds<D>& L, int
     own_out = sown;
     return kt;
   };
-  BlkRows<D> kr, vr;
-  f32x4 nr = {};
-  auto issue = [&](int kt) {
-    kr.load(kb, sk, 32 * kt, Nk, wv);
-    vr.load(vb, sv, 32 * kt, Nk, wv);
-    if (NORM && wv == 0 && l < 8)
-      nr = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+  constexpr int AHEAD = D <= 64 ? 2 : 1;  // tiles in flight past the one being worked on
+  struct Pre {  // a tile's share in flight: its rows and norms, index and the own row's word
+    BlkRows<D, W * SP> kr, vr;
+    f32x4 nr;
+    int kt;
+    uint32_t own;
+  };
+  auto fetch = [&](Pre& p) {
+    p.kt = next_tile(p.own);
+    const int kt = max(p.kt, 0);  // loads on every path: the waits then count them exactly
+    p.kr.load(kb, sk, 32 * kt, Nk, wid);
+    p.vr.load(vb, sv, 32 * kt, Nk, wid);
+    if (NORM && wid == 0 && l < 8)
+      p.nr = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
                                           rows_rsrc(nk + 32 * kt, (uint32_t)(min(32, Nk - 32 * kt) * 4)), 16u * (uint32_t)l, 0, 0));
   };
-  uint32_t cown = 0u;
-  int kt = next_tile(cown);
-  if (kt >= 0) issue(kt);
   int it = 0;
-  while (kt >= 0) {
+  auto step = [&](Pre& p) {
+    const int kt = p.kt;
+    const uint32_t cown = p.own;
     bf16* kst = ring + (it & 1) * STAGE;
     bf16* vst = kst + 32 * D;
-    float* nst = L.norms[it & 1];
-    kr.store(kst, wv);
-    vr.store(vst, wv);
-    if (NORM && wv == 0 && l < 8) *reinterpret_cast<f32x4*>(nst + 4 * l) = nr;
-    uint32_t nown = 0u;
-    const int kt2 = next_tile(nown);
-    if (kt2 >= 0) issue(kt2);  // in flight during this tile's work
+    float* nst = L.vals[it & 1][0];
+    p.kr.store(kst, wid);
+    p.vr.store(vst, wid);
+    if (NORM && wid == 0 && l < 8) *reinterpret_cast<f32x4*>(nst + 4 * l) = p.nr;
+    fetch(p);  // the tile AHEAD steps on, in flight during this tile's work
     lds_barrier();
     ++it;
-    if ((cown >> (kt & 31)) & 1u) {
+    auto products = [&](f32x16& S, f32x16& Dp) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        S = PolBF16::mma(tile_row_frag<D>(kst, t + NT * hh), Q[t], S);
+        Dp = PolBF16::mma(tile_row_frag<D>(vst, t + NT * hh), DO[t], Dp);
+      }
+    };
+    auto tile = [&](const f32x16& S, const f32x16& Dp) {
       ++visited;
       const int k0 = 32 * kt;
       bool anyw = true;  // without a bitmask the counters count the tiles with a weight
-      f32x16 S = f32x16{}, Dp = f32x16{};
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        S = PolBF16::mma(tile_row_frag<D>(kst, t), Q[t], S);
-        Dp = PolBF16::mma(tile_row_frag<D>(vst, t), DO[t], Dp);
-      }
       float rk[16];
       if constexpr (NORM) crow_vals(nst, rk);
       // exact x, branch-free; keys after the query's position, padding keys and rows past Nq
@@ -1068,28 +1119,31 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, DqBlkLds<D>& L, int
         for (int r = 0; r < 16; ++r) X[r] = 8 * (r >> 2) + (r & 3) <= lim ? X[r] : -1.f;
       }
       f32x16 E;
+      float bt = 0.f, lt = 0.f;
       if constexpr (PK == 2) {
         // relu on the bits (a float is > 0 iff its bits as an int32 are): t = max(x, 0) with no
-        // comparison per value; 2 t and t^2 vanish with t.  (Whole-vector bit casts: hipcc
+        // comparison per value; t and t^2 vanish with t.  (Whole-vector bit casts: hipcc
         // compiled a bit cast of one element of an ext_vector to element 0.)
         const f32x16 T = relu16<NORM>(X);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float ds = coef * (T[r] + T[r]) * Dp[r];
-          bsum += ds;
-          if (want_l) lsum = __builtin_fmaf(T[r] * T[r], Dp[r], lsum);
+          const float ds = T[r] * Dp[r];
+          bt += ds;
+          if (want_l) lt = __builtin_fmaf(T[r], ds, lt);
           E[r] = NORM ? ds * rk[r] : ds;
         }
       } else {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const bool pos = X[r] > 0.f;
-          const float ds = pos ? coef * dpow_p<PK>(X[r], pw) * Dp[r] : 0.f;
-          bsum += ds;
-          if (want_l) lsum = __builtin_fmaf(pos ? pow_p<PK>(X[r], pw) : 0.f, Dp[r], lsum);
+          const float ds = pos ? dpow_p<PK>(X[r], pw) * Dp[r] : 0.f;
+          bt += ds;
+          if (want_l) lt = __builtin_fmaf(pos ? pow_p<PK>(X[r], pw) : 0.f, Dp[r], lt);
           E[r] = NORM ? ds * rk[r] : ds;
         }
       }
+      bsum += (double)bt;
+      if (want_l) lsum += (double)lt;
       if (!P.occ) {
         float xm = X[0];
 #pragma unroll
@@ -1100,24 +1154,67 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, DqBlkLds<D>& L, int
       const bf16x8 E0 = PolBF16::pack_c(E, 0), E1 = PolBF16::pack_c(E, 1);
 #pragma unroll
       for (int c = 0; c < ND; ++c) {
-        A[c] = PolBF16::mma(tile_tr_frag<D>(kst, 0, c), E0, A[c]);
-        A[c] = PolBF16::mma(tile_tr_frag<D>(kst, 1, c), E1, A[c]);
+        A[c] = PolBF16::mma(tile_tr_frag<D>(kst, 0, c + ND * hh), E0, A[c]);
+        A[c] = PolBF16::mma(tile_tr_frag<D>(kst, 1, c + ND * hh), E1, A[c]);
       }
+    };
+    const bool own = (cown >> (kt & 31)) & 1u;
+    if constexpr (SP == 1) {
+      if (own) {
+        f32x16 S = f32x16{}, Dp = f32x16{};
+        products(S, Dp);
+        tile(S, Dp);
+      }
+    } else {  // the waves of a tile agree on `own`; every wave takes the barrier
+      f32x16 S = f32x16{}, Dp = f32x16{};
+      if (own) {
+        products(S, Dp);
+        give16(L.xch[wid], S);
+        give16(L.xch[wid] + 16, Dp);
+      }
+      lds_barrier();
+      if (own) tile(take16(L.xch[wid ^ 1], S), take16(L.xch[wid ^ 1] + 16, Dp));
     }
-    cown = nown;  // the own row's word of the next tile
-    kt = kt2;
+  };
+  Pre pa;
+  fetch(pa);
+  if constexpr (AHEAD == 2) {
+    Pre pb;
+    fetch(pb);
+    while (pa.kt >= 0) {
+      step(pa);
+      if (pb.kt < 0) break;
+      step(pb);
+    }
+  } else {
+    while (pa.kt >= 0) step(pa);
+  }
+  float dot = 0.f;  // the query row's x^ . dq^
+  if constexpr (NORM && SP == 2) {
+    if (need) {
+      GradRow<32 * ND> XR;
+      load_grad_row<32 * ND>(base(qslot) + (int64_t)ic * P.s[qslot][2] + 32 * ND * hh, XR);
+      dot = grad_row_dot<32 * ND>(A, XR, rq);
+    }
+    if (g == 0) L.dots[wv][hh][n32] = dot;
+    lds_barrier();
+    dot = L.dots[wv][0][n32] + L.dots[wv][1][n32];
   }
   if (!need) return;
   if (qvalid) {
-    GradRow<D> XR;  // the query row for the normalize backward
-    if constexpr (NORM) load_grad_row<D>(base(qslot) + (int64_t)ic * P.s[qslot][2], XR);
+    GradRow<32 * ND> XR;  // the query row's columns for the normalize backward
+    if constexpr (NORM) {
+      load_grad_row<32 * ND>(base(qslot) + (int64_t)ic * P.s[qslot][2] + 32 * ND * hh, XR);
+      if constexpr (SP == 1) dot = grad_row_dot<32 * ND>(A, XR, rq);
+    }
     const int gslot = br == 0 ? B_DQ1 : B_DQ2;
     bf16* grow = (bf16*)P.grad[br == 0 ? 0 : 2] + (int64_t)b * P.s[gslot][0] + (int64_t)h * P.s[gslot][1] +
-                 (int64_t)i * P.s[gslot][2];
-    store_grad_rows<D, NORM>(A, XR, grow, rq);
+                 (int64_t)i * P.s[gslot][2] + 32 * ND * hh;
+    store_grad_rows<32 * ND, NORM>(A, XR, grow, rq, dot, ds_scale);
   }
-  const float pb = wave_sum(-ci * bsum);
-  const float pl = wave_sum(-lsum);
+  if (hh != 0) return;
+  const float pb = (float)wave_sum(-(double)ci * (double)ds_scale * bsum);
+  const float pl = (float)wave_sum(-lsum);
   if (l == 0) {
     const int64_t lidx = lrow0 + wv;
     P.ws[2 * lidx + 0] = pb;  // slot of (branch, head, query tile), whichever pass takes it
@@ -1132,19 +1229,14 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, DqBlkLds<D>& L, int
 // Key-major: kBwdBlk consecutive key tiles of one head (aligned: one bitmask word holds their
 // bits), streaming per branch the query tiles' Q and dO rows, query norms and tau values.  needm:
 // the block's key tiles to take (at least one).
-template <int D>
-struct DkvBlkLds {
-  bf16 ring[2 * 2 * 32 * D];     // two stages of a Q tile and a dO tile
-  float vals[2][2][32];          // [stage][query norms, tau values]
-  bf16 ktiles[kBwdBlk][32 * D];  // each wave's key rows (swizzled)
-};
 template <int D, int BR, int PK, bool NORM>
-__device__ __forceinline__ void dkv_block(const BwdParams& P, DkvBlkLds<D>& L, int jb, int bh, uint32_t needm) {
-  constexpr int W = kBwdBlk, NT = D / 16, ND = D / 32;
+__device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kKeyBlk<D>>& L, int jb, int bh, uint32_t needm) {
+  constexpr int W = kKeyBlk<D>, SP = kSplit<D>, NT = D / 16 / SP, ND = D / 32 / SP;
   constexpr int STAGE = 2 * 32 * D;  // Q tile, dO tile
   bf16* ring = L.ring;
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
-  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wv = wid / SP, hh = wid % SP;  // the wave's tile of the block, its half of d and of the columns
   const int BH = P.B * P.H, nqt = P.nqt, nkt = P.nkt, Nq = P.Nq, Nk = P.Nk, qoff = P.qoff;
   const int b = bh / P.H, h = bh % P.H;
   const int kt0 = W * jb, kt = kt0 + wv;
@@ -1162,7 +1254,7 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, DkvBlkLds<D>& L, i
   {
     const bf16* r = base(B_V) + (int64_t)jc * P.s[B_V][2];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) V[t] = *reinterpret_cast<const bf16x8*>(r + 16 * t + 8 * g);
+    for (int t = 0; t < NT; ++t) V[t] = *reinterpret_cast<const bf16x8*>(r + 16 * (t + NT * hh) + 8 * g);
   }
   const float beta = *P.beta;
   const float pw = P.p;
@@ -1175,20 +1267,26 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, DkvBlkLds<D>& L, i
   for (int c = 0; c < ND; ++c) AV[c] = f32x16{};
   unsigned visited = 0, computed = 0;
   int it = 0;  // ring position, continued across the branches
-  bf16* kti = L.ktiles[wv];
+  bf16* kti = L.rows[wv];
+  bf16x8 Kf[SP == 2 ? NT : 1];  // a split tile: this branch's key rows
 
 #pragma unroll
-  for (int br = 0; br < BR; ++br) {
+  for (int bi = 0; bi < BR; ++bi) {
+    const int br = BR - 1 - bi;  // the second branch first: dv = dO^T A1 - lambda dO^T A2
     const int qslot = br == 0 ? B_Q1 : B_Q2, kslot = br == 0 ? B_K1 : B_K2;
     const bf16* qb = base(qslot);
     const int64_t sq = P.s[qslot][2];
     const float rk = NORM ? P.norms[norm_base(P, br == 0 ? N_K1 : N_K2, bh) + jc] : 1.f;
     const float* nq = nullptr;
     if constexpr (NORM) nq = P.norms + norm_base(P, br == 0 ? N_Q1 : N_Q2, bh);
-    const float coef = br == 0 ? 1.f : -lam;
+    const float ds_scale = (PK == 2 ? 2.f : 1.f) * (br == 0 ? 1.f : -lam);
     // the wave's key rows (swizzled tile; rows past Nk read as zeros), read as score operands
-    {
-      BlkRows<D> kr4[kBwdBlk];
+    if constexpr (SP == 2) {
+      const bf16* r = base(kslot) + (int64_t)jc * P.s[kslot][2];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) Kf[t] = *reinterpret_cast<const bf16x8*>(r + 16 * (t + NT * hh) + 8 * g);
+    } else {
+      BlkRows<D, kBwdBlk> kr4[kBwdBlk];
 #pragma unroll
       for (int s4 = 0; s4 < kBwdBlk; ++s4) kr4[s4].load(base(kslot), P.s[kslot][2], 32 * min(kt, nkt - 1), Nk, s4);
 #pragma unroll
@@ -1209,7 +1307,7 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, DkvBlkLds<D>& L, i
         const int qtl = q0c + l;
         const bool in = qtl < nqt;
         const uint32_t w = !in ? 0u : P.occ ? P.occ[(row0 + qtl) * P.occ_w + (kt0 >> 5)] : 0xffffffffu;
-        uint32_t bits = (w >> (kt0 & 31)) & 0xfu & needm;
+        uint32_t bits = (w >> (kt0 & 31)) & needm;
         // causal: key tile kt0 + r is seen from query tile qt_first(kt0 + r) on
 #pragma unroll
         for (int r = 0; r < W; ++r)
@@ -1222,45 +1320,51 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, DkvBlkLds<D>& L, i
       own_out = (om >> q) & 1ull;
       return q0c + q;
     };
-    BlkRows<D> qr, dr;
-    float vrq = 1.f, vtq = 0.f;
-    auto issue = [&](int qt) {
-      qr.load(qb, sq, 32 * qt, Nq, wv);
-      dr.load(dob, sdo, 32 * qt, Nq, wv);
-      if (wv == 0 && l < 32) {
+    constexpr int AHEAD = D <= 64 ? 2 : 1;  // tiles in flight past the one being worked on
+    struct Pre {  // a tile's share in flight: its rows, norms and thresholds, index, and whether it is the wave's
+      BlkRows<D, W * SP> qr, dr;
+      float vrq, vtq;
+      int qt;
+      bool own;
+    };
+    auto fetch = [&](Pre& p) {
+      p.qt = next_tile(p.own);
+      const int qt = max(p.qt, 0);  // loads on every path: the waits then count them exactly
+      p.qr.load(qb, sq, 32 * qt, Nq, wid);
+      p.dr.load(dob, sdo, 32 * qt, Nq, wid);
+      if (wid == 0 && l < 32) {
         const int qi = min(32 * qt + l, Nq - 1);
-        vrq = NORM ? nq[qi] : 1.f;
-        vtq = beta * tau_coeff(qoff + 32 * qt + l, P.inv_d);
+        p.vrq = NORM ? nq[qi] : 1.f;
+        p.vtq = beta * tau_coeff(qoff + 32 * qt + l, P.inv_d);
       }
     };
-    bool cown = false;
-    int qt = next_tile(cown);
-    if (qt >= 0) issue(qt);
-    while (qt >= 0) {
+    auto step = [&](Pre& p) {
+      const int qt = p.qt;
+      const bool cown = p.own;
       bf16* qst = ring + (it & 1) * STAGE;
       bf16* dst = qst + 32 * D;
       float* rqs = L.vals[it & 1][0];
       float* tqs = L.vals[it & 1][1];
-      qr.store(qst, wv);
-      dr.store(dst, wv);
-      if (wv == 0 && l < 32) {
-        rqs[l] = vrq;
-        tqs[l] = vtq;
+      p.qr.store(qst, wid);
+      p.dr.store(dst, wid);
+      if (wid == 0 && l < 32) {
+        rqs[l] = p.vrq;
+        tqs[l] = p.vtq;
       }
-      bool nown = false;
-      const int qt2 = next_tile(nown);
-      if (qt2 >= 0) issue(qt2);  // in flight during this tile's work
+      fetch(p);  // the tile AHEAD steps on, in flight during this tile's work
       lds_barrier();
       ++it;
-      if (cown) {
-        ++visited;
-        const int q0 = 32 * qt;
-        f32x16 S = f32x16{}, Dp = f32x16{};
+      auto products = [&](f32x16& S, f32x16& Dp) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-          S = PolBF16::mma(tile_row_frag<D>(qst, t), tile_row_frag<D>(kti, t), S);
-          Dp = PolBF16::mma(tile_row_frag<D>(dst, t), V[t], Dp);
+          if constexpr (SP == 2) S = PolBF16::mma(tile_row_frag<D>(qst, t + NT * hh), Kf[t], S);
+          else S = PolBF16::mma(tile_row_frag<D>(qst, t), tile_row_frag<D>(kti, t), S);
+          Dp = PolBF16::mma(tile_row_frag<D>(dst, t + NT * hh), V[t], Dp);
         }
+      };
+      auto tile = [&](const f32x16& S, const f32x16& Dp) {
+        ++visited;
+        const int q0 = 32 * qt;
         float rq[16], tq[16];
         if constexpr (NORM) crow_vals(rqs, rq);
         crow_vals(tqs, tq);
@@ -1285,16 +1389,16 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, DkvBlkLds<D>& L, i
           const f32x16 T = relu16<NORM>(X);
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            EV[r] = coef * (T[r] * T[r]);
-            const float ds = coef * (T[r] + T[r]) * Dp[r];
+            EV[r] = T[r] * T[r];
+            const float ds = T[r] * Dp[r];
             EK[r] = NORM ? ds * rq[r] : ds;
           }
         } else {
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const bool pos = X[r] > 0.f;
-            EV[r] = pos ? coef * pow_p<PK>(X[r], pw) : 0.f;
-            const float ds = pos ? coef * dpow_p<PK>(X[r], pw) * Dp[r] : 0.f;
+            EV[r] = pos ? pow_p<PK>(X[r], pw) : 0.f;
+            const float ds = pos ? dpow_p<PK>(X[r], pw) * Dp[r] : 0.f;
             EK[r] = NORM ? ds * rq[r] : ds;
           }
         }
@@ -1310,30 +1414,78 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, DkvBlkLds<D>& L, i
         const bf16x8 K0 = PolBF16::pack_c(EK, 0), K1 = PolBF16::pack_c(EK, 1);
 #pragma unroll
         for (int c = 0; c < ND; ++c) {
-          AV[c] = PolBF16::mma(tile_tr_frag<D>(dst, 0, c), V0, AV[c]);
-          AV[c] = PolBF16::mma(tile_tr_frag<D>(dst, 1, c), V1, AV[c]);
-          AK[c] = PolBF16::mma(tile_tr_frag<D>(qst, 0, c), K0, AK[c]);
-          AK[c] = PolBF16::mma(tile_tr_frag<D>(qst, 1, c), K1, AK[c]);
+          AV[c] = PolBF16::mma(tile_tr_frag<D>(dst, 0, c + ND * hh), V0, AV[c]);
+          AV[c] = PolBF16::mma(tile_tr_frag<D>(dst, 1, c + ND * hh), V1, AV[c]);
+          AK[c] = PolBF16::mma(tile_tr_frag<D>(qst, 0, c + ND * hh), K0, AK[c]);
+          AK[c] = PolBF16::mma(tile_tr_frag<D>(qst, 1, c + ND * hh), K1, AK[c]);
         }
+      };
+      if constexpr (SP == 1) {
+        if (cown) {
+          f32x16 S = f32x16{}, Dp = f32x16{};
+          products(S, Dp);
+          tile(S, Dp);
+        }
+      } else {  // the waves of a tile agree on `cown`; every wave takes the barrier
+        f32x16 S = f32x16{}, Dp = f32x16{};
+        if (cown) {
+          products(S, Dp);
+          give16(L.xch[wid], S);
+          give16(L.xch[wid] + 16, Dp);
+        }
+        lds_barrier();
+        if (cown) tile(take16(L.xch[wid ^ 1], S), take16(L.xch[wid ^ 1] + 16, Dp));
       }
-      cown = nown;
-      qt = qt2;
+    };
+    Pre pa;
+    fetch(pa);
+    if constexpr (AHEAD == 2) {
+      Pre pb;
+      fetch(pb);
+      while (pa.qt >= 0) {
+        step(pa);
+        if (pb.qt < 0) break;
+        step(pb);
+      }
+    } else {
+      while (pa.qt >= 0) step(pa);
+    }
+    float dot = 0.f;  // the key row's x^ . dk^
+    if constexpr (NORM && SP == 2) {
+      if (need) {
+        GradRow<32 * ND> XR;
+        load_grad_row<32 * ND>(base(kslot) + (int64_t)jc * P.s[kslot][2] + 32 * ND * hh, XR);
+        dot = grad_row_dot<32 * ND>(AK, XR, rk);
+      }
+      if (g == 0) L.dots[wv][hh][n32] = dot;
+      lds_barrier();
+      dot = L.dots[wv][0][n32] + L.dots[wv][1][n32];
     }
     if (kvalid) {
-      GradRow<D> XR;  // the key row for the normalize backward
-      if constexpr (NORM) load_grad_row<D>(base(kslot) + (int64_t)jc * P.s[kslot][2], XR);
+      GradRow<32 * ND> XR;  // the key row's columns for the normalize backward
+      if constexpr (NORM) {
+        load_grad_row<32 * ND>(base(kslot) + (int64_t)jc * P.s[kslot][2] + 32 * ND * hh, XR);
+        if constexpr (SP == 1) dot = grad_row_dot<32 * ND>(AK, XR, rk);
+      }
       const int gslot = br == 0 ? B_DK1 : B_DK2;
       bf16* grow = (bf16*)P.grad[br == 0 ? 1 : 3] + (int64_t)b * P.s[gslot][0] + (int64_t)h * P.s[gslot][1] +
-                   (int64_t)j * P.s[gslot][2];
-      store_grad_rows<D, NORM>(AK, XR, grow, rk);
+                   (int64_t)j * P.s[gslot][2] + 32 * ND * hh;
+      store_grad_rows<32 * ND, NORM>(AK, XR, grow, rk, dot, ds_scale);
+    }
+    if (BR == 2 && bi == 0) {
+#pragma unroll
+      for (int c = 0; c < ND; ++c)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) AV[c][r] *= -lam;
     }
     lds_barrier();  // every wave is done with its key tile before the next branch's rows
   }
   if (kvalid) {
-    bf16* vrow = (bf16*)P.grad[4] + (int64_t)b * P.s[B_DV][0] + (int64_t)h * P.s[B_DV][1] + (int64_t)j * P.s[B_DV][2];
-    store_grad_rows<D, false>(AV, GradRow<D>{}, vrow, 1.f);
+    bf16* vrow = (bf16*)P.grad[4] + (int64_t)b * P.s[B_DV][0] + (int64_t)h * P.s[B_DV][1] + (int64_t)j * P.s[B_DV][2] +
+                 32 * ND * hh;
+    store_grad_rows<32 * ND, false>(AV, GradRow<32 * ND>{}, vrow, 1.f, 0.f, 1.f);
   }
-  if (P.stats && l == 0 && need) {
+  if (P.stats && l == 0 && need && hh == 0) {
     atomicAdd(P.stats + 0, (unsigned long long)visited);
     atomicAdd(P.stats + 1, (unsigned long long)computed);
   }
@@ -1342,32 +1494,32 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, DkvBlkLds<D>& L, i
 // One workgroup per block of query tiles: longest blocks (last query tiles) of every (head,
 // branch) first, the branches adjacent.
 template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_blk(BwdParams P) {
-  __shared__ __attribute__((aligned(16))) DqBlkLds<D> L;
+__global__ void __launch_bounds__(kQryThreads<D>) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_blk(BwdParams P) {
+  TDA_BLK_LDS(D, kBwdBlk, false);
   const int BH = P.B * P.H, nqb = (P.nqt + kBwdBlk - 1) / kBwdBlk;
   const int bid = blockIdx.x, jb = nqb - 1 - bid / (BR * BH), rem = bid % (BR * BH);
   dq_block<D, BR, PK, NORM>(P, L, jb, BR == 2 ? rem & 1 : 0, BR == 2 ? rem >> 1 : rem);
 }
 
-// Waves per SIMD that the key-major pass is compiled for: one branch without normalisation three
-// at d = 64 and two at d = 128 (2 and 20 VGPRs spilled; dense steps (4, 16, 2048, d) of 242 and 473
-// us against 244 and 539 with one fewer); two branches spill 21 and 38-54 there (467-472 against
-// 501-514 us at d = 64), normalisation 26 and 41, so they run one fewer.
+// Waves per SIMD that the key-major pass is compiled for: the most without spills at d = 64 (three
+// with one branch spill 9 VGPRs: 92 against 86.7 us at (4, 16, 2048, 64)); at d = 128 one, two with
+// one branch and no normalisation (19 VGPRs spilled, yet a dense step (4, 16, 2048, 128) of 473
+// against 539 us).
 template <int D, int BR, bool NORM>
 constexpr int dkv_waves() {
-  return (BR == 2 || NORM ? 1 : 2) + (D <= 64 ? 1 : 0);
+  return D <= 64 || (D == 128 && BR == 1 && !NORM) ? 2 : 1;
 }
 
 // One workgroup per block of key tiles: longest blocks (first key tiles) of every head first.  A
 // key tile takes this pass when a list of its column did not fit (the test bwd_dkv_pairs leaves
 // it by; it writes nothing for such a key tile), or always without lists.
 template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, NORM>()))) bwd_dkv_blk(BwdParams P) {
-  constexpr int W = kBwdBlk;
-  __shared__ __attribute__((aligned(16))) DkvBlkLds<D> L;
+__global__ void __launch_bounds__(kKeyThreads<D>) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, NORM>()))) bwd_dkv_blk(BwdParams P) {
+  constexpr int W = kKeyBlk<D>;
+  TDA_BLK_LDS(D, W, true);
   __shared__ uint32_t needs[W];
   const int l = lane_id();
-  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) / kSplit<D>;
   const int BH = P.B * P.H, nqt = P.nqt;
   const int bid = blockIdx.x, jb = bid / BH, bh = bid % BH, kt = W * jb + wv;
   const uint32_t* counts = P.pairs ? P.pairs + pair_lists(BR, BH, nqt) * 4 * kPairCap : nullptr;
@@ -1405,16 +1557,12 @@ __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_
 // Both block passes over the queue of the key-major pair pass, in one launch: the workgroups
 // take tickets, the key blocks (the longer ones) first, each kind longest blocks first as nearly as
 // the queue's order has it.  With every list fitting the queue is empty and a workgroup leaves
-// after one load (5.0 us); at a threshold scale of 0.5 nearly every block is queued
-// (TDA (2, 16, 1500, 64): 178 us, 2632 us with one wave per query or key tile fetching
+// after one load (4.6 us); at a threshold scale of 0.5 nearly every block is queued
+// (TDA (2, 16, 1500, 64): 151 us, 2632 us with one wave per query or key tile fetching
 // its own rows).
 template <int D, int BR, int PK>
 __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, true>()))) bwd_tiles(BwdParams P) {
-  union Lds {
-    DqBlkLds<D> dq;
-    DkvBlkLds<D> dkv;
-  };
-  __shared__ __attribute__((aligned(16))) Lds L;
+  TDA_BLK_LDS(D, kBwdBlk, true);
   __shared__ uint32_t ticket;
   const uint32_t nk = P.dkvq[0], total = nk + P.dkvq[1];
   if (total == 0u) return;
@@ -1428,13 +1576,12 @@ __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_
     if (t >= total) return;
     if (t < nk) {
       const uint32_t blk = (uint32_t)__builtin_amdgcn_readfirstlane((int)masks[(int64_t)BH * nkb + t]);
-      dkv_block<D, BR, PK, true>(P, L.dkv, (int)(blk % nkb), (int)(blk / nkb),
+      dkv_block<D, BR, PK, true>(P, L, (int)(blk % nkb), (int)(blk / nkb),
                                  (uint32_t)__builtin_amdgcn_readfirstlane((int)masks[blk]));
     } else {
       const uint32_t k = (uint32_t)__builtin_amdgcn_readfirstlane((int)masks[2 * (int64_t)BH * nkb + (t - nk)]);
-      const int rem = (int)(k % (uint32_t)(BR * BH));
-      dq_block<D, BR, PK, true>(P, L.dq, nqb - 1 - (int)(k / (uint32_t)(BR * BH)), BR == 2 ? rem & 1 : 0,
-                                BR == 2 ? rem >> 1 : rem);
+      const int j = (int)(k % (uint32_t)(BR * nqb));
+      dq_block<D, BR, PK, true>(P, L, nqb - 1 - (BR == 2 ? j >> 1 : j), BR == 2 ? j & 1 : 0, (int)(k / (uint32_t)(BR * nqb)));
     }
   }
 }
@@ -1450,24 +1597,31 @@ static int launch_t(const BwdParams& p, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   BwdParams q = p;
   if (!NORM) q.dkvq = nullptr;
-  if (q.pairs) {
-    hipLaunchKernelGGL((bwd_dq_pairs<D, BR, PK, NORM>), dim3((unsigned)qitems), dim3(64), 0, s, q);
-    launched(s, "bwd_dq_pairs");
-    hipLaunchKernelGGL((bwd_dkv_pairs<D, BR, PK, NORM>), dim3((unsigned)kitems), dim3(64), 0, s, q);
-    launched(s, "bwd_dkv_pairs");
+  if constexpr (D <= 128) {
+    if (q.pairs) {
+      hipLaunchKernelGGL((bwd_dq_pairs<D, BR, PK, NORM>), dim3((unsigned)qitems), dim3(64), 0, s, q);
+      launched(s, "bwd_dq_pairs");
+      hipLaunchKernelGGL((bwd_dkv_pairs<D, BR, PK, NORM>), dim3((unsigned)kitems), dim3(64), 0, s, q);
+      launched(s, "bwd_dkv_pairs");
+    }
   }
   const int BH = q.B * q.H;
   const unsigned qblocks = (unsigned)(BR * BH * ((q.nqt + kBwdBlk - 1) / kBwdBlk));
-  const unsigned kblocks = (unsigned)(BH * ((q.nkt + kBwdBlk - 1) / kBwdBlk));
-  if (NORM && q.pairs && q.dkvq) {
-    // as many workgroups as the GPU's 256 CUs hold at dkv_waves waves per SIMD
-    const unsigned most = 256u * dkv_waves<D, BR, true>(), blocks = qblocks + kblocks;
-    hipLaunchKernelGGL((bwd_tiles<D, BR, PK>), dim3(blocks < most ? blocks : most), dim3(64 * kBwdBlk), 0, s, q);
-    launched(s, "bwd_tiles");
-  } else {
-    hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM>), dim3(qblocks), dim3(64 * kBwdBlk), 0, s, q);
+  const unsigned kblocks = (unsigned)(BH * ((q.nkt + kKeyBlk<D> - 1) / kKeyBlk<D>));
+  bool queued = false;
+  if constexpr (NORM && D <= 128) {
+    if (q.pairs && q.dkvq) {
+      // as many workgroups as the GPU's 256 CUs hold at dkv_waves waves per SIMD
+      const unsigned most = 256u * dkv_waves<D, BR, true>(), blocks = qblocks + kblocks;
+      hipLaunchKernelGGL((bwd_tiles<D, BR, PK>), dim3(blocks < most ? blocks : most), dim3(64 * kBwdBlk), 0, s, q);
+      launched(s, "bwd_tiles");
+      queued = true;
+    }
+  }
+  if (!queued) {
+    hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM>), dim3(qblocks), dim3(kQryThreads<D>), 0, s, q);
     launched(s, "bwd_dq_blk");
-    hipLaunchKernelGGL((bwd_dkv_blk<D, BR, PK, NORM>), dim3(kblocks), dim3(64 * kBwdBlk), 0, s, q);
+    hipLaunchKernelGGL((bwd_dkv_blk<D, BR, PK, NORM>), dim3(kblocks), dim3(kKeyThreads<D>), 0, s, q);
     launched(s, "bwd_dkv_blk");
   }
   const int e = (int)hipGetLastError();
@@ -1492,6 +1646,14 @@ static int sel_br(const BwdParams& p, const KernelKey& k, void* s) {
 
 int launch_bwd_fast(const BwdParams& p, const KernelKey& k, void* stream) {
   return k.d == 128 ? sel_br<128>(p, k, stream) : sel_br<64>(p, k, stream);
+}
+
+// head_dim 256 has no pair lists: the block passes over the bitmask (or every causal tile).
+int launch_bwd_blk256(const BwdParams& p0, const KernelKey& k, void* stream) {
+  BwdParams p = p0;
+  p.pairs = nullptr;
+  p.dkvq = nullptr;
+  return sel_br<256>(p, k, stream);
 }
 
 // The pair passes on fp32 rows (the fp32 backward's launcher in tda_bwd.hip runs the tile passes

@@ -199,6 +199,11 @@ __device__ __forceinline__ float wave_sum(float v) {
   v += __shfl_xor(v, 16);
   return v + __shfl_xor(v, 32);
 }
+__device__ __forceinline__ double wave_sum(double v) {  // the same order of additions in every lane's sum
+#pragma unroll
+  for (int m = 1; m < 64; m <<= 1) v += __shfl_xor(v, m);
+  return v;
+}
 // Workgroup barrier for hand-offs through LDS only: the wave's LDS operations complete
 // (lgkmcnt(0)), then s_barrier; the wavefront-scope fences keep the compiler from moving memory
 // operations across it.  __syncthreads()'s workgroup release fence also waits for every
@@ -211,13 +216,7 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-// Wave-wide integer sum (every lane ends with the total).  Call with every lane active.
-__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
-#pragma unroll
-  for (int m = 1; m < 64; m <<= 1) v += (uint32_t)__shfl_xor((int)v, m);
-  return v;
-}
-// Wave-wide OR, the same way.
+// Wave-wide OR (every lane ends with it), by the same steps as wave_sum.  Call with every lane active.
 __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
   v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false);
   v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, false);
@@ -328,7 +327,7 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 // per 16 lanes), with 32 or 64 banks.
 template <int D>
 __device__ __forceinline__ int bswz(int r) {
-  if constexpr (D == 128) return (r ^ (4 * (r & 3))) & 15;
+  if constexpr (D >= 128) return (r ^ (4 * (r & 3))) & 15;  // rows of 256 or 512 bytes: all start at bank 0
   else return ((r ^ (r >> 1)) ^ (2 * (r & 1)) ^ (4 * ((r >> 1) & 1))) & 7;
 }
 

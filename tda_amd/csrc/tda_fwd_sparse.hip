@@ -747,30 +747,37 @@ __device__ __forceinline__ bf16x8 tr_frag(const bf16* p) {
 
 // ------------------------------------------------------------------ fwd_pv_blk
 // The tile pass, over kBlkTiles consecutive query tiles of one head, one wave each.  The waves
-// walk the union of their bitmask rows' kept key tiles in step and share each key tile's K and V
-// rows (and key norms): the workgroup loads them once, each wave a quarter of the rows, one tile
-// ahead into registers, then into a two-stage LDS ring (one barrier per tile: a stage is rewritten
-// two tiles after it was read, and every wave has passed the barrier between).  A wave computes
-// only the tiles its own row keeps.  Once a pair list has passed its cap the wave only counts its
-// non-zero weights (one wave sum at the end) instead of placing them.  K and V tiles load through
-// one descriptor per head at a per-tile offset when the head's offsets fit 31 bits, else through
-// one descriptor per tile.
-// Without normalisation (no screen ran before it) every query tile runs and every causal key tile
-// of a row counts as kept; the row's bitmask words are all written (the words past its last key
-// tile as zeros) and the causal tiles are counted into stats[0].  ZR: the workgroup then clears
-// its even share of the call's zero range.
-// With normalisation it takes the query tiles whose candidate lists overflowed (a count past
-// kCandCap in some branch; fwd_pv_cand took the others): a workgroup with none of them leaves
-// after one round of loads, a wave whose own lists fit only helps to load.  At a threshold scale
-// of 0.5 nearly every list overflows and a third of the kept tiles' weights are zero: bound by the
-// per-element work of the weights (TDA (2, 16, 1500, 64), beta 0.5: 237 us with one wave per query
-// tile, 109 us so); with every list fitting the launch costs 5.1 us.
+// walk the key tiles that any of them takes in step and share each key tile's K and V rows (and key
+// norms): the workgroup loads them once, each wave a quarter of the rows, AHEAD tiles ahead into
+// registers (the loads unconditional: behind a branch the compiler's waits drain every load), then
+// into a two-stage LDS ring (one barrier per tile: a stage is rewritten two tiles after it was
+// read, and every wave has passed the barrier between).  A wave computes only its own tiles.  Once a
+// pair list has passed its cap the wave only counts its non-zero weights.  K and V tiles load
+// through one descriptor per head at a per-tile offset when the head's offsets fit 31 bits, else
+// through one descriptor per tile.  What bounds it is the chain of each tile's step (loads, barrier,
+// fragment reads, products, weights, products), about 1 us however many waves share a SIMD, so
+// instructions out of the step count: the walks below keep no bitmask words in registers (TRA (4,
+// 16, 2048, 64) without normalisation 59 -> 48.5 us with them, the two tiles ahead and weights
+// without their branch's coefficient, which scales the sum once per branch).
+// WALK (no screen ran before it): every query tile, every causal key tile in turn; the row's
+// bitmask words are all written (the words past its last key tile as zeros) and, up to head_dim 128,
+// the causal tiles are counted into stats[0].  ZR: the workgroup then clears its even share of the
+// call's zero range.
+// Without WALK (normalised) it takes the query tiles whose candidate lists overflowed (a count past
+// kCandCap in some branch; fwd_pv_cand took the others), walking the union of their bitmask rows,
+// listed in LDS 64 words at a time; tiles whose weights are all zero lose their bit.  A workgroup
+// with no such tile leaves after one round of loads, a wave whose own lists fit only helps to load.
+// At a threshold scale of 0.5 nearly every list overflows (TDA (2, 16, 1500, 64): 237 us with one
+// wave per query tile, 102 so); with every list fitting the launch costs 4.6 us.
+// SKIP: the A V products of a tile whose weights are all zero are skipped, by a branch around the
+// accumulators (head_dim 256 with normalisation, where 97 % of the tiles are: TDA (2, 8, 1000, 256)
+// 81 us against 249 with two waves per query tile, each forming all scores from its own loads).
 constexpr int kBlkTiles = 4;
 
-template <int D, int BR, int PK, bool NORM, bool ZR = false>
-__global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 3 : 2))) fwd_pv_blk(FwdParams P) {
-  static_assert(!ZR || !NORM, "with normalisation the screen clears the zero range");
-  constexpr bool WALK = !NORM;
+template <int D, int BR, int PK, bool NORM, bool ZR = false, bool WALK = !NORM, bool SKIP = false>
+__global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_per_eu(D <= 64 ? (WALK ? 3 : 2) : D <= 128 ? 2 : 1)))
+fwd_pv_blk(FwdParams P) {
+  static_assert(!ZR || WALK, "the zero range is cleared by the walk");
   constexpr int W = kBlkTiles;
   constexpr int NT = D / 16, ND = D / 32;
   constexpr int VS = D + 32;     // LDS row stride of a V tile: conflict-free transpose reads
@@ -778,11 +785,14 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
   constexpr int CPR = D / 8;     // 16-byte chunks per row
   constexpr int RPI = 64 / CPR;  // rows per load instruction
   constexpr int LPW = 32 / RPI / W;  // load instructions per wave, K and V each
+  constexpr int AHEAD = D <= 64 || (WALK && D <= 128) ? 2 : 1;  // tiles in flight past the one being worked on
   static_assert(LPW >= 1 && LPW * RPI * W == 32, "K/V tile rows split evenly over the waves");
   constexpr int STAGE = 32 * KS + 32 * VS;
   static_assert(2 * STAGE >= W * 32 * KS, "the ring holds the waves' output rows");
   __shared__ __attribute__((aligned(16))) bf16 ring[2 * STAGE];
   __shared__ __attribute__((aligned(16))) float nring[2][32];
+  __shared__ uint16_t wlist[WALK ? 1 : 64 * 32];  // the chunk's tiles: tile | rows that keep it << 11
+  __shared__ uint32_t wwords[WALK ? 1 : W][64];   // the rows' bitmask words of the chunk
 
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -802,9 +812,9 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
       jb = nqb - 1 - bid / BH;
     }
   }
-  // the block's query tiles this pass takes (the same for every wave)
-  uint32_t needm = nqt - W * jb >= W ? (1u << W) - 1u : (1u << (nqt - W * jb)) - 1u;
-  if constexpr (NORM) {
+  // without WALK: the block's query tiles this pass takes (the same for every wave)
+  uint32_t needm = 0u;
+  if constexpr (!WALK) {
     const uint32_t* counts = P.cand + pair_lists(BR, BH, nqt) * kCandCap + (int64_t)bh * nqt + W * jb;
     bool ovf = false;  // lane r of a branch's W lanes: query tile r's list overflowed
     if (l < BR * W && W * jb + l % W < nqt) ovf = counts[(int64_t)(l / W) * BH * nqt + l % W] > (uint32_t)kCandCap;
@@ -814,7 +824,7 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
   }
   const int b = bh / P.H, h = bh % P.H;
   const int qt = W * jb + wv;
-  const bool act = (needm >> wv) & 1u;  // wave-uniform: the other waves only load
+  const bool act = WALK ? qt < nqt : (needm >> wv) & 1u;  // wave-uniform: the other waves only load
   const int qtc = min(qt, nqt - 1);
   const int iq = 32 * qt + n32;
   const bool valid = act && iq < Nq;
@@ -836,8 +846,9 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
   unsigned computed = 0, checked = 0;
   int it = 0;  // ring position, continued across the branches
 
-#pragma unroll
-  for (int br = 0; br < BR; ++br) {
+#pragma unroll(D > 128 ? 1 : BR)
+  for (int bi = 0; bi < BR; ++bi) {
+    const int br = BR - 1 - bi;  // the second branch first: out = -lambda A2 V, then += A1 V
     const int qslot = br ? F_Q2 : F_Q1, kslot = br ? F_K2 : F_K1;
     uint32_t* orow0 = P.occ + ((int64_t)(br * BH + bh) * nqt + W * jb) * P.occ_w;  // the block's first row
     const bf16* khead = (const bf16*)P.in[kslot] + (int64_t)b * P.s[kslot][0] + (int64_t)h * P.s[kslot][1];
@@ -845,7 +856,6 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
     const int64_t sk = P.s[kslot][2], sv = P.s[F_V][2];
     const __amdgpu_buffer_rsrc_t rn =
         make_rsrc(NORM ? P.norms + norm_base(P, br ? N_K2 : N_K1, bh) : nullptr, NORM ? (uint32_t)Nk * 4 : 0u);
-    const float coef = br == 0 ? 1.f : -lam;
     // query fragments straight from the rows (rows past Nq read as zeros), the inverse norm
     bf16x8 Q[NT];
     {
@@ -860,85 +870,50 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
     if constexpr (NORM) rq = P.norms[norm_base(P, br ? N_Q2 : N_Q1, bh) + min(32 * qtc + n32, Nq - 1)];
     const int64_t lidx = ((int64_t)br * BH + bh) * nqt + qtc;
     uint32_t* pent = P.pairs && act ? P.pairs + lidx * (4 * kPairCap) : nullptr;
-    uint32_t npairs = 0, extra = 0;
-
-    // word w of row r of the block, masked to the key tiles the row sees (uniform)
-    auto row_word = [&](int r, int w) -> uint32_t {
-      if (!((needm >> r) & 1u)) return 0u;
-      const int kl = kt_last(W * jb + r, qoff, P.nkt);
-      if (w > (kl >> 5)) return 0u;
-      uint32_t x = WALK ? 0xffffffffu : (uint32_t)__builtin_amdgcn_readfirstlane((int)orow0[(int64_t)r * P.occ_w + w]);
-      if (w == (kl >> 5) && (kl & 31) != 31) x &= (2u << (kl & 31)) - 1u;
-      return x;
+    uint32_t npairs = 0;
+    uint32_t* orow = orow0 + (int64_t)wv * P.occ_w;  // the wave's bitmask row (when active)
+    struct Pre {  // a tile's share in flight
+      u32x4 kr[LPW], vr[LPW];
+      f32x4 nr;
     };
-    // the union walk: next key tile any row keeps, its word, and the own row's word
-    int sw = -1;
-    uint32_t ub = 0u, sown = 0u;
-    auto next_tile = [&](int& w_out, uint32_t& own_out) -> int {
-      while (ub == 0u) {
-        if (++sw > (klast_b >> 5)) return -1;
-        uint32_t u = 0u, o = 0u;
-#pragma unroll
-        for (int r = 0; r < W; ++r) {
-          const uint32_t x = row_word(r, sw);
-          u |= x;
-          o = r == wv ? x : o;
-        }
-        ub = u;
-        sown = o;
-      }
-      const int kt = 32 * sw + __builtin_ctz(ub);
-      ub &= ub - 1u;
-      w_out = sw;
-      own_out = sown;
-      return kt;
-    };
-    u32x4 kr[LPW], vr[LPW];
-    f32x4 nr = {};
     // one descriptor per head and a per-tile offset when the heads' offsets fit 31 bits (uniform),
     // else one descriptor per tile
     const bool whole = head_fits(sk, Nk) && head_fits(sv, Nk);
     const __amdgpu_buffer_rsrc_t rkh = head_rsrc<D>(khead, sk, Nk), rvh = head_rsrc<D>(vhead, sv, Nk);
-    auto issue = [&](int kt) {
+    auto issue = [&](Pre& p, int kt) {
       if (whole) {
         const uint32_t tk = (uint32_t)(32 * kt) * (uint32_t)(2 * sk), tv = (uint32_t)(32 * kt) * (uint32_t)(2 * sv);
 #pragma unroll
-        for (int i = 0; i < LPW; ++i) kr[i] = buf_load16(rkh, tk + (uint32_t)(((vrow0 + RPI * i) * sk + 8 * vch) * 2));
+        for (int i = 0; i < LPW; ++i) p.kr[i] = buf_load16(rkh, tk + (uint32_t)(((vrow0 + RPI * i) * sk + 8 * vch) * 2));
 #pragma unroll
-        for (int i = 0; i < LPW; ++i) vr[i] = buf_load16(rvh, tv + (uint32_t)(((vrow0 + RPI * i) * sv + 8 * vch) * 2));
+        for (int i = 0; i < LPW; ++i) p.vr[i] = buf_load16(rvh, tv + (uint32_t)(((vrow0 + RPI * i) * sv + 8 * vch) * 2));
       } else {
         const __amdgpu_buffer_rsrc_t rk = tile_rsrc<D>(khead, sk, kt, Nk);
         const __amdgpu_buffer_rsrc_t rv = tile_rsrc<D>(vhead, sv, kt, Nk);
 #pragma unroll
-        for (int i = 0; i < LPW; ++i) kr[i] = buf_load16(rk, (uint32_t)(((vrow0 + RPI * i) * sk + 8 * vch) * 2));
+        for (int i = 0; i < LPW; ++i) p.kr[i] = buf_load16(rk, (uint32_t)(((vrow0 + RPI * i) * sk + 8 * vch) * 2));
 #pragma unroll
-        for (int i = 0; i < LPW; ++i) vr[i] = buf_load16(rv, (uint32_t)(((vrow0 + RPI * i) * sv + 8 * vch) * 2));
+        for (int i = 0; i < LPW; ++i) p.vr[i] = buf_load16(rv, (uint32_t)(((vrow0 + RPI * i) * sv + 8 * vch) * 2));
       }
-      if (NORM && wv == 0 && l < 8) nr = __builtin_bit_cast(f32x4, buf_load16(rn, (uint32_t)(32 * kt + 4 * l) * 4));
+      if (NORM && wv == 0 && l < 8) p.nr = __builtin_bit_cast(f32x4, buf_load16(rn, (uint32_t)(32 * kt + 4 * l) * 4));
     };
 
-    int cw = 0;
-    uint32_t cown = 0u;
-    int kt = next_tile(cw, cown);
-    if (kt >= 0) issue(kt);
-    uint32_t keep = cown;  // own word cw with the tiles of no non-zero weight cleared
-    while (kt >= 0) {
+    // the tile in flight into the ring's next stage, and the barrier that makes it readable
+    auto stage = [&](const Pre& p) {
       bf16* kst = ring + (it & 1) * STAGE;
       bf16* vst = kst + 32 * KS;
-      float* nst = nring[it & 1];
 #pragma unroll
       for (int i = 0; i < LPW; ++i) {
-        *reinterpret_cast<u32x4*>(kst + (vrow0 + RPI * i) * KS + 8 * vch) = kr[i];
-        *reinterpret_cast<u32x4*>(vst + (vrow0 + RPI * i) * VS + 8 * vch) = vr[i];
+        *reinterpret_cast<u32x4*>(kst + (vrow0 + RPI * i) * KS + 8 * vch) = p.kr[i];
+        *reinterpret_cast<u32x4*>(vst + (vrow0 + RPI * i) * VS + 8 * vch) = p.vr[i];
       }
-      if (NORM && wv == 0 && l < 8) *reinterpret_cast<f32x4*>(nst + 4 * l) = nr;
-      int nw = 0;
-      uint32_t nown = 0u;
-      const int kt2 = next_tile(nw, nown);
-      if (kt2 >= 0) issue(kt2);  // in flight during this tile's work
-      lds_barrier();
-      ++it;
-      if ((cown >> (kt & 31)) & 1u) {
+      if (NORM && wv == 0 && l < 8) *reinterpret_cast<f32x4*>(nring[it & 1] + 4 * l) = p.nr;
+    };
+    // the wave's work on the staged key tile kt; whether it holds a weight
+    auto tile = [&](int kt) -> bool {
+        const bf16* kst = ring + ((it - 1) & 1) * STAGE;
+        const bf16* vst = kst + 32 * KS;
+        const float* nst = nring[(it - 1) & 1];
         ++checked;
         f32x16 S = {};
         const bf16* kp = kst + n32 * KS + 8 * g;
@@ -965,7 +940,7 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
 #pragma unroll
           for (int r = 0; r < 16; ++r) X[r] = 8 * (r >> 2) + (r & 3) <= lim ? X[r] : -1.f;
         }
-        // weights coef relu(x)^p and the lane's largest x (some weight of the tile is non-zero
+        // weights relu(x)^p and the lane's largest x (some weight of the tile is non-zero
         // iff a lane's is > 0), on the bits: a float is > 0 iff its bits as an int32 are, so the
         // integer max(bits, 0) is relu(x) (no NaN handling to pay for in float max); p other than
         // 1, 2 select on x > 0.  With normalisation a NaN score (a non-finite row) has no weight:
@@ -978,22 +953,19 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
         }
         const i32x16 XB = __builtin_bit_cast(i32x16, X);
         i32x16 TB;
-        int xmb = XB[0];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          TB[r] = NORM ? XB[r] : max(XB[r], 0);
-          if (r) xmb = max(xmb, XB[r]);
-        }
+        for (int r = 0; r < 16; ++r) TB[r] = NORM ? XB[r] : max(XB[r], 0);
         const f32x16 T = __builtin_bit_cast(f32x16, TB);
         f32x16 C;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          if constexpr (PK == 2) C[r] = T[r] * (coef * T[r]);
-          else if constexpr (PK == 1) C[r] = coef * T[r];
-          else C[r] = X[r] > 0.f ? coef * pow_p<PK>(X[r], pw) : 0.f;
+          if constexpr (PK == 2) C[r] = T[r] * T[r];
+          else if constexpr (PK == 1) C[r] = T[r];
+          else C[r] = X[r] > 0.f ? pow_p<PK>(X[r], pw) : 0.f;
         }
-        const bool pos_any = xmb > 0;
+        bool any;
         if (pent) {
+          const uint32_t before = npairs;
           if (npairs < (uint32_t)kPairCap) {
             // list entries of the non-zero weights, in the order (value r, lane); x's bits through
             // a bit cast of the whole vector (hipcc compiled a bit cast of one element of an
@@ -1011,41 +983,147 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
                     u32x4{(uint32_t)(32 * kt + crow(r, g)), (uint32_t)n32, XU[r], kNoSlot};
               npairs += (uint32_t)__builtin_popcountll(bal);
             }
-          } else {
+          } else {  // past the cap: the count alone
 #pragma unroll
-            for (int r = 0; r < 16; ++r) extra += X[r] > 0.f ? 1u : 0u;
+            for (int r = 0; r < 16; ++r) npairs += (uint32_t)__builtin_popcountll(wave_ballot(X[r] > 0.f));
           }
-        }
-        if (wave_ballot(pos_any) == 0ull) {
-          keep &= ~(1u << (kt & 31));
+          any = npairs != before;
         } else {
+          int xmb = XB[0];
+#pragma unroll
+          for (int r = 1; r < 16; ++r) xmb = max(xmb, XB[r]);
+          any = wave_ballot(xmb > 0) != 0ull;
+        }
+        if (any) {
           // pairs of the tile pass are in no column bucket: the key-major backward walks the lists
           if (P.colcnt && l == 0) atomicOr(P.colcnt + (int64_t)bh * P.nkt + kt, kColTaint);
           ++computed;
         }
         // A V on every tile the row keeps (a tile of zero weights adds zero products: the same
         // sums bit for bit, and no branch around the accumulators)
-        const bf16x8 PF0 = PolBF16::pack_c(C, 0), PF1 = PolBF16::pack_c(C, 1);
-        const bf16* vp = vst + voff;
+        if (!SKIP || any) {
+          const bf16x8 PF0 = PolBF16::pack_c(C, 0), PF1 = PolBF16::pack_c(C, 1);
+          const bf16* vp = vst + voff;
 #pragma unroll
-        for (int c = 0; c < ND; ++c) {
-          O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c), PF0, O[c]);
-          O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c + 16 * VS), PF1, O[c]);
+          for (int c = 0; c < ND; ++c) {
+            O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c), PF0, O[c]);
+            O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c + 16 * VS), PF1, O[c]);
+          }
+        }
+        return any;
+    };
+
+    if constexpr (WALK) {  // key tiles 0 .. klast_b in turn
+      const int ktl = act ? kt_last(qt, qoff, P.nkt) : -1;  // the wave's last
+      uint32_t keep = 0u;                                   // the current word: its tiles with a weight
+      auto step = [&](Pre& p, int kt) {
+        stage(p);
+        issue(p, min(kt + AHEAD, klast_b));  // in flight during this tile's work
+        lds_barrier();
+        ++it;
+        if (kt <= ktl && tile(kt)) keep |= 1u << (kt & 31);
+        if ((kt & 31) == 31 || kt == klast_b) {
+          if ((kt >> 5) <= (ktl >> 5) && l == 0) orow[kt >> 5] = keep;
+          keep = 0u;
+        }
+      };
+      Pre pa, pb;
+      issue(pa, 0);
+      if constexpr (AHEAD == 2) {
+        issue(pb, min(1, klast_b));
+        for (int kt = 0; kt <= klast_b; kt += 2) {
+          step(pa, kt);
+          if (kt + 1 > klast_b) break;
+          step(pb, kt + 1);
+        }
+      } else {
+        for (int kt = 0; kt <= klast_b; ++kt) step(pa, kt);
+      }
+    } else {
+      // the union of the rows' kept tiles, listed 64 bitmask words (2048 tiles) at a time
+      const int kl = kt_last(qtc, qoff, P.nkt), nwords = (klast_b >> 5) + 1;
+      for (int w0 = 0; w0 < nwords; w0 += 64) {
+        lds_barrier();  // every wave is done with the previous chunk's list
+        uint32_t own = 0u;  // lane w: word w0 + w of the own row, masked to the key tiles it sees
+        if (act && w0 + l <= (kl >> 5)) {
+          own = orow[w0 + l];
+          if (w0 + l == (kl >> 5) && (kl & 31) != 31) own &= (2u << (kl & 31)) - 1u;
+        }
+        wwords[wv][l] = own;
+        lds_barrier();
+        uint32_t rw[W], u = 0u;
+#pragma unroll
+        for (int r = 0; r < W; ++r) u |= rw[r] = wwords[r][l];
+        int end = __builtin_popcount(u);  // inclusive prefix sum over the lanes
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int x = __shfl_up(end, o);
+          end += l >= o ? x : 0;
+        }
+        const int n = __builtin_amdgcn_readlane(end, 63);
+        // (each wave writes the whole list, the same values, and reads it after its own writes)
+        for (int slot = end - __builtin_popcount(u); wave_ballot(u != 0u) != 0ull; ++slot) {
+          if (u) {
+            const int bb = __builtin_ctz(u);
+            u &= u - 1u;
+            uint32_t rows = 0u;
+#pragma unroll
+            for (int r = 0; r < W; ++r) rows |= ((rw[r] >> bb) & 1u) << r;
+            wlist[slot] = (uint16_t)((uint32_t)(32 * l + bb) | (rows << 11));
+          }
+        }
+        wave_lds_sync();
+        uint32_t ev = 0u;  // 64 entries at a time, one per lane
+        auto entry = [&](int i) -> uint32_t {
+          if ((i & 63) == 0) ev = i + l < n ? wlist[i + l] : 0u;
+          return (uint32_t)__builtin_amdgcn_readlane((int)ev, i & 63);
+        };
+        int at = 0;  // the next entry to issue; past the last one, tile w0's rows (unused)
+        auto next = [&](Pre& p, uint32_t& e) {
+          e = at < n ? entry(at) : 0u;
+          ++at;
+          issue(p, 32 * w0 + (int)(e & 2047u));
+        };
+        auto step = [&](Pre& p, uint32_t& pe) {
+          const uint32_t e = pe, k = e & 2047u;
+          stage(p);
+          next(p, pe);  // in flight during this tile's work
+          lds_barrier();
+          ++it;
+          if (((e >> (11 + wv)) & 1u) && !tile(32 * w0 + (int)k) && l == 0)
+            wwords[wv][k >> 5] &= ~(1u << (k & 31));  // no weight: the tile loses its bit
+        };
+        Pre pa, pb;
+        uint32_t ea = 0u, eb = 0u;
+        if (n) {
+          next(pa, ea);
+          if constexpr (AHEAD == 2) next(pb, eb);
+        }
+        if constexpr (AHEAD == 2) {
+          for (int i = 0; i < n; i += 2) {
+            step(pa, ea);
+            if (i + 1 >= n) break;
+            step(pb, eb);
+          }
+        } else {
+          for (int i = 0; i < n; ++i) step(pa, ea);
+        }
+        wave_lds_sync();
+        if (act && w0 + l <= (kl >> 5)) {
+          const uint32_t now = wwords[wv][l];
+          if (now != own) orow[w0 + l] = now;
         }
       }
-      if (kt2 < 0 || nw != cw) {  // the own row's word cw is done
-        if (act && (WALK || keep != cown) && l == 0) orow0[(int64_t)wv * P.occ_w + cw] = keep;
-        cw = nw;
-        cown = keep = nown;
-      }
-      kt = kt2;
     }
     if (WALK && act && l == 0) {  // the own row's words past its last key tile (no screen wrote them)
-      for (int w = (kt_last(qt, qoff, P.nkt) >> 5) + 1; w < P.occ_w; ++w) orow0[(int64_t)wv * P.occ_w + w] = 0u;
+      for (int w = (kt_last(qt, qoff, P.nkt) >> 5) + 1; w < P.occ_w; ++w) orow[w] = 0u;
     }
-    if (pent) {
-      npairs += wave_sum_u32(extra);
-      if (l == 0) P.pairs[pair_lists(P.nbr, BH, nqt) * 4 * kPairCap + lidx] = npairs;
+    if (pent && l == 0) P.pairs[pair_lists(P.nbr, BH, nqt) * 4 * kPairCap + lidx] = npairs;
+    if (BR == 2 && bi == 0) {
+#pragma unroll
+      for (int c = 0; c < ND; ++c)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) O[c][r] *= -lam;
     }
   }
 
@@ -1086,7 +1164,7 @@ __global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_pe
   if (P.stats && l == 0 && checked) {
     if (WALK) atomicAdd(P.stats + 0, (unsigned long long)checked);  // every causal tile is tested
     atomicAdd(P.stats + 1, (unsigned long long)computed);
-    atomicAdd(P.stats + 2, (unsigned long long)checked);
+    if (D <= 128) atomicAdd(P.stats + 2, (unsigned long long)checked);
   }
 }
 
@@ -1148,6 +1226,7 @@ __global__ void __launch_bounds__(64 * BR) __attribute__((amdgpu_waves_per_eu(3)
   for (int br = 0; br < BR; ++br) fit = fit && nc[br] <= (uint32_t)kCandCap;
   if (!fit) return;  // fwd_pv_blk walks the bitmask tiles (both waves leave: the test is the same)
   if (P.screen_items > (Nq + 255) / 256) {
+    asm volatile("");  // (a side effect: without one hipcc computes the ranks on every path, 2 us at the headline size)
     // the screen split some key ranges over several items, which append in any order: sort each
     // list (lanes 0-31: branch 0, lanes 32-63: branch 1; its keys are distinct) by rank
     const int half = BR == 2 ? (l >> 5) : 0;
@@ -1432,6 +1511,32 @@ int sel_br(const FwdParams& p, const KernelKey& k, hipStream_t s) {
 int launch_fwd_sparse(const FwdParams& p, const KernelKey& k, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   return k.d == 128 ? sel_br<128>(p, k, s) : sel_br<64>(p, k, s);
+}
+
+// head_dim 256 (bf16): no screen and no pair lists; every causal tile through the block pass, after
+// the launcher (tda_wide.hip) wrote the norms table.
+template <int BR, int PK>
+static int launch_blk256_t(const FwdParams& p, bool norm, hipStream_t s) {
+  const unsigned blocks = (unsigned)(p.B * p.H * ((p.nqt + kBlkTiles - 1) / kBlkTiles));
+  if (norm)
+    hipLaunchKernelGGL((fwd_pv_blk<256, BR, PK, true, false, true, true>), dim3(blocks), dim3(64 * kBlkTiles), 0, s, p);
+  else
+    hipLaunchKernelGGL((fwd_pv_blk<256, BR, PK, false>), dim3(blocks), dim3(64 * kBlkTiles), 0, s, p);
+  launched(s, "wide_fwd");
+  return (int)hipGetLastError();
+}
+template <int BR>
+static int launch_blk256_br(const FwdParams& p, const KernelKey& k, hipStream_t s) {
+  switch (k.pkind) {
+    case 2: return launch_blk256_t<BR, 2>(p, k.normalize, s);
+    case 1: return launch_blk256_t<BR, 1>(p, k.normalize, s);
+    default: return launch_blk256_t<BR, 0>(p, k.normalize, s);
+  }
+}
+int launch_fwd_blk256(const FwdParams& p0, const KernelKey& k, void* stream) {
+  FwdParams p = p0;
+  p.pairs = nullptr;  // head_dim 256 leaves the pair buffer alone
+  return k.branches == 2 ? launch_blk256_br<2>(p, k, (hipStream_t)stream) : launch_blk256_br<1>(p, k, (hipStream_t)stream);
 }
 
 // The int8 screen over fp32 rows, for the normalised fp32 pass (fwd_wave in its screened form,

@@ -142,9 +142,11 @@ int launch_bwd(const BwdParams& p, const KernelKey& k, void* stream);
 int launch_bwd_fast(const BwdParams& p, const KernelKey& k, void* stream);
 // fp32 with the forward's pair lists: the query-major and key-major pair passes (tda_bwd_fast.hip)
 int launch_bwd_pairs_f32(const BwdParams& p, const KernelKey& k, void* stream);
-// head_dim 256 (tda_wide.hip): the column-split forward and backward
+// head_dim 256 (tda_wide.hip): fp32 column-split kernels; bf16 the block passes below
 int launch_fwd_wide(const FwdParams& p, const KernelKey& k, void* stream);
 int launch_bwd_wide(const BwdParams& p, const KernelKey& k, void* stream);
+int launch_fwd_blk256(const FwdParams& p, const KernelKey& k, void* stream);
+int launch_bwd_blk256(const BwdParams& p, const KernelKey& k, void* stream);
 // Set the forward's zero range to zero (paths without the screen, which clears it otherwise).
 int launch_zero(const FwdParams& p, void* stream);
 // Sum the (dbeta, dlambda) partial pairs ws[2 * item], item < items, in a fixed order.

@@ -1,4 +1,5 @@
-// tda_wide.hip -- threshold attention at head_dim 256 (fp32 and bf16) for gfx950.
+// tda_wide.hip -- threshold attention at head_dim 256 for gfx950: the fp32 kernels, and the norms
+// table of both dtypes (bf16 runs the block passes of tda_fwd_sparse.hip and tda_bwd_fast.hip).
 //
 // Reference semantics (snap-research/TDA triton_threshold_attention.py, "TTA"): the forward
 // kernel TTA:19-115 and the backward kernels TTA:118-324, whose BLOCK_D is the head_dim for any
@@ -33,45 +34,26 @@ namespace {
 constexpr int WD = 256;  // head_dim of this path
 constexpr int WH = 128;  // output columns of one wave (one half of the row)
 
-template <class Pol> struct WTile;
-template <> struct WTile<PolBF16> { using type = TTileBF16<WH>; };
-template <> struct WTile<PolF32> { using type = TTileF32<WH>; };
+using Pol = PolF32;
 
 // acc += A B^T over the 256 elements of rows ra (A: lane (m, g) supplies row m) and rb (B: lane
 // (n, g) supplies row n); a null row reads as zeros.  Both operands take their elements in the
-// same order, streamed from memory four MFMA steps at a time (nothing resident).
-template <class Pol>
-__device__ __forceinline__ f32x16 dot256(const typename Pol::T* ra, const typename Pol::T* rb, int g, f32x16 acc) {
-  if constexpr (sizeof(typename Pol::T) == 2) {
-    // bf16: step t takes elements 16 t + 8 g .. + 7 (16 steps)
+// same order (lane half g: elements 128 g .. 128 g + 127, one per step), streamed from memory
+// sixteen MFMA steps at a time (nothing resident).
+__device__ __forceinline__ f32x16 dot256(const float* ra, const float* rb, int g, f32x16 acc) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      bf16x8 a[4], b[4];
+  for (int c = 0; c < 8; ++c) {
+    f32x4 a[4], b[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int e = 16 * (4 * c + u) + 8 * g;
-        a[u] = ra ? *reinterpret_cast<const bf16x8*>(ra + e) : bf16x8{};
-        b[u] = rb ? *reinterpret_cast<const bf16x8*>(rb + e) : bf16x8{};
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) acc = Pol::mma(a[u], b[u], acc);
+    for (int u = 0; u < 4; ++u) {
+      const int e = 128 * g + 16 * c + 4 * u;
+      a[u] = ra ? *reinterpret_cast<const f32x4*>(ra + e) : f32x4{0.f, 0.f, 0.f, 0.f};
+      b[u] = rb ? *reinterpret_cast<const f32x4*>(rb + e) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
-  } else {
-    // fp32: lane half g takes elements 128 g .. 128 g + 127, one per step (128 steps)
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      f32x4 a[4], b[4];
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int e = 128 * g + 16 * c + 4 * u;
-        a[u] = ra ? *reinterpret_cast<const f32x4*>(ra + e) : f32x4{0.f, 0.f, 0.f, 0.f};
-        b[u] = rb ? *reinterpret_cast<const f32x4*>(rb + e) : f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int x = 0; x < 4; ++x) acc = Pol::mma(a[u][x], b[u][x], acc);
-    }
+      for (int x = 0; x < 4; ++x) acc = Pol::mma(a[u][x], b[u][x], acc);
   }
   return acc;
 }
@@ -82,31 +64,16 @@ __device__ __forceinline__ TRef<T> half_of(const TRef<T>& x, int hh) {
   return TRef<T>{x.p + WH * hh, x.sb, x.sh, x.st};
 }
 
-template <class Pol, class TT>
-__device__ __forceinline__ void wide_stage(TT& tt, const TRef<const typename Pol::T>& x, int b, int h, int r0, int n) {
-  if constexpr (sizeof(typename Pol::T) == 2) {
-    tt.stage(x, b, h, r0, n);
-    wave_lds_sync();
-  } else {
-    tt.set(x, b, h, r0, n);
-  }
-}
-template <class Pol, class TT>
-__device__ __forceinline__ void wide_release(TT&) {
-  if constexpr (sizeof(typename Pol::T) == 2) wave_lds_sync();
-}
-
 // acc (this wave's 128 columns of a row, transposed C layout: lane = row, value r of column block
 // c = column 32 c + crow(r, g) of the half) += tile^T e, e a 32 x 32 C tile packed as B operands.
-template <class Pol, class TT>
-__device__ __forceinline__ void acc_tile(f32x16 (&acc)[WH / 32], const TT& tt, const f32x16& e) {
-  constexpr int NS = 32 / Pol::KS;
+__device__ __forceinline__ void acc_tile(f32x16 (&acc)[WH / 32], const TRef<const float>& x, int b, int h, int r0,
+                                         int n, const f32x16& e) {
+  TTileF32<WH> tt;
+  tt.set(x, b, h, r0, n);
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const typename Pol::frag bp = Pol::pack_c(e, s);
+  for (int s = 0; s < 16; ++s)
 #pragma unroll
-    for (int c = 0; c < WH / 32; ++c) acc[c] = Pol::mma(tt.frag(s, c), bp, acc[c]);
-  }
+    for (int c = 0; c < WH / 32; ++c) acc[c] = Pol::mma(tt.frag(s, c), e[s], acc[c]);
 }
 
 // Partial dot x^ . acc over this wave's half of the row (x^ = x rinv), the same in both lanes of
@@ -205,10 +172,9 @@ __global__ void __launch_bounds__(256) wide_norms(FwdParams P) {
 // One wave per (query tile, half, head), four independent waves per workgroup, longest query
 // tiles first.  Score tiles S^T = K Q^T (lane = query, values = 16 keys of the tile), as in the
 // d <= 128 kernels; the weights pack into the B operand of out_half^T += V_half^T A^T.
-template <class Pol, int BR, int PK, bool NORM>
+template <int BR, int PK, bool NORM>
 __global__ void __launch_bounds__(256) wide_fwd(FwdParams P) {
-  using T = typename Pol::T;
-  using TT = typename WTile<Pol>::type;
+  using T = float;
   constexpr int ND = WH / 32;
   const int l = lane_id(), n32 = l & 31, g = l >> 5, wv = threadIdx.x >> 6;
   const int BH = P.B * P.H;
@@ -250,9 +216,6 @@ __global__ void __launch_bounds__(256) wide_fwd(FwdParams P) {
   float lam = 0.f;
   if constexpr (BR == 2) lam = clamp01(*P.lam);
 
-  __shared__ __attribute__((aligned(16))) bf16 lds_all[(sizeof(T) == 2) ? 4 * TTileBF16<WH>::ELEMS : 8];
-  TT vt;
-  if constexpr (sizeof(T) == 2) vt.lds = lds_all + wv * TTileBF16<WH>::ELEMS;
 
   f32x16 O[ND];
 #pragma unroll
@@ -266,9 +229,9 @@ __global__ void __launch_bounds__(256) wide_fwd(FwdParams P) {
     const int k0 = kt * 32;
     const int j = k0 + n32;  // key row this lane supplies to the A operand
     const bool jv = j < Nk;
-    f32x16 S1 = dot256<Pol>(jv ? k1.row(b, h, j) : nullptr, qr1, g, f32x16{});
+    f32x16 S1 = dot256(jv ? k1.row(b, h, j) : nullptr, qr1, g, f32x16{});
     f32x16 S2 = f32x16{};
-    if constexpr (BR == 2) S2 = dot256<Pol>(jv ? k2.row(b, h, j) : nullptr, qr2, g, f32x16{});
+    if constexpr (BR == 2) S2 = dot256(jv ? k2.row(b, h, j) : nullptr, qr2, g, f32x16{});
     float rk1 = 1.f, rk2 = 1.f;
     if constexpr (NORM) {
       rk1 = jv ? nk1[j] : 0.f;
@@ -309,9 +272,7 @@ __global__ void __launch_bounds__(256) wide_fwd(FwdParams P) {
         }
         C[r] = a;
       }
-      wide_stage<Pol>(vt, vh, b, h, k0, Nk);
-      acc_tile<Pol>(O, vt, C);
-      wide_release<Pol>(vt);
+      acc_tile(O, vh, b, h, k0, Nk, C);
     }
     if (occrow && (((kt & 31) == 31) || kt == ktl)) {
       if (l == 0) {
@@ -347,10 +308,9 @@ __global__ void __launch_bounds__(256) wide_fwd(FwdParams P) {
 // Dp_ij = dO_i . v_j: dS1 = G1 Dp, dS2 = -lam G2 Dp, dq^_i = sum_j dS_ij rk_j k_j, and
 // dq = (dq^ - q^ (q^ . dq^)) rq; dbeta = -sum_i c_i sum_j (dS1 + dS2), dlambda = -sum A2 Dp.
 // Without the bitmask every causal tile is tested.
-template <class Pol, int BR, int PK, bool NORM>
+template <int BR, int PK, bool NORM>
 __global__ void __launch_bounds__(128) wide_bwd_dq(BwdParams P) {
-  using T = typename Pol::T;
-  using TT = typename WTile<Pol>::type;
+  using T = float;
   constexpr int ND = WH / 32;
   const int l = lane_id(), n32 = l & 31, g = l >> 5, hh = threadIdx.x >> 6;
   const int BH = P.B * P.H;
@@ -392,10 +352,7 @@ __global__ void __launch_bounds__(128) wide_bwd_dq(BwdParams P) {
   const float* nk1 = NORM ? P.norms + norm_base(P, N_K1, bh) : nullptr;
   const float* nk2 = NORM ? P.norms + norm_base(P, N_K2, bh) : nullptr;
 
-  __shared__ __attribute__((aligned(16))) bf16 lds_all[(sizeof(T) == 2) ? 2 * TTileBF16<WH>::ELEMS : 8];
   __shared__ float red[2][2][32];  // [branch][half][row]: the halves' partial row dots
-  TT tile;
-  if constexpr (sizeof(T) == 2) tile.lds = lds_all + hh * TTileBF16<WH>::ELEMS;
   const TRef<const T> k1h = half_of(k1, hh), k2h = half_of(k2, hh);
 
   f32x16 A1[ND], A2[ND];
@@ -418,9 +375,9 @@ __global__ void __launch_bounds__(128) wide_bwd_dq(BwdParams P) {
     const int j = k0 + n32;
     const bool jv = j < Nk;
     f32x16 S1 = f32x16{}, S2 = f32x16{};
-    if (use1) S1 = dot256<Pol>(jv ? k1.row(b, h, j) : nullptr, qr1, g, S1);
-    if (BR == 2 && use2) S2 = dot256<Pol>(jv ? k2.row(b, h, j) : nullptr, qr2, g, S2);
-    const f32x16 Dp = dot256<Pol>(jv ? vv.row(b, h, j) : nullptr, dor, g, f32x16{});
+    if (use1) S1 = dot256(jv ? k1.row(b, h, j) : nullptr, qr1, g, S1);
+    if (BR == 2 && use2) S2 = dot256(jv ? k2.row(b, h, j) : nullptr, qr2, g, S2);
+    const f32x16 Dp = dot256(jv ? vv.row(b, h, j) : nullptr, dor, g, f32x16{});
     f32x16 E1, E2;
     bool any = false;
 #pragma unroll
@@ -451,14 +408,10 @@ __global__ void __launch_bounds__(128) wide_bwd_dq(BwdParams P) {
     if (!occrow && wave_ballot(any) == 0ull) continue;  // the same decision in both halves
     ++computed;
     if (use1) {
-      wide_stage<Pol>(tile, k1h, b, h, k0, Nk);
-      acc_tile<Pol>(A1, tile, E1);
-      wide_release<Pol>(tile);
+      acc_tile(A1, k1h, b, h, k0, Nk, E1);
     }
     if (BR == 2 && use2) {
-      wide_stage<Pol>(tile, k2h, b, h, k0, Nk);
-      acc_tile<Pol>(A2, tile, E2);
-      wide_release<Pol>(tile);
+      acc_tile(A2, k2h, b, h, k0, Nk, E2);
     }
   }
 
@@ -499,10 +452,9 @@ __global__ void __launch_bounds__(128) wide_bwd_dq(BwdParams P) {
 // first; wave hh owns columns 128 hh .. of dk1, dk2 and dv.  Scores S = Q K^T (lane = key,
 // values = 16 queries of the tile): dv_j += sum_i (A1 - lam A2)_ij dO_i, dk^_j += sum_i dS_ij
 // rq_i q_i, then the normalize backward.
-template <class Pol, int BR, int PK, bool NORM>
+template <int BR, int PK, bool NORM>
 __global__ void __launch_bounds__(128) wide_bwd_dkv(BwdParams P) {
-  using T = typename Pol::T;
-  using TT = typename WTile<Pol>::type;
+  using T = float;
   constexpr int ND = WH / 32;
   const int l = lane_id(), n32 = l & 31, g = l >> 5, hh = threadIdx.x >> 6;
   const int BH = P.B * P.H;
@@ -542,10 +494,7 @@ __global__ void __launch_bounds__(128) wide_bwd_dkv(BwdParams P) {
   const float* nq1 = NORM ? P.norms + norm_base(P, N_Q1, bh) : nullptr;
   const float* nq2 = NORM ? P.norms + norm_base(P, N_Q2, bh) : nullptr;
 
-  __shared__ __attribute__((aligned(16))) bf16 lds_all[(sizeof(T) == 2) ? 2 * TTileBF16<WH>::ELEMS : 8];
   __shared__ float red[2][2][32];  // [branch][half][row]
-  TT tile;
-  if constexpr (sizeof(T) == 2) tile.lds = lds_all + hh * TTileBF16<WH>::ELEMS;
   const TRef<const T> q1h = half_of(q1, hh), q2h = half_of(q2, hh), doh = half_of(dO, hh);
 
   f32x16 AV[ND], AK1[ND], AK2[ND];
@@ -568,9 +517,9 @@ __global__ void __launch_bounds__(128) wide_bwd_dkv(BwdParams P) {
     const int ia = q0 + n32;  // query row this lane supplies to the A operand
     const bool iv = ia < Nq;
     f32x16 S1 = f32x16{}, S2 = f32x16{};
-    if (use1) S1 = dot256<Pol>(iv ? q1.row(b, h, ia) : nullptr, kr1, g, S1);
-    if (BR == 2 && use2) S2 = dot256<Pol>(iv ? q2.row(b, h, ia) : nullptr, kr2, g, S2);
-    const f32x16 Dp = dot256<Pol>(iv ? dO.row(b, h, ia) : nullptr, vr, g, f32x16{});
+    if (use1) S1 = dot256(iv ? q1.row(b, h, ia) : nullptr, kr1, g, S1);
+    if (BR == 2 && use2) S2 = dot256(iv ? q2.row(b, h, ia) : nullptr, kr2, g, S2);
+    const f32x16 Dp = dot256(iv ? dO.row(b, h, ia) : nullptr, vr, g, f32x16{});
     f32x16 EV, E1, E2;
     bool any = false;
 #pragma unroll
@@ -602,18 +551,12 @@ __global__ void __launch_bounds__(128) wide_bwd_dkv(BwdParams P) {
     }
     if (!occcol && wave_ballot(any) == 0ull) continue;  // the same decision in both halves
     ++computed;
-    wide_stage<Pol>(tile, doh, b, h, q0, Nq);
-    acc_tile<Pol>(AV, tile, EV);
-    wide_release<Pol>(tile);
+    acc_tile(AV, doh, b, h, q0, Nq, EV);
     if (use1) {
-      wide_stage<Pol>(tile, q1h, b, h, q0, Nq);
-      acc_tile<Pol>(AK1, tile, E1);
-      wide_release<Pol>(tile);
+      acc_tile(AK1, q1h, b, h, q0, Nq, E1);
     }
     if (BR == 2 && use2) {
-      wide_stage<Pol>(tile, q2h, b, h, q0, Nq);
-      acc_tile<Pol>(AK2, tile, E2);
-      wide_release<Pol>(tile);
+      acc_tile(AK2, q2h, b, h, q0, Nq, E2);
     }
   }
 
@@ -641,74 +584,79 @@ __global__ void __launch_bounds__(128) wide_bwd_dkv(BwdParams P) {
 }
 
 // ------------------------------------------------------------------ dispatch
-template <class Pol, int BR, int PK, bool NORM>
+template <class T, int BR>
+void launch_norms(const FwdParams& p, hipStream_t s) {
+  const int64_t rows = (int64_t)BR * p.B * p.H * ((int64_t)p.Nq + p.Nk);
+  hipLaunchKernelGGL((wide_norms<T, BR>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, s, p);
+  launched(s, "wide_norms");
+}
+template <int BR, int PK, bool NORM>
 int wide_fwd_t(const FwdParams& p, void* stream) {
   hipStream_t s = (hipStream_t)stream;
-  if (NORM) {
-    const int64_t rows = (int64_t)BR * p.B * p.H * ((int64_t)p.Nq + p.Nk);
-    hipLaunchKernelGGL((wide_norms<typename Pol::T, BR>), dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, s, p);
-    launched(s, "wide_norms");
-  }
+  if (NORM) launch_norms<float, BR>(p, s);
   const int64_t items = (int64_t)p.B * p.H * p.nqt * 2;
-  hipLaunchKernelGGL((wide_fwd<Pol, BR, PK, NORM>), dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, p);
+  hipLaunchKernelGGL((wide_fwd<BR, PK, NORM>), dim3((unsigned)((items + 3) / 4)), dim3(256), 0, s, p);
   launched(s, "wide_fwd");
   return (int)hipGetLastError();
 }
 
-template <class Pol, int BR, int PK, bool NORM>
+template <int BR, int PK, bool NORM>
 int wide_bwd_t(const BwdParams& p, void* stream) {
   hipStream_t s = (hipStream_t)stream;
   const int64_t qitems = (int64_t)p.B * p.H * p.nqt, kitems = (int64_t)p.B * p.H * p.nkt;
-  hipLaunchKernelGGL((wide_bwd_dq<Pol, BR, PK, NORM>), dim3((unsigned)qitems), dim3(128), 0, s, p);
+  hipLaunchKernelGGL((wide_bwd_dq<BR, PK, NORM>), dim3((unsigned)qitems), dim3(128), 0, s, p);
   launched(s, "wide_bwd_dq");
-  hipLaunchKernelGGL((wide_bwd_dkv<Pol, BR, PK, NORM>), dim3((unsigned)kitems), dim3(128), 0, s, p);
+  hipLaunchKernelGGL((wide_bwd_dkv<BR, PK, NORM>), dim3((unsigned)kitems), dim3(128), 0, s, p);
   launched(s, "wide_bwd_dkv");
   const int e = (int)hipGetLastError();
   return e ? e : launch_bwd_finish(p, BR, qitems, stream);
 }
 
-template <class Pol, int BR, int PK>
+template <int BR, int PK>
 int wfsel_norm(const FwdParams& p, const KernelKey& k, void* s) {
-  return k.normalize ? wide_fwd_t<Pol, BR, PK, true>(p, s) : wide_fwd_t<Pol, BR, PK, false>(p, s);
+  return k.normalize ? wide_fwd_t<BR, PK, true>(p, s) : wide_fwd_t<BR, PK, false>(p, s);
 }
-template <class Pol, int BR>
+template <int BR>
 int wfsel_pk(const FwdParams& p, const KernelKey& k, void* s) {
   switch (k.pkind) {
-    case 2: return wfsel_norm<Pol, BR, 2>(p, k, s);
-    case 1: return wfsel_norm<Pol, BR, 1>(p, k, s);
-    default: return wfsel_norm<Pol, BR, 0>(p, k, s);
+    case 2: return wfsel_norm<BR, 2>(p, k, s);
+    case 1: return wfsel_norm<BR, 1>(p, k, s);
+    default: return wfsel_norm<BR, 0>(p, k, s);
   }
 }
-template <class Pol>
 int wfsel_br(const FwdParams& p, const KernelKey& k, void* s) {
-  return k.branches == 2 ? wfsel_pk<Pol, 2>(p, k, s) : wfsel_pk<Pol, 1>(p, k, s);
+  return k.branches == 2 ? wfsel_pk<2>(p, k, s) : wfsel_pk<1>(p, k, s);
 }
 
-template <class Pol, int BR, int PK>
+template <int BR, int PK>
 int wbsel_norm(const BwdParams& p, const KernelKey& k, void* s) {
-  return k.normalize ? wide_bwd_t<Pol, BR, PK, true>(p, s) : wide_bwd_t<Pol, BR, PK, false>(p, s);
+  return k.normalize ? wide_bwd_t<BR, PK, true>(p, s) : wide_bwd_t<BR, PK, false>(p, s);
 }
-template <class Pol, int BR>
+template <int BR>
 int wbsel_pk(const BwdParams& p, const KernelKey& k, void* s) {
   switch (k.pkind) {
-    case 2: return wbsel_norm<Pol, BR, 2>(p, k, s);
-    case 1: return wbsel_norm<Pol, BR, 1>(p, k, s);
-    default: return wbsel_norm<Pol, BR, 0>(p, k, s);
+    case 2: return wbsel_norm<BR, 2>(p, k, s);
+    case 1: return wbsel_norm<BR, 1>(p, k, s);
+    default: return wbsel_norm<BR, 0>(p, k, s);
   }
 }
-template <class Pol>
 int wbsel_br(const BwdParams& p, const KernelKey& k, void* s) {
-  return k.branches == 2 ? wbsel_pk<Pol, 2>(p, k, s) : wbsel_pk<Pol, 1>(p, k, s);
+  return k.branches == 2 ? wbsel_pk<2>(p, k, s) : wbsel_pk<1>(p, k, s);
 }
 
 }  // namespace
 
 int launch_fwd_wide(const FwdParams& p, const KernelKey& k, void* stream) {
-  return k.dtype == 1 ? wfsel_br<PolBF16>(p, k, stream) : wfsel_br<PolF32>(p, k, stream);
+  if (k.dtype != 1) return wfsel_br(p, k, stream);
+  if (k.normalize) {
+    if (k.branches == 2) launch_norms<bf16, 2>(p, (hipStream_t)stream);
+    else launch_norms<bf16, 1>(p, (hipStream_t)stream);
+  }
+  return launch_fwd_blk256(p, k, stream);
 }
 
 int launch_bwd_wide(const BwdParams& p, const KernelKey& k, void* stream) {
-  return k.dtype == 1 ? wbsel_br<PolBF16>(p, k, stream) : wbsel_br<PolF32>(p, k, stream);
+  return k.dtype == 1 ? launch_bwd_blk256(p, k, stream) : wbsel_br(p, k, stream);
 }
 
 }  // namespace tda

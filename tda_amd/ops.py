@@ -455,9 +455,10 @@ class TDAFunction(torch.autograd.Function):
                 occ_p = base + o_o
                 pairs_p = base + o_p if o_p >= 0 else 0
         all_inputs = ng[0] and ng[1] and ng[4] and (branches == 1 or (ng[2] and ng[3]))
-        if need and bf16 and all_inputs and grad_prealloc_enabled():
+        if need and bf16 and all_inputs and q1.shape[3] <= 128 and grad_prealloc_enabled():
             # the gradients, cleared by this forward while its matrix-core pass runs: the pair
-            # backward then stores only the rows a non-zero weight reaches
+            # backward then stores only the rows a non-zero weight reaches (head_dim 256 has no
+            # pair lists: its backward stores every row)
             srcs = [q1, k1, q2, k2, v] if branches == 2 else [q1, k1, None, None, v]
             gbuf = torch.empty(sum(0 if t is None else t.numel() for t in srcs), dtype=q1.dtype, device=dev)
             zero_p, zero_bytes = gbuf.data_ptr(), gbuf.numel() * gbuf.element_size()

@@ -28,10 +28,11 @@ def _inputs(b, h, nq, nk, d, br, dtype, seed):
     (100, 700, 64, 2, 2.0, 0.5),     # fewer query tiles than key tiles (a key cache)
     (200, 90, 128, 2, 3.0, 0.4),     # fewer key tiles than query tiles
     (33, 4200, 64, 2, 2.0, 0.5),     # more key tiles than the queue holds: no queue
+    (40, 66000, 64, 1, 2.0, 0.7),    # more kept tiles than one listing of the walk (2048)
 ])
 def test_overflowing_lists_against_the_oracle(nq, nk, d, br, p, beta):
     off = max(nk - nq, 0)
-    rows, do = _inputs(1, 3, nq, nk, d, br, torch.bfloat16, 31)
+    rows, do = _inputs(1, 3 if nk < 10000 else 1, nq, nk, d, br, torch.bfloat16, 31)
     leaves = [x.cuda().requires_grad_(True) for x in rows]
     bt = torch.tensor(beta, device="cuda", requires_grad=True)
     lt = torch.tensor(0.4, device="cuda", requires_grad=True)
