@@ -753,10 +753,11 @@ int launch_zero(const FwdParams& p, void* stream) {
   return (int)hipGetLastError();
 }
 
-// head_dim 256 runs tda_wide.hip; otherwise bf16 runs the screen + sparse A.V kernels (tda_fwd_sparse.hip), or with a single query tile
-// the split-key decode kernels (tda_fwd_decode.hip); fp32 runs fwd_wave, after the int8 screen
-// when normalised with more than one query tile.  The screens, and the bf16 block tile pass
-// without normalisation, clear the call's zero range; the other paths launch zero_range.
+// head_dim 256 runs tda_wide.hip; a single query tile the split-key decode kernels
+// (tda_fwd_decode.hip); otherwise bf16 runs the screen + sparse A.V kernels (tda_fwd_sparse.hip) and
+// fp32 the int8 screen, fwd_cand_f32 and fwd_wave when normalised, fwd_wave_blk when not.  The
+// screens, and the bf16 block tile pass without normalisation, clear the call's zero range; the
+// other paths launch zero_range.
 int launch_fwd(const FwdParams& p, const KernelKey& k, void* stream) {
   if (p.zero && p.zero_per_it == 0) {
     // a zero range too large for the screen's per-item slices: cleared whole first
@@ -772,10 +773,13 @@ int launch_fwd(const FwdParams& p, const KernelKey& k, void* stream) {
     e = launch_fwd_wide(p, k, stream);
     return e ? e : launch_zero(p, stream);
   }
-  if (k.dtype == 1 && !(p.nqt == 1 && p.part)) return launch_fwd_sparse(p, k, stream);
-  if (k.dtype == 1) e = launch_fwd_decode(p, k, p.part, stream);
-  else e = sel_d<PolF32>(p, k, stream);
-  const bool screened = k.dtype == 0 && k.normalize && p.k8 && p.nqt > 1;  // the screen cleared it
+  if (p.nqt == 1) {  // (the workspace holds the partial outputs of a single query tile)
+    e = launch_fwd_decode(p, k, p.part, stream);
+    return e ? e : launch_zero(p, stream);
+  }
+  if (k.dtype == 1) return launch_fwd_sparse(p, k, stream);
+  e = sel_d<PolF32>(p, k, stream);
+  const bool screened = k.normalize;  // the screen cleared it
   return e ? e : screened ? 0 : launch_zero(p, stream);
 }
 

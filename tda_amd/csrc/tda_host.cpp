@@ -72,14 +72,15 @@ int64_t occ_words(int64_t bh, int64_t seq_len, int64_t seq_len_kv, int64_t branc
 }
 // Forward workspace: the bitmask scratch (used when the caller asks for no occupancy output;
 // the bf16 forward always builds the bitmask), then, when there is a single query tile
-// (seq_len <= 32), the per-chunk partial outputs of the bf16 decode kernels:
-// [B*H][ceil(key tiles / 32)][seq_len][128] floats (head_dim <= 128) ...
+// (seq_len <= 32), the per-chunk partial outputs of the decode kernels:
+// [B*H][chunks of dec_chunk_tiles key tiles][seq_len][128] floats (head_dim <= 128) ...
 int64_t fwd_occ_bytes(int64_t bh, int64_t seq_len, int64_t seq_len_kv, int64_t branches) {
   return round256(occ_words(bh, seq_len, seq_len_kv, branches) * (int64_t)sizeof(uint32_t));
 }
 int64_t fwd_part_bytes(int64_t bh, int64_t seq_len, int64_t seq_len_kv) {
   if (seq_len > 32) return 0;
-  return round256(bh * ceil_div(ceil_div(seq_len_kv, 32), 32) * seq_len * 128 * (int64_t)sizeof(float));
+  const int64_t nkt = ceil_div(seq_len_kv, 32);
+  return round256(bh * ceil_div(nkt, tda::dec_chunk_tiles(bh, seq_len, nkt)) * seq_len * 128 * (int64_t)sizeof(float));
 }
 // ... or, with more than one query tile, the candidate lists of the bf16 screen.
 // ... and a queue of query tiles for the tile pass (a count block, one item per (head, tile)).

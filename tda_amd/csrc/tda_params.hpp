@@ -125,6 +125,15 @@ struct BwdParams {
   int grads_zeroed;          // the gradient rows hold zeros: the pair passes store named rows only
 };
 
+// Key tiles per workgroup of the decode kernels (tda_fwd_decode.hip), whose partial outputs are
+// [B*H][ceil(nkt / tiles)][Nq][D] floats: 32 (a bitmask word) when that makes the two workgroups per
+// CU that fit, else 8 (a byte of one), so that a short or small cache still spreads over the GPU (8
+// heads, 1000 keys, d = 64, two branches: 8 workgroups and 33 us against 32 and 15 us).  Its
+// partials stay within 4 MiB, so no call grows past the library's own scratch array.
+constexpr int64_t dec_chunk_tiles(int64_t bh, int64_t nq, int64_t nkt) {
+  return bh * ((nkt + 31) / 32) < 512 && bh * ((nkt + 7) / 8) * nq <= 8192 ? 8 : 32;
+}
+
 // Kernel-family launchers (return a hipError_t value).  Template selection happens inside.
 struct KernelKey {
   int dtype;      // 0 f32, 1 bf16
