@@ -123,7 +123,10 @@ typedef struct tda_fwd_args {
                                the larger tda_fwd_workspace_bytes_kv()), 16-byte aligned: holds
                                the tile bitmask when occupancy is NULL and, when seq_len <= 32,
                                the fp32 per-chunk partial outputs of the single-query-tile
-                               (decode) kernels, else the screen's candidate keys per (branch,
+                               (decode) kernels (which split a short or small key cache
+                               finer where workspace_bytes has batch * heads *
+                               ceil(seq_len_kv / 256) * seq_len * 512 bytes more), else the
+                               screen's candidate keys per (branch,
                                head, query tile) and, for normalised calls of either dtype at
                                head_dim 64 or 128 with more than 32 query rows, the key rows
                                quantised to int8 for the screen (head_dim + 8 bytes per key row

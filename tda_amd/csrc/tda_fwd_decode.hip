@@ -309,7 +309,7 @@ __global__ void __launch_bounds__(256) fwd_decode_sum(FwdParams P, const float* 
 template <class Pol, int D, int BR, int PK, bool NORM>
 int launch_decode_t(const FwdParams& p, float* part, hipStream_t s) {
   const int BH = p.B * p.H;
-  const int ct = (int)dec_chunk_tiles(BH, p.Nq, p.nkt), nch = (p.nkt + ct - 1) / ct;
+  const int ct = p.dec_ct, nch = (p.nkt + ct - 1) / ct;
   if (ct == 8)
     hipLaunchKernelGGL((fwd_decode<Pol, D, BR, PK, NORM, 8>), dim3((unsigned)(BH * nch)), dim3(64 * kDecWaves), 0, s, p, part);
   else

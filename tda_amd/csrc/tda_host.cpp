@@ -73,14 +73,16 @@ int64_t occ_words(int64_t bh, int64_t seq_len, int64_t seq_len_kv, int64_t branc
 // Forward workspace: the bitmask scratch (used when the caller asks for no occupancy output;
 // the bf16 forward always builds the bitmask), then, when there is a single query tile
 // (seq_len <= 32), the per-chunk partial outputs of the decode kernels:
-// [B*H][chunks of dec_chunk_tiles key tiles][seq_len][128] floats (head_dim <= 128) ...
+// [B*H][ceil(key tiles / 32)][seq_len][128] floats (head_dim <= 128) ...
 int64_t fwd_occ_bytes(int64_t bh, int64_t seq_len, int64_t seq_len_kv, int64_t branches) {
   return round256(occ_words(bh, seq_len, seq_len_kv, branches) * (int64_t)sizeof(uint32_t));
 }
+int64_t fwd_part_bytes_ct(int64_t bh, int64_t seq_len, int64_t seq_len_kv, int64_t ct) {
+  return round256(bh * ceil_div(ceil_div(seq_len_kv, 32), ct) * seq_len * 128 * (int64_t)sizeof(float));
+}
 int64_t fwd_part_bytes(int64_t bh, int64_t seq_len, int64_t seq_len_kv) {
   if (seq_len > 32) return 0;
-  const int64_t nkt = ceil_div(seq_len_kv, 32);
-  return round256(bh * ceil_div(nkt, tda::dec_chunk_tiles(bh, seq_len, nkt)) * seq_len * 128 * (int64_t)sizeof(float));
+  return fwd_part_bytes_ct(bh, seq_len, seq_len_kv, 32);
 }
 // ... or, with more than one query tile, the candidate lists of the bf16 screen.
 // ... and a queue of query tiles for the tile pass (a count block, one item per (head, tile)).
@@ -299,8 +301,14 @@ int32_t tda_fwd(const tda_fwd_args* a, void* stream) {
   p.occ = a->occupancy ? a->occupancy : static_cast<uint32_t*>(a->workspace);
   char* after_occ = static_cast<char*>(a->workspace) +
                    fwd_occ_bytes(a->batch * a->heads, a->seq_len, c.seq_len_kv, a->branches);
-  if (a->seq_len <= 32) p.part = reinterpret_cast<float*>(after_occ);
-  else {
+  if (a->seq_len <= 32) {
+    // the finer chunks where the caller's workspace has room for their partial outputs
+    const int64_t bh = a->batch * a->heads;
+    const int64_t room = (int64_t)a->workspace_bytes - fwd_occ_bytes(bh, a->seq_len, c.seq_len_kv, a->branches);
+    const int64_t ct = tda::dec_chunk_tiles(bh, a->seq_len, p.nkt);
+    p.part = reinterpret_cast<float*>(after_occ);
+    p.dec_ct = fwd_part_bytes_ct(bh, a->seq_len, c.seq_len_kv, ct) <= room ? (int)ct : 32;
+  } else {
     const int64_t bh = a->batch * a->heads;
     p.cand = reinterpret_cast<uint32_t*>(after_occ);
     p.pvq = reinterpret_cast<uint32_t*>(after_occ + fwd_cand_list_bytes(bh, a->seq_len, a->branches));

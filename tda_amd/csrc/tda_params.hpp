@@ -80,7 +80,8 @@ struct FwdParams {
   float* norms;              // may be null
   uint32_t* occ;             // may be null (bf16: never, the host points it at workspace)
   unsigned long long* stats; // may be null
-  float* part;               // bf16 with one query tile: per-chunk partial outputs (workspace)
+  float* part;               // one query tile: per-chunk partial outputs (workspace)
+  int dec_ct;                // and the key tiles per chunk, 32 or 8 (dec_chunk_tiles)
   uint32_t* pairs;           // may be null: pair lists (bf16)
   uint32_t* colcnt;          // may be null: column bucket counts and entries (in pairs)
   uint32_t* colbuf;
@@ -129,7 +130,8 @@ struct BwdParams {
 // [B*H][ceil(nkt / tiles)][Nq][D] floats: 32 (a bitmask word) when that makes the two workgroups per
 // CU that fit, else 8 (a byte of one), so that a short or small cache still spreads over the GPU (8
 // heads, 1000 keys, d = 64, two branches: 8 workgroups and 33 us against 32 and 15 us).  Its
-// partials stay within 4 MiB, so no call grows past the library's own scratch array.
+// partials stay within 4 MiB.  Only where the caller's workspace has the room (the size functions
+// ask for 32); the Python entry points allocate it.
 constexpr int64_t dec_chunk_tiles(int64_t bh, int64_t nq, int64_t nkt) {
   return bh * ((nkt + 31) / 32) < 512 && bh * ((nkt + 7) / 8) * nq <= 8192 ? 8 : 32;
 }

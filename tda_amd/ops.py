@@ -193,6 +193,10 @@ def _fwd_template(ts, branches, normalize, relu_power, q_offset, zero_bytes):
                 getattr(a, name).stride[:] = t.stride()
         a.zero_bytes = zero_bytes
         ws = _abi.load().tda_fwd_workspace_bytes_for(ctypes.byref(a))
+        b, h, n, d = q1.shape
+        fine = b * h * -(-k1.shape[2] // 256) * n
+        if n <= 32 and d <= 128 and fine <= 8192:
+            ws += 512 * fine  # room for a finer split of the keys of a single query tile
         a.workspace_bytes = (ws + 255) // 256 * 256
         return bytes(a), a.workspace_bytes
 

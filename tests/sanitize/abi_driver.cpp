@@ -146,6 +146,11 @@ int main() {
     CHECK(stub::last_fwd.zero == nullptr && stub::last_fwd.k8 == nullptr);
     a.normalize = 0;  // one query tile and no normalisation: no int8 keys either way
     CHECK(tda_fwd_workspace_bytes_for(&a) == tda_fwd_workspace_bytes_kv(1, 2, 5, 900, 1));
+    // the finer key split of a single query tile only in a workspace with room for its partials
+    a.workspace_bytes = tda_fwd_workspace_bytes_for(&a);
+    CHECK(tda_fwd(&a, nullptr) == TDA_OK && stub::last_fwd.dec_ct == 32);
+    a.workspace_bytes += 2 * 4 * 5 * 512;
+    CHECK(tda_fwd(&a, nullptr) == TDA_OK && stub::last_fwd.dec_ct == 8);
   }
   {
     tda_fwd_args a = fwd_args(1, 2, 100, 64, 2);
