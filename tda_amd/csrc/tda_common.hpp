@@ -349,4 +349,90 @@ __device__ __forceinline__ bf16x8 tile_tr_frag(const bf16* tile, int st, int dsu
   return out;
 }
 
+// ------------------------------------------------------------------ fp32 wave tiles
+// A wave's own 32-row fp32 tile: the next one's rows in flight in registers (load), the current one
+// in the wave's LDS slice (store), read as row fragments (f32_rows_mma) or by columns (f32_cols_mma).
+// Waves per workgroup of the fp32 split passes (one resident tile each): four below 2048 resident
+// tiles (two per SIMD: fewer leave SIMDs idle behind the longest causal row), then two, or one where
+// a row streams at most 16 tiles (the sum over the waves and the uneven deal would cost more than the
+// split gives) and from 4096 tiles at d = 128, where a SIMD holds one wave.  Steps of threshold_rela_triton: (2, 12, 1111, 64) 421 us with four tiles per
+// workgroup, one wave each; 259 with four waves per tile;
+// (2, 16, 2048, 128) 1632 with four, 1502 with two; (4, 16, 2048, 64) 1372 with two, 1432 with one;
+// (8, 32, 512, 64) 426 with two, 411 with one; the
+// differential step (4, 32, 1024, 128) 2980 with two, 2741 with one.
+constexpr int f32_split(int d, int64_t tiles, int streamed) {
+  return tiles < 2048 ? 4 : streamed <= 16 || (d > 64 && tiles >= 4096) ? 1 : 2;
+}
+template <int D>
+constexpr int kF32Stride = D + 4;  // LDS row stride: the row-fragment reads spread over the banks
+// Load instruction u: rows RPI u + l / CPR, 16-byte chunk l % CPR; rows past n read row n - 1 (their
+// products are masked).
+template <int D>
+struct F32Rows {
+  static constexpr int CPR = D / 4, RPI = 64 / CPR, LPW = 32 / RPI;
+  f32x4 v[LPW];
+  __device__ __forceinline__ void load(const TRef<const float>& x, int b, int h, int r0, int n) {
+    const int l = lane_id();
+#pragma unroll
+    for (int u = 0; u < LPW; ++u)
+      v[u] = *reinterpret_cast<const f32x4*>(x.row(b, h, min(r0 + RPI * u + l / CPR, n - 1)) + 4 * (l % CPR));
+  }
+  __device__ __forceinline__ void store(float* tile) const {
+    const int l = lane_id();
+#pragma unroll
+    for (int u = 0; u < LPW; ++u)
+      *reinterpret_cast<f32x4*>(tile + (RPI * u + l / CPR) * kF32Stride<D> + 4 * (l % CPR)) = v[u];
+  }
+};
+// S^T-layout product of a 32-row LDS tile (A operand: lane (m, g) row m, elements g D/2 + t)
+// with a lane's register fragments (B operand, load_rows order): lane n, value r = row crow(r, g).
+template <int D>
+__device__ __forceinline__ f32x16 f32_rows_mma(const float* tile, const float (&bf)[D / 2]) {
+  constexpr int NT = D / 2;
+  const int l = lane_id(), n32 = l & 31, g = l >> 5;
+  const float* p = tile + n32 * kF32Stride<D> + g * NT;
+  f32x16 acc = {};
+#pragma unroll
+  for (int m = 0; m < NT / 4; ++m) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(p + 4 * m);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = PolF32::mma(v[e], bf[4 * m + e], acc);
+  }
+  return acc;
+}
+// acc[c] += tile^T E over the tile's 32 rows (lane n, value r of block c = column 32 c + crow(r, g)):
+// step st takes rows crow(st, 0) and crow(st, 1), E's values st of lane n.
+template <int D>
+__device__ __forceinline__ void f32_cols_mma(const float* tile, const f32x16& E, f32x16 (&acc)[D / 32]) {
+  const int l = lane_id(), n32 = l & 31, g = l >> 5;
+#pragma unroll
+  for (int st = 0; st < 16; ++st) {
+    const float* p = tile + crow(st, g) * kF32Stride<D> + n32;
+#pragma unroll
+    for (int c = 0; c < D / 32; ++c) acc[c] = PolF32::mma(p[32 * c], E[st], acc[c]);
+  }
+}
+// The sum of the workgroup's W accumulators, in wave order, into wave 0's.  The waves' LDS
+// slices (`slice` floats each) carry them; every wave is done with its tiles, and on return wave 0
+// has read them all (a later write to a slice other than wave 0's needs a barrier of its own).
+template <int D, int W>
+__device__ __forceinline__ void f32_split_sum(float* lds, int slice, int wv, f32x16 (&acc)[D / 32]) {
+  if (W == 1) return;
+  const int l = lane_id();
+  if (wv) {
+    wave_lds_sync();
+#pragma unroll
+    for (int c = 0; c < D / 32; ++c)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) lds[wv * slice + (16 * c + r) * 64 + l] = acc[c][r];
+  }
+  __syncthreads();
+  if (wv) return;
+  for (int w = 1; w < W; ++w)
+#pragma unroll
+    for (int c = 0; c < D / 32; ++c)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[c][r] += lds[w * slice + (16 * c + r) * 64 + l];
+}
+
 }  // namespace tda

@@ -294,43 +294,37 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
   }
 }
 
-// ------------------------------------------------------------------ fwd_wave_blk
-// The fp32 pass without normalisation (every causal tile scored) over blocks of four
-// consecutive query tiles of one head, one wave each, as fwd_pv_blk does for bf16: the waves walk
-// the block's causal key tiles in step and share each tile's key rows (every branch) and V rows,
-// which the workgroup loads once (each wave a quarter of the rows, one tile ahead into
-// registers) into LDS; two barriers per tile (the tile is rewritten once every wave is done with
-// it).  A wave scores only the tiles its own query tile sees, with fwd_wave's arithmetic: the
-// key rows' fragments in the load_rows order (lane half g: elements g D/2 .. of row n), V^T one
-// key per lane half and step, the same test, weights, bitmask, counters and output.
-template <int D, int BR, int PK>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1)))
-fwd_wave_blk(FwdParams P) {
+// ------------------------------------------------------------------ fwd_split_f32
+// The fp32 pass without normalisation (every causal tile scored): one query tile per workgroup,
+// its key tiles dealt to the W waves in turn (wave w: key tiles w, w + W, ..), each wave staging
+// its own tiles (K per branch, then V, through one LDS slice; the next tile's rows in flight in
+// registers) with no barrier between them; the sums and the bitmask words meet in LDS.  A wave
+// scores with fwd_wave's arithmetic: row fragments in the load_rows order (lane half g: elements
+// g D/2 .. of row n), V^T one key per lane half and step, the same test and weights.
+// What bounds it is the fp32 products (64 cycles each, 64 per tile at d = 64): one wave per query
+// tile, four tiles to a workgroup, left the workgroup of a head's last tiles running alone: TRA (2, 12,
+// 1111, 64) 99 us so, 58 split; f32_split (tda_common.hpp) has the rule and its figures.
+template <int D, int BR, int PK, int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 64 && BR == 1 ? 2 : 1)))
+fwd_split_f32(FwdParams P) {
   using Pol = PolF32;
-  constexpr int W = 4, NT = D / 2, NS = 16, ND = D / 32;
-  constexpr int KS = D + 4;          // key tile row stride (floats)
-  constexpr int VS = D + 8;          // V tile row stride: rows 4 apart 32 banks apart
-  constexpr int CPR = D / 4;         // 16-byte chunks per row
-  constexpr int RPI = 64 / CPR;      // rows per load instruction
-  constexpr int LPW = 32 / RPI / W;  // load instructions per wave and matrix
-  static_assert(LPW >= 1 && LPW * RPI * W == 32, "tile rows split evenly over the waves");
-  __shared__ __attribute__((aligned(16))) float klds[BR][32 * KS];
-  __shared__ __attribute__((aligned(16))) float vlds[32 * VS];
+  constexpr int NT = D / 2, ND = D / 32;
+  constexpr int SL = 32 * kF32Stride<D>;  // a wave's LDS slice
+  constexpr int OW = 64;                  // bitmask words collected at a time (2048 key tiles)
+  __shared__ __attribute__((aligned(16))) float lds[W * SL];
+  __shared__ uint32_t words[BR][OW];
 
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
   const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int BH = P.B * P.H, Nq = P.Nq, Nk = P.Nk, nqt = P.nqt, qoff = P.qoff;
-  const int nqb = (nqt + W - 1) / W;
-  // longest blocks (last query tiles) of every head first
-  const int bid = blockIdx.x, jb = nqb - 1 - bid / BH, bh = bid % BH;
+  // longest rows (last query tiles) of every head first
+  const int bid = blockIdx.x, qt = nqt - 1 - bid / BH, bh = bid % BH;
   const int b = bh / P.H, h = bh % P.H;
-  const int qt = W * jb + wv;
-  const bool act = qt < nqt;  // wave-uniform: waves past the last query tile only load
   const int i = 32 * qt + n32;
-  const bool qvalid = act && i < Nq;
+  const bool qvalid = i < Nq;
   const int pq = qoff + i;
-  const int ktl = act ? kt_last(qt, qoff, P.nkt) : -1;                       // this wave's last key tile
-  const int ktl_b = kt_last(min(W * jb + W - 1, nqt - 1), qoff, P.nkt);  // the block's
+  const int ktl = kt_last(qt, qoff, P.nkt);
+  float* tile = lds + wv * SL;
 
   const TRef<const float> qr[2] = {{(const float*)P.in[F_Q1], P.s[F_Q1][0], P.s[F_Q1][1], P.s[F_Q1][2]},
                                    {(const float*)P.in[F_Q2], P.s[F_Q2][0], P.s[F_Q2][1], P.s[F_Q2][2]}};
@@ -347,108 +341,91 @@ fwd_wave_blk(FwdParams P) {
   float lam = 0.f;
   if constexpr (BR == 2) lam = clamp01(*P.lam);
 
-  // this wave's rows of a tile: RPI (LPW wv + u) + l / CPR, chunk l % CPR (rows past Nk: Nk - 1)
-  f32x4 kreg[BR][LPW], vreg[LPW];
-  auto issue = [&](int kt) {
-#pragma unroll
-    for (int u = 0; u < LPW; ++u) {
-      const int r = min(32 * kt + RPI * (LPW * wv + u) + l / CPR, Nk - 1);
-#pragma unroll
-      for (int br = 0; br < BR; ++br) kreg[br][u] = *reinterpret_cast<const f32x4*>(kr[br].row(b, h, r) + 4 * (l % CPR));
-      vreg[u] = *reinterpret_cast<const f32x4*>(vv.row(b, h, r) + 4 * (l % CPR));
-    }
-  };
-
+  F32Rows<D> kreg[BR], vreg;
   f32x16 O[ND];
 #pragma unroll
   for (int c = 0; c < ND; ++c) O[c] = f32x16{};
-  uint32_t* occrow = P.occ && act ? P.occ + ((int64_t)bh * nqt + qt) * P.occ_w : nullptr;
+  uint32_t* occrow = P.occ ? P.occ + ((int64_t)bh * nqt + qt) * P.occ_w : nullptr;
   const int64_t occ_br = (int64_t)BH * nqt * P.occ_w;  // distance between the branch planes
-  uint32_t word = 0, word2 = 0;
   unsigned visited = 0, computed = 0;
 
-  issue(0);
-  for (int kt = 0; kt <= ktl_b; ++kt) {
-    lds_barrier();  // every wave is done with the previous tile
+  if (wv <= ktl) {
 #pragma unroll
-    for (int u = 0; u < LPW; ++u) {
-      const int r = RPI * (LPW * wv + u) + l / CPR;
+    for (int br = 0; br < BR; ++br) kreg[br].load(kr[br], b, h, 32 * wv, Nk);
+    vreg.load(vv, b, h, 32 * wv, Nk);
+  }
+  for (int w0 = 0; w0 < P.occ_w; w0 += OW) {  // the same rounds in every wave
+    if (w0 > 0) __syncthreads();              // the previous round's words are stored
+    if (wv == 0) {
 #pragma unroll
-      for (int br = 0; br < BR; ++br) *reinterpret_cast<f32x4*>(klds[br] + r * KS + 4 * (l % CPR)) = kreg[br][u];
-      *reinterpret_cast<f32x4*>(vlds + r * VS + 4 * (l % CPR)) = vreg[u];
+      for (int br = 0; br < BR; ++br) words[br][l] = 0u;
     }
-    if (kt < ktl_b) issue(kt + 1);  // in flight during this tile's products
-    lds_barrier();                  // tile kt in LDS
-    if (kt > ktl) continue;         // (uniform) not seen by this wave's query tile
-    const int k0 = 32 * kt;
-    f32x16 S[BR];
+    __syncthreads();
+    for (int kt = 32 * w0 + wv; kt <= ktl && kt < 32 * (w0 + OW); kt += W) {
+      const int k0 = 32 * kt, kn = 32 * min(kt + W, ktl);  // kn: the next tile's rows (past the last: unused)
+      f32x16 S[BR];
 #pragma unroll
-    for (int br = 0; br < BR; ++br) {
-      S[br] = f32x16{};
-      const float* kp = klds[br] + n32 * KS + g * NT;
-#pragma unroll
-      for (int m = 0; m < NT / 4; ++m) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(kp + 4 * m);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) S[br] = Pol::mma(v[e], Q[br][4 * m + e], S[br]);
+      for (int br = 0; br < BR; ++br) {
+        wave_lds_sync();
+        kreg[br].store(tile);
+        kreg[br].load(kr[br], b, h, kn, Nk);
+        wave_lds_sync();
+        S[br] = f32_rows_mma<D>(tile, Q[br]);
       }
-    }
-    // threshold test: the tile max of the valid scores decides "any x > 0" exactly
-    bool any[2] = {false, false};
-#pragma unroll
-    for (int br = 0; br < BR; ++br) {
-      float m = -INFINITY;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = k0 + crow(r, g);
-        const bool valid = qvalid && key <= pq && key < Nk;
-        m = fmaxf(m, valid ? S[br][r] : -INFINITY);
-      }
-      any[br] = wave_ballot(m - tau > 0.f) != 0ull;
-    }
-    visited += BR;
-    computed += (any[0] ? 1 : 0) + (any[1] ? 1 : 0);
-    if (any[0]) word |= 1u << (kt & 31);
-    if (any[1]) word2 |= 1u << (kt & 31);
-    // the query tile's pairs are in no list: the column bucket of the key tile is incomplete
-    if (P.colcnt && (any[0] || any[1]) && l == 0) atomicOr(P.colcnt + (int64_t)bh * P.nkt + kt, kColTaint);
-    if (any[0] || any[1]) {
+      wave_lds_sync();
+      vreg.store(tile);
+      vreg.load(vv, b, h, kn, Nk);
+      wave_lds_sync();
+      // exact x; keys after the query's position, padding keys and rows past Nq set to -1 (only on
+      // the tiles that have any)
       f32x16 C;
+      bool any[2] = {false, false};
+      const bool edge = k0 + 31 > min(qoff + 32 * qt, Nk - 1) || 32 * qt + 31 >= Nq;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = k0 + crow(r, g);
-        const bool valid = qvalid && key <= pq && key < Nk;
-        const float x1 = __builtin_fmaf(S[0][r], 1.f, -tau);
-        float a = (valid && any[0] && x1 > 0.f) ? pow_p<PK>(x1, pw) : 0.f;
-        if constexpr (BR == 2) {
-          const float x2 = __builtin_fmaf(S[1][r], 1.f, -tau);
-          const float a2 = (valid && any[1] && x2 > 0.f) ? pow_p<PK>(x2, pw) : 0.f;
-          a = __builtin_fmaf(-lam, a2, a);
+      for (int br = 0; br < BR; ++br) {
+        f32x16 X;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) X[r] = __builtin_fmaf(S[br][r], 1.f, -tau);
+        if (edge) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = k0 + crow(r, g);
+            X[r] = qvalid && key <= pq && key < Nk ? X[r] : -1.f;
+          }
         }
-        C[r] = a;
-      }
+        float m = X[0];
 #pragma unroll
-      for (int st = 0; st < NS; ++st) {
-        const float* vp = vlds + crow(st, g) * VS + n32;
+        for (int r = 1; r < 16; ++r) m = fmaxf(m, X[r]);
+        any[br] = wave_ballot(m > 0.f) != 0ull;
 #pragma unroll
-        for (int c = 0; c < ND; ++c) O[c] = Pol::mma(vp[32 * c], C[st], O[c]);
+        for (int r = 0; r < 16; ++r) {
+          const float a = X[r] > 0.f ? pow_p<PK>(X[r], pw) : 0.f;
+          C[r] = br == 0 ? a : __builtin_fmaf(-lam, a, C[r]);
+        }
       }
-    }
-    if (occrow && (((kt & 31) == 31) || kt == ktl)) {
+      visited += BR;
+      computed += (any[0] ? 1 : 0) + (any[1] ? 1 : 0);
+      if (!any[0] && !any[1]) continue;
       if (l == 0) {
-        occrow[kt >> 5] = word;
-        if constexpr (BR == 2) occrow[occ_br + (kt >> 5)] = word2;
+        if (any[0]) atomicOr(&words[0][(kt >> 5) - w0], 1u << (kt & 31));
+        if (BR == 2 && any[1]) atomicOr(&words[BR - 1][(kt >> 5) - w0], 1u << (kt & 31));
+        // the query tile's pairs are in no list: the column bucket of the key tile is incomplete
+        if (P.colcnt) atomicOr(P.colcnt + (int64_t)bh * P.nkt + kt, kColTaint);
       }
-      word = word2 = 0;
+      f32_cols_mma<D>(tile, C, O);
+    }
+    __syncthreads();
+    if (occrow && wv == 0 && w0 + l < P.occ_w) {  // words past the row's last key tile: zeros
+#pragma unroll
+      for (int br = 0; br < BR; ++br) occrow[br * occ_br + w0 + l] = words[br][l];
     }
   }
-  if (!act) return;
-  if (occrow && l == 0) {
-    for (int w = (ktl >> 5) + 1; w < P.occ_w; ++w) {
-      occrow[w] = 0u;
-      if constexpr (BR == 2) occrow[occ_br + w] = 0u;
-    }
+  if (P.stats && l == 0 && visited) {
+    atomicAdd(P.stats + 0, (unsigned long long)visited);
+    atomicAdd(P.stats + 1, (unsigned long long)computed);
   }
+  f32_split_sum<D, W>(lds, SL, wv, O);
+  if (wv) return;
   if (P.pairs && l == 0) {  // this pass writes no pair list: the backward walks the tiles
 #pragma unroll
     for (int br = 0; br < BR; ++br)
@@ -461,10 +438,6 @@ fwd_wave_blk(FwdParams P) {
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         store4(orow + 32 * c + 8 * u + 4 * g, O[c][4 * u], O[c][4 * u + 1], O[c][4 * u + 2], O[c][4 * u + 3]);
-  }
-  if (P.stats && l == 0) {
-    atomicAdd(P.stats + 0, (unsigned long long)visited);
-    atomicAdd(P.stats + 1, (unsigned long long)computed);
   }
 }
 
@@ -707,9 +680,13 @@ static int launch_fwd_t(const FwdParams& p, const KernelKey& k, void* stream) {
     launched(stream, "fwd_cand_f32");
     const unsigned qgrid = (unsigned)(((items < 2048 ? items : 2048) + 3) / 4);
     hipLaunchKernelGGL((fwd_wave<Pol, D, BR, PK, NORM, NORM, NORM>), dim3(qgrid), dim3(256), 0, (hipStream_t)stream, p);
-  } else if (!NORM && p.nqt > 1) {  // blocks of query tiles sharing their key and V tiles
-    const unsigned blocks = (unsigned)(p.B * p.H * ((p.nqt + 3) / 4));
-    hipLaunchKernelGGL((fwd_wave_blk<D, BR, PK>), dim3(blocks), dim3(256), 0, (hipStream_t)stream, p);
+  } else if (!NORM && p.nqt > 1) {  // a query tile per workgroup, its key tiles split over the waves
+    if (f32_split(D, items, p.nkt) == 1)
+      hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 1>), dim3((unsigned)items), dim3(64), 0, (hipStream_t)stream, p);
+    else if (f32_split(D, items, p.nkt) == 2)
+      hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 2>), dim3((unsigned)items), dim3(128), 0, (hipStream_t)stream, p);
+    else
+      hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 4>), dim3((unsigned)items), dim3(256), 0, (hipStream_t)stream, p);
   } else {
     hipLaunchKernelGGL((fwd_wave<Pol, D, BR, PK, NORM>), dim3(grid), dim3(256), 0, (hipStream_t)stream, p);
   }
@@ -755,7 +732,7 @@ int launch_zero(const FwdParams& p, void* stream) {
 
 // head_dim 256 runs tda_wide.hip; a single query tile the split-key decode kernels
 // (tda_fwd_decode.hip); otherwise bf16 runs the screen + sparse A.V kernels (tda_fwd_sparse.hip) and
-// fp32 the int8 screen, fwd_cand_f32 and fwd_wave when normalised, fwd_wave_blk when not.  The
+// fp32 the int8 screen, fwd_cand_f32 and fwd_wave when normalised, fwd_split_f32 when not.  The
 // screens, and the bf16 block tile pass without normalisation, clear the call's zero range; the
 // other paths launch zero_range.
 int launch_fwd(const FwdParams& p, const KernelKey& k, void* stream) {

@@ -2,8 +2,8 @@
 README.md:20-31), where raw dot products of N(0, 1) rows pass their threshold about half the
 time and every causal tile holds weights.  The bf16 forward then runs the block tile pass
 (fwd_pv_blk: four query tiles per workgroup sharing each key tile) and the backward the block
-passes (bwd_dq_blk, bwd_dkv_blk) for every list past its cap; fp32 runs its own block passes
-(fwd_wave_blk, bwd_dq_blk_f32, bwd_dkv_blk_f32).
+passes (bwd_dq_blk, bwd_dkv_blk) for every list past its cap; fp32 runs its own split passes
+(fwd_split_f32, bwd_dq_split_f32, bwd_dkv_split_f32).
 
 Against the CPU oracle (fp64 autograd of the formula): the output and every gradient (dq1,
 dq2, dk1, dk2, dv, dbeta, dlambda) at 2e-2 (bf16) / 1e-4 (fp32) normwise, on shapes whose
@@ -197,7 +197,7 @@ def test_dense_bitmask_counts_and_determinism(branches):
 
 @pytest.mark.parametrize("branches", [1, 2])
 def test_dense_fp32_bitmask_and_offset(branches):
-    """fp32 without normalisation (the fp32 block passes): the gradients with the forward's
+    """fp32 without normalisation (the fp32 split passes): the gradients with the forward's
     bitmask and without one (every causal tile walked) agree bitwise, with a sparse bitmask
     (scaled-down queries: most tiles hold no weight); a second call is bitwise equal; and a
     chunked-prefill offset with keys past the last query position is held to 1e-4 against the
