@@ -874,31 +874,29 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
 // the epilogue and in the dbeta sum), and the branch that counts -lambda in dv runs first, its sum
 // scaled before the other's is added.
 // At d = 256 a tile's row fragments and accumulators do not fit one wave's registers, so two waves
-// share each tile (kSplit): each contracts its half of the d elements of the scores and of dP, adds
-// the other's half through LDS (the same sums in both, so the same decisions) and owns its half of
-// the gradient columns; the normalize backward's row dots are added the same way.
-// TDA (2, 8, 1000, 256): 47 + 107 us against 113 + 224 with two waves per tile fetching their own rows.
-// The split key-major blocks hold two tiles, four waves with a SIMD each (four tiles, two waves per
-// SIMD, spill 76-195 VGPRs).
+// share each tile (kSplit): wave 0 forms the scores and wave 1 dP, each in one chain over the row (the
+// forward's bits, so the same weights), they exchange them through LDS, and each owns half of the
+// gradient columns; the normalize backward's row dots are added through LDS in half order.  There the
+// weights and dS carry their coefficients (-lambda, 2) before their rounding to bf16, and the
+// key-major pass (bwd_dkv_wide) combines both branches' weights in fp32, rounded once for dv.
 template <int D>
 constexpr int kSplit = D > 128 ? 2 : 1;
 template <int D>
-constexpr int kKeyBlk = D > 128 ? 2 : kBwdBlk;
-template <int D>
 constexpr int kQryThreads = 64 * kBwdBlk * kSplit<D>;
-template <int D>
-constexpr int kKeyThreads = 64 * kKeyBlk<D> * kSplit<D>;
 
-// The partial values of a tile's two waves added through LDS: give writes the wave's, take (after
-// a barrier) returns half 0's plus half 1's.
-__device__ __forceinline__ void give16(float (*x)[64], const f32x16& v) {
+// A wave's 16 values through LDS: give writes them, take (after a barrier) reads some wave's.
+__device__ __forceinline__ void give16(f32x4 (*x)[64], const f32x16& v) {
 #pragma unroll
-  for (int r = 0; r < 16; ++r) x[r][lane_id()] = v[r];
+  for (int u = 0; u < 4; ++u) x[u][lane_id()] = f32x4{v[4 * u], v[4 * u + 1], v[4 * u + 2], v[4 * u + 3]};
 }
-__device__ __forceinline__ f32x16 take16(const float (*other)[64], const f32x16& v) {
+__device__ __forceinline__ f32x16 take16(const f32x4 (*x)[64]) {
   f32x16 o;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) o[r] = v[r] + other[r][lane_id()];
+  for (int u = 0; u < 4; ++u) {
+    const f32x4 v = x[u][lane_id()];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[4 * u + e] = v[e];
+  }
   return o;
 }
 
@@ -955,7 +953,7 @@ struct BlkLds {
   bf16* ring;             // two stages of two tiles of D columns
   float (*vals)[2][32];   // [stage]: key norms; query norms and tau values
   bf16 (*rows)[32 * D];   // key-major, one wave per tile: each wave's key rows (swizzled)
-  float (*xch)[32][64];   // a split tile's waves: partial scores and dP
+  f32x4 (*xch)[4][64];    // a split tile's waves: its scores, its dP
   float (*dots)[2][32];   // and row dots
 };
 // Their declaration: W tiles; ROWS as above.
@@ -963,18 +961,18 @@ struct BlkLds {
   __shared__ __attribute__((aligned(16))) bf16 lds_ring[2 * 2 * 32 * D];                      \
   __shared__ __attribute__((aligned(16))) float lds_vals[2][2][32];                           \
   __shared__ __attribute__((aligned(16))) bf16 lds_rows[(ROWS) && kSplit<D> == 1 ? W : 1][(ROWS) && kSplit<D> == 1 ? 32 * D : 8]; \
-  __shared__ __attribute__((aligned(16))) float lds_xch[kSplit<D> == 2 ? 2 * W : 1][kSplit<D> == 2 ? 32 * 64 : 4]; \
+  __shared__ __attribute__((aligned(16))) f32x4 lds_xch[kSplit<D> == 2 ? 2 * W : 1][kSplit<D> == 2 ? 4 * 64 : 1]; \
   __shared__ float lds_dots[W][kSplit<D> == 2 ? 64 : 1];                                      \
   const BlkLds<D, W> L{lds_ring, lds_vals, reinterpret_cast<bf16(*)[32 * D]>(&lds_rows[0][0]),             \
-                       reinterpret_cast<float(*)[32][64]>(&lds_xch[0][0]), reinterpret_cast<float(*)[2][32]>(&lds_dots[0][0])}
+                       reinterpret_cast<f32x4(*)[4][64]>(&lds_xch[0][0]), reinterpret_cast<float(*)[2][32]>(&lds_dots[0][0])}
 template <int D, int BR, int PK, bool NORM>
 __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBwdBlk>& L, int jb, int br, int bh) {
-  constexpr int W = kBwdBlk, SP = kSplit<D>, NT = D / 16 / SP, ND = D / 32 / SP;
+  constexpr int W = kBwdBlk, SP = kSplit<D>, NT = D / 16, ND = D / 32 / SP;
   constexpr int STAGE = 2 * 32 * D;  // K tile, V tile
   bf16* ring = L.ring;
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
   const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int wv = wid / SP, hh = wid % SP;  // the wave's tile of the block, its half of d and of the columns
+  const int wv = wid / SP, hh = wid % SP;  // the wave's tile of the block, its half of the columns
   const int BH = P.B * P.H, nqt = P.nqt, Nq = P.Nq, Nk = P.Nk, qoff = P.qoff;
   const int b = bh / P.H, h = bh % P.H;
   const uint32_t* counts = P.pairs ? P.pairs + pair_lists(BR, BH, nqt) * 4 * kPairCap : nullptr;
@@ -1000,14 +998,14 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBw
     return (const bf16*)P.in[slot] + (int64_t)b * P.s[slot][0] + (int64_t)h * P.s[slot][1];
   };
   const int qslot = br == 0 ? B_Q1 : B_Q2, kslot = br == 0 ? B_K1 : B_K2;
-  bf16x8 DO[NT], Q[NT];
+  bf16x8 DO[SP == 1 ? NT : 1], Q[NT];  // (a split tile: Q holds the wave's operand, wave 1's is dO)
   {
     const bf16* r = base(B_DO) + (int64_t)ic * P.s[B_DO][2];
-    const bf16* rq_ = base(qslot) + (int64_t)ic * P.s[qslot][2];
+    const bf16* rq_ = SP == 2 && hh ? r : base(qslot) + (int64_t)ic * P.s[qslot][2];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      DO[t] = *reinterpret_cast<const bf16x8*>(r + 16 * (t + NT * hh) + 8 * g);
-      Q[t] = *reinterpret_cast<const bf16x8*>(rq_ + 16 * (t + NT * hh) + 8 * g);
+      if constexpr (SP == 1) DO[t] = *reinterpret_cast<const bf16x8*>(r + 16 * t + 8 * g);
+      Q[t] = *reinterpret_cast<const bf16x8*>(rq_ + 16 * t + 8 * g);
     }
   }
   const float rq = NORM ? P.norms[norm_base(P, br == 0 ? N_Q1 : N_Q2, bh) + ic] : 1.f;
@@ -1016,7 +1014,7 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBw
   const float pw = P.p;
   float coef = 1.f;
   if constexpr (BR == 2) coef = br == 0 ? 1.f : -clamp01(*P.lam);
-  const float ds_scale = PK == 2 ? 2.f * coef : coef;
+  const float ds_scale = SP == 2 ? 1.f : PK == 2 ? 2.f * coef : coef;
   const bool want_l = BR == 2 && br == 1;  // dlambda comes from branch 2 alone
   const bf16* vb = base(B_V);
   const int64_t sv = P.s[B_V][2];
@@ -1093,13 +1091,6 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBw
     fetch(p);  // the tile AHEAD steps on, in flight during this tile's work
     lds_barrier();
     ++it;
-    auto products = [&](f32x16& S, f32x16& Dp) {
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        S = PolBF16::mma(tile_row_frag<D>(kst, t + NT * hh), Q[t], S);
-        Dp = PolBF16::mma(tile_row_frag<D>(vst, t + NT * hh), DO[t], Dp);
-      }
-    };
     auto tile = [&](const f32x16& S, const f32x16& Dp) {
       ++visited;
       const int k0 = 32 * kt;
@@ -1120,7 +1111,16 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBw
       }
       f32x16 E;
       float bt = 0.f, lt = 0.f;
-      if constexpr (PK == 2) {
+      if constexpr (SP == 2) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const bool pos = X[r] > 0.f;
+          const float ds = pos ? coef * dpow_p<PK>(X[r], pw) * Dp[r] : 0.f;
+          bt += ds;
+          if (want_l) lt = pos ? __builtin_fmaf(pow_p<PK>(X[r], pw), Dp[r], lt) : lt;
+          E[r] = NORM ? ds * rk[r] : ds;
+        }
+      } else if constexpr (PK == 2) {
         // relu on the bits (a float is > 0 iff its bits as an int32 are): t = max(x, 0) with no
         // comparison per value; t and t^2 vanish with t.  (Whole-vector bit casts: hipcc
         // compiled a bit cast of one element of an ext_vector to element 0.)
@@ -1162,18 +1162,23 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBw
     if constexpr (SP == 1) {
       if (own) {
         f32x16 S = f32x16{}, Dp = f32x16{};
-        products(S, Dp);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          S = PolBF16::mma(tile_row_frag<D>(kst, t), Q[t], S);
+          Dp = PolBF16::mma(tile_row_frag<D>(vst, t), DO[t], Dp);
+        }
         tile(S, Dp);
       }
     } else {  // the waves of a tile agree on `own`; every wave takes the barrier
-      f32x16 S = f32x16{}, Dp = f32x16{};
       if (own) {
-        products(S, Dp);
-        give16(L.xch[wid], S);
-        give16(L.xch[wid] + 16, Dp);
+        const bf16* src = hh ? vst : kst;
+        f32x16 acc = f32x16{};
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc = PolBF16::mma(tile_row_frag<D>(src, t), Q[t], acc);
+        give16(L.xch[wid], acc);
       }
       lds_barrier();
-      if (own) tile(take16(L.xch[wid ^ 1], S), take16(L.xch[wid ^ 1] + 16, Dp));
+      if (own) tile(take16(L.xch[2 * wv]), take16(L.xch[2 * wv + 1]));
     }
   };
   Pre pa;
@@ -1230,13 +1235,12 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBw
 // bits), streaming per branch the query tiles' Q and dO rows, query norms and tau values.  needm:
 // the block's key tiles to take (at least one).
 template <int D, int BR, int PK, bool NORM>
-__device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kKeyBlk<D>>& L, int jb, int bh, uint32_t needm) {
-  constexpr int W = kKeyBlk<D>, SP = kSplit<D>, NT = D / 16 / SP, ND = D / 32 / SP;
+__device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kBwdBlk>& L, int jb, int bh, uint32_t needm) {
+  constexpr int W = kBwdBlk, NT = D / 16, ND = D / 32;
   constexpr int STAGE = 2 * 32 * D;  // Q tile, dO tile
   bf16* ring = L.ring;
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
-  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int wv = wid / SP, hh = wid % SP;  // the wave's tile of the block, its half of d and of the columns
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int BH = P.B * P.H, nqt = P.nqt, nkt = P.nkt, Nq = P.Nq, Nk = P.Nk, qoff = P.qoff;
   const int b = bh / P.H, h = bh % P.H;
   const int kt0 = W * jb, kt = kt0 + wv;
@@ -1254,7 +1258,7 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kK
   {
     const bf16* r = base(B_V) + (int64_t)jc * P.s[B_V][2];
 #pragma unroll
-    for (int t = 0; t < NT; ++t) V[t] = *reinterpret_cast<const bf16x8*>(r + 16 * (t + NT * hh) + 8 * g);
+    for (int t = 0; t < NT; ++t) V[t] = *reinterpret_cast<const bf16x8*>(r + 16 * t + 8 * g);
   }
   const float beta = *P.beta;
   const float pw = P.p;
@@ -1268,7 +1272,6 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kK
   unsigned visited = 0, computed = 0;
   int it = 0;  // ring position, continued across the branches
   bf16* kti = L.rows[wv];
-  bf16x8 Kf[SP == 2 ? NT : 1];  // a split tile: this branch's key rows
 
 #pragma unroll
   for (int bi = 0; bi < BR; ++bi) {
@@ -1281,11 +1284,7 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kK
     if constexpr (NORM) nq = P.norms + norm_base(P, br == 0 ? N_Q1 : N_Q2, bh);
     const float ds_scale = (PK == 2 ? 2.f : 1.f) * (br == 0 ? 1.f : -lam);
     // the wave's key rows (swizzled tile; rows past Nk read as zeros), read as score operands
-    if constexpr (SP == 2) {
-      const bf16* r = base(kslot) + (int64_t)jc * P.s[kslot][2];
-#pragma unroll
-      for (int t = 0; t < NT; ++t) Kf[t] = *reinterpret_cast<const bf16x8*>(r + 16 * (t + NT * hh) + 8 * g);
-    } else {
+    {
       BlkRows<D, kBwdBlk> kr4[kBwdBlk];
 #pragma unroll
       for (int s4 = 0; s4 < kBwdBlk; ++s4) kr4[s4].load(base(kslot), P.s[kslot][2], 32 * min(kt, nkt - 1), Nk, s4);
@@ -1322,7 +1321,7 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kK
     };
     constexpr int AHEAD = D <= 64 ? 2 : 1;  // tiles in flight past the one being worked on
     struct Pre {  // a tile's share in flight: its rows, norms and thresholds, index, and whether it is the wave's
-      BlkRows<D, W * SP> qr, dr;
+      BlkRows<D, W> qr, dr;
       float vrq, vtq;
       int qt;
       bool own;
@@ -1330,9 +1329,9 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kK
     auto fetch = [&](Pre& p) {
       p.qt = next_tile(p.own);
       const int qt = max(p.qt, 0);  // loads on every path: the waits then count them exactly
-      p.qr.load(qb, sq, 32 * qt, Nq, wid);
-      p.dr.load(dob, sdo, 32 * qt, Nq, wid);
-      if (wid == 0 && l < 32) {
+      p.qr.load(qb, sq, 32 * qt, Nq, wv);
+      p.dr.load(dob, sdo, 32 * qt, Nq, wv);
+      if (wv == 0 && l < 32) {
         const int qi = min(32 * qt + l, Nq - 1);
         p.vrq = NORM ? nq[qi] : 1.f;
         p.vtq = beta * tau_coeff(qoff + 32 * qt + l, P.inv_d);
@@ -1345,26 +1344,24 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kK
       bf16* dst = qst + 32 * D;
       float* rqs = L.vals[it & 1][0];
       float* tqs = L.vals[it & 1][1];
-      p.qr.store(qst, wid);
-      p.dr.store(dst, wid);
-      if (wid == 0 && l < 32) {
+      p.qr.store(qst, wv);
+      p.dr.store(dst, wv);
+      if (wv == 0 && l < 32) {
         rqs[l] = p.vrq;
         tqs[l] = p.vtq;
       }
       fetch(p);  // the tile AHEAD steps on, in flight during this tile's work
       lds_barrier();
       ++it;
-      auto products = [&](f32x16& S, f32x16& Dp) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          if constexpr (SP == 2) S = PolBF16::mma(tile_row_frag<D>(qst, t + NT * hh), Kf[t], S);
-          else S = PolBF16::mma(tile_row_frag<D>(qst, t), tile_row_frag<D>(kti, t), S);
-          Dp = PolBF16::mma(tile_row_frag<D>(dst, t + NT * hh), V[t], Dp);
-        }
-      };
-      auto tile = [&](const f32x16& S, const f32x16& Dp) {
+      if (cown) {
         ++visited;
         const int q0 = 32 * qt;
+        f32x16 S = f32x16{}, Dp = f32x16{};
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          S = PolBF16::mma(tile_row_frag<D>(qst, t), tile_row_frag<D>(kti, t), S);
+          Dp = PolBF16::mma(tile_row_frag<D>(dst, t), V[t], Dp);
+        }
         float rq[16], tq[16];
         if constexpr (NORM) crow_vals(rqs, rq);
         crow_vals(tqs, tq);
@@ -1414,27 +1411,11 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kK
         const bf16x8 K0 = PolBF16::pack_c(EK, 0), K1 = PolBF16::pack_c(EK, 1);
 #pragma unroll
         for (int c = 0; c < ND; ++c) {
-          AV[c] = PolBF16::mma(tile_tr_frag<D>(dst, 0, c + ND * hh), V0, AV[c]);
-          AV[c] = PolBF16::mma(tile_tr_frag<D>(dst, 1, c + ND * hh), V1, AV[c]);
-          AK[c] = PolBF16::mma(tile_tr_frag<D>(qst, 0, c + ND * hh), K0, AK[c]);
-          AK[c] = PolBF16::mma(tile_tr_frag<D>(qst, 1, c + ND * hh), K1, AK[c]);
+          AV[c] = PolBF16::mma(tile_tr_frag<D>(dst, 0, c), V0, AV[c]);
+          AV[c] = PolBF16::mma(tile_tr_frag<D>(dst, 1, c), V1, AV[c]);
+          AK[c] = PolBF16::mma(tile_tr_frag<D>(qst, 0, c), K0, AK[c]);
+          AK[c] = PolBF16::mma(tile_tr_frag<D>(qst, 1, c), K1, AK[c]);
         }
-      };
-      if constexpr (SP == 1) {
-        if (cown) {
-          f32x16 S = f32x16{}, Dp = f32x16{};
-          products(S, Dp);
-          tile(S, Dp);
-        }
-      } else {  // the waves of a tile agree on `cown`; every wave takes the barrier
-        f32x16 S = f32x16{}, Dp = f32x16{};
-        if (cown) {
-          products(S, Dp);
-          give16(L.xch[wid], S);
-          give16(L.xch[wid] + 16, Dp);
-        }
-        lds_barrier();
-        if (cown) tile(take16(L.xch[wid ^ 1], S), take16(L.xch[wid ^ 1] + 16, Dp));
       }
     };
     Pre pa;
@@ -1450,27 +1431,17 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kK
     } else {
       while (pa.qt >= 0) step(pa);
     }
-    float dot = 0.f;  // the key row's x^ . dk^
-    if constexpr (NORM && SP == 2) {
-      if (need) {
-        GradRow<32 * ND> XR;
-        load_grad_row<32 * ND>(base(kslot) + (int64_t)jc * P.s[kslot][2] + 32 * ND * hh, XR);
-        dot = grad_row_dot<32 * ND>(AK, XR, rk);
-      }
-      if (g == 0) L.dots[wv][hh][n32] = dot;
-      lds_barrier();
-      dot = L.dots[wv][0][n32] + L.dots[wv][1][n32];
-    }
     if (kvalid) {
-      GradRow<32 * ND> XR;  // the key row's columns for the normalize backward
+      GradRow<D> XR;  // the key row for the normalize backward
+      float dot = 0.f;
       if constexpr (NORM) {
-        load_grad_row<32 * ND>(base(kslot) + (int64_t)jc * P.s[kslot][2] + 32 * ND * hh, XR);
-        if constexpr (SP == 1) dot = grad_row_dot<32 * ND>(AK, XR, rk);
+        load_grad_row<D>(base(kslot) + (int64_t)jc * P.s[kslot][2], XR);
+        dot = grad_row_dot<D>(AK, XR, rk);
       }
       const int gslot = br == 0 ? B_DK1 : B_DK2;
       bf16* grow = (bf16*)P.grad[br == 0 ? 1 : 3] + (int64_t)b * P.s[gslot][0] + (int64_t)h * P.s[gslot][1] +
-                   (int64_t)j * P.s[gslot][2] + 32 * ND * hh;
-      store_grad_rows<32 * ND, NORM>(AK, XR, grow, rk, dot, ds_scale);
+                   (int64_t)j * P.s[gslot][2];
+      store_grad_rows<D, NORM>(AK, XR, grow, rk, dot, ds_scale);
     }
     if (BR == 2 && bi == 0) {
 #pragma unroll
@@ -1481,11 +1452,10 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kK
     lds_barrier();  // every wave is done with its key tile before the next branch's rows
   }
   if (kvalid) {
-    bf16* vrow = (bf16*)P.grad[4] + (int64_t)b * P.s[B_DV][0] + (int64_t)h * P.s[B_DV][1] + (int64_t)j * P.s[B_DV][2] +
-                 32 * ND * hh;
-    store_grad_rows<32 * ND, false>(AV, GradRow<32 * ND>{}, vrow, 1.f, 0.f, 1.f);
+    bf16* vrow = (bf16*)P.grad[4] + (int64_t)b * P.s[B_DV][0] + (int64_t)h * P.s[B_DV][1] + (int64_t)j * P.s[B_DV][2];
+    store_grad_rows<D, false>(AV, GradRow<D>{}, vrow, 1.f, 0.f, 1.f);
   }
-  if (P.stats && l == 0 && need && hh == 0) {
+  if (P.stats && l == 0 && need) {
     atomicAdd(P.stats + 0, (unsigned long long)visited);
     atomicAdd(P.stats + 1, (unsigned long long)computed);
   }
@@ -1507,19 +1477,19 @@ __global__ void __launch_bounds__(kQryThreads<D>) __attribute__((amdgpu_waves_pe
 // against 539 us).
 template <int D, int BR, bool NORM>
 constexpr int dkv_waves() {
-  return D <= 64 || (D == 128 && BR == 1 && !NORM) ? 2 : 1;
+  return D <= 64 || (BR == 1 && !NORM) ? 2 : 1;
 }
 
 // One workgroup per block of key tiles: longest blocks (first key tiles) of every head first.  A
 // key tile takes this pass when a list of its column did not fit (the test bwd_dkv_pairs leaves
 // it by; it writes nothing for such a key tile), or always without lists.
 template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(kKeyThreads<D>) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, NORM>()))) bwd_dkv_blk(BwdParams P) {
-  constexpr int W = kKeyBlk<D>;
+__global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, NORM>()))) bwd_dkv_blk(BwdParams P) {
+  constexpr int W = kBwdBlk;
   TDA_BLK_LDS(D, W, true);
   __shared__ uint32_t needs[W];
   const int l = lane_id();
-  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) / kSplit<D>;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int BH = P.B * P.H, nqt = P.nqt;
   const int bid = blockIdx.x, jb = bid / BH, bh = bid % BH, kt = W * jb + wv;
   const uint32_t* counts = P.pairs ? P.pairs + pair_lists(BR, BH, nqt) * 4 * kPairCap : nullptr;
@@ -1552,6 +1522,238 @@ __global__ void __launch_bounds__(kKeyThreads<D>) __attribute__((amdgpu_waves_pe
   for (int r = 0; r < W; ++r) needm |= needs[r] ? 1u << r : 0u;
   needm = (uint32_t)__builtin_amdgcn_readfirstlane((int)needm);
   if (needm) dkv_block<D, BR, PK, NORM>(P, L, jb, bh, needm);
+}
+
+// Key-major at head_dim 256: kWideKeys key tiles of one head, 2 BR waves each (branch br, half hh),
+// walking the query tiles that any of them has in either branch (their bitmask bits, or every causal
+// one) and staging the Q rows of every branch and dO, one tile ahead.  Wave (br, 0) of a tile forms
+// branch br's scores, wave (0, 1) dP; all take them from LDS, and wave (br, hh) owns half of dk_br's
+// columns and a share of dv's.  At most 256 registers with two branches: accumulators past those live in
+// the accumulation registers, and a branch around them copies them all (B2 H8 N1000: 83 us so, 166 with
+// one wave per half, both branches in it; the query-major pass 46).
+constexpr int kWideKeys = 2;
+
+// tile_row_frag<256> and tile_tr_frag<256> from one byte offset per lane each: with rows of 512 bytes the
+// swizzle's exclusive or with a step's chunk is one of the offset with a constant.  keep_here makes the
+// offsets values of the loop's body (held as loop invariants, one register per step, they spill).
+struct WideTile {
+  int row, tr;
+  __device__ __forceinline__ WideTile() {
+    const int l = lane_id(), m = l & 31, g = l >> 5, j = l & 15, r = 4 * (l >> 5) + (j >> 2);
+    row = 512 * m + 16 * (g ^ bswz<256>(m));
+    tr = 512 * r + 16 * ((2 * ((l >> 4) & 1) + ((j & 3) >> 1)) ^ bswz<256>(r)) + 8 * (j & 1);
+  }
+  __device__ __forceinline__ void keep_here() { asm volatile("" : "+v"(row), "+v"(tr)); }
+  __device__ __forceinline__ bf16x8 row_frag(const bf16* tile, int t) const {
+    return *reinterpret_cast<const bf16x8*>(reinterpret_cast<const char*>(tile) + (row ^ (32 * (t & 7))) + 256 * (t >> 3));
+  }
+  __device__ __forceinline__ bf16x8 tr_frag(const bf16* tile, int st, int dsub) const {
+    bf16x8 out;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const char* p = reinterpret_cast<const char*>(tile) + (tr ^ (16 * ((4 * (dsub & 3)) ^ (8 * u)))) + 8192 * st + 4096 * u + 256 * (dsub >> 2);
+      const bf16x4 w = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(s16x4, p)));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[4 * u + e] = w[e];
+    }
+    return out;
+  }
+};
+
+template <int BR, int PK, bool NORM>
+__global__ void __launch_bounds__(128 * BR * kWideKeys) __attribute__((amdgpu_waves_per_eu(BR))) bwd_dkv_wide(BwdParams P) {
+  constexpr int D = 256, W = kWideKeys, NT = D / 16, NW = 2 * BR;  // NW: waves per key tile
+  constexpr int NDK = D / 64, NDV = D / 32 / NW;                   // a wave's column blocks of dk, of dv
+  constexpr int TILE = 32 * D, STAGE = (BR + 1) * TILE;            // Q of every branch, dO
+  constexpr int RT = BR == 2 ? NT - 6 : NT;                        // steps of the resident operand in registers
+  __shared__ __attribute__((aligned(16))) bf16 ring[2 * STAGE];
+  __shared__ __attribute__((aligned(16))) float vals[2][BR + 1][32];  // [stage]: query norms per branch, tau values
+  __shared__ __attribute__((aligned(16))) f32x4 xch[W][BR + 1][4][64];  // a tile's scores per branch, its dP
+  __shared__ float dots[W][BR][2][32];                                 // the halves' row dots
+  __shared__ __attribute__((aligned(16))) bf16x8 rest[BR == 2 ? W * (BR + 1) : 1][BR == 2 ? NT - RT : 1][64];
+  const int l = lane_id(), n32 = l & 31, g = l >> 5;
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wv = wid / NW, sub = wid % NW, br = sub >> 1, hh = sub & 1;
+  const int BH = P.B * P.H, nqt = P.nqt, nkt = P.nkt, Nq = P.Nq, Nk = P.Nk, qoff = P.qoff;
+  // longest blocks (first key tiles) of every head first
+  const int bid = blockIdx.x, kt0 = W * (bid / BH), bh = bid % BH, kt = kt0 + wv;
+  const int b = bh / P.H, h = bh % P.H;
+  const int j = 32 * kt + n32, jc = min(j, Nk - 1);
+  const bool kvalid = j < Nk;
+  const int qtf_b = qt_first(kt0, qoff);  // first query tile of the block
+  const uint32_t actm = nkt - kt0 >= W ? (1u << W) - 1u : (1u << (nkt - kt0)) - 1u;  // key tiles there are
+  auto base = [&](int slot) {
+    return (const bf16*)P.in[slot] + (int64_t)b * P.s[slot][0] + (int64_t)h * P.s[slot][1];
+  };
+  const int kslot = br == 0 ? B_K1 : B_K2;
+  // this wave's resident operand: its branch's K rows, or (wave (0, 1)) the V rows; with two branches
+  // its last steps wait in LDS (in registers they spill)
+  bf16x8 R[RT];
+  const int chain = (BR + 1) * wv + (hh ? BR : br);  // (wave (1, 1) has none: wave (0, 1)'s, the same values)
+  {
+    const int slot = hh ? B_V : kslot;
+    const bf16* r = base(slot) + (int64_t)jc * P.s[slot][2] + 8 * g;
+#pragma unroll
+    for (int t = 0; t < RT; ++t) R[t] = *reinterpret_cast<const bf16x8*>(r + 16 * t);
+#pragma unroll
+    for (int t = RT; t < NT; ++t) rest[chain][t - RT][l] = *reinterpret_cast<const bf16x8*>(r + 16 * t);
+  }
+  float rk[BR];
+#pragma unroll
+  for (int b2 = 0; b2 < BR; ++b2) rk[b2] = NORM ? P.norms[norm_base(P, b2 == 0 ? N_K1 : N_K2, bh) + jc] : 1.f;
+  const float beta = *P.beta;
+  const float pw = P.p;
+  float lam = 0.f;
+  if constexpr (BR == 2) lam = clamp01(*P.lam);
+  const float coef = br == 0 ? 1.f : -lam;
+  f32x16 AV[NDV], AK[NDK];
+#pragma unroll
+  for (int c = 0; c < NDV; ++c) AV[c] = f32x16{};
+#pragma unroll
+  for (int c = 0; c < NDK; ++c) AK[c] = f32x16{};
+  unsigned visited = 0, computed = 0;
+
+  // union walk over query tiles qtf_b .. nqt - 1, 64 per round: lane q tests query tile q0c + q
+  int q0c = qtf_b - 64;
+  uint64_t um = 0ull, om[BR];
+  auto next_tile = [&](uint32_t& own) -> int {  // own: bit b2, the wave's key tile in branch b2
+    own = 0u;
+    while (um == 0ull) {
+      q0c += 64;
+      if (q0c >= nqt) return -1;
+      const int qtl = q0c + l;
+      uint32_t any = 0u;
+#pragma unroll
+      for (int b2 = 0; b2 < BR; ++b2) {
+        const int64_t row = ((int64_t)b2 * BH + bh) * nqt + qtl;
+        uint32_t bits = qtl >= nqt ? 0u : P.occ ? P.occ[row * P.occ_w + (kt0 >> 5)] >> (kt0 & 31) : 0xffffffffu;
+        bits &= actm;
+        // causal: key tile kt0 + r is seen from query tile qt_first(kt0 + r) on
+#pragma unroll
+        for (int r = 0; r < W; ++r)
+          if (qtl < qt_first(kt0 + r, qoff)) bits &= ~(1u << r);
+        om[b2] = wave_ballot((bits >> wv) & 1u);
+        any |= bits;
+      }
+      um = wave_ballot(any != 0u);
+    }
+    const int q = __builtin_ctzll(um);
+    um &= um - 1ull;
+#pragma unroll
+    for (int b2 = 0; b2 < BR; ++b2) own |= (uint32_t)((om[b2] >> q) & 1ull) << b2;
+    return q0c + q;
+  };
+  BlkRows<D, W * NW> qr[BR], dr;  // the wave's share of the tile in flight
+  float vrq[BR], vtq = 0.f;
+  int qt;
+  uint32_t own;
+  auto fetch = [&]() {
+    qt = next_tile(own);
+    const int q0 = 32 * max(qt, 0);  // loads on every path: the waits then count them exactly
+#pragma unroll
+    for (int b2 = 0; b2 < BR; ++b2) {
+      const int slot = b2 == 0 ? B_Q1 : B_Q2;
+      qr[b2].load(base(slot), P.s[slot][2], q0, Nq, wid);
+      if (NORM && wid == 0 && l < 32) vrq[b2] = P.norms[norm_base(P, b2 == 0 ? N_Q1 : N_Q2, bh) + min(q0 + l, Nq - 1)];
+    }
+    dr.load(base(B_DO), P.s[B_DO][2], q0, Nq, wid);
+    if (wid == 0 && l < 32) vtq = beta * tau_coeff(qoff + q0 + l, P.inv_d);
+  };
+  WideTile wt;
+  fetch();
+#pragma unroll 1
+  for (int it = 0; qt >= 0; ++it) {
+    const int q0 = 32 * qt;
+    const uint32_t cown = own;
+    bf16* st = ring + (it & 1) * STAGE;
+    bf16* dst = st + BR * TILE;
+    float (*vs)[32] = vals[it & 1];
+#pragma unroll
+    for (int b2 = 0; b2 < BR; ++b2) {
+      qr[b2].store(st + b2 * TILE, wid);
+      if (NORM && wid == 0 && l < 32) vs[b2][l] = vrq[b2];
+    }
+    dr.store(dst, wid);
+    if (wid == 0 && l < 32) vs[BR][l] = vtq;
+    fetch();  // the next tile, in flight during this one's work
+    lds_barrier();
+    wt.keep_here();
+    if (hh ? br == 0 && cown : (cown >> br) & 1u) {
+      const bf16* src = hh ? dst : st + br * TILE;
+      give16(xch[wv][hh ? BR : br], mma_chain<NT>([&](int t) { return wt.row_frag(src, t); }, [&](int t) { return t < RT ? R[t] : rest[chain][t - RT][l]; }));
+    }
+    lds_barrier();
+    if (!cown) continue;  // (the waves of a tile agree)
+    ++visited;
+    const bool edge = 32 * kt + 31 > qoff + q0 || q0 + 31 >= Nq || 32 * kt + 31 >= Nk;
+    // query crow(r, g) sees the key iff c_r >= lo and exists iff c_r < hi (c_r = 8 (r / 4) + r % 4)
+    const int lo = (kvalid ? j - qoff - q0 : 64) - 4 * g, hi = Nq - q0 - 4 * g;
+    f32x16 EV = f32x16{}, E = f32x16{};
+    bool any = false;
+#pragma unroll
+    for (int b2 = 0; b2 < BR; ++b2) {
+      if (!((cown >> b2) & 1u)) continue;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {  // four values at a time: all sixteen's operands at once spill
+        const f32x4 S = xch[wv][b2][u][l], Dp = xch[wv][BR][u][l];
+        const f32x4 tq = *reinterpret_cast<const f32x4*>(vs[BR] + 8 * u + 4 * g);
+        f32x4 rq = {1.f, 1.f, 1.f, 1.f};
+        if constexpr (NORM) rq = *reinterpret_cast<const f32x4*>(vs[b2] + 8 * u + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int c = 8 * u + e, r = 4 * u + e;
+          float x = __builtin_fmaf(NORM ? S[e] * rk[b2] : S[e], rq[e], -tq[e]);
+          if (edge) x = c >= lo && c < hi ? x : -1.f;
+          const bool pos = x > 0.f;
+          const float w = pos ? pow_p<PK>(x, pw) : 0.f;
+          EV[r] = b2 == 0 ? w : __builtin_fmaf(-lam, w, EV[r]);
+          any |= pos;
+          if (BR == 1 || b2 == br) {
+            const float ds = pos ? coef * dpow_p<PK>(x, pw) * Dp[e] : 0.f;
+            E[r] = NORM ? ds * rq[e] : ds;
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (!P.occ && wave_ballot(any) == 0ull) continue;  // the same decision in every wave of the tile
+    ++computed;
+    const bf16x8 V0 = PolBF16::pack_c(EV, 0), V1 = PolBF16::pack_c(EV, 1);
+#pragma unroll
+    for (int c = 0; c < NDV; ++c) {
+      AV[c] = PolBF16::mma(wt.tr_frag(dst, 0, c + NDV * sub), V0, AV[c]);
+      AV[c] = PolBF16::mma(wt.tr_frag(dst, 1, c + NDV * sub), V1, AV[c]);
+    }
+    if ((cown >> br) & 1u) {
+      const bf16x8 K0 = PolBF16::pack_c(E, 0), K1 = PolBF16::pack_c(E, 1);
+      const bf16* src = st + br * TILE;
+#pragma unroll
+      for (int c = 0; c < NDK; ++c) {
+        AK[c] = PolBF16::mma(wt.tr_frag(src, 0, c + NDK * hh), K0, AK[c]);
+        AK[c] = PolBF16::mma(wt.tr_frag(src, 1, c + NDK * hh), K1, AK[c]);
+      }
+    }
+  }
+  const float rkb = br == 0 ? rk[0] : rk[BR - 1];
+  GradRow<32 * NDK> XR;  // the key row's columns for the normalize backward
+  if constexpr (NORM) {
+    load_grad_row<32 * NDK>(base(kslot) + (int64_t)jc * P.s[kslot][2] + 32 * NDK * hh, XR);
+    const float part = grad_row_dot<32 * NDK>(AK, XR, rkb);
+    if (g == 0) dots[wv][br][hh][n32] = part;
+    lds_barrier();
+  }
+  if (kvalid) {
+    auto grow = [&](int gi, int slot) {
+      return (bf16*)P.grad[gi] + (int64_t)b * P.s[slot][0] + (int64_t)h * P.s[slot][1] + (int64_t)j * P.s[slot][2];
+    };
+    store_grad_rows<32 * NDV, false>(AV, GradRow<32 * NDV>{}, grow(4, B_DV) + 32 * NDV * sub, 1.f, 0.f, 1.f);
+    store_grad_rows<32 * NDK, NORM>(AK, XR, grow(br == 0 ? 1 : 3, br == 0 ? B_DK1 : B_DK2) + 32 * NDK * hh, rkb,
+                                    NORM ? dots[wv][br][0][n32] + dots[wv][br][1][n32] : 0.f, 1.f);
+  }
+  if (P.stats && l == 0 && sub == 0) {
+    atomicAdd(P.stats + 0, (unsigned long long)visited);
+    atomicAdd(P.stats + 1, (unsigned long long)computed);
+  }
 }
 
 // Both block passes over the queue of the key-major pair pass, in one launch: the workgroups
@@ -1607,7 +1809,8 @@ static int launch_t(const BwdParams& p, void* stream) {
   }
   const int BH = q.B * q.H;
   const unsigned qblocks = (unsigned)(BR * BH * ((q.nqt + kBwdBlk - 1) / kBwdBlk));
-  const unsigned kblocks = (unsigned)(BH * ((q.nkt + kKeyBlk<D> - 1) / kKeyBlk<D>));
+  constexpr int KB = D <= 128 ? kBwdBlk : kWideKeys;
+  const unsigned kblocks = (unsigned)(BH * ((q.nkt + KB - 1) / KB));
   bool queued = false;
   if constexpr (NORM && D <= 128) {
     if (q.pairs && q.dkvq) {
@@ -1621,7 +1824,10 @@ static int launch_t(const BwdParams& p, void* stream) {
   if (!queued) {
     hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM>), dim3(qblocks), dim3(kQryThreads<D>), 0, s, q);
     launched(s, "bwd_dq_blk");
-    hipLaunchKernelGGL((bwd_dkv_blk<D, BR, PK, NORM>), dim3(kblocks), dim3(kKeyThreads<D>), 0, s, q);
+    if constexpr (D <= 128)
+      hipLaunchKernelGGL((bwd_dkv_blk<D, BR, PK, NORM>), dim3(kblocks), dim3(64 * kBwdBlk), 0, s, q);
+    else
+      hipLaunchKernelGGL((bwd_dkv_wide<BR, PK, NORM>), dim3(kblocks), dim3(128 * BR * kWideKeys), 0, s, q);
     launched(s, "bwd_dkv_blk");
   }
   const int e = (int)hipGetLastError();

@@ -349,6 +349,33 @@ __device__ __forceinline__ bf16x8 tile_tr_frag(const bf16* tile, int st, int dsu
   return out;
 }
 
+// One chain of NT bf16 products, acc += a(t) b(t), its operands read a group of four steps ahead of
+// their use and no further: left to itself the compiler reads them all at once, and in a kernel that
+// fills the register file the spills' reloads then wait for every load in flight.
+template <int NT, class FA, class FB>
+__device__ __forceinline__ f32x16 mma_chain(FA&& fa, FB&& fb) {
+  constexpr int G = 4;
+  bf16x8 a[2][G], b[2][G];
+  f32x16 acc = {};
+#pragma unroll
+  for (int t0 = -G; t0 < NT; t0 += G) {
+    if (t0 + G < NT) {
+#pragma unroll
+      for (int u = 0; u < G; ++u) {
+        a[(t0 / G + 1) & 1][u] = fa(t0 + G + u);
+        b[(t0 / G + 1) & 1][u] = fb(t0 + G + u);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (t0 >= 0) {
+#pragma unroll
+      for (int u = 0; u < G; ++u) acc = PolBF16::mma(a[(t0 / G) & 1][u], b[(t0 / G) & 1][u], acc);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  return acc;
+}
+
 // ------------------------------------------------------------------ fp32 wave tiles
 // A wave's own 32-row fp32 tile: the next one's rows in flight in registers (load), the current one
 // in the wave's LDS slice (store), read as row fragments (f32_rows_mma) or by columns (f32_cols_mma).

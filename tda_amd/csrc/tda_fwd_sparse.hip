@@ -760,23 +760,55 @@ __device__ __forceinline__ bf16x8 tr_frag(const bf16* p) {
 // 16, 2048, 64) without normalisation 59 -> 48.5 us with them, the two tiles ahead and weights
 // without their branch's coefficient, which scales the sum once per branch).
 // WALK (no screen ran before it): every query tile, every causal key tile in turn; the row's
-// bitmask words are all written (the words past its last key tile as zeros) and, up to head_dim 128,
-// the causal tiles are counted into stats[0].  ZR: the workgroup then clears its even share of the
-// call's zero range.
+// bitmask words are all written (the words past its last key tile as zeros) and the causal tiles
+// are counted into stats[0].  ZR: the workgroup then clears its even share of the call's zero range.
 // Without WALK (normalised) it takes the query tiles whose candidate lists overflowed (a count past
 // kCandCap in some branch; fwd_pv_cand took the others), walking the union of their bitmask rows,
 // listed in LDS 64 words at a time; tiles whose weights are all zero lose their bit.  A workgroup
 // with no such tile leaves after one round of loads, a wave whose own lists fit only helps to load.
 // At a threshold scale of 0.5 nearly every list overflows (TDA (2, 16, 1500, 64): 237 us with one
 // wave per query tile, 102 so); with every list fitting the launch costs 4.6 us.
-// SKIP: the A V products of a tile whose weights are all zero are skipped, by a branch around the
-// accumulators (head_dim 256 with normalisation, where 97 % of the tiles are: TDA (2, 8, 1000, 256)
-// 81 us against 249 with two waves per query tile, each forming all scores from its own loads).
 constexpr int kBlkTiles = 4;
 
-template <int D, int BR, int PK, bool NORM, bool ZR = false, bool WALK = !NORM, bool SKIP = false>
-__global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_per_eu(D <= 64 ? (WALK ? 3 : 2) : D <= 128 ? 2 : 1)))
+// Block and head of workgroup `bid`: longest blocks (last query tiles) of every head first; one
+// head's blocks on one XCD when the heads fill the eight XCDs.
+__device__ __forceinline__ void blk_order(int bid, int BH, int nqb, int& bh, int& jb) {
+  if (BH % 8 == 0) {
+    const int x = bid & 7, j = bid >> 3, hg = BH / 8;
+    bh = x + 8 * (j % hg);
+    jb = nqb - 1 - j / hg;
+  } else {
+    bh = bid % BH;
+    jb = nqb - 1 - bid / BH;
+  }
+}
+// D columns (from column c0) of query tile qt's output rows through the wave's LDS slice (row stride
+// D + 8): lane (n, g) holds elements 32c + crow(r, g) of row n; the stores are 16 bytes per lane.
+template <int D>
+__device__ __forceinline__ void blk_store_out(const FwdParams& P, const f32x16 (&O)[D / 32], bf16* ost, int b, int h, int qt,
+                                              int c0 = 0) {
+  constexpr int KS = D + 8, CPR = D / 8, RPI = 64 / CPR;
+  const int l = lane_id(), n32 = l & 31, g = l >> 5;
+#pragma unroll
+  for (int c = 0; c < D / 32; ++c)
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      store4(ost + n32 * KS + 32 * c + 8 * u + 4 * g, O[c][4 * u], O[c][4 * u + 1], O[c][4 * u + 2], O[c][4 * u + 3]);
+  wave_lds_sync();
+  bf16* ohead = (bf16*)P.out + (int64_t)b * P.s[F_OUT][0] + (int64_t)h * P.s[F_OUT][1] + c0;
+#pragma unroll
+  for (int i = 0; i < 32 / RPI; ++i) {
+    const int r = l / CPR + RPI * i, row = 32 * qt + r;
+    if (row < P.Nq)
+      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(ost + r * KS + 8 * (l % CPR)),
+                                  reinterpret_cast<u32x4*>(ohead + (int64_t)row * P.s[F_OUT][2] + 8 * (l % CPR)));
+  }
+}
+
+template <int D, int BR, int PK, bool NORM, bool ZR = false>
+__global__ void __launch_bounds__(64 * kBlkTiles) __attribute__((amdgpu_waves_per_eu(D <= 64 ? (NORM ? 2 : 3) : 2)))
 fwd_pv_blk(FwdParams P) {
+  constexpr bool WALK = !NORM;
   static_assert(!ZR || WALK, "the zero range is cleared by the walk");
   constexpr int W = kBlkTiles;
   constexpr int NT = D / 16, ND = D / 32;
@@ -785,7 +817,7 @@ fwd_pv_blk(FwdParams P) {
   constexpr int CPR = D / 8;     // 16-byte chunks per row
   constexpr int RPI = 64 / CPR;  // rows per load instruction
   constexpr int LPW = 32 / RPI / W;  // load instructions per wave, K and V each
-  constexpr int AHEAD = D <= 64 || (WALK && D <= 128) ? 2 : 1;  // tiles in flight past the one being worked on
+  constexpr int AHEAD = D <= 64 || WALK ? 2 : 1;  // tiles in flight past the one being worked on
   static_assert(LPW >= 1 && LPW * RPI * W == 32, "K/V tile rows split evenly over the waves");
   constexpr int STAGE = 32 * KS + 32 * VS;
   static_assert(2 * STAGE >= W * 32 * KS, "the ring holds the waves' output rows");
@@ -799,19 +831,7 @@ fwd_pv_blk(FwdParams P) {
   const int BH = P.B * P.H, Nq = P.Nq, Nk = P.Nk, nqt = P.nqt, qoff = P.qoff;
   const int nqb = (nqt + W - 1) / W;
   int bh, jb;
-  {
-    // longest blocks (last query tiles) of every head first; one head's blocks on one XCD when
-    // the heads fill the eight XCDs
-    const int bid = blockIdx.x;
-    if (BH % 8 == 0) {
-      const int x = bid & 7, j = bid >> 3, hg = BH / 8;
-      bh = x + 8 * (j % hg);
-      jb = nqb - 1 - j / hg;
-    } else {
-      bh = bid % BH;
-      jb = nqb - 1 - bid / BH;
-    }
-  }
+  blk_order(blockIdx.x, BH, nqb, bh, jb);
   // without WALK: the block's query tiles this pass takes (the same for every wave)
   uint32_t needm = 0u;
   if constexpr (!WALK) {
@@ -846,7 +866,7 @@ fwd_pv_blk(FwdParams P) {
   unsigned computed = 0, checked = 0;
   int it = 0;  // ring position, continued across the branches
 
-#pragma unroll(D > 128 ? 1 : BR)
+#pragma unroll
   for (int bi = 0; bi < BR; ++bi) {
     const int br = BR - 1 - bi;  // the second branch first: out = -lambda A2 V, then += A1 V
     const int qslot = br ? F_Q2 : F_Q1, kslot = br ? F_K2 : F_K1;
@@ -1001,14 +1021,12 @@ fwd_pv_blk(FwdParams P) {
         }
         // A V on every tile the row keeps (a tile of zero weights adds zero products: the same
         // sums bit for bit, and no branch around the accumulators)
-        if (!SKIP || any) {
-          const bf16x8 PF0 = PolBF16::pack_c(C, 0), PF1 = PolBF16::pack_c(C, 1);
-          const bf16* vp = vst + voff;
+        const bf16x8 PF0 = PolBF16::pack_c(C, 0), PF1 = PolBF16::pack_c(C, 1);
+        const bf16* vp = vst + voff;
 #pragma unroll
-          for (int c = 0; c < ND; ++c) {
-            O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c), PF0, O[c]);
-            O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c + 16 * VS), PF1, O[c]);
-          }
+        for (int c = 0; c < ND; ++c) {
+          O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c), PF0, O[c]);
+          O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c + 16 * VS), PF1, O[c]);
         }
         return any;
     };
@@ -1138,33 +1156,205 @@ fwd_pv_blk(FwdParams P) {
     for (uint32_t u = threadIdx.x; u < zn; u += 64 * W) __builtin_nontemporal_store(u32x4{0u, 0u, 0u, 0u}, zbase + u);
   }
 
-  // Output rows through LDS (the wave's slice of the ring, free once every wave has passed the
-  // barrier below): lane (n, g) holds elements 32c + crow(r, g) of row n; stores then cover whole
-  // rows, 16 bytes per lane.
-  __syncthreads();
+  __syncthreads();  // every wave is done with the ring: its slices hold the output rows
   if (!act) return;
-  bf16* ost = ring + wv * 32 * KS;
-#pragma unroll
-  for (int c = 0; c < ND; ++c)
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      store4(ost + n32 * KS + 32 * c + 8 * u + 4 * g, O[c][4 * u], O[c][4 * u + 1], O[c][4 * u + 2], O[c][4 * u + 3]);
-  wave_lds_sync();
-  {
-    bf16* ohead = (bf16*)P.out + (int64_t)b * P.s[F_OUT][0] + (int64_t)h * P.s[F_OUT][1];
-    constexpr int OL = 32 / RPI;
-#pragma unroll
-    for (int i = 0; i < OL; ++i) {
-      const int r = l / CPR + RPI * i, row = 32 * qt + r;
-      if (row < Nq)
-        __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(ost + r * KS + 8 * vch),
-                                    reinterpret_cast<u32x4*>(ohead + (int64_t)row * P.s[F_OUT][2] + 8 * vch));
-    }
-  }
+  blk_store_out<D>(P, O, ring + wv * 32 * KS, b, h, qt);
   if (P.stats && l == 0 && checked) {
     if (WALK) atomicAdd(P.stats + 0, (unsigned long long)checked);  // every causal tile is tested
     atomicAdd(P.stats + 1, (unsigned long long)computed);
-    if (D <= 128) atomicAdd(P.stats + 2, (unsigned long long)checked);
+    atomicAdd(P.stats + 2, (unsigned long long)checked);
+  }
+}
+
+// ------------------------------------------------------------------ fwd_blk256
+// head_dim 256: no screen and no pair lists; kBlkTiles query tiles of one head per workgroup, every
+// causal key tile in turn, both branches' key tiles and the value tile staged together (as fwd_pv_blk
+// stages them, one tile ahead).  A tile's weights A1 - lambda A2 are combined in fp32 and rounded to
+// bf16 once; a tile without a weight adds nothing.  One chain of products per score row, keys as the
+// A operand: the backward passes form the same bits.
+// kWideFwdWaves waves per query tile, each owning a share of the output's columns.  Two: with two
+// branches wave w forms branch w's weights and they exchange them through LDS; with one both form
+// them.  They fit 256 registers, two waves per SIMD, and skip the A V products of a tile without a
+// weight (at beta = 1 most are).  B2 H8 N1000 at beta = 1: 62 us with two branches (133 with one wave
+// per tile: its 512 registers put the accumulators where a branch around them copies them all), 47 with
+// one (one wave per tile: 40 to 105, as the compiler happens to keep or copy them).  Without normalisation a single branch has weights nearly everywhere: one wave
+// per tile with no branch, a tile without a weight reading zeros for V: 53 us.
+template <int BR, bool NORM>
+constexpr int kWideFwdWaves = BR == 2 || NORM ? 2 : 1;
+
+template <int BR, int PK, bool NORM>
+__global__ void __launch_bounds__((64 * kBlkTiles * kWideFwdWaves<BR, NORM>))
+__attribute__((amdgpu_waves_per_eu((kWideFwdWaves<BR, NORM>)))) fwd_blk256(FwdParams P) {
+  constexpr int D = 256, W = kBlkTiles, NW = kWideFwdWaves<BR, NORM>, NT = D / 16, ND = D / 32 / NW;
+  constexpr int VS = D + 32, KS = D + 8, CPR = D / 8, RPI = 64 / CPR, LPW = 32 / RPI / (NW * W);
+  constexpr int STAGE = 32 * (BR * KS + VS);
+  constexpr bool SKIP = NW == 2;
+  constexpr int OS = D / NW + 8;  // row stride of a wave's output slice
+  static_assert(2 * STAGE >= NW * W * 32 * OS, "the ring holds the waves' output rows");
+  __shared__ __attribute__((aligned(16))) bf16 ring[2 * STAGE];
+  __shared__ __attribute__((aligned(16))) float nring[2][BR][32];
+  __shared__ __attribute__((aligned(16))) f32x4 xch[BR == 2 ? 2 * W : 1][4][64];  // two branches: the waves' weights
+  __shared__ uint32_t xany[2 * W];                                             // and whether there are any
+  __shared__ __attribute__((aligned(16))) bf16 zeros[SKIP ? 8 : 32 * VS];  // a value tile of zeros
+
+  const int l = lane_id(), n32 = l & 31, g = l >> 5;
+  const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int wv = wid / NW, part = wid % NW, br = BR == 2 ? part : 0;  // query tile, share of the columns, branch
+  const int BH = P.B * P.H, Nq = P.Nq, Nk = P.Nk, nqt = P.nqt, qoff = P.qoff;
+  int bh, jb;
+  blk_order(blockIdx.x, BH, (nqt + W - 1) / W, bh, jb);
+  const int b = bh / P.H, h = bh % P.H;
+  const int qt = W * jb + wv, qtc = min(qt, nqt - 1);
+  const bool act = qt < nqt;  // wave-uniform: waves past the last query tile only load
+  const int iq = 32 * qt + n32, pq = qoff + iq;
+  const bool valid = act && iq < Nq;
+  const bool rowpad = 32 * qt + 31 >= Nq;  // the query tile has rows past Nq (uniform)
+  const int klast_b = kt_last(min(W * jb + W - 1, nqt - 1), qoff, P.nkt);  // the block's last key tile
+  const int ktl = act ? kt_last(qt, qoff, P.nkt) : -1;                     // the wave's
+  const float tau = *P.beta * tau_coeff(pq, P.inv_d);
+  const float pw = P.p;
+  float lam = 0.f;
+  if constexpr (BR == 2) lam = clamp01(*P.lam);
+  const int row0 = RPI * LPW * wid + l / CPR, ch = l % CPR;  // this wave's rows of a staged tile
+  const int bk = l >> 4, jj = l & 15;
+  const int voff = (4 * (bk >> 1) + (jj >> 2)) * VS + 16 * (bk & 1) + 4 * (jj & 3) + 32 * ND * part;
+
+  // this lane's query row in the wave's branch (rows past Nq read as zeros) and its inverse norm
+  bf16x8 Q[NT];
+  float rq = 1.f;
+  {
+    const int qs = br ? F_Q2 : F_Q1;
+    const int64_t sq = P.s[qs][2];
+    const __amdgpu_buffer_rsrc_t rs =
+        tile_rsrc<D>((const bf16*)P.in[qs] + (int64_t)b * P.s[qs][0] + (int64_t)h * P.s[qs][1], sq, qtc, Nq);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) Q[t] = __builtin_bit_cast(bf16x8, buf_load16(rs, (uint32_t)((n32 * sq + 16 * t + 8 * g) * 2)));
+    if constexpr (NORM) rq = P.norms[norm_base(P, br ? N_Q2 : N_Q1, bh) + min(32 * qtc + n32, Nq - 1)];
+  }
+  uint32_t* orow = P.occ + ((int64_t)(br * BH + bh) * nqt + qtc) * P.occ_w;  // the tile's bitmask row in the branch
+  const bf16* khead[BR];
+#pragma unroll
+  for (int x = 0; x < BR; ++x) {
+    const int ks = x ? F_K2 : F_K1;
+    khead[x] = (const bf16*)P.in[ks] + (int64_t)b * P.s[ks][0] + (int64_t)h * P.s[ks][1];
+  }
+  const bf16* vhead = (const bf16*)P.in[F_V] + (int64_t)b * P.s[F_V][0] + (int64_t)h * P.s[F_V][1];
+
+  u32x4 kr[BR][LPW], vr[LPW];  // this wave's share of the tile in flight
+  f32x4 nr[BR];
+  auto issue = [&](int kt) {
+#pragma unroll
+    for (int x = 0; x < BR; ++x) {
+      const int64_t sk = P.s[x ? F_K2 : F_K1][2];
+      const __amdgpu_buffer_rsrc_t rk = tile_rsrc<D>(khead[x], sk, kt, Nk);
+#pragma unroll
+      for (int i = 0; i < LPW; ++i) kr[x][i] = buf_load16(rk, (uint32_t)(((row0 + RPI * i) * sk + 8 * ch) * 2));
+      if (NORM && wid == 0 && l < 8)
+        nr[x] = __builtin_bit_cast(f32x4, buf_load16(make_rsrc(P.norms + norm_base(P, x ? N_K2 : N_K1, bh), (uint32_t)Nk * 4),
+                                                     (uint32_t)(32 * kt + 4 * l) * 4));
+    }
+    const int64_t sv = P.s[F_V][2];
+    const __amdgpu_buffer_rsrc_t rv = tile_rsrc<D>(vhead, sv, kt, Nk);
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) vr[i] = buf_load16(rv, (uint32_t)(((row0 + RPI * i) * sv + 8 * ch) * 2));
+  };
+
+  f32x16 O[ND];
+#pragma unroll
+  for (int c = 0; c < ND; ++c) O[c] = f32x16{};
+  unsigned checked = 0, computed = 0;
+  uint32_t keep = 0u;  // the current bitmask word: its tiles with a weight
+  issue(0);
+  if (!SKIP) {
+    for (int x = threadIdx.x; x < 32 * VS / 8; x += 64 * NW * W) *reinterpret_cast<u32x4*>(zeros + 8 * x) = u32x4{0u, 0u, 0u, 0u};
+  }
+#pragma unroll 1
+  for (int kt = 0; kt <= klast_b; ++kt) {
+    bf16* st = ring + (kt & 1) * STAGE;
+    bf16* vst = st + BR * 32 * KS;
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) {
+#pragma unroll
+      for (int x = 0; x < BR; ++x) *reinterpret_cast<u32x4*>(st + (32 * x + row0 + RPI * i) * KS + 8 * ch) = kr[x][i];
+      *reinterpret_cast<u32x4*>(vst + (row0 + RPI * i) * VS + 8 * ch) = vr[i];
+    }
+    if (NORM && wid == 0 && l < 8) {
+#pragma unroll
+      for (int x = 0; x < BR; ++x) *reinterpret_cast<f32x4*>(nring[kt & 1][x] + 4 * l) = nr[x];
+    }
+    issue(min(kt + 1, klast_b));  // in flight during this tile's work
+    lds_barrier();
+    f32x16 C = f32x16{};
+    bool any = false;
+    if (kt <= ktl) {
+      const bf16* kp = st + (32 * br + n32) * KS + 8 * g;
+      const f32x16 S = mma_chain<NT>([&](int t) { return *reinterpret_cast<const bf16x8*>(kp + 16 * t); }, [&](int t) { return Q[t]; });
+      // exact x; keys after the query's position, padding keys and query rows past Nq set to -1 (only
+      // on the tiles that have any); a NaN score has no weight
+      f32x16 X;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        f32x4 rk = {1.f, 1.f, 1.f, 1.f};
+        if constexpr (NORM) rk = *reinterpret_cast<const f32x4*>(nring[kt & 1][br] + 8 * u + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) X[4 * u + e] = __builtin_fmaf(NORM ? S[4 * u + e] * rk[e] : S[4 * u + e], rq, -tau);
+      }
+      if (32 * kt + 31 > min(qoff + 32 * qt, Nk - 1) || rowpad) {
+        const int lim = (valid ? min(pq, Nk - 1) - 32 * kt : -1) - 4 * g;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) X[r] = 8 * (r >> 2) + (r & 3) <= lim ? X[r] : -1.f;
+      }
+      bool pos = false;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const bool p = X[r] > 0.f;
+        C[r] = p ? pow_p<PK>(X[r], pw) : 0.f;
+        pos |= p;
+      }
+      any = wave_ballot(pos) != 0ull;
+      ++checked;
+      keep |= any ? 1u << (kt & 31) : 0u;
+      computed += any ? 1u : 0u;
+      if constexpr (BR == 2) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) xch[wid][u][l] = f32x4{C[4 * u], C[4 * u + 1], C[4 * u + 2], C[4 * u + 3]};
+        if (l == 0) xany[wid] = any ? 1u : 0u;
+      }
+    }
+    if constexpr (BR == 2) {  // (the next weights are written past the next tile's first barrier)
+      lds_barrier();
+      if (kt <= ktl) {
+        any = (uint32_t)__builtin_amdgcn_readfirstlane((int)(xany[2 * wv] | xany[2 * wv + 1])) != 0u;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const f32x4 a1 = xch[2 * wv][u][l], a2 = xch[2 * wv + 1][u][l];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) C[4 * u + e] = __builtin_fmaf(-lam, a2[e], a1[e]);
+        }
+      }
+    }
+    if (!SKIP || any) {  // O += V^T C
+      const bf16x8 PF0 = PolBF16::pack_c(C, 0), PF1 = PolBF16::pack_c(C, 1);
+      const bf16* vp = (SKIP || any ? vst : zeros) + voff;
+#pragma unroll
+      for (int c = 0; c < ND; ++c) {
+        O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c), PF0, O[c]);
+        O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c + 16 * VS), PF1, O[c]);
+      }
+    }
+    if ((kt & 31) == 31 || kt == klast_b) {
+      if ((kt >> 5) <= (ktl >> 5) && l == 0 && br == part) orow[kt >> 5] = keep;
+      keep = 0u;
+    }
+  }
+  __syncthreads();  // every wave is done with the ring: its slices hold the output rows
+  if (!act) return;
+  if (l == 0 && br == part)  // the bitmask words past the row's last key tile
+    for (int w = (ktl >> 5) + 1; w < P.occ_w; ++w) orow[w] = 0u;
+  blk_store_out<D / NW>(P, O, ring + wid * 32 * OS, b, h, qt, 32 * ND * part);
+  if (P.stats && l == 0 && br == part) {
+    atomicAdd(P.stats + 0, (unsigned long long)checked);  // every causal tile is tested
+    atomicAdd(P.stats + 1, (unsigned long long)computed);
   }
 }
 
@@ -1513,15 +1703,14 @@ int launch_fwd_sparse(const FwdParams& p, const KernelKey& k, void* stream) {
   return k.d == 128 ? sel_br<128>(p, k, s) : sel_br<64>(p, k, s);
 }
 
-// head_dim 256 (bf16): no screen and no pair lists; every causal tile through the block pass, after
-// the launcher (tda_wide.hip) wrote the norms table.
+// head_dim 256 (bf16), after the launcher (tda_wide.hip) wrote the norms table.
 template <int BR, int PK>
 static int launch_blk256_t(const FwdParams& p, bool norm, hipStream_t s) {
   const unsigned blocks = (unsigned)(p.B * p.H * ((p.nqt + kBlkTiles - 1) / kBlkTiles));
   if (norm)
-    hipLaunchKernelGGL((fwd_pv_blk<256, BR, PK, true, false, true, true>), dim3(blocks), dim3(64 * kBlkTiles), 0, s, p);
+    hipLaunchKernelGGL((fwd_blk256<BR, PK, true>), dim3(blocks), dim3(64 * kBlkTiles * kWideFwdWaves<BR, true>), 0, s, p);
   else
-    hipLaunchKernelGGL((fwd_pv_blk<256, BR, PK, false>), dim3(blocks), dim3(64 * kBlkTiles), 0, s, p);
+    hipLaunchKernelGGL((fwd_blk256<BR, PK, false>), dim3(blocks), dim3(64 * kBlkTiles * kWideFwdWaves<BR, false>), 0, s, p);
   launched(s, "wide_fwd");
   return (int)hipGetLastError();
 }
@@ -1533,9 +1722,7 @@ static int launch_blk256_br(const FwdParams& p, const KernelKey& k, hipStream_t 
     default: return launch_blk256_t<BR, 0>(p, k.normalize, s);
   }
 }
-int launch_fwd_blk256(const FwdParams& p0, const KernelKey& k, void* stream) {
-  FwdParams p = p0;
-  p.pairs = nullptr;  // head_dim 256 leaves the pair buffer alone
+int launch_fwd_blk256(const FwdParams& p, const KernelKey& k, void* stream) {
   return k.branches == 2 ? launch_blk256_br<2>(p, k, (hipStream_t)stream) : launch_blk256_br<1>(p, k, (hipStream_t)stream);
 }
 
