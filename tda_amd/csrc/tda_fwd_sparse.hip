@@ -1019,14 +1019,17 @@ fwd_pv_blk(FwdParams P) {
           if (P.colcnt && l == 0) atomicOr(P.colcnt + (int64_t)bh * P.nkt + kt, kColTaint);
           ++computed;
         }
-        // A V on every tile the row keeps (a tile of zero weights adds zero products: the same
-        // sums bit for bit, and no branch around the accumulators)
-        const bf16x8 PF0 = PolBF16::pack_c(C, 0), PF1 = PolBF16::pack_c(C, 1);
-        const bf16* vp = vst + voff;
+        // A V.  With normalisation a kept tile without a weight adds nothing, whatever its value rows
+        // hold; the walk of every tile adds its zero products (the same sums for finite rows, and no
+        // branch around the accumulators).
+        if (WALK || any) {
+          const bf16x8 PF0 = PolBF16::pack_c(C, 0), PF1 = PolBF16::pack_c(C, 1);
+          const bf16* vp = vst + voff;
 #pragma unroll
-        for (int c = 0; c < ND; ++c) {
-          O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c), PF0, O[c]);
-          O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c + 16 * VS), PF1, O[c]);
+          for (int c = 0; c < ND; ++c) {
+            O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c), PF0, O[c]);
+            O[c] = PolBF16::mma(tr_frag<VS>(vp + 32 * c + 16 * VS), PF1, O[c]);
+          }
         }
         return any;
     };
