@@ -917,6 +917,25 @@ __device__ __forceinline__ f32x16 relu16(f32x16 x) {
   return x;
 }
 
+// dP as the p = 2 passes multiply it by t = relu(x): with normalisation 0 at a pair without a weight where
+// dP is not finite (a value row that no weight meets).  Only a tile that has such a value pays for the
+// selection: bwd_tiles, TDA (2, 16, 1500, 64) at beta 0.5, 162 us so, 166 with it on every tile.
+template <bool NORM>
+__device__ __forceinline__ f32x16 finite_dp(f32x16 dp, const f32x16& t) {
+  if constexpr (NORM) {
+    auto m3 = [](float a, float b, float c) {  // NaN if any is
+      return __builtin_elementwise_maximum(__builtin_elementwise_maximum(fabsf(a), fabsf(b)), fabsf(c));
+    };
+    const float a = m3(dp[0], dp[1], dp[2]), b = m3(dp[3], dp[4], dp[5]), c = m3(dp[6], dp[7], dp[8]);
+    const float d = m3(dp[9], dp[10], dp[11]), e = m3(dp[12], dp[13], dp[14]);
+    if (wave_ballot(!(m3(m3(a, b, c), m3(d, e, dp[15]), dp[15]) < INFINITY)) != 0ull) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dp[r] = t[r] > 0.f ? dp[r] : 0.f;
+    }
+  }
+  return dp;
+}
+
 // This wave's share (of NW waves) of a 32-row tile of D columns: rows RPI (LPW wv + i) + l / CH,
 // chunk l % CH.
 template <int D, int NW>
@@ -1124,10 +1143,10 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBw
         // relu on the bits (a float is > 0 iff its bits as an int32 are): t = max(x, 0) with no
         // comparison per value; t and t^2 vanish with t.  (Whole-vector bit casts: hipcc
         // compiled a bit cast of one element of an ext_vector to element 0.)
-        const f32x16 T = relu16<NORM>(X);
+        const f32x16 T = relu16<NORM>(X), dP = finite_dp<NORM>(Dp, T);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const float ds = T[r] * Dp[r];
+          const float ds = T[r] * dP[r];
           bt += ds;
           if (want_l) lt = __builtin_fmaf(T[r], ds, lt);
           E[r] = NORM ? ds * rk[r] : ds;
@@ -1138,7 +1157,7 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBw
           const bool pos = X[r] > 0.f;
           const float ds = pos ? dpow_p<PK>(X[r], pw) * Dp[r] : 0.f;
           bt += ds;
-          if (want_l) lt = __builtin_fmaf(pos ? pow_p<PK>(X[r], pw) : 0.f, Dp[r], lt);
+          if (want_l) lt = pos ? __builtin_fmaf(pow_p<PK>(X[r], pw), Dp[r], lt) : lt;
           E[r] = NORM ? ds * rk[r] : ds;
         }
       }
@@ -1383,11 +1402,11 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kB
         }
         f32x16 EV, EK;
         if constexpr (PK == 2) {  // relu on the bits, as in bwd_dq_blk
-          const f32x16 T = relu16<NORM>(X);
+          const f32x16 T = relu16<NORM>(X), dP = finite_dp<NORM>(Dp, T);
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             EV[r] = T[r] * T[r];
-            const float ds = T[r] * Dp[r];
+            const float ds = T[r] * dP[r];
             EK[r] = NORM ? ds * rq[r] : ds;
           }
         } else {

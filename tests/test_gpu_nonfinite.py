@@ -1,5 +1,6 @@
 """Non-finite values of v where no weight meets them, in the normalised bf16 tile passes (lists that
-overflow): a tile whose weights are all zero adds nothing to the output, whatever v holds there."""
+overflow): a tile whose weights are all zero adds nothing to the output, and a pair without a weight
+adds nothing to a gradient, whatever v holds there."""
 import pytest
 import torch
 
@@ -8,6 +9,7 @@ from oracle.formula import rel_err, tda_grads
 
 pytestmark = pytest.mark.gpu
 TOL = 2e-2  # bf16 weights, results and gradients (2^-9 each)
+NAMES = {1: ["dq1", "dk1", "dv"], 2: ["dq1", "dq2", "dk1", "dk2", "dv"]}
 
 
 def _call(rows, beta, lam, p, br):
@@ -19,6 +21,38 @@ def _call(rows, beta, lam, p, br):
 def _oracle_rows(rows, br):
     rows = [x.double().cpu() for x in rows]
     return rows if br == 2 else [rows[0], None, rows[1], None, rows[2]]
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("d,br,p", [(64, 1, 2.0), (64, 2, 2.0), (128, 2, 2.0), (128, 1, 1.5), (256, 2, 2.0)])
+def test_value_rows_without_a_weight(d, br, p, bad):
+    """One key points away from every query (no weight in its column); its value row is not finite.
+    Every gradient is what a finite row there gives."""
+    n, j = 260, 70
+    g = torch.Generator("cpu").manual_seed(61)
+    mk = lambda: torch.randn((1, 2, n, d), generator=g)  # noqa: E731
+    qs, ks = [mk() for _ in range(br)], [mk() for _ in range(br)]
+    for q, k in zip(qs, ks):
+        q[..., 0] = 3.0 + q[..., 0].abs()
+        k[..., j, :] = 0.0
+        k[..., j, 0] = -4.0
+    rows = [x.bfloat16() for x in (*qs, *ks, mk())]
+    do = mk().bfloat16()
+    finite = [x.clone() for x in rows]
+    finite[-1][..., j, :] = 0.0
+    ref = tda_grads(*_oracle_rows(finite, br), do.double(), 0.4, 0.5, p, True, br)
+    assert ref["dbeta"].abs() > 0
+    rows[-1][..., j, :] = bad
+    leaves = [x.cuda().requires_grad_(True) for x in rows]
+    bt, lt = (torch.tensor(x, device="cuda", requires_grad=True) for x in (0.4, 0.5))
+    out = _call(leaves, bt, lt, p, br)
+    out.backward(do.cuda())
+    for leaf, name in zip(leaves, NAMES[br]):
+        assert torch.isfinite(leaf.grad).all(), name
+        assert rel_err(leaf.grad, ref[name]) <= TOL, name
+    assert abs(bt.grad.item() - ref["dbeta"].item()) <= 1e-3 * abs(ref["dbeta"].item()) + 1e-5
+    if br == 2:
+        assert abs(lt.grad.item() - ref["dlambda"].item()) <= 1e-3 * abs(ref["dlambda"].item()) + 1e-5
 
 
 @pytest.mark.parametrize("d,br", [(64, 1), (64, 2), (128, 1), (128, 2), (256, 2)])
