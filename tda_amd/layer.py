@@ -66,21 +66,34 @@ class ThresholdDifferentialAttention(nn.Module):
         else:
             self.lambda_param = None
 
-    def project(self, x: torch.Tensor):
-        """The (B, H, N, d) views of the projected q1, q2, k1, k2, v (q, k, v for TRA).  One
-        unbind, whose backward stacks the parts' gradients in one pass: indexing each part had its
-        backward fill, copy into and add up a whole projection's gradient per part (90 us of a
-        587 us step at (2, 1024), 16 heads of 64; the step now 507 us)."""
+    def _projection(self, x: torch.Tensor) -> torch.Tensor:
         b, n, _ = x.shape
-        y = self.in_proj(x).view(b, n, self.n_proj, self.num_heads, self.head_dim)
-        return [part.transpose(1, 2) for part in y.unbind(2)]
+        return self.in_proj(x).view(b, n, self.n_proj, self.num_heads, self.head_dim)
+
+    def project(self, x: torch.Tensor):
+        """The (B, H, N, d) views of the projected q1, q2, k1, k2, v (q, k, v for TRA).  A caller may
+        edit a view in place."""
+        y = self._projection(x)
+        return [y[:, :, i].transpose(1, 2) for i in range(self.n_proj)]
+
+    _own_project = project
+
+    def _parts(self, x: torch.Tensor):
+        """project(x), whoever defines it.  The class's own views are seen by the operator alone here, so
+        they come from one unbind: its backward stacks the parts' gradients in one pass, where
+        indexing fills, copies into and adds up a whole projection's gradient per part (14 kernels,
+        90 us of GPU time, of a training step at (2, 1024), 16 heads of 64).  autograd forbids
+        editing an unbind's results in place."""
+        if getattr(self.project, "__func__", None) is not ThresholdDifferentialAttention._own_project:
+            return self.project(x)
+        return [part.transpose(1, 2) for part in self._projection(x).unbind(2)]
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """x: (batch, seq_len, embed_dim), causal over seq_len."""
         if x.dim() != 3 or x.shape[-1] != self.embed_dim:
             raise ValueError(f"x must have shape (batch, seq_len, {self.embed_dim}), got {tuple(x.shape)}")
         b, n, _ = x.shape
-        parts = self.project(x)
+        parts = self._parts(x)
         if self.differential:
             q1, q2, k1, k2, v = parts
             o = differential_threshold_rela_triton(q1, q2, k1, k2, v, self.beta, self.lambda_param,

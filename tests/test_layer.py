@@ -55,6 +55,62 @@ def test_projections_are_views_and_output_layout():
     assert c.is_contiguous()
 
 
+def test_projected_parts_can_be_edited_in_place():
+    """An in-place step on a part (a rotary embedding, say) works in autograd, and gives the gradients
+    of the same step out of place."""
+    m = _layer(embed_dim=128, num_heads=2)
+    x = torch.randn(2, 7, 128)
+    scale = torch.rand(7, 1) + 0.5
+
+    def grads(edit):
+        parts = m.project(x)
+        parts = edit(parts)
+        loss = sum(((i + 1) * p * p).sum() for i, p in enumerate(parts))
+        return torch.autograd.grad(loss, list(m.in_proj.parameters()))
+
+    def in_place(parts):
+        parts[0].mul_(scale)
+        parts[2].add_(parts[0])
+        return parts
+
+    want = grads(lambda p: [p[0] * scale, p[1], p[2] + p[0] * scale, p[3], p[4]])
+    for got, ref in zip(grads(in_place), want):
+        torch.testing.assert_close(got, ref)
+
+
+@pytest.mark.parametrize("how", ["subclass", "instance", "class"])
+def test_forward_uses_an_overridden_project(how, monkeypatch):
+    """forward() takes its parts from project(), overridden in a subclass, on the instance or on the class
+    (the operator replaced by the formula: this runs on the CPU)."""
+    import types
+
+    from tda_amd import ThresholdDifferentialAttention, layer
+    monkeypatch.setattr(layer, "differential_threshold_rela_triton",
+                        lambda q1, q2, k1, k2, v, beta, lam, p, norm: tda(q1, q2, k1, k2, v, beta, lam, p, norm))
+
+    own = ThresholdDifferentialAttention.project
+
+    def project(self, x):
+        parts = own(self, x)
+        parts[4].mul_(2.0)
+        return parts
+
+    torch.manual_seed(3)
+    m = _layer(embed_dim=64, num_heads=1, beta_init=0.2)
+    x = torch.randn(1, 9, 64)
+    plain = m(x)
+    if how == "subclass":
+        m.__class__ = type("Doubled", (ThresholdDifferentialAttention,), {"project": project})
+    elif how == "class":
+        monkeypatch.setattr(ThresholdDifferentialAttention, "project", project)
+    else:
+        m.project = types.MethodType(project, m)
+    out = m(x)
+    torch.testing.assert_close(out, 2.0 * plain)
+    out.sum().backward()
+    assert m.in_proj.weight.grad.abs().max() > 0
+
+
 def _oracle_layer(m, x, differential):
     """The same layer from the oracle formula, in float64 on the CPU, with m's weights."""
     W = m.in_proj.weight.detach().double().cpu().requires_grad_(True)
