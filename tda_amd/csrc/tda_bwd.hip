@@ -649,6 +649,7 @@ bwd_dq_split_f32(BwdParams P) {
       atomicAdd(P.stats + 1, (unsigned long long)computed);
     }
   }
+  wave_lds_sync();  // with one wave no barrier follows: lane 1 reads what lane 0 wrote
   f32_split_sum<D, W>(lds, SL, wv, A);
   if (wv) return;
   const int gslot = br == 0 ? B_DQ1 : B_DQ2;

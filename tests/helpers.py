@@ -27,5 +27,42 @@ def oracle_out(q1, q2, k1, k2, v, beta, lam, p, normalize, branches, heads=None,
                        float(beta), float(lam), p, normalize, branches=branches, heads=heads, dtype=dtype)
 
 
+def rel_norm(y, ref) -> float:
+    """2-norm of the difference over the 2-norm of the reference."""
+    y, ref = y.detach().double().cpu(), ref.detach().double().cpu()
+    return ((y - ref).norm() / ref.norm().clamp_min(1e-300)).item()
+
+
+def grads_on_gpu(rows, dout, beta, lam, p, normalize, branches, q_offset=0):
+    """tda_grads of every head, evaluated in float64 on the GPU a batch entry at a time: a dict of out,
+    the rows' gradients and the scalars', and for the scalars beta_scale and lambda_scale, the sums of
+    their per-row contributions' magnitudes (what the rounding of sums of both signs is measured
+    against)."""
+    from oracle.formula import tda, tra
+    names = ["dq1", "dq2", "dk1", "dk2", "dv"] if branches == 2 else ["dq1", "dk1", "dv"]
+    n = rows[0].shape[2]
+    res = {k: [] for k in ["out", *names]}
+    res.update(dbeta=0.0, dlambda=0.0, beta_scale=0.0, lambda_scale=0.0)
+    for b in range(rows[0].shape[0]):
+        xs = [x.detach()[b:b + 1].double().cuda().requires_grad_(True) for x in rows]
+        bt = torch.full((n,), float(beta), dtype=torch.float64, device="cuda", requires_grad=True)
+        if branches == 2:
+            lt = torch.full((n, 1), float(lam), dtype=torch.float64, device="cuda", requires_grad=True)
+            out = tda(*xs, bt, lt, p, normalize, q_offset=q_offset)
+            g = torch.autograd.grad(out, [*xs, bt, lt], dout[b:b + 1].double().cuda())
+            res["dlambda"] += g[-1].sum().item()
+            res["lambda_scale"] += g[-1].abs().sum().item()
+            g = g[:-1]
+        else:
+            out = tra(*xs, bt, p, normalize, q_offset=q_offset)
+            g = torch.autograd.grad(out, [*xs, bt], dout[b:b + 1].double().cuda())
+        res["dbeta"] += g[-1].sum().item()
+        res["beta_scale"] += g[-1].abs().sum().item()
+        res["out"].append(out.detach())
+        for name, x in zip(names, g):
+            res[name].append(x)
+    return {k: torch.cat(v) if isinstance(v, list) else v for k, v in res.items()}
+
+
 def heads_of(x, heads):
     return torch.stack([x[b, h] for (b, h) in heads])

@@ -1,15 +1,17 @@
 """fp32 without normalisation: the split passes, one resident tile per workgroup, its streamed tiles
 dealt to four, two or one waves (f32_split in tda_common.hpp: below 2048 resident tiles four; from
 there two, and one for rows of at most 16 tiles or from 4096 tiles at d = 128), against the formula in
-64 bits.  Sizes on both sides of each line, fewer streamed tiles than waves, ragged last tiles, a key
+64 bits, every head and the gradients of beta and lambda.  Sizes on both sides of each line, fewer streamed tiles than waves, ragged last tiles, a key
 cache longer than the queries, and rows past one bitmask round (2048 key tiles).  1e-4 normwise: fp32
 products and sums of at most 65600 terms of random signs (2^-24 sqrt(65600) = 1.5e-5), the power's
-factor two, and the cancellation in score - tau."""
+factor two, and the cancellation in score - tau; the scalars 1e-6 of the sum of their rows' contributions
+(sums of both signs, over the tiles in fp64)."""
 import pytest
 import torch
 
 import tda_amd
-from oracle.formula import rel_err, tda_grads
+from oracle.formula import rel_err
+from tests.helpers import grads_on_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -21,27 +23,29 @@ pytestmark = pytest.mark.gpu
     (16, 32, 128, 128, 64, 1, 2.0),  # 2048 tiles, short rows: one wave
     (8, 15, 545, 545, 64, 1, 2.0),   # 2160 tiles of 18: two waves
     (8, 31, 545, 545, 128, 1, 2.0),  # 4464 tiles of 18 at d = 128: one wave
+    (16, 32, 128, 128, 64, 2, 2.0),  # two branches, one wave
+    (8, 15, 545, 545, 64, 2, 2.0),   # two branches, two waves
+    (8, 15, 545, 545, 128, 1, 1.5),  # d = 128: two waves
+    (8, 15, 545, 545, 128, 2, 2.0),  # d = 128: two waves, one in the query-major pass (4320 tiles)
 ])
 def test_against_the_formula(b, h, nq, nk, d, br, p):
     g = torch.Generator("cuda").manual_seed(nq + d)
     rows = [torch.randn((b, h, n, d), generator=g, device="cuda") for n in (nq, nq, nk, nk, nk, nq)]
-    heads = sorted({0, b * h - 1})  # the heads that the formula checks
-    q1, q2, k1, k2, v = (x.requires_grad_(True) for x in rows[:5])
+    q1, q2, k1, k2, v, do = rows
+    leaves = [x.requires_grad_(True) for x in ([q1, q2, k1, k2, v] if br == 2 else [q1, k1, v])]
+    bt, lt = (torch.tensor(x, device="cuda", requires_grad=True) for x in (1.0, 0.4))
     if br == 2:
-        out = tda_amd.differential_threshold_rela_triton(q1, q2, k1, k2, v, 1.0, 0.4, relu_power=p, normalize=False)
-        leaves = [q1, q2, k1, k2, v]
+        out = tda_amd.differential_threshold_rela_triton(*leaves, bt, lt, relu_power=p, normalize=False)
     else:
-        out = tda_amd.threshold_rela_triton(q1, k1, v, 1.0, relu_power=p, normalize=False)
-        leaves = [q1, k1, v]
-    grads = torch.autograd.grad(out, leaves, rows[5])
-    names = ["dq1", "dq2", "dk1", "dk2", "dv"] if br == 2 else ["dq1", "dk1", "dv"]
-    for bh in heads:
-        i, j = divmod(bh, h)
-        one = [x.detach()[i:i + 1, j:j + 1].double().cpu() for x in rows]
-        ref = tda_grads(*one, 1.0, 0.4, p, False, br, q_offset=nk - nq)
-        assert rel_err(out[i:i + 1, j:j + 1], ref["out"]) < 1e-4
-        for name, x in zip(names, grads):
-            assert rel_err(x[i:i + 1, j:j + 1], ref[name]) < 1e-4, name
+        out = tda_amd.threshold_rela_triton(*leaves, bt, relu_power=p, normalize=False)
+    out.backward(do)
+    ref = grads_on_gpu(leaves, do, 1.0, 0.4, p, False, br, q_offset=nk - nq)
+    assert rel_err(out, ref["out"]) < 1e-4
+    for x, name in zip(leaves, ["dq1", "dq2", "dk1", "dk2", "dv"] if br == 2 else ["dq1", "dk1", "dv"]):
+        assert rel_err(x.grad, ref[name]) < 1e-4, name
+    assert abs(bt.grad.item() - ref["dbeta"]) <= 1e-6 * ref["beta_scale"]
+    if br == 2:
+        assert abs(lt.grad.item() - ref["dlambda"]) <= 1e-6 * ref["lambda_scale"]
 
 
 def test_rows_longer_than_a_bitmask_round():
