@@ -1,13 +1,14 @@
 """Normalised calls whose threshold scale lets a few per cent of the weights through: the candidate
 and pair lists overflow, so the tile passes (fwd_pv_blk after the screen; bwd_tiles over the queue
 of blocks, or bwd_dq_blk and bwd_dkv_blk without a queue) take most query and key tiles, beside
-some that still fit.  Output and every gradient against the fp64 oracle."""
+some that still fit.  Output and every gradient, beta's and lambda's too, against the fp64 oracle."""
 import pytest
 import torch
 
 import tda_amd
 from oracle.formula import rel_err, tda_grads
 from tda_amd import ops
+from tests.helpers import grads_on_gpu, rel_norm
 
 pytestmark = pytest.mark.gpu
 TOL = 2e-2  # bf16 weights, results and gradients (2^-9 each) in sums of up to a few hundred terms
@@ -50,6 +51,32 @@ def test_overflowing_lists_against_the_oracle(nq, nk, d, br, p, beta):
         assert rel_err(leaf.grad, ref[name]) <= TOL, name
     # the scalars are sums of terms of both signs, each with the rounding of bf16 products' inputs only
     assert abs(bt.grad.item() - ref["dbeta"].item()) <= 1e-3 * abs(ref["dbeta"].item()) + 1e-5
+    if br == 2:
+        assert abs(lt.grad.item() - ref["dlambda"].item()) <= 1e-3 * abs(ref["dlambda"].item()) + 1e-5
+
+
+@pytest.mark.parametrize("b,h,n,d,br,blocks", [(2, 16, 1500, 64, 2, 512), (3, 12, 1100, 128, 1, 256)])
+def test_more_queued_blocks_than_workgroups(b, h, n, d, br, blocks):
+    """bwd_tiles with more blocks in its queue than the GPU holds workgroups (`blocks`): they take
+    further tickets, key blocks and then query blocks, in the same LDS.  Every head, in the 2-norm: bf16
+    weights and results, 2^-9 at most each."""
+    rows, do = _inputs(b, h, n, n, d, br, torch.bfloat16, 33)
+    leaves = [x.cuda().requires_grad_(True) for x in rows]
+    bt, lt = (torch.tensor(x, device="cuda", requires_grad=True) for x in (0.5, 0.4))
+    if br == 2:
+        out = tda_amd.differential_threshold_rela_triton(*leaves, bt, lt, normalize=True)
+    else:
+        out = tda_amd.threshold_rela_triton(*leaves, bt, normalize=True)
+    out.backward(do.cuda())
+    tiles = -(-n // 32)
+    assert b * h * -(-tiles // 4) * (br + 1) * 0.8 > blocks  # (the first blocks' lists may fit)
+    ref = grads_on_gpu(rows, do, 0.5, 0.4, 2.0, True, br)
+    assert rel_norm(out, ref["out"]) <= 2.0 ** -8
+    for leaf, name in zip(leaves, ["dq1", "dq2", "dk1", "dk2", "dv"] if br == 2 else ["dq1", "dk1", "dv"]):
+        assert rel_norm(leaf.grad, ref[name]) <= 2.0 ** -8, name
+    assert abs(bt.grad.item() - ref["dbeta"]) <= 1e-5 * ref["beta_scale"]
+    if br == 2:
+        assert abs(lt.grad.item() - ref["dlambda"]) <= 1e-5 * ref["lambda_scale"]
 
 
 @pytest.mark.parametrize("d,br", [(64, 2), (128, 1)])
