@@ -258,6 +258,33 @@ def test_bwd_norms_optional_without_normalize():
     assert lib.tda_validate_bwd(ctypes.byref(a)) == _abi.OK
 
 
+def test_python_workspace_has_room_for_the_finer_decode_split():
+    """The Python entry points' forward workspace holds the partial outputs of 8-tile chunks wherever
+    the launcher would take them (include/tda.h, workspace), and is the documented size elsewhere."""
+    from tda_amd import ops
+    lib = _lib()
+    r256 = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    finer = 0
+    for b, h, n, nk, d, dt in [(1, 8, 1, 1000, 64, torch.bfloat16), (1, 1, 1, 1, 64, torch.float32),
+                               (2, 2, 32, 1025, 128, torch.bfloat16), (1, 3, 7, 257, 64, torch.float32),
+                               (1, 2, 16, 65536, 128, torch.bfloat16), (1, 2, 16, 65537, 128, torch.bfloat16),
+                               (16, 32, 1, 97, 64, torch.bfloat16), (7, 73, 1, 97, 64, torch.float32),
+                               (1, 32, 32, 4096, 128, torch.bfloat16), (1, 8, 33, 1000, 64, torch.bfloat16),
+                               (1, 8, 1, 1000, 256, torch.bfloat16)]:
+        q, k = torch.empty((b, h, n, d), dtype=dt, device="meta"), torch.empty((b, h, nk, d), dtype=dt, device="meta")
+        tpl, ws = ops._fwd_template((q, k, None, None, k, q), 1, False, 2.0, max(nk - n, 0), 0)
+        a = _abi.TdaFwdArgs.from_buffer_copy(tpl)
+        documented = lib.tda_fwd_workspace_bytes_for(ctypes.byref(a))
+        assert documented > 0 and a.workspace_bytes == ws
+        bh, nkt = b * h, -(-nk // 32)
+        if n <= 32 and d <= 128 and bh * -(-nkt // 32) < 512 and bh * -(-nkt // 8) * n <= 8192:
+            finer += 1
+            assert ws >= documented - r256(bh * -(-nkt // 32) * n * 512) + r256(bh * -(-nkt // 8) * n * 512)
+        elif n > 32 or d > 128:
+            assert ws == r256(documented)
+    assert finer == 6
+
+
 def test_buffer_sizes():
     lib = _lib()
     assert lib.tda_occupancy_words(4, 16, 4096, 2) == 2 * 64 * 128 * 4

@@ -7,6 +7,8 @@ not need contribute exact zeros; to rounding for a bf16 block of one query tile,
 the decode kernels); decode (one query at the last position) and other shapes
 against the CPU oracle with the position offset; gradients against fp64 autograd of the
 oracle formula; the tile counters against the causal tile ranges."""
+import ctypes
+
 import pytest
 import torch
 
@@ -134,17 +136,33 @@ def test_offset_tile_counters(dt):
     assert st.tiles_nonzero == int(st.occupancy.sum())
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f32"])
+@pytest.mark.parametrize("chunk", [8, 32])
 @pytest.mark.parametrize("nq", [1, 7, 32])
 @pytest.mark.parametrize("nk,where", [(200, "last"), (5000, "last"), (5000, "middle")])
-def test_decode_side_outputs(nq, nk, where):
-    """bf16 with one query tile takes the split-key decode kernels: output, norms table, tile
-    bitmask and counters against the oracle (5000 keys = 157 key tiles = 5 chunks summed in
-    order), and the backward driven by its bitmask equals the backward that tests every tile."""
-    from tda_amd import ops
+def test_decode_side_outputs(nq, nk, where, chunk, dt, monkeypatch):
+    """One query tile takes the split-key decode kernels: output, norms table, tile bitmask and
+    counters against the oracle, and the backward driven by its bitmask equals the backward that
+    tests every tile.  In chunks of 8 key tiles, for whose partial outputs the Python entry points
+    make room (5000 keys = 157 key tiles = 20 chunks summed in order), and of 32, in a workspace of
+    the documented size (5 chunks; a wave's eight tiles per chunk and branch, the bitmask's whole
+    words)."""
+    from tda_amd import _abi, ops
     from oracle.formula import tau
+    dtype = DT[dt]
+    if chunk == 32:
+        template = ops._fwd_template
+
+        def documented(*args):
+            a = _abi.TdaFwdArgs.from_buffer_copy(template(*args)[0])
+            a.workspace_bytes = _abi.load().tda_fwd_workspace_bytes_for(ctypes.byref(a))
+            assert a.workspace_bytes < template(*args)[1]
+            return bytes(a), a.workspace_bytes
+
+        monkeypatch.setattr(ops, "_fwd_template", documented)
     off = nk - nq if where == "last" else nk // 2
-    q1, q2, do = make_inputs((1, 3, nq, 128), 59, 3, torch.bfloat16)
-    k1, k2, v = make_inputs((1, 3, nk, 128), 60, 3, torch.bfloat16)
+    q1, q2, do = make_inputs((1, 3, nq, 128), 59, 3, dtype)
+    k1, k2, v = make_inputs((1, 3, nk, 128), 60, 3, dtype)
     beta = torch.full((), 0.7, device="cuda")
     lam = torch.full((), 0.5, device="cuda")
     norms, occ = ops.side_buffers(q1.shape, 2, True, "cuda", nk)
@@ -153,7 +171,7 @@ def test_decode_side_outputs(nq, nk, where):
                       q_offset=off)
     ref = _oracle(q1, q2, k1, k2, v, 0.7, 0.5, 2.0, True, 2, off)
     assert ref.abs().max() > 0
-    assert rel_err(out, ref) <= TOL[torch.bfloat16]
+    assert rel_err(out, ref) <= TOL[dtype]
     BH, nkt = 3, (nk + 31) // 32
     nrm = norms.cpu()
     slots = [(q1, nq), (k1, nk), (q2, nq), (k2, nk)]
@@ -181,7 +199,8 @@ def test_decode_side_outputs(nq, nk, where):
     assert mism <= 2, mism  # only threshold ties within rounding may differ
     visited, computed, checked = (int(x) for x in stats.tolist())
     assert visited == 2 * BH * (last + 1)
-    assert computed == checked == int(bits.sum())
+    assert computed == int(bits.sum())
+    assert checked == (computed if dt == "bf16" else 0)  # (fp32 has no screened count)
     assert 0 < computed < visited
     a = ops.backward(q1, k1, q2, k2, v, do, beta, lam, 2.0, True, 2, norms=norms, occupancy=occ, q_offset=off)
     b = ops.backward(q1, k1, q2, k2, v, do, beta, lam, 2.0, True, 2, norms=norms, occupancy=None, q_offset=off)
