@@ -22,7 +22,7 @@ Superset behaviour (all results identical where the reference is defined):
     when Nq = Nk, which is the reference's case.
 Only the causal form exists, as in the reference.  Supported head_dim: 16, 32, 64, 128, 256
 (the reference takes any power of two >= 16, TTA:348, :366-368).  The kernels run d = 64, 128
-and 256 (256: column-split kernels, each wave owning half of the output columns);
+and 256 (256: a wave owns half of the output's or a gradient's columns);
 d = 16 and 32 are computed at d = 64 with the rows zero-padded (dot products and norms
 unchanged) and beta scaled by sqrt(64 / d), so that tau = beta sqrt(2 ln(P+1) / d) is the same
 threshold; the padding's gradients are dropped and beta's gradient flows through the scaling.

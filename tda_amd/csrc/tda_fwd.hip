@@ -2,25 +2,21 @@
 //
 // Reference semantics (snap-research/TDA triton_threshold_attention.py, "TTA"):
 //   forward kernel TTA:19-115, differential composition TTA:489-519.
-// Every 32x32 (query tile, key tile) pair on or below the diagonal is visited; the scores of
-// both branches are formed on the matrix cores, thresholded in registers, and the A.V
+// The fp32 kernels (head_dim up to 128, more than one query tile) and the dispatch of every forward.
+// The scores of both branches are formed on the matrix cores, thresholded in registers, and the A.V
 // product is issued only when a wave-wide ballot finds a non-zero entry (ReLU leaves almost
 // every tile empty: TDA is ultra-sparse).  The two branches share one accumulator:
 // out = sum_j (A1_ij - clamp(lambda) A2_ij) v_j, so the differential combine is free.
-#include <type_traits>
-
 #include "tda_common.hpp"
 #include "tda_params.hpp"
 #include "tda_pos.hpp"
 
 namespace tda {
 
-template <class Pol, int D> struct TTileSel;
-template <int D> struct TTileSel<PolBF16, D> { using type = TTileBF16<D>; };
-template <int D> struct TTileSel<PolF32, D> { using type = TTileF32<D>; };
-
-// One wave per 32-row query tile, four independent waves per workgroup.  Work items are
-// ordered longest-first (the last query tiles have the most causal key tiles).
+// ------------------------------------------------------------------ fwd_wave
+// fp32 with normalisation, after key_prep and fwd_screen_i8 ran on the same inputs: the query tiles
+// the candidate pass (fwd_cand_f32) queued, whose candidate lists did not fit.  One wave per 32-row query
+// tile, four independent waves per workgroup, taking the queue's tiles in turn.
 //
 // Layouts (see tda_common.hpp): the score tile is computed transposed, S^T = K Q^T, with the
 // key rows as the A operand (row fragments loaded from HBM per key tile) and the wave's query
@@ -28,43 +24,29 @@ template <int D> struct TTileSel<PolF32, D> { using type = TTileF32<D>; };
 // so the per-query threshold, inverse norm and the causal test are per-lane scalars, and the
 // thresholded tile packs directly into the B operand of O^T += V^T A^T.
 //
-// SCR (fp32, normalised, after key_prep and fwd_screen_i8 ran on the same inputs): the screen's
-// bitmask names every key tile holding a non-zero weight (a superset), so the wave visits only
-// those tiles; the inverse norms come from the table the screen and key_prep wrote (the values
-// the screen's bound is stated for), and the bitmask words are rewritten exactly.
-//
-// QUEUE (with SCR): only the query tiles the fp32 candidate pass (fwd_cand_f32) queued, whose
-// candidate lists did not fit; the waves take them in turn.
-template <class Pol, int D, int BR, int PK, bool NORM, bool SCR>
-__device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh, int wv);
+// The screen's bitmask names every key tile holding a non-zero weight (a superset), so the wave
+// visits only those tiles; the inverse norms come from the table the screen and key_prep wrote (the
+// values the screen's bound is stated for), and the bitmask words are rewritten exactly.
+template <int D, int BR, int PK>
+__device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh);
 
-template <class Pol, int D, int BR, int PK, bool NORM, bool SCR = false, bool QUEUE = false>
+template <int D, int BR, int PK>
 __global__ void __launch_bounds__(256) fwd_wave(FwdParams P) {
-  static_assert(!QUEUE || SCR, "the queue comes from the screened candidate pass");
-  const int wv = threadIdx.x >> 6;
-  const int BH = P.B * P.H;
-  if constexpr (QUEUE) {
-    const uint32_t queued = P.pvq[0];
-    for (uint32_t k = blockIdx.x * 4u + (uint32_t)wv; k < queued; k += gridDim.x * 4u) {
-      const int v = (int)P.pvq[1 + k];
-      fwd_wave_tile<Pol, D, BR, PK, NORM, SCR>(P, v % P.nqt, v / P.nqt, wv);
-    }
-    return;
+  const uint32_t queued = P.pvq[0];
+  for (uint32_t k = blockIdx.x * 4u + (threadIdx.x >> 6); k < queued; k += gridDim.x * 4u) {
+    const int v = (int)P.pvq[1 + k];
+    fwd_wave_tile<D, BR, PK>(P, v % P.nqt, v / P.nqt);
   }
-  const int64_t item = (int64_t)blockIdx.x * 4 + wv;
-  if (item >= (int64_t)BH * P.nqt) return;  // whole wave leaves; no workgroup barriers below
-  fwd_wave_tile<Pol, D, BR, PK, NORM, SCR>(P, P.nqt - 1 - (int)(item / BH), (int)(item % BH), wv);
 }
 
-template <class Pol, int D, int BR, int PK, bool NORM, bool SCR>
-__device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh, int wv) {
-  static_assert(!SCR || NORM, "the screened pass is the normalised one");
+template <int D, int BR, int PK>
+__device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh) {
+  using Pol = PolF32;
   using T = typename Pol::T;
   using frag = typename Pol::frag;
   constexpr int NT = D / Pol::KS;  // MFMA steps over d
   constexpr int NS = 32 / Pol::KS; // MFMA steps over a 32-key tile
   constexpr int ND = D / 32;       // 32-wide column blocks of the output
-  using TT = typename TTileSel<Pol, D>::type;
 
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
   const int BH = P.B * P.H;
@@ -92,66 +74,50 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
     }
   }
   float rq1 = 1.f, rq2 = 1.f;
-  if constexpr (SCR) {
-    if (qvalid) {
-      rq1 = P.norms[norm_base(P, N_Q1, bh) + i];
-      if constexpr (BR == 2) rq2 = P.norms[norm_base(P, N_Q2, bh) + i];
-    }
-  } else if constexpr (NORM) {
-    rq1 = inv_norm(row_sumsq<Pol, NT>(Q1));
-    if constexpr (BR == 2) rq2 = inv_norm(row_sumsq<Pol, NT>(Q2));
-    if (P.norms && qvalid && g == 0) {
-      P.norms[norm_base(P, N_Q1, bh) + i] = rq1;
-      if constexpr (BR == 2) P.norms[norm_base(P, N_Q2, bh) + i] = rq2;
-    }
+  if (qvalid) {
+    rq1 = P.norms[norm_base(P, N_Q1, bh) + i];
+    if constexpr (BR == 2) rq2 = P.norms[norm_base(P, N_Q2, bh) + i];
   }
   const float pw = P.p;
   const float tau = (*P.beta) * tau_coeff(pq, P.inv_d);
   float lam = 0.f;
   if constexpr (BR == 2) lam = clamp01(*P.lam);
 
-  __shared__ __attribute__((aligned(16))) bf16 lds_all[(sizeof(T) == 2) ? 4 * TTileBF16<D>::ELEMS : 8];
-  TT vt;
-  if constexpr (sizeof(T) == 2) vt.lds = lds_all + wv * TTileBF16<D>::ELEMS;
+  TTileF32<D> vt;
 
   f32x16 O[ND];
 #pragma unroll
   for (int c = 0; c < ND; ++c) O[c] = f32x16{};
 
   // bitmask rows [branch][B*H][query tile][word] of this query tile
-  uint32_t* occrow = P.occ ? P.occ + ((int64_t)bh * P.nqt + qt) * P.occ_w : nullptr;
+  uint32_t* occrow = P.occ + ((int64_t)bh * P.nqt + qt) * P.occ_w;
   const int64_t occ_br = (int64_t)BH * P.nqt * P.occ_w;  // distance between the branch planes
   uint32_t word = 0, word2 = 0;
-  unsigned visited = 0, computed = 0, checked = 0;
+  unsigned computed = 0, checked = 0;
 
   for (int kt = 0; kt <= ktl; ++kt) {
-    bool use1 = true, use2 = true;  // SCR: the branches the screen kept this tile in
-    if constexpr (SCR) {
-      // the screen's bits of this word (per branch), read before this wave rewrites the word
-      const uint32_t s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)occrow[kt >> 5]);
-      const uint32_t s2 = BR == 2 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)occrow[occ_br + (kt >> 5)]) : 0u;
-      const uint32_t keep = (s1 | s2) & (~0u << (kt & 31));  // kept tiles kt .. of the word
-      const int next = keep ? (kt & ~31) + __builtin_ctz(keep) : (kt | 31) + 1;
-      if (next > kt) {  // skipped tiles hold no weight: close the word if it ends among them
-        const int wend = kt | 31;
-        if (next > wend || next > ktl) {
-          if (l == 0) {
-            occrow[kt >> 5] = word;
-            if constexpr (BR == 2) occrow[occ_br + (kt >> 5)] = word2;
-          }
-          word = word2 = 0;
-          kt = wend;
-          continue;
+    // the screen's bits of this word (per branch), read before this wave rewrites the word
+    const uint32_t s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)occrow[kt >> 5]);
+    const uint32_t s2 = BR == 2 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)occrow[occ_br + (kt >> 5)]) : 0u;
+    const uint32_t keep = (s1 | s2) & (~0u << (kt & 31));  // kept tiles kt .. of the word
+    const int next = keep ? (kt & ~31) + __builtin_ctz(keep) : (kt | 31) + 1;
+    if (next > kt) {  // skipped tiles hold no weight: close the word if it ends among them
+      const int wend = kt | 31;
+      if (next > wend || next > ktl) {
+        if (l == 0) {
+          occrow[kt >> 5] = word;
+          if constexpr (BR == 2) occrow[occ_br + (kt >> 5)] = word2;
         }
-        kt = next;
+        word = word2 = 0;
+        kt = wend;
+        continue;
       }
-      use1 = (s1 >> (kt & 31)) & 1u;
-      use2 = (s2 >> (kt & 31)) & 1u;
-      checked += (use1 ? 1u : 0u) + (use2 ? 1u : 0u);
+      kt = next;
     }
+    const bool use1 = (s1 >> (kt & 31)) & 1u, use2 = (s2 >> (kt & 31)) & 1u;  // the branches that keep the tile
+    checked += (use1 ? 1u : 0u) + (use2 ? 1u : 0u);
     const int k0 = kt * 32;
     const int j = k0 + n32;  // key row this lane loads for the A operand
-    const bool kfirst = qt == qt_first(kt, qoff);  // the first query tile to see kt writes its norms
     f32x16 S1 = f32x16{}, S2 = f32x16{};
     float rk1r[16] = {}, rk2r[16] = {};
     // a branch the screen did not keep here holds no weight in the tile: no scores for it
@@ -161,14 +127,9 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
       Pol::template load_rows<NT>(r1, g, K1);
 #pragma unroll
       for (int t = 0; t < NT; ++t) S1 = Pol::mma(K1[t], Q1[t], S1);
-      if constexpr (NORM) {
-        float rk;
-        if constexpr (SCR) rk = j < Nk ? P.norms[norm_base(P, N_K1, bh) + j] : 0.f;
-        else rk = inv_norm(row_sumsq<Pol, NT>(K1));
-        if (!SCR && P.norms && kfirst && g == 0 && j < Nk) P.norms[norm_base(P, N_K1, bh) + j] = rk;
+      const float rk = j < Nk ? P.norms[norm_base(P, N_K1, bh) + j] : 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) rk1r[r] = __shfl(rk, crow(r, g));
-      }
+      for (int r = 0; r < 16; ++r) rk1r[r] = __shfl(rk, crow(r, g));
     }
     if (BR == 2 && use2) {
       frag K2[NT];
@@ -176,14 +137,9 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
       Pol::template load_rows<NT>(r2, g, K2);
 #pragma unroll
       for (int t = 0; t < NT; ++t) S2 = Pol::mma(K2[t], Q2[t], S2);
-      if constexpr (NORM) {
-        float rk;
-        if constexpr (SCR) rk = j < Nk ? P.norms[norm_base(P, N_K2, bh) + j] : 0.f;
-        else rk = inv_norm(row_sumsq<Pol, NT>(K2));
-        if (!SCR && P.norms && kfirst && g == 0 && j < Nk) P.norms[norm_base(P, N_K2, bh) + j] = rk;
+      const float rk = j < Nk ? P.norms[norm_base(P, N_K2, bh) + j] : 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) rk2r[r] = __shfl(rk, crow(r, g));
-      }
+      for (int r = 0; r < 16; ++r) rk2r[r] = __shfl(rk, crow(r, g));
     }
 
     // Threshold test.  x = fma(s * rk_j, rq_i, -tau_i) is monotone in s * rk_j, so the tile
@@ -193,17 +149,16 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
     for (int r = 0; r < 16; ++r) {
       const int key = k0 + crow(r, g);
       const bool valid = qvalid && key <= pq && key < Nk;
-      if constexpr (NORM) S1[r] *= rk1r[r];
+      S1[r] *= rk1r[r];
       m1 = fmaxf(m1, valid ? S1[r] : -INFINITY);
       if constexpr (BR == 2) {
-        if constexpr (NORM) S2[r] *= rk2r[r];
+        S2[r] *= rk2r[r];
         m2 = fmaxf(m2, valid ? S2[r] : -INFINITY);
       }
     }
     const bool any1 = use1 && wave_ballot(__builtin_fmaf(m1, rq1, -tau) > 0.f) != 0ull;
     bool any2 = false;
     if constexpr (BR == 2) any2 = use2 && wave_ballot(__builtin_fmaf(m2, rq2, -tau) > 0.f) != 0ull;
-    visited += BR;
     computed += (any1 ? 1 : 0) + (any2 ? 1 : 0);
     if (any1) word |= 1u << (kt & 31);
     if (any2) word2 |= 1u << (kt & 31);
@@ -224,21 +179,15 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
         }
         C[r] = a;
       }
-      if constexpr (sizeof(T) == 2) {
-        vt.stage(vv, b, h, k0, Nk);
-        wave_lds_sync();
-      } else {
-        vt.set(vv, b, h, k0, Nk);
-      }
+      vt.set(vv, b, h, k0, Nk);
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
         const frag bp = Pol::pack_c(C, s);
 #pragma unroll
         for (int c = 0; c < ND; ++c) O[c] = Pol::mma(vt.frag(s, c), bp, O[c]);
       }
-      if constexpr (sizeof(T) == 2) wave_lds_sync();
     }
-    if (occrow && (((kt & 31) == 31) || kt == ktl)) {
+    if ((kt & 31) == 31 || kt == ktl) {
       if (l == 0) {
         occrow[kt >> 5] = word;
         if constexpr (BR == 2) occrow[occ_br + (kt >> 5)] = word2;
@@ -246,7 +195,7 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
       word = word2 = 0;
     }
   }
-  if (occrow && l == 0) {
+  if (l == 0) {
     for (int w = (ktl >> 5) + 1; w < P.occ_w; ++w) {
       occrow[w] = 0u;
       if constexpr (BR == 2) occrow[occ_br + w] = 0u;
@@ -258,28 +207,6 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
       P.pairs[pair_lists(BR, BH, P.nqt) * 4 * kPairCap + ((int64_t)br * BH + bh) * P.nqt + qt] = kPairOverflow;
   }
 
-  // Key tiles no query tile sees (keys past the last query position): their inverse norms
-  // still go to the table (the backward's normalize epilogue reads every key row's), written
-  // by the last query tile's wave (with SCR key_prep wrote every key row's).
-  if constexpr (NORM && !SCR) {
-    if (P.norms && qt == P.nqt - 1) {
-      for (int kt = ktl + 1; kt < P.nkt; ++kt) {
-        const int j = 32 * kt + n32;
-        frag K[NT];
-        const T* r1 = (j < Nk) ? k1.row(b, h, j) : nullptr;
-        Pol::template load_rows<NT>(r1, g, K);
-        const float rka = inv_norm(row_sumsq<Pol, NT>(K));
-        if (g == 0 && j < Nk) P.norms[norm_base(P, N_K1, bh) + j] = rka;
-        if constexpr (BR == 2) {
-          const T* r2 = (j < Nk) ? k2.row(b, h, j) : nullptr;
-          Pol::template load_rows<NT>(r2, g, K);
-          const float rkb = inv_norm(row_sumsq<Pol, NT>(K));
-          if (g == 0 && j < Nk) P.norms[norm_base(P, N_K2, bh) + j] = rkb;
-        }
-      }
-    }
-  }
-
   if (qvalid) {
     T* orow = out.row(b, h, i);
 #pragma unroll
@@ -288,9 +215,9 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
       for (int u = 0; u < 4; ++u)
         store4(orow + 32 * c + 8 * u + 4 * g, O[c][4 * u], O[c][4 * u + 1], O[c][4 * u + 2], O[c][4 * u + 3]);
   }
-  if (P.stats && l == 0) {  // with SCR the screen counted the causal tiles; `checked`: its kept ones
-    atomicAdd(P.stats + (SCR ? 2 : 0), (unsigned long long)(SCR ? checked : visited));
+  if (P.stats && l == 0) {  // (the screen counted the causal tiles; checked: those it kept)
     atomicAdd(P.stats + 1, (unsigned long long)computed);
+    atomicAdd(P.stats + 2, (unsigned long long)checked);
   }
 }
 
@@ -663,56 +590,49 @@ __global__ void __launch_bounds__(64 * BR) fwd_cand_f32(FwdParams P) {
 }
 
 // ------------------------------------------------------------------ dispatch
-// Normalised fp32 calls with more than one query tile and the int8 keys' workspace run the int8
-// screen first (key_prep and fwd_screen_i8 on the fp32 rows, tda_fwd_sparse.hip), then the
-// screened fwd_wave.
-template <class Pol, int D, int BR, int PK, bool NORM>
+// fp32 with more than one query tile.  Normalised: the int8 screen with candidate lists (key_prep and
+// fwd_screen_i8 on the fp32 rows, tda_fwd_sparse.hip), the candidate pass, then the tile pass over the
+// query tiles whose lists overflowed.  Without: a query tile per workgroup, its key tiles split over
+// the waves.
+template <int D, int BR, int PK, bool NORM>
 static int launch_fwd_t(const FwdParams& p, const KernelKey& k, void* stream) {
-  static_assert(std::is_same<Pol, PolF32>::value, "the fp32 dispatch (bf16 runs tda_fwd_sparse.hip)");
   const int64_t items = (int64_t)p.B * p.H * p.nqt;
-  const unsigned grid = (unsigned)((items + 3) / 4);
-  if (NORM && p.k8 && p.nqt > 1 && p.cand) {
-    // the int8 screen with candidate lists, the candidate pass, then the tile pass over the query
-    // tiles whose lists overflowed
+  if constexpr (NORM) {
     const int e = launch_fwd_screen_f32(p, k, stream);
     if (e) return e;
     hipLaunchKernelGGL((fwd_cand_f32<D, BR, PK>), dim3((unsigned)items), dim3(64 * BR), 0, (hipStream_t)stream, p);
     launched(stream, "fwd_cand_f32");
     const unsigned qgrid = (unsigned)(((items < 2048 ? items : 2048) + 3) / 4);
-    hipLaunchKernelGGL((fwd_wave<Pol, D, BR, PK, NORM, NORM, NORM>), dim3(qgrid), dim3(256), 0, (hipStream_t)stream, p);
-  } else if (!NORM && p.nqt > 1) {  // a query tile per workgroup, its key tiles split over the waves
-    if (f32_split(D, items, p.nkt) == 1)
-      hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 1>), dim3((unsigned)items), dim3(64), 0, (hipStream_t)stream, p);
-    else if (f32_split(D, items, p.nkt) == 2)
-      hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 2>), dim3((unsigned)items), dim3(128), 0, (hipStream_t)stream, p);
-    else
-      hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 4>), dim3((unsigned)items), dim3(256), 0, (hipStream_t)stream, p);
+    hipLaunchKernelGGL((fwd_wave<D, BR, PK>), dim3(qgrid), dim3(256), 0, (hipStream_t)stream, p);
+  } else if (f32_split(D, items, p.nkt) == 1) {
+    hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 1>), dim3((unsigned)items), dim3(64), 0, (hipStream_t)stream, p);
+  } else if (f32_split(D, items, p.nkt) == 2) {
+    hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 2>), dim3((unsigned)items), dim3(128), 0, (hipStream_t)stream, p);
   } else {
-    hipLaunchKernelGGL((fwd_wave<Pol, D, BR, PK, NORM>), dim3(grid), dim3(256), 0, (hipStream_t)stream, p);
+    hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 4>), dim3((unsigned)items), dim3(256), 0, (hipStream_t)stream, p);
   }
   launched(stream, "fwd_wave");
   return (int)hipGetLastError();
 }
 
-template <class Pol, int D, int BR, int PK>
+template <int D, int BR, int PK>
 static int sel_norm(const FwdParams& p, const KernelKey& k, void* s) {
-  return k.normalize ? launch_fwd_t<Pol, D, BR, PK, true>(p, k, s) : launch_fwd_t<Pol, D, BR, PK, false>(p, k, s);
+  return k.normalize ? launch_fwd_t<D, BR, PK, true>(p, k, s) : launch_fwd_t<D, BR, PK, false>(p, k, s);
 }
-template <class Pol, int D, int BR>
+template <int D, int BR>
 static int sel_pk(const FwdParams& p, const KernelKey& k, void* s) {
   switch (k.pkind) {
-    case 2: return sel_norm<Pol, D, BR, 2>(p, k, s);
-    case 1: return sel_norm<Pol, D, BR, 1>(p, k, s);
-    default: return sel_norm<Pol, D, BR, 0>(p, k, s);
+    case 2: return sel_norm<D, BR, 2>(p, k, s);
+    case 1: return sel_norm<D, BR, 1>(p, k, s);
+    default: return sel_norm<D, BR, 0>(p, k, s);
   }
 }
-template <class Pol, int D>
+template <int D>
 static int sel_br(const FwdParams& p, const KernelKey& k, void* s) {
-  return k.branches == 2 ? sel_pk<Pol, D, 2>(p, k, s) : sel_pk<Pol, D, 1>(p, k, s);
+  return k.branches == 2 ? sel_pk<D, 2>(p, k, s) : sel_pk<D, 1>(p, k, s);
 }
-template <class Pol>
 static int sel_d(const FwdParams& p, const KernelKey& k, void* s) {
-  return k.d == 128 ? sel_br<Pol, 128>(p, k, s) : sel_br<Pol, 64>(p, k, s);
+  return k.d == 128 ? sel_br<128>(p, k, s) : sel_br<64>(p, k, s);
 }
 
 // The zero range of a call whose path has no screen (which clears it otherwise): 16 bytes per
@@ -730,8 +650,8 @@ int launch_zero(const FwdParams& p, void* stream) {
   return (int)hipGetLastError();
 }
 
-// head_dim 256 runs tda_wide.hip; a single query tile the split-key decode kernels
-// (tda_fwd_decode.hip); otherwise bf16 runs the screen + sparse A.V kernels (tda_fwd_sparse.hip) and
+// head_dim 256 runs tda_wide.hip (fp32) or fwd_blk256 after its norms kernel (bf16); a single query
+// tile the split-key decode kernels (tda_fwd_decode.hip); otherwise bf16 runs the screen + sparse A.V kernels (tda_fwd_sparse.hip) and
 // fp32 the int8 screen, fwd_cand_f32 and fwd_wave when normalised, fwd_split_f32 when not.  The
 // screens, and the bf16 block tile pass without normalisation, clear the call's zero range; the
 // other paths launch zero_range.
@@ -746,7 +666,7 @@ int launch_fwd(const FwdParams& p, const KernelKey& k, void* stream) {
     return launch_fwd(q, k, stream);
   }
   int e;
-  if (k.d == 256) {  // both dtypes: the column-split kernels of tda_wide.hip (no screen)
+  if (k.d == 256) {  // no screen
     e = launch_fwd_wide(p, k, stream);
     return e ? e : launch_zero(p, stream);
   }
@@ -755,7 +675,7 @@ int launch_fwd(const FwdParams& p, const KernelKey& k, void* stream) {
     return e ? e : launch_zero(p, stream);
   }
   if (k.dtype == 1) return launch_fwd_sparse(p, k, stream);
-  e = sel_d<PolF32>(p, k, stream);
+  e = sel_d(p, k, stream);
   const bool screened = k.normalize;  // the screen cleared it
   return e ? e : screened ? 0 : launch_zero(p, stream);
 }

@@ -28,7 +28,7 @@
 namespace tda {
 namespace {
 
-constexpr int kDecWaves = 4;  // waves per workgroup; key tiles per chunk = 32
+constexpr int kDecWaves = 4;  // waves per workgroup
 
 // Sum of squares of a row held as NT bf16x8 fragments per lane half (the row's two halves in
 // lanes n and n + 32): bf16 pairs by dot2 (each product exact in fp32), two chains over the

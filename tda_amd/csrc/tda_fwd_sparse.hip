@@ -18,13 +18,13 @@
 //               candidate keys (the keys of its passing lanes).
 //   fwd_pv_cand one wave per branch of a query tile whose candidate lists fit: the score tile
 //               of its rows against the candidate keys (the same MFMA sequence and operand
-//               values as fwd_pv, so the same scores), the exact weights and coef A V over the
+//               values as fwd_pv_blk, so the same scores), the exact weights and coef A V over the
 //               candidates' V rows, the branches' sums added through LDS; the bitmask row is
 //               rewritten exactly.
 //   fwd_pv_blk  the tile pass for the query tiles whose lists overflowed, four consecutive query
 //               tiles per workgroup sharing each key tile's rows: walks the set bits of both
 //               branches, recomputes the score tile, forms the exact weights ReLU(x)^p with the
-//               causal mask, and accumulates out += coef A V.  Tiles whose exact weights are all
+//               causal mask, and accumulates A V per branch.  Tiles whose exact weights are all
 //               zero lose their bit, so the bitmask ends exact.
 // Without normalisation one launch, fwd_pv_blk over every query tile: scores every causal key tile and forms the weights, A V and the exact
 // bitmask itself (a screen would compute the same bf16 scores once more); its workgroups also
@@ -369,7 +369,7 @@ __global__ void __launch_bounds__(256) key_prep(FwdParams P, int BR) {
     const int64_t lists = pair_lists(BR, BH, P.nqt), nthr = (int64_t)gridDim.x * 256;
     uint32_t* counts = P.cand + lists * kCandCap;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < lists; i += nthr) counts[i] = 0u;
-    if (blockIdx.x == 0 && threadIdx.x == 0) P.pvq[0] = 0u;
+    if (sizeof(T) == 4 && blockIdx.x == 0 && threadIdx.x == 0) P.pvq[0] = 0u;  // the fp32 tile pass's queue
     if (P.colcnt)  // the column buckets' counts (the candidate pass appends)
       for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < (int64_t)BH * P.nkt; i += nthr) P.colcnt[i] = 0u;
   }
@@ -1364,10 +1364,10 @@ __attribute__((amdgpu_waves_per_eu((kWideFwdWaves<BR, NORM>)))) fwd_blk256(FwdPa
 // ------------------------------------------------------------------ fwd_pv_cand
 // The exact pass of the query tiles whose candidate-key lists (every branch, normalised scores)
 // fit: per branch the score tile of the query rows against the candidate keys' rows (row c =
-// candidate c, rows past the count zero) is computed with the MFMA sequence of fwd_pv, its
+// candidate c, rows past the count zero) is computed with the MFMA sequence of fwd_pv_blk, its
 // operands loaded straight from the rows (the same values in the same operands: bitwise the same
 // scores); the candidates' V rows go to a swizzled LDS tile by direct loads, and the exact
-// weights with the causal mask accumulate coef A V as in fwd_pv.  One gather round per branch
+// weights with the causal mask, times the branch's coefficient, accumulate A V.  One gather round per branch
 // replaces one per kept key tile.  With two branches each runs on its own wave of the workgroup
 // (half the dependent loads per wave; LDS per wave as with one) and the second wave's sum is
 // added to the first's through LDS before the first stores the rows.  The bitmask row is rewritten from the key tiles
@@ -1618,7 +1618,7 @@ __global__ void __launch_bounds__(64 * BR) __attribute__((amdgpu_waves_per_eu(3)
   // 2 (k ^ osig(n)) + (g ^ otau(n)) of the row: the two halves of chunk k share a 16-byte slot
   // (swapped when otau(n) = 1) and the 32 rows of a half-wave's store fall on distinct banks (with
   // the tile's 16-byte swizzle they met in pairs, two extra cycles per store); the row reads then
-  // take 16-byte slots, and the stores cover whole rows (streaming stores, as in fwd_pv: nothing
+  // take 16-byte slots, and the stores cover whole rows (streaming stores, as in fwd_pv_blk: nothing
   // here reads the output again).
   auto osig = [](int r) { return (r >> 1) & (CPR - 1); };
   auto otau = [](int r) { return D == 128 ? (r & 1) : ((r >> 4) & 1); };

@@ -1,5 +1,6 @@
-"""head_dim 256 (the reference takes any power of two, TTA:29, :366-368, :431): the column-split
-kernels of tda_amd/csrc/tda_wide.hip against the CPU oracle on the same inputs.
+"""head_dim 256 (the reference takes any power of two, TTA:29, :366-368, :431): the fp32
+kernels of tda_amd/csrc/tda_wide.hip and the bf16 ones (fwd_blk256, bwd_dq_blk, bwd_dkv_wide) against
+the CPU oracle on the same inputs.
 
 fp32 <= 1e-4 and bf16 <= 2e-2 (normwise relative error), forward and every gradient (dq1, dq2,
 dk1, dk2, dv, dbeta, dlambda), normalize on and off, through both public functions and
