@@ -1779,7 +1779,7 @@ __global__ void __launch_bounds__(128 * BR * kWideKeys) __attribute__((amdgpu_wa
 // take tickets, the key blocks (the longer ones) first, each kind longest blocks first as nearly as
 // the queue's order has it.  With every list fitting the queue is empty and a workgroup leaves
 // after one load (4.6 us); at a threshold scale of 0.5 nearly every block is queued
-// (TDA (2, 16, 1500, 64): 151 us, 2632 us with one wave per query or key tile fetching
+// (TDA (2, 16, 1500, 64): 162 us, 2632 us with one wave per query or key tile fetching
 // its own rows).
 template <int D, int BR, int PK>
 __global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, true>()))) bwd_tiles(BwdParams P) {

@@ -767,7 +767,7 @@ __device__ __forceinline__ bf16x8 tr_frag(const bf16* p) {
 // listed in LDS 64 words at a time; tiles whose weights are all zero lose their bit.  A workgroup
 // with no such tile leaves after one round of loads, a wave whose own lists fit only helps to load.
 // At a threshold scale of 0.5 nearly every list overflows (TDA (2, 16, 1500, 64): 237 us with one
-// wave per query tile, 102 so); with every list fitting the launch costs 4.6 us.
+// wave per query tile, 108 so); with every list fitting the launch costs 4.6 us.
 constexpr int kBlkTiles = 4;
 
 // Block and head of workgroup `bid`: longest blocks (last query tiles) of every head first; one
