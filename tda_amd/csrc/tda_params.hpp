@@ -129,8 +129,10 @@ struct BwdParams {
 // Key tiles per workgroup of the decode kernels (tda_fwd_decode.hip), whose partial outputs are
 // [B*H][ceil(nkt / tiles)][Nq][D] floats: 32 (a bitmask word) when that makes the two workgroups per
 // CU that fit, else 8 (a byte of one), so that a short or small cache still spreads over the GPU (8
-// heads, 1000 keys, d = 64, two branches: 8 workgroups and 33 us against 32 and 15 us).  Its
-// partials stay within 4 MiB.  Only where the caller's workspace has the room (the size functions
+// heads, 1000 keys, d = 64, two branches: 8 workgroups and 33 us against 32 and 15 us).  At that line
+// 32 wins: one query on (4, 32, 4096, 128), 512 workgroups, 55 us per call against 69.  The partials
+// of 8 stay within 4 MiB, a bound on the workspace rather than the crossing: 32 queries on (1, 32,
+// 4096, 128), 16 MiB of them, take 44 us with 32 and 40 with 8 (fp32 138 and 101).  Only where the caller's workspace has the room (the size functions
 // ask for 32); the Python entry points allocate it.
 constexpr int64_t dec_chunk_tiles(int64_t bh, int64_t nq, int64_t nkt) {
   return bh * ((nkt + 31) / 32) < 512 && bh * ((nkt + 7) / 8) * nq <= 8192 ? 8 : 32;

@@ -81,9 +81,9 @@ class ThresholdDifferentialAttention(nn.Module):
     def _parts(self, x: torch.Tensor):
         """project(x), whoever defines it.  The class's own views are seen by the operator alone here, so
         they come from one unbind: its backward stacks the parts' gradients in one pass, where
-        indexing fills, copies into and adds up a whole projection's gradient per part (14 kernels,
-        90 us of GPU time, of a training step at (2, 1024), 16 heads of 64).  autograd forbids
-        editing an unbind's results in place."""
+        indexing fills, copies into and adds up a whole projection's gradient per part (a training step
+        at (2, 1024), 16 heads of 64: 15 kernels and 268 us of GPU time against 28 and 340).
+        autograd forbids editing an unbind's results in place."""
         if getattr(self.project, "__func__", None) is not ThresholdDifferentialAttention._own_project:
             return self.project(x)
         return [part.transpose(1, 2) for part in self._projection(x).unbind(2)]
