@@ -14,9 +14,11 @@
 namespace tda {
 
 // ------------------------------------------------------------------ fwd_wave
-// fp32 with normalisation, after key_prep and fwd_screen_i8 ran on the same inputs: the query tiles
-// the candidate pass (fwd_cand_f32) queued, whose candidate lists did not fit.  One wave per 32-row query
-// tile, four independent waves per workgroup, taking the queue's tiles in turn.
+// fp32, one wave per 32-row query tile, four independent waves per workgroup, in two forms.
+// fwd_wave, with normalisation, after key_prep and fwd_screen_i8 ran on the same inputs (SCR): the waves
+// take in turn the query tiles the candidate pass (fwd_cand_f32) queued, whose candidate lists did not
+// fit.  fwd_wave_heads: a single query tile per head, a wave each, over every key tile it sees
+// (one_wave_heads has the rule and its figures).
 //
 // Layouts (see tda_common.hpp): the score tile is computed transposed, S^T = K Q^T, with the
 // key rows as the A operand (row fragments loaded from HBM per key tile) and the wave's query
@@ -24,10 +26,10 @@ namespace tda {
 // so the per-query threshold, inverse norm and the causal test are per-lane scalars, and the
 // thresholded tile packs directly into the B operand of O^T += V^T A^T.
 //
-// The screen's bitmask names every key tile holding a non-zero weight (a superset), so the wave
+// SCR: the screen's bitmask names every key tile holding a non-zero weight (a superset), so the wave
 // visits only those tiles; the inverse norms come from the table the screen and key_prep wrote (the
 // values the screen's bound is stated for), and the bitmask words are rewritten exactly.
-template <int D, int BR, int PK>
+template <int D, int BR, int PK, bool NORM, bool SCR>
 __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh);
 
 template <int D, int BR, int PK>
@@ -35,12 +37,19 @@ __global__ void __launch_bounds__(256) fwd_wave(FwdParams P) {
   const uint32_t queued = P.pvq[0];
   for (uint32_t k = blockIdx.x * 4u + (threadIdx.x >> 6); k < queued; k += gridDim.x * 4u) {
     const int v = (int)P.pvq[1 + k];
-    fwd_wave_tile<D, BR, PK>(P, v % P.nqt, v / P.nqt);
+    fwd_wave_tile<D, BR, PK, true, true>(P, v % P.nqt, v / P.nqt);
   }
 }
 
-template <int D, int BR, int PK>
+template <int D, int BR, int PK, bool NORM>
+__global__ void __launch_bounds__(256) fwd_wave_heads(FwdParams P) {
+  const int64_t bh = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (bh < (int64_t)P.B * P.H) fwd_wave_tile<D, BR, PK, NORM, false>(P, 0, (int)bh);
+}
+
+template <int D, int BR, int PK, bool NORM, bool SCR>
 __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh) {
+  static_assert(!SCR || NORM, "the screened pass is the normalised one");
   using Pol = PolF32;
   using T = typename Pol::T;
   using frag = typename Pol::frag;
@@ -74,9 +83,18 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
     }
   }
   float rq1 = 1.f, rq2 = 1.f;
-  if (qvalid) {
-    rq1 = P.norms[norm_base(P, N_Q1, bh) + i];
-    if constexpr (BR == 2) rq2 = P.norms[norm_base(P, N_Q2, bh) + i];
+  if constexpr (SCR) {
+    if (qvalid) {
+      rq1 = P.norms[norm_base(P, N_Q1, bh) + i];
+      if constexpr (BR == 2) rq2 = P.norms[norm_base(P, N_Q2, bh) + i];
+    }
+  } else if constexpr (NORM) {
+    rq1 = inv_norm(row_sumsq<Pol, NT>(Q1));
+    if constexpr (BR == 2) rq2 = inv_norm(row_sumsq<Pol, NT>(Q2));
+    if (qvalid && g == 0) {
+      P.norms[norm_base(P, N_Q1, bh) + i] = rq1;
+      if constexpr (BR == 2) P.norms[norm_base(P, N_Q2, bh) + i] = rq2;
+    }
   }
   const float pw = P.p;
   const float tau = (*P.beta) * tau_coeff(pq, P.inv_d);
@@ -93,29 +111,33 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
   uint32_t* occrow = P.occ + ((int64_t)bh * P.nqt + qt) * P.occ_w;
   const int64_t occ_br = (int64_t)BH * P.nqt * P.occ_w;  // distance between the branch planes
   uint32_t word = 0, word2 = 0;
-  unsigned computed = 0, checked = 0;
+  unsigned visited = 0, computed = 0, checked = 0;
 
   for (int kt = 0; kt <= ktl; ++kt) {
-    // the screen's bits of this word (per branch), read before this wave rewrites the word
-    const uint32_t s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)occrow[kt >> 5]);
-    const uint32_t s2 = BR == 2 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)occrow[occ_br + (kt >> 5)]) : 0u;
-    const uint32_t keep = (s1 | s2) & (~0u << (kt & 31));  // kept tiles kt .. of the word
-    const int next = keep ? (kt & ~31) + __builtin_ctz(keep) : (kt | 31) + 1;
-    if (next > kt) {  // skipped tiles hold no weight: close the word if it ends among them
-      const int wend = kt | 31;
-      if (next > wend || next > ktl) {
-        if (l == 0) {
-          occrow[kt >> 5] = word;
-          if constexpr (BR == 2) occrow[occ_br + (kt >> 5)] = word2;
+    bool use1 = true, use2 = true;  // the branches that the screen kept this tile in
+    if constexpr (SCR) {
+      // the screen's bits of this word (per branch), read before this wave rewrites the word
+      const uint32_t s1 = (uint32_t)__builtin_amdgcn_readfirstlane((int)occrow[kt >> 5]);
+      const uint32_t s2 = BR == 2 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)occrow[occ_br + (kt >> 5)]) : 0u;
+      const uint32_t keep = (s1 | s2) & (~0u << (kt & 31));  // kept tiles kt .. of the word
+      const int next = keep ? (kt & ~31) + __builtin_ctz(keep) : (kt | 31) + 1;
+      if (next > kt) {  // skipped tiles hold no weight: close the word if it ends among them
+        const int wend = kt | 31;
+        if (next > wend || next > ktl) {
+          if (l == 0) {
+            occrow[kt >> 5] = word;
+            if constexpr (BR == 2) occrow[occ_br + (kt >> 5)] = word2;
+          }
+          word = word2 = 0;
+          kt = wend;
+          continue;
         }
-        word = word2 = 0;
-        kt = wend;
-        continue;
+        kt = next;
       }
-      kt = next;
+      use1 = (s1 >> (kt & 31)) & 1u;
+      use2 = (s2 >> (kt & 31)) & 1u;
+      checked += (use1 ? 1u : 0u) + (use2 ? 1u : 0u);
     }
-    const bool use1 = (s1 >> (kt & 31)) & 1u, use2 = (s2 >> (kt & 31)) & 1u;  // the branches that keep the tile
-    checked += (use1 ? 1u : 0u) + (use2 ? 1u : 0u);
     const int k0 = kt * 32;
     const int j = k0 + n32;  // key row this lane loads for the A operand
     f32x16 S1 = f32x16{}, S2 = f32x16{};
@@ -127,9 +149,14 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
       Pol::template load_rows<NT>(r1, g, K1);
 #pragma unroll
       for (int t = 0; t < NT; ++t) S1 = Pol::mma(K1[t], Q1[t], S1);
-      const float rk = j < Nk ? P.norms[norm_base(P, N_K1, bh) + j] : 0.f;
+      if constexpr (NORM) {
+        float rk;
+        if constexpr (SCR) rk = j < Nk ? P.norms[norm_base(P, N_K1, bh) + j] : 0.f;
+        else rk = inv_norm(row_sumsq<Pol, NT>(K1));
+        if (!SCR && g == 0 && j < Nk) P.norms[norm_base(P, N_K1, bh) + j] = rk;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) rk1r[r] = __shfl(rk, crow(r, g));
+        for (int r = 0; r < 16; ++r) rk1r[r] = __shfl(rk, crow(r, g));
+      }
     }
     if (BR == 2 && use2) {
       frag K2[NT];
@@ -137,9 +164,14 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
       Pol::template load_rows<NT>(r2, g, K2);
 #pragma unroll
       for (int t = 0; t < NT; ++t) S2 = Pol::mma(K2[t], Q2[t], S2);
-      const float rk = j < Nk ? P.norms[norm_base(P, N_K2, bh) + j] : 0.f;
+      if constexpr (NORM) {
+        float rk;
+        if constexpr (SCR) rk = j < Nk ? P.norms[norm_base(P, N_K2, bh) + j] : 0.f;
+        else rk = inv_norm(row_sumsq<Pol, NT>(K2));
+        if (!SCR && g == 0 && j < Nk) P.norms[norm_base(P, N_K2, bh) + j] = rk;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) rk2r[r] = __shfl(rk, crow(r, g));
+        for (int r = 0; r < 16; ++r) rk2r[r] = __shfl(rk, crow(r, g));
+      }
     }
 
     // Threshold test.  x = fma(s * rk_j, rq_i, -tau_i) is monotone in s * rk_j, so the tile
@@ -149,16 +181,17 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
     for (int r = 0; r < 16; ++r) {
       const int key = k0 + crow(r, g);
       const bool valid = qvalid && key <= pq && key < Nk;
-      S1[r] *= rk1r[r];
+      if constexpr (NORM) S1[r] *= rk1r[r];
       m1 = fmaxf(m1, valid ? S1[r] : -INFINITY);
       if constexpr (BR == 2) {
-        S2[r] *= rk2r[r];
+        if constexpr (NORM) S2[r] *= rk2r[r];
         m2 = fmaxf(m2, valid ? S2[r] : -INFINITY);
       }
     }
     const bool any1 = use1 && wave_ballot(__builtin_fmaf(m1, rq1, -tau) > 0.f) != 0ull;
     bool any2 = false;
     if constexpr (BR == 2) any2 = use2 && wave_ballot(__builtin_fmaf(m2, rq2, -tau) > 0.f) != 0ull;
+    visited += BR;
     computed += (any1 ? 1 : 0) + (any2 ? 1 : 0);
     if (any1) word |= 1u << (kt & 31);
     if (any2) word2 |= 1u << (kt & 31);
@@ -207,6 +240,23 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
       P.pairs[pair_lists(BR, BH, P.nqt) * 4 * kPairCap + ((int64_t)br * BH + bh) * P.nqt + qt] = kPairOverflow;
   }
 
+  // Key tiles the query tile does not see: their inverse norms still go to the table (the backward's
+  // normalize epilogue reads every key row's); with SCR key_prep wrote every key row's.
+  if constexpr (NORM && !SCR) {
+    for (int kt = ktl + 1; kt < P.nkt; ++kt) {
+      const int j = 32 * kt + n32;
+      frag K[NT];
+      Pol::template load_rows<NT>(j < Nk ? k1.row(b, h, j) : nullptr, g, K);
+      const float rka = inv_norm(row_sumsq<Pol, NT>(K));
+      if (g == 0 && j < Nk) P.norms[norm_base(P, N_K1, bh) + j] = rka;
+      if constexpr (BR == 2) {
+        Pol::template load_rows<NT>(j < Nk ? k2.row(b, h, j) : nullptr, g, K);
+        const float rkb = inv_norm(row_sumsq<Pol, NT>(K));
+        if (g == 0 && j < Nk) P.norms[norm_base(P, N_K2, bh) + j] = rkb;
+      }
+    }
+  }
+
   if (qvalid) {
     T* orow = out.row(b, h, i);
 #pragma unroll
@@ -215,9 +265,9 @@ __device__ __forceinline__ void fwd_wave_tile(const FwdParams& P, int qt, int bh
       for (int u = 0; u < 4; ++u)
         store4(orow + 32 * c + 8 * u + 4 * g, O[c][4 * u], O[c][4 * u + 1], O[c][4 * u + 2], O[c][4 * u + 3]);
   }
-  if (P.stats && l == 0) {  // (the screen counted the causal tiles; checked: those it kept)
+  if (P.stats && l == 0) {  // with SCR the screen counted the causal tiles; checked: those it kept
+    atomicAdd(P.stats + (SCR ? 2 : 0), (unsigned long long)(SCR ? checked : visited));
     atomicAdd(P.stats + 1, (unsigned long long)computed);
-    atomicAdd(P.stats + 2, (unsigned long long)checked);
   }
 }
 
@@ -590,14 +640,34 @@ __global__ void __launch_bounds__(64 * BR) fwd_cand_f32(FwdParams P) {
 }
 
 // ------------------------------------------------------------------ dispatch
-// fp32 with more than one query tile.  Normalised: the int8 screen with candidate lists (key_prep and
+// A single fp32 query tile per head: whether a wave per head beats the split-key decode kernels, whose
+// workgroups of four waves each hold a CU's four SIMDs, leave idle waves at fewer than four key tiles,
+// and need a second launch for the sum.  It does at one or two key tiles, and the longer caches the more
+// of the GPU's 1024 SIMDs the heads fill: decode / wave times 1.6 - 2.1 at one tile of up to 256
+// heads and 4 - 8 from 1024 on; at four tiles 0.45 - 1.0 up to 256 heads; at 512 heads 0.8 - 1.4 (d = 64)
+// and 1.25 - 1.8 (d = 128, two branches) at four, 0.95 - 1.3 at eight (d = 128); at 1024 heads 1.1 -
+// 2.2 at eight, at sixteen 1.1 - 1.4 but for d = 64 without normalisation (0.85), at 63 1.0 - 1.2 for
+// d = 128 and 0.7 - 0.95 for 64; at 2048 1.0 - 1.3 at 63 tiles.  Past sixteen tiles it pays where the
+// heads nearly fill whole rounds of the SIMDs.
+static bool one_wave_heads(int d, bool norm, int64_t heads, int nkt) {
+  const int64_t rounds = (heads + 1023) / 1024;
+  const bool full = 6 * heads >= 5 * 1024 * rounds;
+  if (full && heads >= (d > 64 ? 1024 : 2048)) return true;
+  if (heads >= 1024) return nkt <= (full && norm ? 16 : 8);
+  return nkt <= (heads >= 512 && (norm || d > 64) ? (norm && d > 64 ? 8 : 4) : 2);
+}
+
+// fp32 with more than one query tile, or one per head a wave each.  Normalised with more than one: the
+// int8 screen with candidate lists (key_prep and
 // fwd_screen_i8 on the fp32 rows, tda_fwd_sparse.hip), the candidate pass, then the tile pass over the
 // query tiles whose lists overflowed.  Without: a query tile per workgroup, its key tiles split over
 // the waves.
 template <int D, int BR, int PK, bool NORM>
 static int launch_fwd_t(const FwdParams& p, const KernelKey& k, void* stream) {
   const int64_t items = (int64_t)p.B * p.H * p.nqt;
-  if constexpr (NORM) {
+  if (p.nqt == 1) {
+    hipLaunchKernelGGL((fwd_wave_heads<D, BR, PK, NORM>), dim3((unsigned)((items + 3) / 4)), dim3(256), 0, (hipStream_t)stream, p);
+  } else if constexpr (NORM) {
     const int e = launch_fwd_screen_f32(p, k, stream);
     if (e) return e;
     hipLaunchKernelGGL((fwd_cand_f32<D, BR, PK>), dim3((unsigned)items), dim3(64 * BR), 0, (hipStream_t)stream, p);
@@ -651,7 +721,8 @@ int launch_zero(const FwdParams& p, void* stream) {
 }
 
 // head_dim 256 runs tda_wide.hip (fp32) or fwd_blk256 after its norms kernel (bf16); a single query
-// tile the split-key decode kernels (tda_fwd_decode.hip); otherwise bf16 runs the screen + sparse A.V kernels (tda_fwd_sparse.hip) and
+// tile the split-key decode kernels (tda_fwd_decode.hip), or in fp32 a wave per head where that is
+// faster (one_wave_heads); otherwise bf16 runs the screen + sparse A.V kernels (tda_fwd_sparse.hip) and
 // fp32 the int8 screen, fwd_cand_f32 and fwd_wave when normalised, fwd_split_f32 when not.  The
 // screens, and the bf16 block tile pass without normalisation, clear the call's zero range; the
 // other paths launch zero_range.
@@ -670,13 +741,14 @@ int launch_fwd(const FwdParams& p, const KernelKey& k, void* stream) {
     e = launch_fwd_wide(p, k, stream);
     return e ? e : launch_zero(p, stream);
   }
-  if (p.nqt == 1) {  // (the workspace holds the partial outputs of a single query tile)
+  if (p.nqt == 1 && !(k.dtype == 0 && one_wave_heads(k.d, k.normalize, (int64_t)p.B * p.H, p.nkt))) {
+    // (the workspace holds the partial outputs of a single query tile)
     e = launch_fwd_decode(p, k, p.part, stream);
     return e ? e : launch_zero(p, stream);
   }
   if (k.dtype == 1) return launch_fwd_sparse(p, k, stream);
   e = sel_d(p, k, stream);
-  const bool screened = k.normalize;  // the screen cleared it
+  const bool screened = k.normalize && p.nqt > 1;  // the screen cleared it
   return e ? e : screened ? 0 : launch_zero(p, stream);
 }
 
