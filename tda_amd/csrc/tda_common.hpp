@@ -377,40 +377,47 @@ __device__ __forceinline__ f32x16 mma_chain(FA&& fa, FB&& fb) {
 }
 
 // ------------------------------------------------------------------ fp32 wave tiles
-// A wave's own 32-row fp32 tile: the next one's rows in flight in registers (load), the current one
-// in the wave's LDS slice (store), read as row fragments (f32_rows_mma) or by columns (f32_cols_mma).
-// Waves per workgroup of the fp32 split passes (one resident tile each): four below 2048 resident
-// tiles (two per SIMD: fewer leave SIMDs idle behind the longest causal row), then two, or one where
-// a row streams at most 16 tiles (the sum over the waves and the uneven deal would cost more than the
-// split gives) and from 4096 tiles at d = 128, where a SIMD holds one wave.  Steps of threshold_rela_triton: (2, 12, 1111, 64) 421 us with four tiles per
-// workgroup, one wave each; 259 with four waves per tile;
-// (2, 16, 2048, 128) 1632 with four, 1502 with two; (4, 16, 2048, 64) 1372 with two, 1432 with one;
-// (8, 32, 512, 64) 426 with two, 411 with one; the
-// differential step (4, 32, 1024, 128) 2980 with two, 2741 with one.
-constexpr int f32_split(int d, int64_t tiles, int streamed) {
-  return tiles < 2048 ? 4 : streamed <= 16 || (d > 64 && tiles >= 4096) ? 1 : 2;
+// A 32-row fp32 tile in LDS, a wave's own (NW = 1) or shared by NW waves, each moving its share of the
+// rows: the next one's rows in flight in registers (load), the current one in LDS (store), read as row
+// fragments (f32_rows_mma) or by columns (f32_cols_mma).
+// How the fp32 passes without normalisation share out `tiles` resident tiles that stream up to `streamed`
+// tiles each, on a GPU that holds `slots` waves of theirs (1024 SIMDs, one or two waves each): the number
+// of waves a workgroup deals one resident tile's streamed tiles to, or 0 for the block pass, four resident
+// tiles to a workgroup, one wave each, sharing the streamed rows.  Splitting a tile fills idle SIMDs and
+// shortens the chain behind the longest causal row; sharing saves row traffic, which counts once the
+// SIMDs are full.  Device times of the split with 1 / 2 / 4 waves over the block pass's, forward and backward
+// of 4 - 1024 heads, 2 - 32 tiles, both head_dims, one and two branches: four waves 0.30 - 0.61 up to a quarter of
+// the slots (from 4 tiles on) and 0.35 - 0.78 up to half of them (from 8 tiles on); two 0.7 - 0.95 at 2 - 3
+// tiles and up to the slots 0.6 - 1.0, once 1.16 (256 heads of 4); one 0.75 - 1.03 up to 2.5 times the slots
+// and 0.6 - 1.1 at up to 12 tiles; past both lines 1.0 - 1.43 with one, more with two and four.
+constexpr int f32_split(int64_t slots, int64_t tiles, int streamed) {
+  if ((streamed >= 4 && 4 * tiles <= slots) || (streamed >= 8 && 2 * tiles <= slots)) return 4;
+  if (tiles <= slots) return 2;
+  return 2 * tiles <= 5 * slots || streamed <= 12 ? 1 : 0;
 }
 template <int D>
 constexpr int kF32Stride = D + 4;  // LDS row stride: the row-fragment reads spread over the banks
-// Load instruction u: rows RPI u + l / CPR, 16-byte chunk l % CPR; rows past n read row n - 1 (their
+// Load instruction u of wave wv: rows RPI (LPW wv + u) + l / CPR, 16-byte chunk l % CPR; rows past n read row n - 1 (their
 // products are masked).
-template <int D>
+template <int D, int NW = 1>
 struct F32Rows {
-  static constexpr int CPR = D / 4, RPI = 64 / CPR, LPW = 32 / RPI;
+  static constexpr int CPR = D / 4, RPI = 64 / CPR, LPW = 32 / RPI / NW;
+  static_assert(LPW >= 1 && LPW * RPI * NW == 32, "tile rows split evenly over the waves");
   f32x4 v[LPW];
-  __device__ __forceinline__ void load(const TRef<const float>& x, int b, int h, int r0, int n) {
+  __device__ __forceinline__ void load(const TRef<const float>& x, int b, int h, int r0, int n, int wv = 0) {
     const int l = lane_id();
 #pragma unroll
     for (int u = 0; u < LPW; ++u)
-      v[u] = *reinterpret_cast<const f32x4*>(x.row(b, h, min(r0 + RPI * u + l / CPR, n - 1)) + 4 * (l % CPR));
+      v[u] = *reinterpret_cast<const f32x4*>(x.row(b, h, min(r0 + RPI * (LPW * wv + u) + l / CPR, n - 1)) + 4 * (l % CPR));
   }
-  __device__ __forceinline__ void store(float* tile) const {
+  __device__ __forceinline__ void store(float* tile, int wv = 0) const {
     const int l = lane_id();
 #pragma unroll
     for (int u = 0; u < LPW; ++u)
-      *reinterpret_cast<f32x4*>(tile + (RPI * u + l / CPR) * kF32Stride<D> + 4 * (l % CPR)) = v[u];
+      *reinterpret_cast<f32x4*>(tile + (RPI * (LPW * wv + u) + l / CPR) * kF32Stride<D> + 4 * (l % CPR)) = v[u];
   }
 };
+constexpr int kF32Blk = 4;  // resident tiles (waves) per workgroup of the fp32 block passes
 // S^T-layout product of a 32-row LDS tile (A operand: lane (m, g) row m, elements g D/2 + t)
 // with a lane's register fragments (B operand, load_rows order): lane n, value r = row crow(r, g).
 template <int D>

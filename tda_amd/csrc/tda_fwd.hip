@@ -418,6 +418,150 @@ fwd_split_f32(FwdParams P) {
   }
 }
 
+// ------------------------------------------------------------------ fwd_blk_f32
+// The same pass for grids that fill the GPU over and over with long rows (f32_split has the line): blocks
+// of four consecutive query tiles of one head, one wave each, walking the block's causal key tiles in step
+// and sharing each tile's key rows (every branch) and V rows, which the workgroup loads once (each wave a
+// quarter of the rows, one tile ahead into registers) into LDS; two barriers per tile (it is rewritten
+// once every wave is done with it).  A wave scores only the tiles its own query tile sees, with
+// fwd_split_f32's arithmetic.  Bound by the fp32 products; forward of 1024 heads of 1000 rows, d = 128,
+// one branch: 2442 us, 3486 with a wave per tile and no sharing.
+template <int D, int BR, int PK>
+__global__ void __launch_bounds__(64 * kF32Blk) __attribute__((amdgpu_waves_per_eu(D <= 64 ? 2 : 1)))
+fwd_blk_f32(FwdParams P) {
+  using Pol = PolF32;
+  constexpr int W = kF32Blk, NT = D / 2, ND = D / 32;
+  __shared__ __attribute__((aligned(16))) float klds[BR][32 * kF32Stride<D>];
+  __shared__ __attribute__((aligned(16))) float vlds[32 * kF32Stride<D>];
+
+  const int l = lane_id(), n32 = l & 31, g = l >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int BH = P.B * P.H, Nq = P.Nq, Nk = P.Nk, nqt = P.nqt, qoff = P.qoff;
+  const int nqb = (nqt + W - 1) / W;
+  // longest blocks (last query tiles) of every head first
+  const int bid = blockIdx.x, jb = nqb - 1 - bid / BH, bh = bid % BH;
+  const int b = bh / P.H, h = bh % P.H;
+  const int qt = W * jb + wv;
+  const bool act = qt < nqt;  // wave-uniform: waves past the last query tile only load
+  const int i = 32 * qt + n32;
+  const bool qvalid = act && i < Nq;
+  const int pq = qoff + i;
+  const int ktl = act ? kt_last(qt, qoff, P.nkt) : -1;                       // this wave's last key tile
+  const int ktl_b = kt_last(min(W * jb + W - 1, nqt - 1), qoff, P.nkt);  // the block's
+
+  const TRef<const float> qr[2] = {{(const float*)P.in[F_Q1], P.s[F_Q1][0], P.s[F_Q1][1], P.s[F_Q1][2]},
+                                   {(const float*)P.in[F_Q2], P.s[F_Q2][0], P.s[F_Q2][1], P.s[F_Q2][2]}};
+  const TRef<const float> kr[2] = {{(const float*)P.in[F_K1], P.s[F_K1][0], P.s[F_K1][1], P.s[F_K1][2]},
+                                   {(const float*)P.in[F_K2], P.s[F_K2][0], P.s[F_K2][1], P.s[F_K2][2]}};
+  const TRef<const float> vv{(const float*)P.in[F_V], P.s[F_V][0], P.s[F_V][1], P.s[F_V][2]};
+  const TRef<float> out{(float*)P.out, P.s[F_OUT][0], P.s[F_OUT][1], P.s[F_OUT][2]};
+
+  float Q[BR][NT];
+#pragma unroll
+  for (int br = 0; br < BR; ++br) Pol::template load_rows<NT>(qvalid ? qr[br].row(b, h, i) : nullptr, g, Q[br]);
+  const float pw = P.p;
+  const float tau = (*P.beta) * tau_coeff(pq, P.inv_d);
+  float lam = 0.f;
+  if constexpr (BR == 2) lam = clamp01(*P.lam);
+
+  F32Rows<D, W> kreg[BR], vreg;  // this wave's share of the next tile's rows
+  auto issue = [&](int kt) {
+#pragma unroll
+    for (int br = 0; br < BR; ++br) kreg[br].load(kr[br], b, h, 32 * kt, Nk, wv);
+    vreg.load(vv, b, h, 32 * kt, Nk, wv);
+  };
+
+  f32x16 O[ND];
+#pragma unroll
+  for (int c = 0; c < ND; ++c) O[c] = f32x16{};
+  uint32_t* occrow = P.occ && act ? P.occ + ((int64_t)bh * nqt + qt) * P.occ_w : nullptr;
+  const int64_t occ_br = (int64_t)BH * nqt * P.occ_w;  // distance between the branch planes
+  uint32_t word = 0, word2 = 0;
+  unsigned visited = 0, computed = 0;
+
+  issue(0);
+  for (int kt = 0; kt <= ktl_b; ++kt) {
+    lds_barrier();  // every wave is done with the previous tile
+#pragma unroll
+    for (int br = 0; br < BR; ++br) kreg[br].store(klds[br], wv);
+    vreg.store(vlds, wv);
+    if (kt < ktl_b) issue(kt + 1);  // in flight during this tile's products
+    lds_barrier();                  // tile kt in LDS
+    if (kt > ktl) continue;         // (uniform) not seen by this wave's query tile
+    const int k0 = 32 * kt;
+    f32x16 S[BR];
+#pragma unroll
+    for (int br = 0; br < BR; ++br) S[br] = f32_rows_mma<D>(klds[br], Q[br]);
+    // threshold test: the tile max of the valid scores decides "any x > 0" exactly
+    bool any[2] = {false, false};
+#pragma unroll
+    for (int br = 0; br < BR; ++br) {
+      float m = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = k0 + crow(r, g);
+        const bool valid = qvalid && key <= pq && key < Nk;
+        m = fmaxf(m, valid ? S[br][r] : -INFINITY);
+      }
+      any[br] = wave_ballot(m - tau > 0.f) != 0ull;
+    }
+    visited += BR;
+    computed += (any[0] ? 1 : 0) + (any[1] ? 1 : 0);
+    if (any[0]) word |= 1u << (kt & 31);
+    if (any[1]) word2 |= 1u << (kt & 31);
+    // the query tile's pairs are in no list: the column bucket of the key tile is incomplete
+    if (P.colcnt && (any[0] || any[1]) && l == 0) atomicOr(P.colcnt + (int64_t)bh * P.nkt + kt, kColTaint);
+    if (any[0] || any[1]) {
+      f32x16 C;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = k0 + crow(r, g);
+        const bool valid = qvalid && key <= pq && key < Nk;
+        const float x1 = __builtin_fmaf(S[0][r], 1.f, -tau);
+        float a = (valid && any[0] && x1 > 0.f) ? pow_p<PK>(x1, pw) : 0.f;
+        if constexpr (BR == 2) {
+          const float x2 = __builtin_fmaf(S[1][r], 1.f, -tau);
+          const float a2 = (valid && any[1] && x2 > 0.f) ? pow_p<PK>(x2, pw) : 0.f;
+          a = __builtin_fmaf(-lam, a2, a);
+        }
+        C[r] = a;
+      }
+      f32_cols_mma<D>(vlds, C, O);
+    }
+    if (occrow && (((kt & 31) == 31) || kt == ktl)) {
+      if (l == 0) {
+        occrow[kt >> 5] = word;
+        if constexpr (BR == 2) occrow[occ_br + (kt >> 5)] = word2;
+      }
+      word = word2 = 0;
+    }
+  }
+  if (!act) return;
+  if (occrow && l == 0) {
+    for (int w = (ktl >> 5) + 1; w < P.occ_w; ++w) {
+      occrow[w] = 0u;
+      if constexpr (BR == 2) occrow[occ_br + w] = 0u;
+    }
+  }
+  if (P.pairs && l == 0) {  // this pass writes no pair list: the backward walks the tiles
+#pragma unroll
+    for (int br = 0; br < BR; ++br)
+      P.pairs[pair_lists(BR, BH, nqt) * 4 * kPairCap + ((int64_t)br * BH + bh) * nqt + qt] = kPairOverflow;
+  }
+  if (qvalid) {
+    float* orow = out.row(b, h, i);
+#pragma unroll
+    for (int c = 0; c < ND; ++c)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        store4(orow + 32 * c + 8 * u + 4 * g, O[c][4 * u], O[c][4 * u + 1], O[c][4 * u + 2], O[c][4 * u + 3]);
+  }
+  if (P.stats && l == 0) {
+    atomicAdd(P.stats + 0, (unsigned long long)visited);
+    atomicAdd(P.stats + 1, (unsigned long long)computed);
+  }
+}
+
 // ------------------------------------------------------------------ fwd_cand_f32
 // The fp32 exact pass over the screen's candidate keys (normalised, more than one query tile):
 // one workgroup per query tile whose candidate lists (every branch) fit, one wave per branch.
@@ -661,7 +805,7 @@ static bool one_wave_heads(int d, bool norm, int64_t heads, int nkt) {
 // int8 screen with candidate lists (key_prep and
 // fwd_screen_i8 on the fp32 rows, tda_fwd_sparse.hip), the candidate pass, then the tile pass over the
 // query tiles whose lists overflowed.  Without: a query tile per workgroup, its key tiles split over
-// the waves.
+// the waves, or a block of four (f32_split).
 template <int D, int BR, int PK, bool NORM>
 static int launch_fwd_t(const FwdParams& p, const KernelKey& k, void* stream) {
   const int64_t items = (int64_t)p.B * p.H * p.nqt;
@@ -674,12 +818,17 @@ static int launch_fwd_t(const FwdParams& p, const KernelKey& k, void* stream) {
     launched(stream, "fwd_cand_f32");
     const unsigned qgrid = (unsigned)(((items < 2048 ? items : 2048) + 3) / 4);
     hipLaunchKernelGGL((fwd_wave<D, BR, PK>), dim3(qgrid), dim3(256), 0, (hipStream_t)stream, p);
-  } else if (f32_split(D, items, p.nkt) == 1) {
-    hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 1>), dim3((unsigned)items), dim3(64), 0, (hipStream_t)stream, p);
-  } else if (f32_split(D, items, p.nkt) == 2) {
-    hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 2>), dim3((unsigned)items), dim3(128), 0, (hipStream_t)stream, p);
   } else {
-    hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 4>), dim3((unsigned)items), dim3(256), 0, (hipStream_t)stream, p);
+    hipStream_t s = (hipStream_t)stream;
+    switch (f32_split(D <= 64 && BR == 1 ? 2048 : 1024, items, p.nkt)) {
+      case 4: hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 4>), dim3((unsigned)items), dim3(256), 0, s, p); break;
+      case 2: hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 2>), dim3((unsigned)items), dim3(128), 0, s, p); break;
+      case 1: hipLaunchKernelGGL((fwd_split_f32<D, BR, PK, 1>), dim3((unsigned)items), dim3(64), 0, s, p); break;
+      default: {
+        const int64_t blocks = (int64_t)p.B * p.H * ((p.nqt + kF32Blk - 1) / kF32Blk);
+        hipLaunchKernelGGL((fwd_blk_f32<D, BR, PK>), dim3((unsigned)blocks), dim3(64 * kF32Blk), 0, s, p);
+      }
+    }
   }
   launched(stream, "fwd_wave");
   return (int)hipGetLastError();
@@ -723,7 +872,7 @@ int launch_zero(const FwdParams& p, void* stream) {
 // head_dim 256 runs tda_wide.hip (fp32) or fwd_blk256 after its norms kernel (bf16); a single query
 // tile the split-key decode kernels (tda_fwd_decode.hip), or in fp32 a wave per head where that is
 // faster (one_wave_heads); otherwise bf16 runs the screen + sparse A.V kernels (tda_fwd_sparse.hip) and
-// fp32 the int8 screen, fwd_cand_f32 and fwd_wave when normalised, fwd_split_f32 when not.  The
+// fp32 the int8 screen, fwd_cand_f32 and fwd_wave when normalised, fwd_split_f32 or fwd_blk_f32 when not.  The
 // screens, and the bf16 block tile pass without normalisation, clear the call's zero range; the
 // other paths launch zero_range.
 int launch_fwd(const FwdParams& p, const KernelKey& k, void* stream) {

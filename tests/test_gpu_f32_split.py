@@ -1,11 +1,13 @@
 """fp32 without normalisation: the split passes, one resident tile per workgroup, its streamed tiles
-dealt to four, two or one waves (f32_split in tda_common.hpp: below 2048 resident tiles four; from
-there two, and one for rows of at most 16 tiles or from 4096 tiles at d = 128), against the formula in
+dealt to four, two or one waves, and the block passes, four resident tiles per workgroup (f32_split in
+tda_common.hpp: by the resident tiles against the 1024 or 2048 waves the GPU holds, and the streamed tiles), against the formula in
 64 bits, every head and the gradients of beta and lambda.  Sizes on both sides of each line, fewer streamed tiles than waves, ragged last tiles, a key
 cache longer than the queries, and rows past one bitmask round (2048 key tiles).  1e-4 normwise: fp32
 products and sums of at most 65600 terms of random signs (2^-24 sqrt(65600) = 1.5e-5), the power's
 factor two, and the cancellation in score - tau; the scalars 1e-6 of the sum of their rows' contributions
-(sums of both signs, over the tiles in fp64)."""
+(sums of both signs, over the tiles in fp64).
+Powers above 1: the derivative of p = 1 steps at the threshold, where a score within rounding of it moves a
+whole term."""
 import pytest
 import torch
 
@@ -20,13 +22,20 @@ pytestmark = pytest.mark.gpu
     (1, 2, 33, 33, 64, 1, 2.0),      # two tiles: two of the four waves idle
     (1, 3, 161, 161, 128, 2, 1.5),   # six tiles, ragged
     (2, 2, 40, 700, 64, 2, 2.0),     # two query tiles on a longer key cache
-    (16, 32, 128, 128, 64, 1, 2.0),  # 2048 tiles, short rows: one wave
-    (8, 15, 545, 545, 64, 1, 2.0),   # 2160 tiles of 18: two waves
-    (8, 31, 545, 545, 128, 1, 2.0),  # 4464 tiles of 18 at d = 128: one wave
+    (16, 32, 128, 128, 64, 1, 2.0),  # 2048 tiles: two waves
+    (8, 15, 545, 545, 64, 1, 2.0),   # 2160 tiles of 18: one wave
+    (8, 31, 545, 545, 128, 1, 2.0),  # 4464 tiles of 18 at d = 128: blocks of four, the last of two
     (16, 32, 128, 128, 64, 2, 2.0),  # two branches, one wave
-    (8, 15, 545, 545, 64, 2, 2.0),   # two branches, two waves
-    (8, 15, 545, 545, 128, 1, 1.5),  # d = 128: two waves
-    (8, 15, 545, 545, 128, 2, 2.0),  # d = 128: two waves, one in the query-major pass (4320 tiles)
+    (8, 15, 545, 545, 64, 2, 2.0),   # two branches, one wave
+    (8, 15, 545, 545, 128, 1, 1.5),  # d = 128: one wave
+    (8, 15, 545, 545, 128, 2, 2.0),  # d = 128: one wave, blocks in the query-major pass (4320 tiles)
+    (4, 10, 545, 545, 64, 2, 2.0),   # 720 tiles of 18: two waves
+    (4, 10, 545, 545, 128, 1, 1.5),  # d = 128: two waves
+    (4, 10, 545, 545, 128, 2, 2.0),  # two waves, one in the query-major pass (1440 tiles)
+    (8, 41, 545, 545, 64, 1, 2.0),   # 5904 tiles of 18: blocks
+    (8, 21, 449, 545, 64, 2, 1.5),   # two branches, queries past the first keys: blocks, one wave in the query-major pass
+    (8, 21, 545, 545, 64, 2, 2.0),   # two branches: blocks everywhere
+    (8, 21, 500, 640, 128, 2, 2.0),  # d = 128: blocks
 ])
 def test_against_the_formula(b, h, nq, nk, d, br, p):
     g = torch.Generator("cuda").manual_seed(nq + d)
