@@ -622,13 +622,23 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
   }
 
   if (queue) {
+    // up to 64 blocks at a time, one addition to the counter for all of them (additions to one
+    // counter come 11 ns apart: 24576 blocks of 8192 heads 281 us)
     const int nb = BR * ((P.nqt + kBwdBlk - 1) / kBwdBlk);
-    for (int j = kt; j < nb; j += P.nkt) {
-      if (j != kt) qcount = query_block_count<BR>(P, counts, bh, j);
-      if (wave_ballot(qcount > (uint32_t)kPairCap) != 0ull && l == 0) {
-        const int64_t nkb = (int64_t)BH * ((P.nkt + kBwdBlk - 1) / kBwdBlk);
-        P.dkvq[kTileqHead + 2 * nkb + atomicAdd(P.dkvq + 1, 1u)] = (uint32_t)(bh * nb + j);
+    for (int j0 = kt; j0 < nb; j0 += 64 * P.nkt) {
+      uint64_t hit = 0ull;
+      for (int it = 0; it < 64 && j0 + it * P.nkt < nb; ++it) {
+        const int j = j0 + it * P.nkt;
+        if (j != kt) qcount = query_block_count<BR>(P, counts, bh, j);
+        if (wave_ballot(qcount > (uint32_t)kPairCap) != 0ull) hit |= 1ull << it;
       }
+      if (hit == 0ull) continue;
+      uint32_t at = 0u;
+      if (l == 0) at = atomicAdd(P.dkvq + 1, (uint32_t)__builtin_popcountll(hit));
+      at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+      const int64_t nkb = (int64_t)BH * ((P.nkt + kBwdBlk - 1) / kBwdBlk);
+      if ((hit >> l) & 1ull)
+        P.dkvq[kTileqHead + 2 * nkb + at + (uint32_t)__builtin_popcountll(hit & ((1ull << l) - 1ull))] = (uint32_t)(bh * nb + j0 + l * P.nkt);
     }
   }
 
@@ -881,8 +891,8 @@ __global__ void __launch_bounds__(64) bwd_dkv_pairs(BwdParams P) {
 // key-major pass (bwd_dkv_wide) combines both branches' weights in fp32, rounded once for dv.
 template <int D>
 constexpr int kSplit = D > 128 ? 2 : 1;
-template <int D>
-constexpr int kQryThreads = 64 * kBwdBlk * kSplit<D>;
+template <int D, int W>
+constexpr int kQryThreads = 64 * W * kSplit<D>;
 
 // A wave's 16 values through LDS: give writes them, take (after a barrier) reads some wave's.
 __device__ __forceinline__ void give16(f32x4 (*x)[64], const f32x16& v) {
@@ -963,7 +973,7 @@ struct BlkRows {
   }
 };
 
-// Query-major: kBwdBlk query tiles of one (branch, head), streaming K, V and the key norms.  The
+// Query-major: W query tiles (kBwdBlk, or fewer where no head has more) of one (branch, head), streaming K, V and the key norms.  The
 // block takes its tiles whose lists did not fit (or all, without lists).
 //
 // The block functions' LDS, arrays of the kernel.
@@ -984,9 +994,9 @@ struct BlkLds {
   __shared__ float lds_dots[W][kSplit<D> == 2 ? 64 : 1];                                      \
   const BlkLds<D, W> L{lds_ring, lds_vals, reinterpret_cast<bf16(*)[32 * D]>(&lds_rows[0][0]),             \
                        reinterpret_cast<f32x4(*)[4][64]>(&lds_xch[0][0]), reinterpret_cast<float(*)[2][32]>(&lds_dots[0][0])}
-template <int D, int BR, int PK, bool NORM>
-__device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBwdBlk>& L, int jb, int br, int bh) {
-  constexpr int W = kBwdBlk, SP = kSplit<D>, NT = D / 16, ND = D / 32 / SP;
+template <int D, int BR, int PK, bool NORM, int W>
+__device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, W>& L, int jb, int br, int bh) {
+  constexpr int SP = kSplit<D>, NT = D / 16, ND = D / 32 / SP;
   constexpr int STAGE = 2 * 32 * D;  // K tile, V tile
   bf16* ring = L.ring;
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
@@ -1081,7 +1091,7 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBw
     own_out = sown;
     return kt;
   };
-  constexpr int AHEAD = D <= 64 ? 2 : 1;  // tiles in flight past the one being worked on
+  constexpr int AHEAD = D <= 64 && W > 2 ? 2 : 1;  // tiles in flight past the one being worked on
   struct Pre {  // a tile's share in flight: its rows and norms, index and the own row's word
     BlkRows<D, W * SP> kr, vr;
     f32x4 nr;
@@ -1250,12 +1260,12 @@ __device__ __forceinline__ void dq_block(const BwdParams& P, const BlkLds<D, kBw
   }
 }
 
-// Key-major: kBwdBlk consecutive key tiles of one head (aligned: one bitmask word holds their
-// bits), streaming per branch the query tiles' Q and dO rows, query norms and tau values.  needm:
+// Key-major: W consecutive key tiles (kBwdBlk, or fewer where no head has more) of one head (aligned: one
+// bitmask word holds their bits), streaming per branch the query tiles' Q and dO rows, query norms and tau values.  needm:
 // the block's key tiles to take (at least one).
-template <int D, int BR, int PK, bool NORM>
-__device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kBwdBlk>& L, int jb, int bh, uint32_t needm) {
-  constexpr int W = kBwdBlk, NT = D / 16, ND = D / 32;
+template <int D, int BR, int PK, bool NORM, int W>
+__device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, W>& L, int jb, int bh, uint32_t needm) {
+  constexpr int NT = D / 16, ND = D / 32;
   constexpr int STAGE = 2 * 32 * D;  // Q tile, dO tile
   bf16* ring = L.ring;
   const int l = lane_id(), n32 = l & 31, g = l >> 5;
@@ -1304,11 +1314,11 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kB
     const float ds_scale = (PK == 2 ? 2.f : 1.f) * (br == 0 ? 1.f : -lam);
     // the wave's key rows (swizzled tile; rows past Nk read as zeros), read as score operands
     {
-      BlkRows<D, kBwdBlk> kr4[kBwdBlk];
+      BlkRows<D, W> kr4[W];
 #pragma unroll
-      for (int s4 = 0; s4 < kBwdBlk; ++s4) kr4[s4].load(base(kslot), P.s[kslot][2], 32 * min(kt, nkt - 1), Nk, s4);
+      for (int s4 = 0; s4 < W; ++s4) kr4[s4].load(base(kslot), P.s[kslot][2], 32 * min(kt, nkt - 1), Nk, s4);
 #pragma unroll
-      for (int s4 = 0; s4 < kBwdBlk; ++s4) kr4[s4].store(kti, s4);
+      for (int s4 = 0; s4 < W; ++s4) kr4[s4].store(kti, s4);
     }
     f32x16 AK[ND];
 #pragma unroll
@@ -1338,7 +1348,7 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kB
       own_out = (om >> q) & 1ull;
       return q0c + q;
     };
-    constexpr int AHEAD = D <= 64 ? 2 : 1;  // tiles in flight past the one being worked on
+    constexpr int AHEAD = D <= 64 && W > 2 ? 2 : 1;  // tiles in flight past the one being worked on
     struct Pre {  // a tile's share in flight: its rows, norms and thresholds, index, and whether it is the wave's
       BlkRows<D, W> qr, dr;
       float vrq, vtq;
@@ -1482,10 +1492,10 @@ __device__ __forceinline__ void dkv_block(const BwdParams& P, const BlkLds<D, kB
 
 // One workgroup per block of query tiles: longest blocks (last query tiles) of every (head,
 // branch) first, the branches adjacent.
-template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(kQryThreads<D>) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_blk(BwdParams P) {
-  TDA_BLK_LDS(D, kBwdBlk, false);
-  const int BH = P.B * P.H, nqb = (P.nqt + kBwdBlk - 1) / kBwdBlk;
+template <int D, int BR, int PK, bool NORM, int W>
+__global__ void __launch_bounds__((kQryThreads<D, W>)) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_blk(BwdParams P) {
+  TDA_BLK_LDS(D, W, false);
+  const int BH = P.B * P.H, nqb = (P.nqt + W - 1) / W;
   const int bid = blockIdx.x, jb = nqb - 1 - bid / (BR * BH), rem = bid % (BR * BH);
   dq_block<D, BR, PK, NORM>(P, L, jb, BR == 2 ? rem & 1 : 0, BR == 2 ? rem >> 1 : rem);
 }
@@ -1502,9 +1512,8 @@ constexpr int dkv_waves() {
 // One workgroup per block of key tiles: longest blocks (first key tiles) of every head first.  A
 // key tile takes this pass when a list of its column did not fit (the test bwd_dkv_pairs leaves
 // it by; it writes nothing for such a key tile), or always without lists.
-template <int D, int BR, int PK, bool NORM>
-__global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, NORM>()))) bwd_dkv_blk(BwdParams P) {
-  constexpr int W = kBwdBlk;
+template <int D, int BR, int PK, bool NORM, int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, NORM>()))) bwd_dkv_blk(BwdParams P) {
   TDA_BLK_LDS(D, W, true);
   __shared__ uint32_t needs[W];
   const int l = lane_id();
@@ -1781,19 +1790,26 @@ __global__ void __launch_bounds__(128 * BR * kWideKeys) __attribute__((amdgpu_wa
 // after one load (4.6 us); at a threshold scale of 0.5 nearly every block is queued
 // (TDA (2, 16, 1500, 64): 162 us, 2632 us with one wave per query or key tile fetching
 // its own rows).
-template <int D, int BR, int PK>
-__global__ void __launch_bounds__(64 * kBwdBlk) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, true>()))) bwd_tiles(BwdParams P) {
-  TDA_BLK_LDS(D, kBwdBlk, true);
+// W = 1 or 2 where no head has more query or key tiles: the other waves of four would have no tile, and
+// hold the registers of a block that has.  Its blocks are of one length and are taken in turn: the
+// tickets of one counter come 11 ns apart.  With the pair passes, 8192 heads of 32 rows at a threshold
+// scale of 0.4: TRA d = 64 280 us, d = 128 433 (with four waves 403, 690); TDA 404 and 691 (732, 1281).
+template <int D, int BR, int PK, int W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(dkv_waves<D, BR, true>()))) bwd_tiles(BwdParams P) {
+  TDA_BLK_LDS(D, W, true);
   __shared__ uint32_t ticket;
   const uint32_t nk = P.dkvq[0], total = nk + P.dkvq[1];
   if (total == 0u) return;
   const int BH = P.B * P.H, nqb = (P.nqt + kBwdBlk - 1) / kBwdBlk, nkb = (P.nkt + kBwdBlk - 1) / kBwdBlk;
   const uint32_t* masks = P.dkvq + kTileqHead;
-  while (true) {
+  for (uint32_t turn = blockIdx.x;; turn += gridDim.x) {
+    uint32_t t = turn;
     __syncthreads();  // every wave is done with the previous block's LDS and ticket
-    if (threadIdx.x == 0) ticket = atomicAdd(P.dkvq + 2, 1u);
-    __syncthreads();
-    const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)ticket);
+    if constexpr (W == kBwdBlk) {
+      if (threadIdx.x == 0) ticket = atomicAdd(P.dkvq + 2, 1u);
+      __syncthreads();
+      t = (uint32_t)__builtin_amdgcn_readfirstlane((int)ticket);
+    }
     if (t >= total) return;
     if (t < nk) {
       const uint32_t blk = (uint32_t)__builtin_amdgcn_readfirstlane((int)masks[(int64_t)BH * nkb + t]);
@@ -1827,26 +1843,45 @@ static int launch_t(const BwdParams& p, void* stream) {
     }
   }
   const int BH = q.B * q.H;
-  const unsigned qblocks = (unsigned)(BR * BH * ((q.nqt + kBwdBlk - 1) / kBwdBlk));
+  const unsigned qblocks = (unsigned)(BR * BH * ((q.nqt + kBwdBlk - 1) / kBwdBlk));  // (one block of one tile too)
   constexpr int KB = D <= 128 ? kBwdBlk : kWideKeys;
   const unsigned kblocks = (unsigned)(BH * ((q.nkt + KB - 1) / KB));
   bool queued = false;
   if constexpr (NORM && D <= 128) {
     if (q.pairs && q.dkvq) {
       // as many workgroups as the GPU's 256 CUs hold at dkv_waves waves per SIMD
-      const unsigned most = 256u * dkv_waves<D, BR, true>(), blocks = qblocks + kblocks;
-      hipLaunchKernelGGL((bwd_tiles<D, BR, PK>), dim3(blocks < most ? blocks : most), dim3(64 * kBwdBlk), 0, s, q);
+      const int tiles = q.nqt > q.nkt ? q.nqt : q.nkt, W = tiles == 1 ? 1 : tiles == 2 ? 2 : kBwdBlk;
+      // (of W = 1 as many as its 21 and 41 KB of LDS let in: more would wait for the first ones' whole share)
+      const unsigned most = 256u * (W == 1 ? (D <= 64 ? 7 : 3) : dkv_waves<D, BR, true>() * (kBwdBlk / W)), blocks = qblocks + kblocks;
+      const dim3 grid(blocks < most ? blocks : most);
+      if (W == 1)
+        hipLaunchKernelGGL((bwd_tiles<D, BR, PK, 1>), grid, dim3(64), 0, s, q);
+      else if (W == 2)
+        hipLaunchKernelGGL((bwd_tiles<D, BR, PK, 2>), grid, dim3(128), 0, s, q);
+      else
+        hipLaunchKernelGGL((bwd_tiles<D, BR, PK, kBwdBlk>), grid, dim3(64 * kBwdBlk), 0, s, q);
       launched(s, "bwd_tiles");
       queued = true;
     }
   }
   if (!queued) {
-    hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM>), dim3(qblocks), dim3(kQryThreads<D>), 0, s, q);
+    bool one = false;  // a head's only tile: a block of one, as in bwd_tiles
+    if constexpr (!NORM && D <= 64) {  // (d = 128: 189 us in blocks of four, 228 so, 8192 heads of 16 rows)
+      one = q.nqt == 1;
+      if (one) hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM, 1>), dim3(qblocks), dim3(kQryThreads<D, 1>), 0, s, q);
+    }
+    if (!one) hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM, kBwdBlk>), dim3(qblocks), dim3(kQryThreads<D, kBwdBlk>), 0, s, q);
     launched(s, "bwd_dq_blk");
-    if constexpr (D <= 128)
-      hipLaunchKernelGGL((bwd_dkv_blk<D, BR, PK, NORM>), dim3(kblocks), dim3(64 * kBwdBlk), 0, s, q);
-    else
+    one = false;
+    if constexpr (!NORM && D <= 128) {
+      one = q.nkt == 1;
+      if (one) hipLaunchKernelGGL((bwd_dkv_blk<D, BR, PK, NORM, 1>), dim3(kblocks), dim3(64), 0, s, q);
+    }
+    if constexpr (D <= 128) {
+      if (!one) hipLaunchKernelGGL((bwd_dkv_blk<D, BR, PK, NORM, kBwdBlk>), dim3(kblocks), dim3(64 * kBwdBlk), 0, s, q);
+    } else {
       hipLaunchKernelGGL((bwd_dkv_wide<BR, PK, NORM>), dim3(kblocks), dim3(128 * BR * kWideKeys), 0, s, q);
+    }
     launched(s, "bwd_dkv_blk");
   }
   const int e = (int)hipGetLastError();

@@ -1,0 +1,45 @@
+"""bf16 training steps over many heads of one or two tiles: the block passes that take fewer tiles per
+workgroup there (bwd_tiles with a queue longer than its grid, bwd_dq_blk, bwd_dkv_blk), against
+the formula in 64 bits, every head.  2e-2: bf16 rows, weights and gradients, as in the parity tests."""
+import pytest
+import torch
+
+import tda_amd
+from oracle.formula import rel_err
+from tests.helpers import TOL, grads_on_gpu, rel_norm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("b,h,nq,nk,d,br,norm,p,beta", [
+    (16, 64, 32, 32, 64, 2, True, 2.0, 0.3),    # one tile: up to 3072 queued blocks, 1792 workgroups
+    (16, 64, 17, 17, 64, 1, True, 1.5, 0.3),
+    (8, 64, 31, 31, 128, 2, True, 2.0, 0.3),    # 768 workgroups
+    (8, 64, 32, 32, 128, 1, True, 1.5, 0.3),
+    (16, 64, 33, 33, 64, 2, True, 2.0, 0.3),    # two tiles: 1024 workgroups
+    (8, 64, 64, 64, 128, 2, True, 1.5, 0.3),    # 512
+    (8, 64, 20, 50, 64, 2, True, 2.0, 0.3),     # one query tile, two key tiles
+    (8, 64, 65, 65, 64, 2, True, 2.0, 0.3),     # three: blocks of four
+    (4, 64, 32, 32, 64, 2, False, 2.0, 0.5), (4, 64, 9, 9, 128, 1, False, 1.5, 0.5),
+    (4, 64, 32, 70, 64, 1, False, 2.0, 0.5),    # one query tile, three key tiles
+    (4, 64, 32, 70, 128, 2, False, 2.0, 0.5),
+])
+def test_against_the_formula(b, h, nq, nk, d, br, norm, p, beta):
+    g = torch.Generator("cpu").manual_seed(61)
+    rows = [torch.randn((b, h, n, d), generator=g).bfloat16().cuda() for n in ([nq, nq, nk, nk, nk] if br == 2 else [nq, nk, nk])]
+    do = torch.randn((b, h, nq, d), generator=g).bfloat16().cuda()
+    leaves = [x.requires_grad_(True) for x in rows]
+    bt, lt = (torch.tensor(x, device="cuda", requires_grad=True) for x in (beta, 0.4))
+    if br == 2:
+        out = tda_amd.differential_threshold_rela_triton(*leaves, bt, lt, relu_power=p, normalize=norm)
+    else:
+        out = tda_amd.threshold_rela_triton(*leaves, bt, relu_power=p, normalize=norm)
+    out.backward(do)
+    ref = grads_on_gpu(leaves, do, beta, 0.4, p, norm, br, q_offset=nk - nq)
+    tol = TOL[torch.bfloat16]
+    assert rel_err(out, ref["out"]) < tol and rel_norm(out, ref["out"]) < tol
+    for x, name in zip(leaves, ["dq1", "dq2", "dk1", "dk2", "dv"] if br == 2 else ["dq1", "dk1", "dv"]):
+        assert rel_err(x.grad, ref[name]) < tol and rel_norm(x.grad, ref[name]) < tol, name
+    assert abs(bt.grad.item() - ref["dbeta"]) <= tol * ref["beta_scale"]
+    if br == 2:
+        assert abs(lt.grad.item() - ref["dlambda"]) <= tol * ref["lambda_scale"]
