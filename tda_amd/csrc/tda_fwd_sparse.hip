@@ -1180,22 +1180,25 @@ fwd_pv_blk(FwdParams P) {
 // them.  They fit 256 registers, two waves per SIMD, and skip the A V products of a tile without a
 // weight (at beta = 1 most are).  B2 H8 N1000 at beta = 1: 62 us with two branches (133 with one wave
 // per tile: its 512 registers put the accumulators where a branch around them copies them all), 47 with
-// one (one wave per tile: 40 to 105, as the compiler happens to keep or copy them).  Without normalisation a single branch has weights nearly everywhere: one wave
-// per tile with no branch, a tile without a weight reading zeros for V: 53 us.
+// one (one wave per tile: 40 to 105, as the compiler happens to keep or copy them).  Without normalisation a single
+// branch has weights nearly everywhere: one wave per tile with no branch, a tile without a weight reading zeros for V: 53 us.
 template <int BR, bool NORM>
 constexpr int kWideFwdWaves = BR == 2 || NORM ? 2 : 1;
 
-template <int BR, int PK, bool NORM>
-__global__ void __launch_bounds__((64 * kBlkTiles * kWideFwdWaves<BR, NORM>))
+// W = 1 where every head has one query and one key tile: a ring of one stage, so that a CU holds more
+// heads at a time (of four waves, or pairs, three would have no tile).  Forward of 8192 heads of 32 rows: two branches 236 us, one 130
+// (W = 4: 467, 239), without normalisation 153 and 96 (411, 256).
+template <int BR, int PK, bool NORM, int W>
+__global__ void __launch_bounds__((64 * W * kWideFwdWaves<BR, NORM>))
 __attribute__((amdgpu_waves_per_eu((kWideFwdWaves<BR, NORM>)))) fwd_blk256(FwdParams P) {
-  constexpr int D = 256, W = kBlkTiles, NW = kWideFwdWaves<BR, NORM>, NT = D / 16, ND = D / 32 / NW;
+  constexpr int D = 256, RING = W == 1 ? 1 : 2, NW = kWideFwdWaves<BR, NORM>, NT = D / 16, ND = D / 32 / NW;
   constexpr int VS = D + 32, KS = D + 8, CPR = D / 8, RPI = 64 / CPR, LPW = 32 / RPI / (NW * W);
   constexpr int STAGE = 32 * (BR * KS + VS);
   constexpr bool SKIP = NW == 2;
   constexpr int OS = D / NW + 8;  // row stride of a wave's output slice
-  static_assert(2 * STAGE >= NW * W * 32 * OS, "the ring holds the waves' output rows");
-  __shared__ __attribute__((aligned(16))) bf16 ring[2 * STAGE];
-  __shared__ __attribute__((aligned(16))) float nring[2][BR][32];
+  static_assert(RING * STAGE >= NW * W * 32 * OS, "the ring holds the waves' output rows");
+  __shared__ __attribute__((aligned(16))) bf16 ring[RING * STAGE];
+  __shared__ __attribute__((aligned(16))) float nring[RING][BR][32];
   __shared__ __attribute__((aligned(16))) f32x4 xch[BR == 2 ? 2 * W : 1][4][64];  // two branches: the waves' weights
   __shared__ uint32_t xany[2 * W];                                             // and whether there are any
   __shared__ __attribute__((aligned(16))) bf16 zeros[SKIP ? 8 : 32 * VS];  // a value tile of zeros
@@ -1212,8 +1215,8 @@ __attribute__((amdgpu_waves_per_eu((kWideFwdWaves<BR, NORM>)))) fwd_blk256(FwdPa
   const int iq = 32 * qt + n32, pq = qoff + iq;
   const bool valid = act && iq < Nq;
   const bool rowpad = 32 * qt + 31 >= Nq;  // the query tile has rows past Nq (uniform)
-  const int klast_b = kt_last(min(W * jb + W - 1, nqt - 1), qoff, P.nkt);  // the block's last key tile
-  const int ktl = act ? kt_last(qt, qoff, P.nkt) : -1;                     // the wave's
+  const int klast_b = W == 1 ? 0 : kt_last(min(W * jb + W - 1, nqt - 1), qoff, P.nkt);  // the block's last key tile
+  const int ktl = W == 1 ? 0 : act ? kt_last(qt, qoff, P.nkt) : -1;                     // the wave's
   const float tau = *P.beta * tau_coeff(pq, P.inv_d);
   const float pw = P.p;
   float lam = 0.f;
@@ -1273,7 +1276,8 @@ __attribute__((amdgpu_waves_per_eu((kWideFwdWaves<BR, NORM>)))) fwd_blk256(FwdPa
   }
 #pragma unroll 1
   for (int kt = 0; kt <= klast_b; ++kt) {
-    bf16* st = ring + (kt & 1) * STAGE;
+    const int slot = RING == 2 ? kt & 1 : 0;  // (one stage: one key tile)
+    bf16* st = ring + slot * STAGE;
     bf16* vst = st + BR * 32 * KS;
 #pragma unroll
     for (int i = 0; i < LPW; ++i) {
@@ -1283,9 +1287,9 @@ __attribute__((amdgpu_waves_per_eu((kWideFwdWaves<BR, NORM>)))) fwd_blk256(FwdPa
     }
     if (NORM && wid == 0 && l < 8) {
 #pragma unroll
-      for (int x = 0; x < BR; ++x) *reinterpret_cast<f32x4*>(nring[kt & 1][x] + 4 * l) = nr[x];
+      for (int x = 0; x < BR; ++x) *reinterpret_cast<f32x4*>(nring[slot][x] + 4 * l) = nr[x];
     }
-    issue(min(kt + 1, klast_b));  // in flight during this tile's work
+    if (RING == 2) issue(min(kt + 1, klast_b));  // in flight during this tile's work
     lds_barrier();
     f32x16 C = f32x16{};
     bool any = false;
@@ -1298,7 +1302,7 @@ __attribute__((amdgpu_waves_per_eu((kWideFwdWaves<BR, NORM>)))) fwd_blk256(FwdPa
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         f32x4 rk = {1.f, 1.f, 1.f, 1.f};
-        if constexpr (NORM) rk = *reinterpret_cast<const f32x4*>(nring[kt & 1][br] + 8 * u + 4 * g);
+        if constexpr (NORM) rk = *reinterpret_cast<const f32x4*>(nring[slot][br] + 8 * u + 4 * g);
 #pragma unroll
         for (int e = 0; e < 4; ++e) X[4 * u + e] = __builtin_fmaf(NORM ? S[4 * u + e] * rk[e] : S[4 * u + e], rq, -tau);
       }
@@ -1710,10 +1714,15 @@ int launch_fwd_sparse(const FwdParams& p, const KernelKey& k, void* stream) {
 template <int BR, int PK>
 static int launch_blk256_t(const FwdParams& p, bool norm, hipStream_t s) {
   const unsigned blocks = (unsigned)(p.B * p.H * ((p.nqt + kBlkTiles - 1) / kBlkTiles));
-  if (norm)
-    hipLaunchKernelGGL((fwd_blk256<BR, PK, true>), dim3(blocks), dim3(64 * kBlkTiles * kWideFwdWaves<BR, true>), 0, s, p);
+  const bool one = p.nqt == 1 && p.nkt == 1;
+  if (norm && one)
+    hipLaunchKernelGGL((fwd_blk256<BR, PK, true, 1>), dim3(blocks), dim3(64 * kWideFwdWaves<BR, true>), 0, s, p);
+  else if (norm)
+    hipLaunchKernelGGL((fwd_blk256<BR, PK, true, kBlkTiles>), dim3(blocks), dim3(64 * kBlkTiles * kWideFwdWaves<BR, true>), 0, s, p);
+  else if (one)
+    hipLaunchKernelGGL((fwd_blk256<BR, PK, false, 1>), dim3(blocks), dim3(64 * kWideFwdWaves<BR, false>), 0, s, p);
   else
-    hipLaunchKernelGGL((fwd_blk256<BR, PK, false>), dim3(blocks), dim3(64 * kBlkTiles * kWideFwdWaves<BR, false>), 0, s, p);
+    hipLaunchKernelGGL((fwd_blk256<BR, PK, false, kBlkTiles>), dim3(blocks), dim3(64 * kBlkTiles * kWideFwdWaves<BR, false>), 0, s, p);
   launched(s, "wide_fwd");
   return (int)hipGetLastError();
 }

@@ -1,6 +1,7 @@
 """bf16 training steps over many heads of one or two tiles: the block passes that take fewer tiles per
-workgroup there (bwd_tiles with a queue longer than its grid, bwd_dq_blk, bwd_dkv_blk), against
-the formula in 64 bits, every head.  2e-2: bf16 rows, weights and gradients, as in the parity tests."""
+workgroup there (bwd_tiles with a queue longer than its grid, bwd_dq_blk, bwd_dkv_blk, the head_dim 256
+forward), against the formula in 64 bits, every head.  2e-2: bf16 rows, weights and gradients, as in
+the parity tests."""
 import pytest
 import torch
 
@@ -23,6 +24,9 @@ pytestmark = pytest.mark.gpu
     (4, 64, 32, 32, 64, 2, False, 2.0, 0.5), (4, 64, 9, 9, 128, 1, False, 1.5, 0.5),
     (4, 64, 32, 70, 64, 1, False, 2.0, 0.5),    # one query tile, three key tiles
     (4, 64, 32, 70, 128, 2, False, 2.0, 0.5),
+    (4, 32, 32, 32, 256, 2, True, 2.0, 0.3), (4, 32, 1, 1, 256, 2, False, 2.0, 0.0),
+    (4, 32, 17, 17, 256, 1, True, 1.5, 0.3), (4, 32, 31, 31, 256, 1, False, 2.0, 0.3),
+    (4, 32, 20, 33, 256, 1, False, 2.0, 0.3),   # one query tile, two key tiles
 ])
 def test_against_the_formula(b, h, nq, nk, d, br, norm, p, beta):
     g = torch.Generator("cpu").manual_seed(61)
