@@ -1496,7 +1496,8 @@ template <int D, int BR, int PK, bool NORM, int W>
 __global__ void __launch_bounds__((kQryThreads<D, W>)) __attribute__((amdgpu_waves_per_eu(2))) bwd_dq_blk(BwdParams P) {
   TDA_BLK_LDS(D, W, false);
   const int BH = P.B * P.H, nqb = (P.nqt + W - 1) / W;
-  const int bid = blockIdx.x, jb = nqb - 1 - bid / (BR * BH), rem = bid % (BR * BH);
+  if (D > 128 && blockIdx.y && grid_bid<kQryThreads<D, W>>() >= (uint32_t)(BR * BH) * (uint32_t)nqb) return;
+  const int bid = D > 128 ? (int)grid_bid<kQryThreads<D, W>>() : blockIdx.x, jb = nqb - 1 - bid / (BR * BH), rem = bid % (BR * BH);
   dq_block<D, BR, PK, NORM>(P, L, jb, BR == 2 ? rem & 1 : 0, BR == 2 ? rem >> 1 : rem);
 }
 
@@ -1604,7 +1605,8 @@ __global__ void __launch_bounds__(128 * BR * kWideKeys) __attribute__((amdgpu_wa
   const int wv = wid / NW, sub = wid % NW, br = sub >> 1, hh = sub & 1;
   const int BH = P.B * P.H, nqt = P.nqt, nkt = P.nkt, Nq = P.Nq, Nk = P.Nk, qoff = P.qoff;
   // longest blocks (first key tiles) of every head first
-  const int bid = blockIdx.x, kt0 = W * (bid / BH), bh = bid % BH, kt = kt0 + wv;
+  if (blockIdx.y && grid_bid<64 * W * NW>() >= (uint32_t)BH * (uint32_t)((nkt + W - 1) / W)) return;
+  const int bid = (int)grid_bid<64 * W * NW>(), kt0 = W * (bid / BH), bh = bid % BH, kt = kt0 + wv;
   const int b = bh / P.H, h = bh % P.H;
   const int j = 32 * kt + n32, jc = min(j, Nk - 1);
   const bool kvalid = j < Nk;
@@ -1870,7 +1872,8 @@ static int launch_t(const BwdParams& p, void* stream) {
       one = q.nqt == 1;
       if (one) hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM, 1>), dim3(qblocks), dim3(kQryThreads<D, 1>), 0, s, q);
     }
-    if (!one) hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM, kBwdBlk>), dim3(qblocks), dim3(kQryThreads<D, kBwdBlk>), 0, s, q);
+    const dim3 qgrid = D > 128 ? grid_of<kQryThreads<D, kBwdBlk>>(qblocks) : dim3(qblocks);
+    if (!one) hipLaunchKernelGGL((bwd_dq_blk<D, BR, PK, NORM, kBwdBlk>), qgrid, dim3(kQryThreads<D, kBwdBlk>), 0, s, q);
     launched(s, "bwd_dq_blk");
     one = false;
     if constexpr (!NORM && D <= 128) {
@@ -1880,7 +1883,7 @@ static int launch_t(const BwdParams& p, void* stream) {
     if constexpr (D <= 128) {
       if (!one) hipLaunchKernelGGL((bwd_dkv_blk<D, BR, PK, NORM, kBwdBlk>), dim3(kblocks), dim3(64 * kBwdBlk), 0, s, q);
     } else {
-      hipLaunchKernelGGL((bwd_dkv_wide<BR, PK, NORM>), dim3(kblocks), dim3(128 * BR * kWideKeys), 0, s, q);
+      hipLaunchKernelGGL((bwd_dkv_wide<BR, PK, NORM>), grid_of<128 * BR * kWideKeys>(kblocks), dim3(128 * BR * kWideKeys), 0, s, q);
     }
     launched(s, "bwd_dkv_blk");
   }

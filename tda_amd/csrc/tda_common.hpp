@@ -216,6 +216,17 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+// A launch holds at most 2^32 - 1 work-items along x: grid_of lays more workgroups out over y too, the
+// last row partly past the end (grid_bid >= blocks: such a workgroup returns at once).
+template <int THREADS>
+inline dim3 grid_of(int64_t blocks) {
+  constexpr int64_t most = 0xffffffffll / THREADS;
+  return blocks <= most ? dim3((unsigned)blocks) : dim3((unsigned)most, (unsigned)((blocks + most - 1) / most));
+}
+template <int THREADS>
+__device__ __forceinline__ uint32_t grid_bid() {
+  return blockIdx.y * (uint32_t)(0xffffffffll / THREADS) + blockIdx.x;
+}
 // Wave-wide OR (every lane ends with it), by the same steps as wave_sum.  Call with every lane active.
 __device__ __forceinline__ uint32_t wave_or(uint32_t v) {
   v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, false);

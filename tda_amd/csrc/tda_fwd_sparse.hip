@@ -1208,7 +1208,8 @@ __attribute__((amdgpu_waves_per_eu((kWideFwdWaves<BR, NORM>)))) fwd_blk256(FwdPa
   const int wv = wid / NW, part = wid % NW, br = BR == 2 ? part : 0;  // query tile, share of the columns, branch
   const int BH = P.B * P.H, Nq = P.Nq, Nk = P.Nk, nqt = P.nqt, qoff = P.qoff;
   int bh, jb;
-  blk_order(blockIdx.x, BH, (nqt + W - 1) / W, bh, jb);
+  if (blockIdx.y && grid_bid<64 * W * NW>() >= (uint32_t)BH * (uint32_t)((nqt + W - 1) / W)) return;
+  blk_order((int)grid_bid<64 * W * NW>(), BH, (nqt + W - 1) / W, bh, jb);
   const int b = bh / P.H, h = bh % P.H;
   const int qt = W * jb + wv, qtc = min(qt, nqt - 1);
   const bool act = qt < nqt;  // wave-uniform: waves past the last query tile only load
@@ -1716,13 +1717,13 @@ static int launch_blk256_t(const FwdParams& p, bool norm, hipStream_t s) {
   const unsigned blocks = (unsigned)(p.B * p.H * ((p.nqt + kBlkTiles - 1) / kBlkTiles));
   const bool one = p.nqt == 1 && p.nkt == 1;
   if (norm && one)
-    hipLaunchKernelGGL((fwd_blk256<BR, PK, true, 1>), dim3(blocks), dim3(64 * kWideFwdWaves<BR, true>), 0, s, p);
+    hipLaunchKernelGGL((fwd_blk256<BR, PK, true, 1>), (grid_of<64 * kWideFwdWaves<BR, true>>(blocks)), dim3(64 * kWideFwdWaves<BR, true>), 0, s, p);
   else if (norm)
-    hipLaunchKernelGGL((fwd_blk256<BR, PK, true, kBlkTiles>), dim3(blocks), dim3(64 * kBlkTiles * kWideFwdWaves<BR, true>), 0, s, p);
+    hipLaunchKernelGGL((fwd_blk256<BR, PK, true, kBlkTiles>), (grid_of<64 * kBlkTiles * kWideFwdWaves<BR, true>>(blocks)), dim3(64 * kBlkTiles * kWideFwdWaves<BR, true>), 0, s, p);
   else if (one)
-    hipLaunchKernelGGL((fwd_blk256<BR, PK, false, 1>), dim3(blocks), dim3(64 * kWideFwdWaves<BR, false>), 0, s, p);
+    hipLaunchKernelGGL((fwd_blk256<BR, PK, false, 1>), (grid_of<64 * kWideFwdWaves<BR, false>>(blocks)), dim3(64 * kWideFwdWaves<BR, false>), 0, s, p);
   else
-    hipLaunchKernelGGL((fwd_blk256<BR, PK, false, kBlkTiles>), dim3(blocks), dim3(64 * kBlkTiles * kWideFwdWaves<BR, false>), 0, s, p);
+    hipLaunchKernelGGL((fwd_blk256<BR, PK, false, kBlkTiles>), (grid_of<64 * kBlkTiles * kWideFwdWaves<BR, false>>(blocks)), dim3(64 * kBlkTiles * kWideFwdWaves<BR, false>), 0, s, p);
   launched(s, "wide_fwd");
   return (int)hipGetLastError();
 }

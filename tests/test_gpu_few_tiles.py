@@ -47,3 +47,22 @@ def test_against_the_formula(b, h, nq, nk, d, br, norm, p, beta):
     assert abs(bt.grad.item() - ref["dbeta"]) <= tol * ref["beta_scale"]
     if br == 2:
         assert abs(lt.grad.item() - ref["dlambda"]) <= tol * ref["lambda_scale"]
+
+
+def test_more_work_items_than_one_grid_dimension_holds():
+    """head_dim 256, 2^23 + 3 heads of one row: the query-major pass has 512 work-items per head, past
+    2^32 - 1.  The first heads and the last against the formula at N = 1 (the threshold is 0 there): out =
+    relu(q.k)^2 v, dq = 2 relu(q.k) (dout.v) k, in fp64; 2^-7 in the 2-norm: bf16 products' operands (dS) and
+    results, 2^-9 each."""
+    n = 2 ** 23 + 3
+    g = torch.Generator("cuda").manual_seed(67)
+    q, k, v, do = (torch.randn((1, n, 1, 256), generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(4))
+    q.requires_grad_(True), k.requires_grad_(True), v.requires_grad_(True)
+    out = tda_amd.threshold_rela_triton(q, k, v, 1.0, relu_power=2.0, normalize=False)
+    dq, dk, dv = torch.autograd.grad(out, [q, k, v], do)
+    for at in (slice(0, 64), slice(n - 64, n)):
+        qd, kd, vd, dd = (x.detach()[0, at, 0].double() for x in (q, k, v, do))
+        x = (qd * kd).sum(-1, keepdim=True).clamp(min=0)
+        dp = (dd * vd).sum(-1, keepdim=True)
+        for got, want in ((out, x * x * vd), (dq, 2 * x * dp * kd), (dk, 2 * x * dp * qd), (dv, x * x * dd)):
+            assert rel_norm(got[0, at, 0], want) < 2.0 ** -7
